@@ -10,6 +10,9 @@ through the boundary of include/fitre_*.h, on device memory that torch holds:
   curvature  computeOmegaZAndLambdaDelta + computeNaturalGradient: factors, damped inverses, natural gradient
   dense      computeGradient + gaussNewtonHessianVec of the fully connected family
 
+exact() says what they should return, from plain torch arithmetic in 64 bits on the inputs that prepare() made.  It covers
+losses, probabilities, gradients, Hessian-vector products and, where no running statistics are in it, the activation store.
+
 A ReLU at zero and two equal cells under a max pool send whole gradient entries elsewhere when a forward pass differs in
 its last bit, which says nothing about the pass.  So in "step", "hessian" and "curvature" what the backward side reads
 as z is a float64 forward pass made by torch and rounded, the same for every implementation, and the forward pass of a
@@ -31,6 +34,7 @@ from fitre_amd.harness import build_alexnet, build_lenet, build_vgg11, input_dim
 ACTS = {"none": S.CNN_ACT_NONE, "softplus": S.CNN_ACT_SOFTPLUS, "elu": S.CNN_ACT_ELU, "relu": S.CNN_ACT_RELU, "swish": S.CNN_ACT_SWISH}
 AUTOENCODER = (784, 512, 256, 64, 256, 512, 784)  # 28x28 images squeezed to 64 numbers and back
 DAMPING = 1e-3
+CIFAR10_STATISTICS = ((0.4914, 0.4822, 0.4465), (0.2470, 0.2435, 0.2616))  # means and deviations of the input pipeline
 DEVICE = "cuda:0"
 
 
@@ -194,39 +198,47 @@ def _activate(code, x):
     return F.softplus(x, threshold=700.0) if code == S.CNN_ACT_SOFTPLUS else x
 
 
-def _fill_z(st):
-    """The activation store of a training forward pass (the slabs of include/fitre_nn.h), from float64 arithmetic."""
-    m, n, w = st.model, st.n, st.weights.double()
+def _unfolded(x, c, wm):
+    """The convolution of c as a product with laid-out patches, some images at a time: [N][Cout][A][B]."""
+    some = max(1, (1 << 27) // (wm.shape[1] * c.outWidth * c.outHeight))
+    parts = []
+    for a in range(0, x.shape[0], some):
+        cols = F.unfold(x[a:a + some], c.kSize, padding=c.padding, stride=c.stride).transpose(0, 1)
+        parts.append((wm @ cols.reshape(wm.shape[1], -1)).reshape(c.outChannels, -1, c.outWidth, c.outHeight).transpose(0, 1))
+    return torch.cat(parts)
 
-    def put(at, t):
-        st.z[at:at + t.numel()] = t.reshape(-1).float()
+
+def _network(st, w, x, put=lambda at, t: None, running=None):
+    """Logits of the network in float64 for images x [N][C][A][B] and flat weights w.  put(at, t) is told every stage of the
+    activation store (the slabs of include/fitre_nn.h); running: the store whose running statistics normalise."""
+    m, n = st.model, x.shape[0]
 
     def bias(i, out):
         return w[m.bOffsets[i]:m.bOffsets[i] + out] if m.bias else torch.zeros(out, dtype=torch.float64, device=DEVICE)
 
-    x = st.batch.double().transpose(0, 1)  # [N][C][A][B]; the store is [C][N][A][B]
     for i in range(m.cLayers):
         c, p, slab = m.convLayer[i], m.poolLayer[i], m.zOffsets[i + 1]
         k = c.inChannels * c.kSize ** 2
         wm = w[m.wOffsets[i]:m.wOffsets[i] + k * c.outChannels].reshape(c.outChannels, k)
-        y = torch.empty(n, c.outChannels, c.outWidth, c.outHeight, dtype=torch.float64, device=DEVICE)
-        some = max(1, (1 << 27) // (k * c.outWidth * c.outHeight))  # images whose patches are laid out at a time
-        for a in range(0, n, some):
-            cols = F.unfold(x[a:a + some], c.kSize, padding=c.padding, stride=c.stride).transpose(0, 1)
-            part = (wm @ cols.reshape(k, -1)).reshape(c.outChannels, -1, c.outWidth, c.outHeight)
-            y[a:a + some] = part.transpose(0, 1) + bias(i, c.outChannels).reshape(1, -1, 1, 1)
+        y = _unfolded(x, c, wm) + bias(i, c.outChannels).reshape(1, -1, 1, 1)
         put(slab, y.transpose(0, 1))
         if c.batchNorm:
             at = slab + c.batchNormOffset
             mean, var = y.mean((0, 2, 3)), y.var((0, 2, 3), unbiased=False)
+            if running is not None:
+                mean, var = (running[at + o:at + o + c.outChannels].double() for o in (c.runningMeansOffset, c.runningVariancesOffset))
             y = (y - mean.reshape(1, -1, 1, 1)) / torch.sqrt(var.reshape(1, -1, 1, 1) + 1e-5)
             put(at, y.transpose(0, 1))
             put(at + c.meansOffset, mean)
             put(at + c.variancesOffset, var)
         x = _activate(m.actFuns[i], y)
         put(slab + c.activationOffset, x.transpose(0, 1))
+        if p.type == S.MAX_POOL:  # the cell that is taken is the largest of the rounded ones
+            at = F.max_pool2d(x.detach().float(), p.pSize, p.stride, p.padding, return_indices=True)[1]
+            x = x.flatten(2).gather(2, at.flatten(2)).reshape(at.shape)
+        elif p.type == S.AVG_POOL:
+            x = F.avg_pool2d(x, p.pSize, p.stride, p.padding)
         if p.type != S.NO_POOL:
-            x = (F.max_pool2d if p.type == S.MAX_POOL else F.avg_pool2d)(x, p.pSize, p.stride, p.padding)
             put(slab + c.poolOffset, x.transpose(0, 1))
     x = x.transpose(2, 3).reshape(n, -1)  # the linear layers read [N][C][B][A], written over the last slab's output
     put(m.zOffsets[m.cLayers] + m.convLayer[m.cLayers - 1].outputOffset, x)
@@ -237,10 +249,22 @@ def _fill_z(st):
         put(at + f.offset, x)
         x = _activate(f.actFun, x)
         put(at, x)
-    p = torch.softmax(x, 1)
+    return x
+
+
+def _store(z):
+    """put() of _network that writes into z, rounded to its type."""
+    def put(at, t):
+        z[at:at + t.numel()] = t.detach().reshape(-1).to(z.dtype)
+    return put
+
+
+def _fill_z(st):
+    """The activation store, probabilities and loss errors of a training forward pass, from float64 arithmetic."""
+    p = torch.softmax(_network(st, st.weights.double(), st.batch.double().transpose(0, 1), _store(st.z)), 1)
     st.probs[:p.numel()] = p.reshape(-1).float()
-    p[torch.arange(n), st.labels.long() - 1] -= 1
-    st.errors[:p.numel()] = (p / n).reshape(-1).float()
+    p[torch.arange(st.n), st.labels.long() - 1] -= 1
+    st.errors[:p.numel()] = (p / st.n).reshape(-1).float()
 
 
 def _forward(st, z):
@@ -265,7 +289,8 @@ def prepare(case, seed):
         images, n = case["images"], case["batch"]
         x = _images(images, 3, 32, 32, st.gen).mul_(64).add_(128).clamp_(0, 255).round_().reshape(images, -1)
         y = torch.randint(1, 11, (images,), device=DEVICE, generator=st.gen).float()
-        d.testSetX, d.testSetY, d.testSizeX, d.testSizeY = st.hold(x), st.hold(y), images, images
+        st.test_x, st.test_y = x, y
+        d.testSetX, d.testSetY, d.testSizeX, d.testSizeY = x.data_ptr(), y.data_ptr(), images, images
         st.both = torch.zeros(2 * n * 3072, device=DEVICE)  # a batch as it is stored, and as the network reads it
         d.sampledTrainX = st.both.data_ptr()
         st.batch_labels = torch.zeros(n, device=DEVICE)
@@ -357,6 +382,94 @@ def run(st):
     L.cnn.gaussNewtonHessianVec(C.byref(m), C.byref(st.data), st.z.data_ptr(), st.dx.data_ptr(), st.v.data_ptr(), st.weights.data_ptr(),
                                 C.byref(st.hv_scratch), S.FULL_DATASET)
     return dict(loss=st.loss.value, error=st.error.value, gradient=st.grad, z=st.z, dx=st.dx, gauss_newton=st.hv[:m.pSize])
+
+
+# ---------------------------------------------------------------- the same in 64 bits
+def _padded(t, like):
+    out = torch.zeros(like.numel(), dtype=torch.float64, device=DEVICE)
+    out[:t.numel()] = t.detach().reshape(-1)
+    return out
+
+
+def exact(case, seed):
+    do = case["do"]
+    if do == "curvature":
+        return None  # factors, damping and inverses of nine layers by the rules of the framework: its tests' oracle has them
+    st = prepare(case, seed)
+    if do == "dense":
+        return _exact_dense(st)
+    if do == "evaluate":
+        return _exact_evaluate(st)
+    w = st.weights.double().requires_grad_()
+    z = torch.zeros(st.z.numel(), dtype=torch.float64, device=DEVICE)
+    logits = _network(st, w, st.batch.double().transpose(0, 1), _store(z))
+    labels = st.labels.long() - 1
+    loss = F.cross_entropy(logits, labels)
+    if do == "hessian":
+        g, = torch.autograd.grad(loss, w, create_graph=True)
+        return dict(hv=torch.autograd.grad((g * st.v.double()).sum(), w)[0])
+    g, = torch.autograd.grad(loss, w)
+    if do == "gradient":
+        g = g + 5e-4 * st.weights.double()
+    p = torch.softmax(logits.detach(), 1)
+    errors = p.clone()
+    errors[torch.arange(st.n), labels] -= 1
+    # a probability below the smallest float makes the 32-bit loss a matter of how it is clamped
+    loss = loss.item() if p.min().item() > 1e-30 else None
+    return dict(loss=loss, probs=_padded(p, st.probs), errors=_padded(errors / st.n, st.errors), gradient=g,
+                z=None if case["bn"] else z, dx=None)
+
+
+def _exact_evaluate(st):
+    """Batches through the running statistics that prepare() left; probabilities of the last, short one."""
+    d, n, total = st.data, st.case["batch"], st.data.testSizeX
+    x, y = st.test_x.double().reshape(total, 3, 32, 32), st.test_y.long() - 1
+    mean, std = (torch.tensor(t, dtype=torch.float64, device=DEVICE).reshape(1, 3, 1, 1) for t in CIFAR10_STATISTICS)
+    x = (x / 255 - mean) / std
+    w, running, loss, hits = st.weights.double(), st.z.clone(), 0.0, 0
+    probs = st.probs.double()  # the rows past the last batch are what was there before
+    for a in range(0, total, n):
+        logits, labels = _network(st, w, x[a:a + n], running=running), y[a:a + n]
+        loss += F.cross_entropy(logits, labels, reduction="sum").item()
+        hits += (logits.argmax(1) == labels).sum().item()
+        probs[:logits.numel()] = torch.softmax(logits, 1).reshape(-1)
+    return dict(loss=loss / total, accuracy=100.0 * hits / total, probs=probs, z=None)
+
+
+def _exact_dense(st):
+    """Loss, gradient and Gauss-Newton product; the last keeps the reference's term of the top layer, -(1/n) of the product of
+    that layer's direction and the errors, back-propagated through the layers below."""
+    m, n, x, v = st.model, st.x.shape[0], st.x.double(), st.v.double()
+    z = torch.zeros(st.z.numel(), dtype=torch.float64, device=DEVICE)
+
+    def layers(w, top):
+        h = x
+        for i in range(top):
+            a, b, size = m.wOffsets[i], m.bOffsets[i], m.layerSizes[i + 1]
+            h = h @ w[a:a + m.layerSizes[i] * size].reshape(m.layerSizes[i], size) + w[b:b + size]
+            if i + 1 == m.numLayers:
+                return h
+            h = torch.sigmoid(h) if m.actFuns[i] == S.ACT_LOGISTIC else h
+            _store(z)(m.zOffsets[i + 1], h)
+        return h
+
+    w, top = st.weights.double().requires_grad_(), m.numLayers
+    logits = layers(w, top)
+    out = torch.sigmoid(logits)
+    _store(z)(m.zOffsets[top], out)
+    loss = -(x * logits - F.softplus(logits)).sum() / n
+    g, = torch.autograd.grad(loss, w, retain_graph=True)
+    u = torch.zeros_like(logits, requires_grad=True)
+    jt, = torch.autograd.grad(logits, w, u, create_graph=True)  # J'u, whose derivative by u takes v to Jv
+    jv, = torch.autograd.grad(jt, u, v)
+    out = out.detach()
+    gn, = torch.autograd.grad(logits, w, out * (1 - out) * jv / n)
+    size = m.layerSizes[top]
+    below = layers(w, top - 1)
+    a = m.wOffsets[top - 1]
+    vw = v[a:a + m.layerSizes[top - 1] * size].reshape(-1, size)
+    gn = gn - torch.autograd.grad(below, w, (x - out) @ vw.t() / n)[0]
+    return dict(loss=loss.item(), error=((x - out) ** 2).sum().item() / n, gradient=g, z=z, dx=None, gauss_newton=gn)
 
 
 # ---------------------------------------------------------------- what a pass cannot do without
