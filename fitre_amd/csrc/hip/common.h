@@ -193,6 +193,20 @@ __device__ __forceinline__ float act_derivative(int actFun, float zi, float zo)
 	}
 }
 
+// the activation functions, as fitre_hip_activation_forward evaluates them
+__device__ __forceinline__ float act_forward_value(int actFun, float x)
+{
+	switch (actFun) {
+	case CNN_ACT_RELU: return x < 0.f ? 0.f : x;
+	case CNN_ACT_SOFTPLUS: return x < 20.f ? logf(1.f + expf(x)) : x;
+	case CNN_ACT_ELU: return x < 0.f ? (expf(x) - 1.f) : x;
+	case CNN_ACT_SWISH: return x / (1.f + expf(-x));
+	case ACT_LOGISTIC: return 1.f / (1.f + expf(-x));
+	case ACT_TANH: return tanhf(x);
+	default: return x;
+	}
+}
+
 // strict-> scan of four values in order, starting below every finite float
 __device__ __forceinline__ int scan2x2(float v0, float v1, float v2, float v3)
 {

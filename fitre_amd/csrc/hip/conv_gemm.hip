@@ -8,6 +8,7 @@
 #include "conv_thin.h"
 #include "linear_small.h"
 #include "linear_tail.h"
+#include "linear_forward.h"
 #include "linear_skinny.h"
 
 namespace fitre {
@@ -993,6 +994,40 @@ int fitre_hip_linear_weight_grad(int in, int out, int n, const float *delta, con
 	int rc = gemm_ex(0, 1, out, in, n, 1.f, delta, out, zin, in, 0.f, dW, out, nullptr, 0, FITRE_KC_FC_GEMM, ws, wsBytes);
 	if (rc || !db) return rc;
 	return fitre_hip_row_sum(delta, out, n, db);
+}
+
+// ---- forward pass of a run of small layers ----------------------------------------------------
+int fitre_hip_fc_tail_forward_fits(int layers, const fitre_fc_forward_layer *l, int n)
+{
+	if (!l || n < 1 || layers < 1 || layers > kFwdTailLayers) return 0;
+	long weights = 0;
+	for (int f = 0; f < layers; f++) {
+		if (l[f].in < 1 || l[f].out < 1 || l[f].in > kFwdTailMaxIn || l[f].out > kFwdTailMaxOut) return 0;
+		if (f > 0 && l[f].in != l[f - 1].out) return 0;
+		weights += (long)l[f].in * l[f].out;
+	}
+	return weights <= kFwdTailMaxWeights && (double)weights * n <= kFwdTailMaxWork;
+}
+
+int fitre_hip_fc_tail_forward(int layers, const fitre_fc_forward_layer *l, int n, const float *x)
+{
+	FITRE_NEED_INIT();
+	FITRE_REQUIRE(l && x && n > 0, "fitre_hip_fc_tail_forward: null pointer or non-positive batch");
+	FITRE_REQUIRE(fitre_hip_fc_tail_forward_fits(layers, l, n), "fitre_hip_fc_tail_forward: these layers do not fit one launch");
+	FwdTailParams p{};
+	p.layers = layers, p.samples = n, p.x = x;
+	double macs = 0.0;
+	for (int f = 0; f < layers; f++) {
+		FITRE_REQUIRE(l[f].W && l[f].pre && l[f].post, "fitre_hip_fc_tail_forward: null pointer");
+		FITRE_REQUIRE(act_known(l[f].act), "fitre_hip_fc_tail_forward: unknown activation code %d", l[f].act);
+		int logWidth = 0;
+		while ((1 << logWidth) < l[f].out) logWidth++;
+		p.l[f] = FwdTailLayer{ l[f].in, l[f].out, l[f].act, logWidth, l[f].W, l[f].bias, l[f].pre, l[f].post };
+		macs += (double)l[f].in * l[f].out * n;
+	}
+	LaunchScope scope(FITRE_KC_FC_GEMM, 2.0 * macs, 0);
+	fc_tail_forward_kernel<<<(unsigned)((n + kFwdTailSamples - 1) / kFwdTailSamples), kFwdTailThreads, 0, stream()>>>(p);
+	return check_launch("fc_tail_forward_kernel");
 }
 
 static int tail_samples(int n) { return n >= 512 ? kTailMaxSamples : 4; }

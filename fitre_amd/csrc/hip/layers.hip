@@ -701,19 +701,6 @@ bn_normalize_kernel(const float *x, const float *mean, const float *variance, fl
 	}
 }
 
-// the activation functions, as fitre_hip_activation_forward evaluates them
-__device__ __forceinline__ float act_forward_value(int actFun, float x)
-{
-	switch (actFun) {
-	case CNN_ACT_RELU: return x < 0.f ? 0.f : x;
-	case CNN_ACT_SOFTPLUS: return x < 20.f ? logf(1.f + expf(x)) : x;
-	case CNN_ACT_ELU: return x < 0.f ? (expf(x) - 1.f) : x;
-	case CNN_ACT_SWISH: return x / (1.f + expf(-x));
-	case ACT_LOGISTIC: return 1.f / (1.f + expf(-x));
-	case ACT_TANH: return tanhf(x);
-	default: return x;
-	}
-}
 __device__ __forceinline__ float4 act_forward4(int actFun, float4 v)
 {
 	return make_float4(act_forward_value(actFun, v.x), act_forward_value(actFun, v.y), act_forward_value(actFun, v.z),

@@ -240,6 +240,21 @@ real cnnForward(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, r
 	for (int l = 0; l < model->lLayers; l++) {
 		if (l != 0) outputOffset = 0;
 		const FC_LAYER *f = &model->fcLayer[l];
+		/* the layers from here up in one launch, where they are small enough (LeNet's three, VGG's one, the upper two of the
+		 * CIFAR AlexNet) */
+		fitre_fc_forward_layer rest[4];
+		const int left = model->lLayers - l;
+		for (int k = 0; k < left && left <= 4; k++) {
+			const FC_LAYER *g = &model->fcLayer[l + k];
+			real *post = z + zOffsets[l + k + 1 + nc];
+			fitre_fc_forward_layer t = { g->in, g->out, g->actFun, weights + wOffsets[l + k + nc],
+				                         (model->bias == 0) ? NULL : weights + bOffsets[l + k + nc], post + (long)g->out * n, post };
+			rest[k] = t;
+		}
+		if (left <= 4 && fitre_hip_fc_tail_forward_fits(left, rest, n)) {
+			HIP_CALL(fitre_hip_fc_tail_forward(left, rest, n, z + zOffsets[l + nc] + outputOffset));
+			break;
+		}
 		real *out = z + zOffsets[l + 1 + nc];
 		const long count = (long)f->out * n;
 		/* W z + b, then the saved copy behind it, then the activation in place */

@@ -148,6 +148,12 @@ class fitre_matrix(C.Structure):
                 ("onesRow", C.c_long), ("onesCol", C.c_long), ("onesValue", C.c_double)]
 
 
+class fitre_fc_forward_layer(C.Structure):
+    """One layer of fitre_hip_fc_tail_forward (include/fitre_hip.h)."""
+    _fields_ = [("in_", C.c_int), ("out", C.c_int), ("act", C.c_int), ("W", C.c_void_p), ("bias", C.c_void_p), ("pre", C.c_void_p),
+                ("post", C.c_void_p)]
+
+
 class fitre_fc_tail_layer(C.Structure):
     """One layer of fitre_hip_fc_tail_backward (include/fitre_hip.h)."""
     _fields_ = [("in_", C.c_int), ("out", C.c_int), ("act", C.c_int), ("W", C.c_void_p), ("zPre", C.c_void_p),

@@ -448,6 +448,19 @@ int fitre_hip_linear_input_grad(int in, int out, int n, const float *W, const fl
 int fitre_hip_linear_weight_grad(int in, int out, int n, const float *delta, const float *zin, float *dW, float *db,
                                  void *ws, size_t wsBytes);
 
+/* The forward pass of one to four small fully connected layers that follow each other (layers[0] reads x, in x n), in one
+ * launch: pre = W z + b, post = act(pre), and post is the next layer's input (functions/cnn_forward.cu:250-340 for every
+ * layer).  _fits: at most 2048 inputs and 1024 outputs a layer, 98304 weights together,
+ * 1.3e8 multiply-adds. */
+typedef struct fitre_fc_forward_layer {
+	int in, out;
+	int act;
+	const float *W, *bias; /* out x in, column-major; out (may be NULL) */
+	float *pre, *post;     /* out x n each */
+} fitre_fc_forward_layer;
+int fitre_hip_fc_tail_forward_fits(int layers, const fitre_fc_forward_layer *l, int n);
+int fitre_hip_fc_tail_forward(int layers, const fitre_fc_forward_layer *l, int n, const float *x);
+
 /* The backward products of a whole tail of small fully connected layers (layers[0] the lowest) in two launches (three
  * when the batch is above 512): every layer's delta (after its activation derivative) into its slot, dW = delta * zin',
  * db = delta * 1, and the lowest layer's input gradient W' * delta into `features` -- in a convolution layer's layout
