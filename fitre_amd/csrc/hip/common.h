@@ -207,6 +207,22 @@ __device__ __forceinline__ float act_forward_value(int actFun, float x)
 	}
 }
 
+// strict-> scan of a 2 x 2 window in memory order, as the pooling kernels scan it
+__device__ __forceinline__ float max2x2(float v0, float v1, float v2, float v3)
+{
+	float best = -FLT_MAX;
+	if (v0 > best) best = v0;
+	if (v1 > best) best = v1;
+	if (v2 > best) best = v2;
+	if (v3 > best) best = v3;
+	return best;
+}
+// a 2 x 2 window as pool_forward_kernel pools it
+__device__ __forceinline__ float pool2x2(bool average, float v0, float v1, float v2, float v3)
+{
+	return average ? (((v0 + v1) + v2) + v3) / 4.f : max2x2(v0, v1, v2, v3);
+}
+
 // strict-> scan of four values in order, starting below every finite float
 __device__ __forceinline__ int scan2x2(float v0, float v1, float v2, float v3)
 {

@@ -706,29 +706,22 @@ __device__ __forceinline__ float4 act_forward4(int actFun, float4 v)
 	return make_float4(act_forward_value(actFun, v.x), act_forward_value(actFun, v.y), act_forward_value(actFun, v.z),
 	                   act_forward_value(actFun, v.w));
 }
-// strict-> scan of a 2 x 2 window in memory order, as the pooling kernels scan it
-__device__ __forceinline__ float max2x2(float v0, float v1, float v2, float v3)
-{
-	float best = -FLT_MAX;
-	if (v0 > best) best = v0;
-	if (v1 > best) best = v1;
-	if (v2 > best) best = v2;
-	if (v3 > best) best = v3;
-	return best;
-}
-
 // Normalisation, activation and 2x2 / stride 2 max pooling of a layer in one pass over its convolution output: x is
 // read once and zhat, the activation output and the pooled output are written (the three separate passes read four
 // tensors for the same three results).  One (channel, segment) per workgroup.  `partial`: the per-segment sums of x and
 // x^2 of channel_partial_kernel<2> (segmentsIn per channel) -- every workgroup of a channel adds them up in the same
 // order, the first one also stores the statistics; null: statMean / statVar hold the statistics to use.  zhat null: no
 // normalisation (x goes into the activation as it is).  POOL 0: the unit of work is a 2 x 4 patch (B % 4 == 0, A even);
-// POOL 2: no pooling, the unit is a 16-byte group.
+// POOL 1: one pooled cell (A and B even: the 2 x 2 maps at VGG's end, LeNet's 10 x 10), and with toFc the pooled output
+// goes to the linear layers' order [N][C][b][a] at once; POOL 2: no pooling, the unit is a 16-byte group.  average: the
+// windows' mean instead of their maximum, summed as pool_forward_kernel sums it.
+// The last layer of VGG-11 at batch 256 took seven launches of 4.7 us apiece (statistics, normalisation, activation,
+// pooling, permutation, copy, beside the sums), each of them launch-bound at 0.5 MB; it is two now.
 template <int POOL>
 __global__ void __launch_bounds__(kRedBlock)
 bn_act_pool_forward_kernel(const float *x, const double *partial, int segmentsIn, float momentum, float *mean, float *variance,
                            float *runMean, float *runVar, const float *statMean, const float *statVar, float epsilon, int samples,
-                           int inA, int inB, int actFun, float *zhat, float *actOut, float *poolOut)
+                           int inA, int inB, int actFun, float *zhat, float *actOut, float *poolOut, bool average, bool toFc)
 {
 	const int c = blockIdx.y;
 	const long perChannel = (long)samples * inA * inB;
@@ -772,6 +765,32 @@ bn_act_pool_forward_kernel(const float *x, const double *partial, int segmentsIn
 			}
 			*reinterpret_cast<float4 *>(actOut + base + 4 * i) = act_forward4(actFun, a);
 		}
+	} else if constexpr (POOL == 1) {
+		const int outA = inA / 2, outB = inB / 2, perMap = outA * outB;
+		const long cells = (long)samples * perMap;
+		const long per = (cells + gridDim.x - 1) / gridDim.x;
+		const long lo = (long)blockIdx.x * per;
+		const long hi = (lo + per < cells) ? lo + per : cells;
+		for (long i = lo + threadIdx.x; i < hi; i += kRedBlock) {
+			const long map = i / perMap;
+			const int rem = (int)(i - map * perMap);
+			const int oa = rem / outB, ob = rem - oa * outB;
+			const size_t in = base + (size_t)map * inA * inB + (size_t)(2 * oa) * inB + 2 * ob;
+			float2 a0 = *reinterpret_cast<const float2 *>(x + in);
+			float2 a1 = *reinterpret_cast<const float2 *>(x + in + inB);
+			if (zhat) {
+				a0.x = (a0.x - mu) * inv, a0.y = (a0.y - mu) * inv, a1.x = (a1.x - mu) * inv, a1.y = (a1.y - mu) * inv;
+				*reinterpret_cast<float2 *>(zhat + in) = a0;
+				*reinterpret_cast<float2 *>(zhat + in + inB) = a1;
+			}
+			const float2 r0 = make_float2(act_forward_value(actFun, a0.x), act_forward_value(actFun, a0.y));
+			const float2 r1 = make_float2(act_forward_value(actFun, a1.x), act_forward_value(actFun, a1.y));
+			*reinterpret_cast<float2 *>(actOut + in) = r0;
+			*reinterpret_cast<float2 *>(actOut + in + inB) = r1;
+			const float v = pool2x2(average, r0.x, r0.y, r1.x, r1.y);
+			if (toFc) poolOut[((size_t)map * gridDim.y + c) * perMap + (size_t)ob * outA + oa] = v;
+			else poolOut[((size_t)c * samples + map) * perMap + rem] = v;
+		}
 	} else {
 		const int outB2 = inB / 4, outA = inA / 2, outB = inB / 2;
 		const int perMap = outA * outB2;
@@ -797,7 +816,7 @@ bn_act_pool_forward_kernel(const float *x, const double *partial, int segmentsIn
 			*reinterpret_cast<float4 *>(actOut + in) = r0;
 			*reinterpret_cast<float4 *>(actOut + in + inB) = r1;
 			*reinterpret_cast<float2 *>(poolOut + pBase + (size_t)map * outA * outB + (size_t)oa * outB + 2 * pb) =
-			    make_float2(max2x2(r0.x, r0.y, r1.x, r1.y), max2x2(r0.z, r0.w, r1.z, r1.w));
+			    make_float2(pool2x2(average, r0.x, r0.y, r1.x, r1.y), pool2x2(average, r0.z, r0.w, r1.z, r1.w));
 		}
 	}
 }
@@ -1837,7 +1856,7 @@ int fitre_hip_batch_norm_forward(const float *in, int channels, long perChannel,
 	return check_launch("batch_norm_forward");
 }
 
-int fitre_hip_bn_act_pool_forward(const float *in, int channels, int samples, int inA, int inB, float *zhat, float *mean,
+static int bn_act_pool_forward(bool toFc, const float *in, int channels, int samples, int inA, int inB, float *zhat, float *mean,
                                   float *variance, float *runningMean, float *runningVariance, float epsilon, float momentum,
                                   int train, int actFun, float *actOut, int poolType, int ksize, int stride, int padding, int outA,
                                   int outB, float *poolOut, void *ws, size_t wsBytes)
@@ -1854,11 +1873,27 @@ int fitre_hip_bn_act_pool_forward(const float *in, int channels, int samples, in
 		rc = check_channels("fitre_hip_bn_act_pool_forward", channels, perChannel, ws, wsBytes);
 		if (rc) return rc;
 	}
-	const bool pool2 = poolType == MAX_POOL && ksize == 2 && stride == 2 && padding == 0 && inB % 4 == 0 && inA % 2 == 0 &&
-	                   outA == inA / 2 && outB == inB / 2 && (((uintptr_t)poolOut) & 7) == 0;
-	const bool fused = (poolType == NO_POOL || pool2) && perChannel % 4 == 0 && channels <= 65535 && aligned16(in) && aligned16(actOut) &&
-	                   (!zhat || aligned16(zhat));
-	if (!fused) {
+	const int pooledA = poolType == NO_POOL ? inA : outA, pooledB = poolType == NO_POOL ? inB : outB;
+	float *const last = poolType == NO_POOL ? actOut : poolOut;
+	const size_t lastBytes = sizeof(float) * (size_t)channels * samples * pooledA * pooledB;
+	FITRE_REQUIRE(!toFc || (ws && wsBytes >= lastBytes), "fitre_hip_bn_act_pool_forward_fc: workspace of %zu bytes is smaller than the %zu required",
+	              wsBytes, lastBytes);
+	const bool vec = perChannel % 4 == 0 && channels <= 65535 && aligned16(in) && aligned16(actOut) && (!zhat || aligned16(zhat));
+	const bool pool2 = (poolType == MAX_POOL || poolType == AVG_POOL) && ksize == 2 && stride == 2 && padding == 0 && inA % 2 == 0 &&
+	                   inB % 2 == 0 && outA == inA / 2 && outB == inB / 2;
+	const bool average = poolType == AVG_POOL;
+	// 2: whole 16-byte groups, pooled or permuted by launches of their own; 0: 2 x 4 patches, four neighbouring cells a
+	// thread; 1: pooled cells, for rows that are no whole number of patches and where the output is permuted on the way
+	const int unit = !pool2 || poolType == NO_POOL ? 2 : ((inB % 4 == 0 && !toFc && (((uintptr_t)poolOut) & 7) == 0) ? 0 : 1);
+	const bool poolApart = unit == 2 && poolType != NO_POOL, permuteApart = toFc && unit != 1;
+	auto steps_apart = [&]() -> int {
+		int rc2 = FITRE_OK;
+		if (poolApart) rc2 = fitre_hip_pool_forward(poolType, actOut, channels, samples, inA, inB, ksize, stride, padding, outA, outB, poolOut);
+		if (rc2 || !permuteApart) return rc2;
+		rc2 = fitre_hip_conv_to_fc(last, channels, samples, pooledA, pooledB, (float *)ws);
+		return rc2 ? rc2 : fitre_hip_copy_d2d(last, ws, lastBytes);
+	};
+	if (!vec) {
 		const float *actIn = in;
 		if (zhat) {
 			rc = fitre_hip_batch_norm_forward(in, channels, perChannel, zhat, mean, variance, runningMean, runningVariance, epsilon, momentum,
@@ -1867,8 +1902,18 @@ int fitre_hip_bn_act_pool_forward(const float *in, int channels, int samples, in
 			actIn = zhat;
 		}
 		rc = fitre_hip_activation_forward(actFun, actIn, actOut, count);
-		if (rc || poolType == NO_POOL) return rc;
-		return fitre_hip_pool_forward(poolType, actOut, channels, samples, inA, inB, ksize, stride, padding, outA, outB, poolOut);
+		if (rc) return rc;
+		if (poolType != NO_POOL) {
+			rc = fitre_hip_pool_forward(poolType, actOut, channels, samples, inA, inB, ksize, stride, padding, outA, outB, poolOut);
+			if (rc) return rc;
+		}
+		if (!toFc) return FITRE_OK;
+		rc = fitre_hip_conv_to_fc(last, channels, samples, pooledA, pooledB, (float *)ws);
+		return rc ? rc : fitre_hip_copy_d2d(last, ws, lastBytes);
+	}
+	if (poolApart) { // a shape the pooling step refuses is refused before anything is written
+		rc = check_pool_shape("fitre_hip_bn_act_pool_forward", channels, samples, inA, inB, ksize, stride, padding, outA, outB);
+		if (rc) return rc;
 	}
 	const int S = segments_for(channels, perChannel);
 	double *partial = nullptr;
@@ -1878,17 +1923,37 @@ int fitre_hip_bn_act_pool_forward(const float *in, int channels, int samples, in
 		LaunchScope scope(FITRE_KC_BN_FWD, 4.0 * (double)count);
 		channel_partial_kernel<2, true><<<grid, kRedBlock, 0, stream()>>>(in, nullptr, perChannel, partial);
 	}
-	const double moved = 4.0 * (double)count * (zhat ? 3 : 2) + (poolType == NO_POOL ? 0.0 : (double)count);
-	LaunchScope scope(zhat ? FITRE_KC_BN_FWD : FITRE_KC_ACT_FWD, moved);
-	if (poolType == NO_POOL)
-		bn_act_pool_forward_kernel<2><<<grid, kRedBlock, 0, stream()>>>(in, partial, S, momentum, mean, variance, runningMean, runningVariance,
-		                                                                runningMean, runningVariance, epsilon, samples, inA, inB, actFun,
-		                                                                zhat, actOut, poolOut);
-	else
-		bn_act_pool_forward_kernel<0><<<grid, kRedBlock, 0, stream()>>>(in, partial, S, momentum, mean, variance, runningMean, runningVariance,
-		                                                                runningMean, runningVariance, epsilon, samples, inA, inB, actFun,
-		                                                                zhat, actOut, poolOut);
-	return check_launch("bn_act_pool_forward_kernel");
+	{
+		const double moved = 4.0 * (double)count * (zhat ? 3 : 2) + (unit == 2 ? 0.0 : (double)count);
+		LaunchScope scope(zhat ? FITRE_KC_BN_FWD : FITRE_KC_ACT_FWD, moved);
+		auto launch = [&](auto kernel) {
+			kernel<<<grid, kRedBlock, 0, stream()>>>(in, partial, S, momentum, mean, variance, runningMean, runningVariance, runningMean,
+			                                         runningVariance, epsilon, samples, inA, inB, actFun, zhat, actOut, poolOut, average, toFc);
+		};
+		if (unit == 2) launch(bn_act_pool_forward_kernel<2>);
+		else if (unit == 1) launch(bn_act_pool_forward_kernel<1>);
+		else launch(bn_act_pool_forward_kernel<0>);
+	}
+	rc = check_launch("bn_act_pool_forward_kernel");
+	return rc ? rc : steps_apart();
+}
+
+int fitre_hip_bn_act_pool_forward(const float *in, int channels, int samples, int inA, int inB, float *zhat, float *mean,
+                                  float *variance, float *runningMean, float *runningVariance, float epsilon, float momentum,
+                                  int train, int actFun, float *actOut, int poolType, int ksize, int stride, int padding, int outA,
+                                  int outB, float *poolOut, void *ws, size_t wsBytes)
+{
+	return bn_act_pool_forward(false, in, channels, samples, inA, inB, zhat, mean, variance, runningMean, runningVariance, epsilon, momentum,
+	                           train, actFun, actOut, poolType, ksize, stride, padding, outA, outB, poolOut, ws, wsBytes);
+}
+
+int fitre_hip_bn_act_pool_forward_fc(const float *in, int channels, int samples, int inA, int inB, float *zhat, float *mean,
+                                     float *variance, float *runningMean, float *runningVariance, float epsilon, float momentum,
+                                     int train, int actFun, float *actOut, int poolType, int ksize, int stride, int padding, int outA,
+                                     int outB, float *poolOut, void *ws, size_t wsBytes)
+{
+	return bn_act_pool_forward(true, in, channels, samples, inA, inB, zhat, mean, variance, runningMean, runningVariance, epsilon, momentum,
+	                           train, actFun, actOut, poolType, ksize, stride, padding, outA, outB, poolOut, ws, wsBytes);
 }
 
 // The launches of the stand-alone batch-norm backward step; `partial` holds the per-(channel, segment) sums.

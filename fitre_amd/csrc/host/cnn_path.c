@@ -218,7 +218,8 @@ real cnnForward(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, r
 		{
 			real *bnOut = has_bn(cv) ? slab + cv->batchNormOffset : NULL;
 			const int pooled = pl->type != NO_POOL;
-			HIP_CALL(fitre_hip_bn_act_pool_forward(
+			/* the last layer's output leaves in the linear layers' order: [C][N][a*B+b] -> [N][C][b*A+a] */
+			HIP_CALL((l == nc - 1 ? fitre_hip_bn_act_pool_forward_fc : fitre_hip_bn_act_pool_forward)(
 			    slab, cv->outChannels, n, pooled ? pl->width : cv->outWidth, pooled ? pl->height : cv->outHeight, bnOut,
 			    bnOut ? bnOut + cv->meansOffset : NULL, bnOut ? bnOut + cv->variancesOffset : NULL,
 			    bnOut ? bnOut + cv->runningMeansOffset : NULL, bnOut ? bnOut + cv->runningVariancesOffset : NULL,
@@ -227,14 +228,8 @@ real cnnForward(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, r
 		}
 	}
 
-	/* [C][N][a*B+b] -> [N][C][b*A+a], in place through the workspace */
 	const CONV_LAYER *last = &model->convLayer[nc - 1];
-	int extA, extB;
-	feature_extent(model, &extA, &extB);
-	real *feat = z + zOffsets[nc] + last->outputOffset;
-	const size_t featCount = (size_t)extA * extB * n * last->outChannels;
-	HIP_CALL(fitre_hip_conv_to_fc(feat, last->outChannels, n, extA, extB, (real *)ws));
-	HIP_CALL(fitre_hip_copy_d2d(feat, ws, sizeof(real) * featCount));
+	const real *feat = z + zOffsets[nc] + last->outputOffset;
 
 	int outputOffset = last->outputOffset;
 	for (int l = 0; l < model->lLayers; l++) {

@@ -225,6 +225,12 @@ int fitre_hip_bn_act_pool_forward(const float *in, int channels, int samples, in
                                   float *variance, float *runningMean, float *runningVariance, float epsilon,
                                   float momentum, int train, int actFun, float *actOut, int poolType, int ksize,
                                   int stride, int padding, int outA, int outB, float *poolOut, void *ws, size_t wsBytes);
+/* The same for the last convolution layer: its output (poolOut, or actOut without a pool) is left in the linear layers'
+ * order, as fitre_hip_conv_to_fc gives it.  Workspace: at least that output's size beside the batch norm's. */
+int fitre_hip_bn_act_pool_forward_fc(const float *in, int channels, int samples, int inA, int inB, float *zhat, float *mean,
+                                     float *variance, float *runningMean, float *runningVariance, float epsilon,
+                                     float momentum, int train, int actFun, float *actOut, int poolType, int ksize,
+                                     int stride, int padding, int outA, int outB, float *poolOut, void *ws, size_t wsBytes);
 /* out = (m*delta - sum(delta) - zhat*sum(delta*zhat)) / (m*sqrt(eps+var)), m = perChannel.  :550-621.
  * biasGrad (may be NULL) receives the per-channel sum of out. */
 int fitre_hip_batch_norm_backward(const float *delta, const float *zhat, const float *variance,

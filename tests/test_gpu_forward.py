@@ -3,8 +3,8 @@ import numpy as np
 import pytest
 
 from fitre_amd import lib as L
-from fitre_amd.structs import (ACT_LINEAR, ACT_LOGISTIC, ACT_TANH, CNN_ACT_ELU, CNN_ACT_NONE, CNN_ACT_RELU, CNN_ACT_SOFTPLUS,
-                               CNN_ACT_SWISH)
+from fitre_amd.structs import (ACT_LINEAR, ACT_LOGISTIC, ACT_TANH, AVG_POOL, CNN_ACT_ELU, CNN_ACT_NONE, CNN_ACT_RELU,
+                               CNN_ACT_SOFTPLUS, CNN_ACT_SWISH, MAX_POOL, NO_POOL)
 
 pytestmark = pytest.mark.gpu
 hip = L.hip
@@ -67,3 +67,53 @@ def test_what_a_run_of_layers_refuses(dev):
         return hip.fitre_hip_fc_tail_forward_fits(len(dims), arr, n)
     assert fits([(2048, 48)]) and not fits([(2049, 40)]) and not fits([(8, 1025)]) and not fits([(2048, 49)])
     assert not fits([(8, 8), (9, 8)]) and not fits([(4, 4)] * 5) and not fits([(8, 8)], 0) and not fits([(512, 128)], 4096)
+
+
+# channels, samples, A, B, window, stride, padding, kind: pooled cells (2 x 2 maps, rows of ten, one cell only), patches, windows
+# that are pooled apart, no pool, and counts that are no multiple of four
+LAST = [(16, 77, 2, 2, 2, 2, 0, MAX_POOL), (16, 33, 10, 10, 2, 2, 0, MAX_POOL), (5, 9, 6, 10, 2, 2, 0, AVG_POOL), (1, 1, 2, 2, 2, 2, 0, AVG_POOL),
+        (6, 5, 4, 8, 2, 2, 0, MAX_POOL), (6, 4, 4, 8, 2, 2, 0, AVG_POOL), (4, 8, 7, 7, 3, 2, 0, MAX_POOL), (4, 8, 8, 8, 3, 2, 1, MAX_POOL),
+        (3, 7, 4, 6, 0, 0, 0, NO_POOL), (3, 7, 3, 5, 0, 0, 0, NO_POOL), (3, 3, 5, 7, 2, 2, 0, MAX_POOL)]
+
+
+@pytest.mark.parametrize("act", [CNN_ACT_RELU, CNN_ACT_SWISH])
+@pytest.mark.parametrize("bn,train", [(True, 1), (True, 0), (False, 1)])
+@pytest.mark.parametrize("geom", LAST)
+def test_last_layer_in_the_linear_layers_order(dev, geom, bn, train, act):
+    """fitre_hip_bn_act_pool_forward_fc and the plain form against normalisation, activation, pooling and permutation as
+    launches of their own: the same bits where the statistics are (one workgroup's share of a channel here)."""
+    c, n, a, b, k, s, p, kind = geom
+    oa, ob = ((a + 2 * p - k) // s + 1, (b + 2 * p - k) // s + 1) if kind != NO_POOL else (a, b)
+    per, count, pooled = n * a * b, c * n * a * b, c * n * oa * ob
+    rng = np.random.default_rng(count + kind)
+    px = dev.upload((3 * rng.standard_normal(count) + 1).astype(np.float32))
+    nb = max(hip.fitre_hip_batch_norm_workspace(c, per), 4 * max(count, pooled))
+    ws = dev.alloc(nb)
+
+    def buffers():
+        return [dev.upload(np.full(size, 0.5, np.float32)) for size in (count, count, pooled, c, c, c, c)]
+
+    def fetch(bufs, order):
+        got = [dev.download(q, size) for q, size in zip(bufs, (count, count, pooled, c, c, c, c))]
+        return [got[i] for i in order]
+
+    sep = buffers()
+    src = px
+    if bn:
+        ok(hip.fitre_hip_batch_norm_forward(px, c, per, sep[0], *sep[3:], 1e-5, 0.9, train, ws, nb))
+        src = sep[0]
+    ok(hip.fitre_hip_activation_forward(act, src, sep[1], count))
+    if kind != NO_POOL:
+        ok(hip.fitre_hip_pool_forward(kind, sep[1], c, n, a, b, k, s, p, oa, ob, sep[2]))
+    fc = dev.upload(np.zeros(pooled, np.float32))
+    ok(hip.fitre_hip_conv_to_fc(sep[1] if kind == NO_POOL else sep[2], c, n, oa, ob, fc))
+    for call, permuted in ((hip.fitre_hip_bn_act_pool_forward, False), (hip.fitre_hip_bn_act_pool_forward_fc, True)):
+        one = buffers()
+        ok(call(px, c, n, a, b, one[0] if bn else None, *(one[3:] if bn else [None] * 4), 1e-5, 0.9, train, act, one[1], kind, k, s, p, oa,
+                ob, one[2] if kind != NO_POOL else None, ws, nb))
+        for i in (0, 3, 4, 5, 6):
+            np.testing.assert_array_equal(dev.download(one[i], count if i == 0 else c), dev.download(sep[i], count if i == 0 else c))
+        last = 1 if kind == NO_POOL else 2
+        for i, size in ((1, count), (2, pooled)):
+            want = fc if permuted and i == last else sep[i]
+            np.testing.assert_array_equal(dev.download(one[i], size), dev.download(want, size))
