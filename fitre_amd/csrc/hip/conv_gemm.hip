@@ -6,6 +6,7 @@
 #include "conv_common.h"
 #include "conv_quad.h"
 #include "conv_thin.h"
+#include "conv_thin_forward.h"
 #include "linear_small.h"
 #include "linear_tail.h"
 #include "linear_forward.h"
@@ -573,6 +574,7 @@ int fitre_hip_conv_forward(const fitre_conv_shape *s, const float *x, const floa
 	if (rc) return rc;
 	FITRE_REQUIRE(x && w && y, "fitre_hip_conv_forward: null pointer");
 	if (c3_pos_eligible(s, false)) return launch_c3_pos<false>(s, x, w, bias, y, ws, wsBytes);
+	if (thin_fwd_eligible(s)) return launch_thin_forward(s, x, w, bias, y, nullptr);
 	const int I = s->outChannels, J = s->samples * s->outA * s->outB, R = s->inChannels * s->ksize * s->ksize;
 	GemmPlan plan = plan_gemm(I, J, R, false, 0, true);
 	PlainParams pa{ w, (uint32_t)((size_t)I * R * sizeof(float)), R, I };
@@ -581,6 +583,30 @@ int fitre_hip_conv_forward(const fitre_conv_shape *s, const float *x, const floa
 	rc = attach_patch_table(pb, plan.bn);
 	if (rc) return rc;
 	return launch_gemm<PlainKContig, PatchRowContig>(pa, pb, out, I, J, R, plan, ws, wsBytes, FITRE_KC_CONV_FWD, conv_flops(s));
+}
+
+// the convolution, activation and pool of a layer without batch norm
+int fitre_hip_conv_act_pool_forward(const fitre_conv_shape *s, const float *x, const float *w, const float *bias, float *y, int actFun,
+                                    float *actOut, int poolType, int ksize, int stride, int padding, int poolA, int poolB, float *poolOut,
+                                    int toFc, void *ws, size_t wsBytes)
+{
+	FITRE_NEED_INIT();
+	int rc = check_conv("fitre_hip_conv_act_pool_forward", s);
+	if (rc) return rc;
+	FITRE_REQUIRE(x && w && y && actOut, "fitre_hip_conv_act_pool_forward: null pointer");
+	FITRE_REQUIRE(act_known(actFun), "fitre_hip_conv_act_pool_forward: unknown activation code %d", actFun);
+	FITRE_REQUIRE(poolType == NO_POOL || poolOut, "fitre_hip_conv_act_pool_forward: null pooled output");
+	if ((poolType == MAX_POOL || poolType == AVG_POOL) && ksize == 2 && stride == 2 && padding == 0 && s->outA % 2 == 0 && s->outB % 2 == 0 &&
+	    poolA == s->outA / 2 && poolB == s->outB / 2 && !c3_pos_eligible(s, false) && thin_fwd_eligible(s)) {
+		ThinFwdParams fold{};
+		fold.act = actFun, fold.average = poolType == AVG_POOL, fold.toFc = toFc != 0, fold.actOut = actOut, fold.poolOut = poolOut;
+		return launch_thin_forward(s, x, w, bias, y, &fold);
+	}
+	rc = fitre_hip_conv_forward(s, x, w, bias, y, ws, wsBytes);
+	if (rc) return rc;
+	return (toFc ? fitre_hip_bn_act_pool_forward_fc : fitre_hip_bn_act_pool_forward)(
+	    y, s->outChannels, s->samples, s->outA, s->outB, nullptr, nullptr, nullptr, nullptr, nullptr, 0.f, 0.f, 0, actFun, actOut, poolType,
+	    ksize, stride, padding, poolA, poolB, poolOut, ws, wsBytes);
 }
 
 // ---- weight gradient: I = Cout, J = Cin*k*k, R = positions -------------------

@@ -336,6 +336,11 @@ typedef struct fitre_conv_shape {
 size_t fitre_hip_conv_forward_workspace(const fitre_conv_shape *s);
 int fitre_hip_conv_forward(const fitre_conv_shape *s, const float *x, const float *w, const float *bias,
                            float *y, void *ws, size_t wsBytes);
+/* The same and then, for a layer without batch norm, fitre_hip_bn_act_pool_forward (toFc: _fc) with a null zhat on y: one
+ * launch for few channels and a 2 x 2 / stride 2 pool, the separate ones otherwise. */
+int fitre_hip_conv_act_pool_forward(const fitre_conv_shape *s, const float *x, const float *w, const float *bias, float *y,
+                                    int actFun, float *actOut, int poolType, int ksize, int stride, int padding, int poolA,
+                                    int poolB, float *poolOut, int toFc, void *ws, size_t wsBytes);
 /* dW[Cout][Cin*k*k] = sum over (n,a,b) of patch(x) * delta.  Replaces im2col + GEMM of
  * functions/cnn_backward.cu:771-783. */
 size_t fitre_hip_conv_weight_grad_workspace(const fitre_conv_shape *s);

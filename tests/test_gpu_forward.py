@@ -1,6 +1,9 @@
 """The fused steps of the forward pass (include/fitre_hip.h) against float64 numpy on the same float32 operands."""
+import ctypes as C
+
 import numpy as np
 import pytest
+import torch
 
 from fitre_amd import lib as L
 from fitre_amd.structs import (ACT_LINEAR, ACT_LOGISTIC, ACT_TANH, AVG_POOL, CNN_ACT_ELU, CNN_ACT_NONE, CNN_ACT_RELU,
@@ -117,3 +120,56 @@ def test_last_layer_in_the_linear_layers_order(dev, geom, bn, train, act):
         for i, size in ((1, count), (2, pooled)):
             want = fc if permuted and i == last else sep[i]
             np.testing.assert_array_equal(dev.download(one[i], size), dev.download(want, size))
+
+
+# samples, cin, cout, A, B, window, padding: LeNet's two layers (with and without border, images that share a workgroup and a
+# remainder of them, the channel groups of one, two and four), odd rows and columns, one channel, sixteen of each, 3 x 3
+# windows without a border, and shapes that stay on the tile engine (more channels, seven-wide windows)
+THIN = [(7, 3, 6, 32, 32, 5, 0), (130, 6, 16, 14, 14, 5, 0), (2100, 6, 16, 14, 14, 5, 0), (9, 3, 6, 28, 28, 5, 2), (5, 1, 1, 6, 6, 5, 0),
+        (6, 16, 16, 7, 11, 5, 2), (11, 5, 7, 9, 6, 3, 0), (3, 2, 3, 5, 5, 5, 1), (4, 4, 4, 30, 9, 5, 4), (3, 3, 20, 12, 12, 5, 0), (3, 2, 4, 14, 14, 7, 0)]
+
+
+@pytest.mark.parametrize("act", [CNN_ACT_RELU, CNN_ACT_SWISH])
+@pytest.mark.parametrize("kind,to_fc", [(MAX_POOL, 1), (AVG_POOL, 0), (NO_POOL, 0)])
+@pytest.mark.parametrize("geom", THIN)
+def test_thin_convolution_with_activation_and_pool(dev, geom, kind, to_fc, act):
+    """fitre_hip_conv_act_pool_forward: the convolution against float64, then activation, pool and permutation as launches
+    of their own on what it wrote, the same bits."""
+    from fitre_amd.structs import fitre_conv_shape
+    n, ci, co, a, b, k, pad = geom
+    oa, ob = a + 2 * pad - k + 1, b + 2 * pad - k + 1
+    pa, pb = (oa // 2, ob // 2) if kind != NO_POOL else (oa, ob)
+    rng = np.random.default_rng(n + ci * co + a)
+    x = rng.standard_normal((ci, n, a, b)).astype(np.float32)
+    w = (rng.standard_normal((co, ci, k, k)) / np.sqrt(ci * k * k)).astype(np.float32)
+    bias = rng.standard_normal(co).astype(np.float32)
+    count, pooled = co * n * oa * ob, co * n * pa * pb
+    shape = fitre_conv_shape(n, ci, co, a, b, oa, ob, k, 1, pad)
+    nb = max(hip.fitre_hip_conv_forward_workspace(C.byref(shape)), 4 * count)
+    ws = dev.alloc(nb)
+    px, pw = dev.upload(x.reshape(-1)), dev.upload(w.reshape(-1))
+    for with_bias in (True, False):
+        y, ao, po = (dev.upload(np.full(size + 4, 7.0, np.float32)) for size in (count, count, pooled))
+        ok(hip.fitre_hip_conv_act_pool_forward(C.byref(shape), px, pw, dev.upload(bias) if with_bias else None, y, act, ao, kind, 2, 2, 0,
+                                               pa, pb, po if kind != NO_POOL else None, to_fc, ws, nb))
+        got = dev.download(y, count + 4)
+        np.testing.assert_array_equal(got[-4:], 7.0)
+        want = torch.nn.functional.conv2d(torch.from_numpy(x).double().transpose(0, 1), torch.from_numpy(w).double(),
+                                          torch.from_numpy(bias).double() if with_bias else None, padding=pad).transpose(0, 1).numpy()
+        # a float32 sum of ci * k * k terms of size one over their root, 2^-24 a step
+        assert np.abs(got[:-4] - want.reshape(-1)).max() <= (ci * k * k + 16) * 2.0 ** -24 * max(1.0, np.abs(want).max())
+        ref, pref = dev.zeros(count), dev.zeros(pooled)
+        ok(hip.fitre_hip_activation_forward(act, y, ref, count))
+        last = ref
+        if kind != NO_POOL:
+            ok(hip.fitre_hip_pool_forward(kind, ref, co, n, oa, ob, 2, 2, 0, pa, pb, pref))
+            last = pref
+        np.testing.assert_array_equal(dev.download(ao, count), dev.download(ref, count))
+        if to_fc:
+            out = dev.zeros(pooled)
+            ok(hip.fitre_hip_conv_to_fc(last, co, n, pa, pb, out))
+            last = out
+        if kind != NO_POOL:
+            got = dev.download(po, pooled + 4)
+            np.testing.assert_array_equal(got[:-4], dev.download(last, pooled))
+            np.testing.assert_array_equal(got[-4:], 7.0)
