@@ -268,6 +268,21 @@ struct LaunchScope {
 
 int check_launch(const char *what);
 
+// A convolution output that is still the partials of a split product: x (bias added) is to be written from them.
+struct SplitSource {
+	const float *base; // partials, laid out like x
+	int splits;
+	long stride;
+	const float *bias; // per channel, or null
+	float *x;
+	double *partial; // room for the batch-norm sums (fitre_hip_batch_norm_workspace bytes) where they are taken
+};
+// fitre_hip_bn_act_pool_forward(_fc) on such an output.  16-byte aligned tensors, channels of a multiple of four cells.
+int bn_act_pool_forward_split(bool toFc, const SplitSource &split, int channels, int samples, int inA, int inB, float *zhat, float *mean,
+                              float *variance, float *runningMean, float *runningVariance, float epsilon, float momentum, int train, int actFun,
+                              float *actOut, int poolType, int ksize, int stride, int padding, int outA, int outB, float *poolOut, void *ws,
+                              size_t wsBytes);
+
 // ---- integer division by a run-time constant ------------------------------
 // q = n / d for 0 <= n < 2^31 via one 32x32->64 multiply.
 struct FastDiv {

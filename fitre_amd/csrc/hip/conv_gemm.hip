@@ -585,28 +585,63 @@ int fitre_hip_conv_forward(const fitre_conv_shape *s, const float *x, const floa
 	return launch_gemm<PlainKContig, PatchRowContig>(pa, pb, out, I, J, R, plan, ws, wsBytes, FITRE_KC_CONV_FWD, conv_flops(s));
 }
 
-// the convolution, activation and pool of a layer without batch norm
-int fitre_hip_conv_act_pool_forward(const fitre_conv_shape *s, const float *x, const float *w, const float *bias, float *y, int actFun,
-                                    float *actOut, int poolType, int ksize, int stride, int padding, int poolA, int poolB, float *poolOut,
-                                    int toFc, void *ws, size_t wsBytes)
+// the convolution, batch norm (zhat null: none), activation and pool of a layer
+size_t fitre_hip_conv_bn_act_pool_workspace(const fitre_conv_shape *s, int batchNorm)
+{
+	if (!s) return 0;
+	const size_t conv = (fitre_hip_conv_forward_workspace(s) + 255) & ~(size_t)255;
+	return conv + (batchNorm ? fitre_hip_batch_norm_workspace(s->outChannels, (long)s->samples * s->outA * s->outB) : 0);
+}
+
+int fitre_hip_conv_bn_act_pool_forward(const fitre_conv_shape *s, const float *x, const float *w, const float *bias, float *y, float *zhat,
+                                       float *mean, float *variance, float *runningMean, float *runningVariance, float epsilon,
+                                       float momentum, int train, int actFun, float *actOut, int poolType, int ksize, int stride, int padding,
+                                       int poolA, int poolB, float *poolOut, int toFc, void *ws, size_t wsBytes)
 {
 	FITRE_NEED_INIT();
-	int rc = check_conv("fitre_hip_conv_act_pool_forward", s);
+	int rc = check_conv("fitre_hip_conv_bn_act_pool_forward", s);
 	if (rc) return rc;
-	FITRE_REQUIRE(x && w && y && actOut, "fitre_hip_conv_act_pool_forward: null pointer");
-	FITRE_REQUIRE(act_known(actFun), "fitre_hip_conv_act_pool_forward: unknown activation code %d", actFun);
-	FITRE_REQUIRE(poolType == NO_POOL || poolOut, "fitre_hip_conv_act_pool_forward: null pooled output");
-	if ((poolType == MAX_POOL || poolType == AVG_POOL) && ksize == 2 && stride == 2 && padding == 0 && s->outA % 2 == 0 && s->outB % 2 == 0 &&
-	    poolA == s->outA / 2 && poolB == s->outB / 2 && !c3_pos_eligible(s, false) && thin_fwd_eligible(s)) {
+	FITRE_REQUIRE(x && w && y && actOut, "fitre_hip_conv_bn_act_pool_forward: null pointer");
+	FITRE_REQUIRE(!zhat || (mean && variance && runningMean && runningVariance), "fitre_hip_conv_bn_act_pool_forward: null statistics");
+	FITRE_REQUIRE(act_known(actFun), "fitre_hip_conv_bn_act_pool_forward: unknown activation code %d", actFun);
+	FITRE_REQUIRE(poolType == NO_POOL || poolOut, "fitre_hip_conv_bn_act_pool_forward: null pooled output");
+	const bool c3 = c3_pos_eligible(s, false);
+	if (!zhat && !c3 && (poolType == MAX_POOL || poolType == AVG_POOL) && ksize == 2 && stride == 2 && padding == 0 && s->outA % 2 == 0 &&
+	    s->outB % 2 == 0 && poolA == s->outA / 2 && poolB == s->outB / 2 && thin_fwd_eligible(s)) {
 		ThinFwdParams fold{};
 		fold.act = actFun, fold.average = poolType == AVG_POOL, fold.toFc = toFc != 0, fold.actOut = actOut, fold.poolOut = poolOut;
 		return launch_thin_forward(s, x, w, bias, y, &fold);
 	}
-	rc = fitre_hip_conv_forward(s, x, w, bias, y, ws, wsBytes);
-	if (rc) return rc;
+	const long perChannel = (long)s->samples * s->outA * s->outB;
+	const uintptr_t at = (uintptr_t)y | (uintptr_t)actOut | (uintptr_t)zhat | (uintptr_t)ws;
+	const size_t sums = zhat ? fitre_hip_batch_norm_workspace(s->outChannels, perChannel) : 0;
+	if (c3 && ws && (at & 15) == 0 && perChannel % 4 == 0 && s->outChannels <= 65535 && wsBytes >= sums + 4096) {
+		// the batch-norm sums behind the split partials, which the pass that takes them still reads
+		const size_t convBytes = (wsBytes - sums) & ~(size_t)255;
+		int splits = 1;
+		rc = launch_c3_pos<false>(s, x, w, bias, y, ws, convBytes, &splits);
+		if (rc) return rc;
+		if (splits > 1) {
+			const SplitSource src{ (const float *)ws, splits, (long)s->outChannels * perChannel, bias, y, (double *)((char *)ws + convBytes) };
+			return bn_act_pool_forward_split(toFc != 0, src, s->outChannels, s->samples, s->outA, s->outB, zhat, mean, variance, runningMean,
+			                                 runningVariance, epsilon, momentum, train, actFun, actOut, poolType, ksize, stride, padding, poolA,
+			                                 poolB, poolOut, ws, wsBytes);
+		}
+	} else {
+		rc = fitre_hip_conv_forward(s, x, w, bias, y, ws, wsBytes);
+		if (rc) return rc;
+	}
 	return (toFc ? fitre_hip_bn_act_pool_forward_fc : fitre_hip_bn_act_pool_forward)(
-	    y, s->outChannels, s->samples, s->outA, s->outB, nullptr, nullptr, nullptr, nullptr, nullptr, 0.f, 0.f, 0, actFun, actOut, poolType,
-	    ksize, stride, padding, poolA, poolB, poolOut, ws, wsBytes);
+	    y, s->outChannels, s->samples, s->outA, s->outB, zhat, mean, variance, runningMean, runningVariance, epsilon, momentum, train, actFun, actOut,
+	    poolType, ksize, stride, padding, poolA, poolB, poolOut, ws, wsBytes);
+}
+
+int fitre_hip_conv_act_pool_forward(const fitre_conv_shape *s, const float *x, const float *w, const float *bias, float *y, int actFun,
+                                    float *actOut, int poolType, int ksize, int stride, int padding, int poolA, int poolB, float *poolOut,
+                                    int toFc, void *ws, size_t wsBytes)
+{
+	return fitre_hip_conv_bn_act_pool_forward(s, x, w, bias, y, nullptr, nullptr, nullptr, nullptr, nullptr, 0.f, 0.f, 0, actFun, actOut,
+	                                          poolType, ksize, stride, padding, poolA, poolB, poolOut, toFc, ws, wsBytes);
 }
 
 // ---- weight gradient: I = Cout, J = Cin*k*k, R = positions -------------------

@@ -4,6 +4,7 @@
 #include <float.h>
 #include <math.h>
 #include "common.h"
+#include <type_traits>
 #include "fitre_nn.h"
 
 namespace fitre {
@@ -715,24 +716,94 @@ __device__ __forceinline__ float4 act_forward4(int actFun, float4 v)
 // POOL 1: one pooled cell (A and B even: the 2 x 2 maps at VGG's end, LeNet's 10 x 10), and with toFc the pooled output
 // goes to the linear layers' order [N][C][b][a] at once; POOL 2: no pooling, the unit is a 16-byte group.  average: the
 // windows' mean instead of their maximum, summed as pool_forward_kernel sums it.
+// SRC: where x comes from.  0: it is there.  1: it is still the unsummed split-K partials of the convolution (SplitSource),
+// summed in split order in double as splitk_reduce_kernel sums them, and x is written on the way: one launch and one read
+// of x less (statistics known, or no normalisation).  2: the same where one workgroup has a whole channel (at most 4096
+// cells: the 4 x 4 and 2 x 2 maps): it sums x, takes the channel's statistics from it and goes on, three launches in one.
+// VGG-16 at batch 128 has ten split layers, each a reduction of 9 to 13 us and 4.7 us of sums before this pass.
 // The last layer of VGG-11 at batch 256 took seven launches of 4.7 us apiece (statistics, normalisation, activation,
 // pooling, permutation, copy, beside the sums), each of them launch-bound at 0.5 MB; it is two now.
-template <int POOL>
+// four cells of x from the partials of a split product
+__device__ __forceinline__ float4 split_sum4(const SplitSource &src, size_t at, float bias)
+{
+	double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+	const float *p = src.base + at;
+	int k = 0;
+	for (; k + 4 <= src.splits; k += 4) { // four independent reads in flight
+		float4 t[4];
+#pragma unroll
+		for (int u = 0; u < 4; u++) t[u] = *reinterpret_cast<const float4 *>(p + (size_t)(k + u) * src.stride);
+#pragma unroll
+		for (int u = 0; u < 4; u++) s0 += (double)t[u].x, s1 += (double)t[u].y, s2 += (double)t[u].z, s3 += (double)t[u].w;
+	}
+	for (; k < src.splits; k++) {
+		const float4 t = *reinterpret_cast<const float4 *>(p + (size_t)k * src.stride);
+		s0 += (double)t.x, s1 += (double)t.y, s2 += (double)t.z, s3 += (double)t.w;
+	}
+	return make_float4((float)s0 + bias, (float)s1 + bias, (float)s2 + bias, (float)s3 + bias);
+}
+__device__ __forceinline__ float2 split_sum2(const SplitSource &src, size_t at, float bias)
+{
+	double s0 = 0.0, s1 = 0.0;
+	for (int k = 0; k < src.splits; k++) {
+		const float2 t = *reinterpret_cast<const float2 *>(src.base + at + (size_t)k * src.stride);
+		s0 += (double)t.x, s1 += (double)t.y;
+	}
+	return make_float2((float)s0 + bias, (float)s1 + bias);
+}
+// x = the sum of a split product's partials over this workgroup's segment of a channel, and the segment's sums of x and
+// x^2 in the order of channel_partial_kernel<2>
+__device__ __forceinline__ void split_segment(const SplitSource &src, size_t base, float bias, long lo, long hi, double &sum, double &squares, double *lds)
+{
+	double s0 = 0.0, s1 = 0.0;
+	for (long i = lo + 4 * (long)threadIdx.x; i + 3 < hi; i += 4 * kRedBlock) {
+		const float4 a = split_sum4(src, base + i, bias);
+		*reinterpret_cast<float4 *>(src.x + base + i) = a;
+		const float t0 = (a.x + a.y) + (a.z + a.w);
+		s0 += (double)t0;
+		s1 += (double)a.x * a.x + (double)a.y * a.y + (double)a.z * a.z + (double)a.w * a.w;
+	}
+	sum = block_sum<kRedBlock>(s0, lds);
+	squares = block_sum<kRedBlock>(s1, lds);
+}
+__global__ void __launch_bounds__(kRedBlock) split_sums_kernel(const SplitSource src, long perChannel, double *partial)
+{
+	__shared__ double lds[kRedBlock / kWave];
+	const int c = blockIdx.y;
+	long lo, hi;
+	segment_range(perChannel, lo, hi); // perChannel % 4 == 0
+	double sum, squares;
+	split_segment(src, (size_t)c * perChannel, src.bias ? src.bias[c] : 0.f, lo, hi, sum, squares, lds);
+	if (threadIdx.x == 0) {
+		const size_t slot = ((size_t)c * gridDim.x + blockIdx.x) * 2;
+		partial[slot] = sum;
+		partial[slot + 1] = squares;
+	}
+}
+
+template <int POOL, int SRC>
 __global__ void __launch_bounds__(kRedBlock)
-bn_act_pool_forward_kernel(const float *x, const double *partial, int segmentsIn, float momentum, float *mean, float *variance,
+bn_act_pool_forward_kernel(const SplitSource src, const float *x, const double *partial, int segmentsIn, float momentum, float *mean, float *variance,
                            float *runMean, float *runVar, const float *statMean, const float *statVar, float epsilon, int samples,
                            int inA, int inB, int actFun, float *zhat, float *actOut, float *poolOut, bool average, bool toFc)
 {
 	const int c = blockIdx.y;
 	const long perChannel = (long)samples * inA * inB;
+	const float bias = (SRC != 0 && src.bias) ? src.bias[c] : 0.f;
 	float mu = 0.f, inv = 1.f;
 	if (zhat) {
 		float var;
-		if (partial) {
+		if (SRC == 2 || partial) {
 			double s = 0.0, ss = 0.0;
-			for (int k = 0; k < segmentsIn; k++) {
-				s += partial[((size_t)c * segmentsIn + k) * 2];
-				ss += partial[((size_t)c * segmentsIn + k) * 2 + 1];
+			if constexpr (SRC == 2) {
+				__shared__ double lds[kRedBlock / kWave];
+				split_segment(src, (size_t)c * perChannel, bias, 0, perChannel, s, ss, lds);
+				__syncthreads(); // x is read back below by other threads of this workgroup
+			} else {
+				for (int k = 0; k < segmentsIn; k++) {
+					s += partial[((size_t)c * segmentsIn + k) * 2];
+					ss += partial[((size_t)c * segmentsIn + k) * 2 + 1];
+				}
 			}
 			const double m = s / (double)perChannel;
 			double v = ss / (double)perChannel - m * m;
@@ -752,13 +823,35 @@ bn_act_pool_forward_kernel(const float *x, const double *partial, int segmentsIn
 		inv = 1.f / sqrtf(var + epsilon);
 	}
 	const size_t base = (size_t)c * perChannel;
+	auto load4 = [&](size_t at) -> float4 {
+		if constexpr (SRC == 1) {
+			const float4 v = split_sum4(src, at, bias);
+			*reinterpret_cast<float4 *>(src.x + at) = v;
+			return v;
+		} else if constexpr (SRC == 2) {
+			return *reinterpret_cast<const float4 *>(src.x + at);
+		} else {
+			return *reinterpret_cast<const float4 *>(x + at);
+		}
+	};
+	auto load2 = [&](size_t at) -> float2 {
+		if constexpr (SRC == 1) {
+			const float2 v = split_sum2(src, at, bias);
+			*reinterpret_cast<float2 *>(src.x + at) = v;
+			return v;
+		} else if constexpr (SRC == 2) {
+			return *reinterpret_cast<const float2 *>(src.x + at);
+		} else {
+			return *reinterpret_cast<const float2 *>(x + at);
+		}
+	};
 	if constexpr (POOL == 2) {
 		const long groups = perChannel / 4;
 		const long per = (groups + gridDim.x - 1) / gridDim.x;
 		const long lo = (long)blockIdx.x * per;
 		const long hi = (lo + per < groups) ? lo + per : groups;
 		for (long i = lo + threadIdx.x; i < hi; i += kRedBlock) {
-			float4 a = *reinterpret_cast<const float4 *>(x + base + 4 * i);
+			float4 a = load4(base + 4 * i);
 			if (zhat) {
 				a.x = (a.x - mu) * inv, a.y = (a.y - mu) * inv, a.z = (a.z - mu) * inv, a.w = (a.w - mu) * inv;
 				*reinterpret_cast<float4 *>(zhat + base + 4 * i) = a;
@@ -776,8 +869,8 @@ bn_act_pool_forward_kernel(const float *x, const double *partial, int segmentsIn
 			const int rem = (int)(i - map * perMap);
 			const int oa = rem / outB, ob = rem - oa * outB;
 			const size_t in = base + (size_t)map * inA * inB + (size_t)(2 * oa) * inB + 2 * ob;
-			float2 a0 = *reinterpret_cast<const float2 *>(x + in);
-			float2 a1 = *reinterpret_cast<const float2 *>(x + in + inB);
+			float2 a0 = load2(in);
+			float2 a1 = load2(in + inB);
 			if (zhat) {
 				a0.x = (a0.x - mu) * inv, a0.y = (a0.y - mu) * inv, a1.x = (a1.x - mu) * inv, a1.y = (a1.y - mu) * inv;
 				*reinterpret_cast<float2 *>(zhat + in) = a0;
@@ -804,8 +897,8 @@ bn_act_pool_forward_kernel(const float *x, const double *partial, int segmentsIn
 			const int rem = (int)(i - map * perMap);
 			const int oa = rem / outB2, pb = rem - oa * outB2;
 			const size_t in = base + (size_t)map * inA * inB + (size_t)(2 * oa) * inB + 4 * pb;
-			float4 a0 = *reinterpret_cast<const float4 *>(x + in);
-			float4 a1 = *reinterpret_cast<const float4 *>(x + in + inB);
+			float4 a0 = load4(in);
+			float4 a1 = load4(in + inB);
 			if (zhat) {
 				a0.x = (a0.x - mu) * inv, a0.y = (a0.y - mu) * inv, a0.z = (a0.z - mu) * inv, a0.w = (a0.w - mu) * inv;
 				a1.x = (a1.x - mu) * inv, a1.y = (a1.y - mu) * inv, a1.z = (a1.z - mu) * inv, a1.w = (a1.w - mu) * inv;
@@ -1856,7 +1949,7 @@ int fitre_hip_batch_norm_forward(const float *in, int channels, long perChannel,
 	return check_launch("batch_norm_forward");
 }
 
-static int bn_act_pool_forward(bool toFc, const float *in, int channels, int samples, int inA, int inB, float *zhat, float *mean,
+static int bn_act_pool_forward(bool toFc, const SplitSource *split, const float *in, int channels, int samples, int inA, int inB, float *zhat, float *mean,
                                   float *variance, float *runningMean, float *runningVariance, float epsilon, float momentum,
                                   int train, int actFun, float *actOut, int poolType, int ksize, int stride, int padding, int outA,
                                   int outB, float *poolOut, void *ws, size_t wsBytes)
@@ -1869,7 +1962,7 @@ static int bn_act_pool_forward(bool toFc, const float *in, int channels, int sam
 	FITRE_REQUIRE(channels > 0 && samples > 0 && inA > 0 && inB > 0, "fitre_hip_bn_act_pool_forward: non-positive shape");
 	const long perChannel = (long)samples * inA * inB, count = perChannel * channels;
 	int rc;
-	if (zhat) {
+	if (zhat && !split) {
 		rc = check_channels("fitre_hip_bn_act_pool_forward", channels, perChannel, ws, wsBytes);
 		if (rc) return rc;
 	}
@@ -1893,6 +1986,7 @@ static int bn_act_pool_forward(bool toFc, const float *in, int channels, int sam
 		rc2 = fitre_hip_conv_to_fc(last, channels, samples, pooledA, pooledB, (float *)ws);
 		return rc2 ? rc2 : fitre_hip_copy_d2d(last, ws, lastBytes);
 	};
+	if (split && !vec) return fail(FITRE_E_UNSUPPORTED, "bn_act_pool_forward: partials of a misaligned or odd tensor");
 	if (!vec) {
 		const float *actIn = in;
 		if (zhat) {
@@ -1918,32 +2012,60 @@ static int bn_act_pool_forward(bool toFc, const float *in, int channels, int sam
 	const int S = segments_for(channels, perChannel);
 	double *partial = nullptr;
 	const dim3 grid(S, channels);
-	if (zhat && train) {
-		partial = (double *)ws;
-		LaunchScope scope(FITRE_KC_BN_FWD, 4.0 * (double)count);
-		channel_partial_kernel<2, true><<<grid, kRedBlock, 0, stream()>>>(in, nullptr, perChannel, partial);
+	int source = 0; // the kernel's SRC
+	if (split && !(zhat && train)) source = 1;
+	else if (split && S == 1) source = 2;
+	if (zhat && train && source == 0) {
+		LaunchScope scope(FITRE_KC_BN_FWD, 4.0 * (double)count * (split ? split->splits + 1 : 1));
+		if (split) {
+			partial = split->partial;
+			split_sums_kernel<<<grid, kRedBlock, 0, stream()>>>(*split, perChannel, partial);
+		} else {
+			partial = (double *)ws;
+			channel_partial_kernel<2, true><<<grid, kRedBlock, 0, stream()>>>(in, nullptr, perChannel, partial);
+		}
 	}
 	{
-		const double moved = 4.0 * (double)count * (zhat ? 3 : 2) + (unit == 2 ? 0.0 : (double)count);
+		const double moved = 4.0 * (double)count * ((zhat ? 3 : 2) + (source ? split->splits : 0)) + (unit == 2 ? 0.0 : (double)count);
 		LaunchScope scope(zhat ? FITRE_KC_BN_FWD : FITRE_KC_ACT_FWD, moved);
 		auto launch = [&](auto kernel) {
-			kernel<<<grid, kRedBlock, 0, stream()>>>(in, partial, S, momentum, mean, variance, runningMean, runningVariance, runningMean,
-			                                         runningVariance, epsilon, samples, inA, inB, actFun, zhat, actOut, poolOut, average, toFc);
+			kernel<<<grid, kRedBlock, 0, stream()>>>(split ? *split : SplitSource{}, in, partial, S, momentum, mean, variance, runningMean,
+			                                         runningVariance, runningMean, runningVariance, epsilon, samples, inA, inB, actFun, zhat,
+			                                         actOut, poolOut, average, toFc);
 		};
-		if (unit == 2) launch(bn_act_pool_forward_kernel<2>);
-		else if (unit == 1) launch(bn_act_pool_forward_kernel<1>);
-		else launch(bn_act_pool_forward_kernel<0>);
+		auto pick = [&](auto src) {
+			constexpr int SRC = decltype(src)::value;
+			if (unit == 2) launch(bn_act_pool_forward_kernel<2, SRC>);
+			else if (unit == 1) launch(bn_act_pool_forward_kernel<1, SRC>);
+			else launch(bn_act_pool_forward_kernel<0, SRC>);
+		};
+		if (source == 2) pick(std::integral_constant<int, 2>{});
+		else if (source == 1) pick(std::integral_constant<int, 1>{});
+		else pick(std::integral_constant<int, 0>{});
 	}
 	rc = check_launch("bn_act_pool_forward_kernel");
 	return rc ? rc : steps_apart();
 }
+
+} // extern "C"
+
+int fitre::bn_act_pool_forward_split(bool toFc, const SplitSource &split, int channels, int samples, int inA, int inB, float *zhat, float *mean,
+                                     float *variance, float *runningMean, float *runningVariance, float epsilon, float momentum, int train,
+                                     int actFun, float *actOut, int poolType, int ksize, int stride, int padding, int outA, int outB,
+                                     float *poolOut, void *ws, size_t wsBytes)
+{
+	return bn_act_pool_forward(toFc, &split, split.x, channels, samples, inA, inB, zhat, mean, variance, runningMean, runningVariance, epsilon,
+	                           momentum, train, actFun, actOut, poolType, ksize, stride, padding, outA, outB, poolOut, ws, wsBytes);
+}
+
+extern "C" {
 
 int fitre_hip_bn_act_pool_forward(const float *in, int channels, int samples, int inA, int inB, float *zhat, float *mean,
                                   float *variance, float *runningMean, float *runningVariance, float epsilon, float momentum,
                                   int train, int actFun, float *actOut, int poolType, int ksize, int stride, int padding, int outA,
                                   int outB, float *poolOut, void *ws, size_t wsBytes)
 {
-	return bn_act_pool_forward(false, in, channels, samples, inA, inB, zhat, mean, variance, runningMean, runningVariance, epsilon, momentum,
+	return bn_act_pool_forward(false, nullptr, in, channels, samples, inA, inB, zhat, mean, variance, runningMean, runningVariance, epsilon, momentum,
 	                           train, actFun, actOut, poolType, ksize, stride, padding, outA, outB, poolOut, ws, wsBytes);
 }
 
@@ -1952,7 +2074,7 @@ int fitre_hip_bn_act_pool_forward_fc(const float *in, int channels, int samples,
                                      int train, int actFun, float *actOut, int poolType, int ksize, int stride, int padding, int outA,
                                      int outB, float *poolOut, void *ws, size_t wsBytes)
 {
-	return bn_act_pool_forward(true, in, channels, samples, inA, inB, zhat, mean, variance, runningMean, runningVariance, epsilon, momentum,
+	return bn_act_pool_forward(true, nullptr, in, channels, samples, inA, inB, zhat, mean, variance, runningMean, runningVariance, epsilon, momentum,
 	                           train, actFun, actOut, poolType, ksize, stride, padding, outA, outB, poolOut, ws, wsBytes);
 }
 

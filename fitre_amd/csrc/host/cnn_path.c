@@ -63,8 +63,7 @@ static size_t forward_ws_bytes(const CNN_MODEL *model, int batch)
 	for (int i = 0; i < model->cLayers; i++) {
 		const CONV_LAYER *c = &model->convLayer[i];
 		fitre_conv_shape s = conv_shape(c, batch);
-		need = max_sz(need, fitre_hip_conv_forward_workspace(&s));
-		if (has_bn(c)) need = max_sz(need, fitre_hip_batch_norm_workspace(c->outChannels, (long)batch * c->outWidth * c->outHeight));
+		need = max_sz(need, fitre_hip_conv_bn_act_pool_workspace(&s, has_bn(c)) + 256);
 	}
 	if (model->cLayers > 0) {
 		int extA, extB;
@@ -212,22 +211,15 @@ real cnnForward(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, r
 		fitre_conv_shape shape = conv_shape(cv, n);
 
 		const real *bias = (model->bias == 0) ? NULL : weights + bOffsets[l];
-		if (!has_bn(cv)) {
-			HIP_CALL(fitre_hip_conv_act_pool_forward(&shape, in, weights + wOffsets[l], bias, slab, model->actFuns[l], actOut, pl->type,
-			                                         pl->pSize, pl->stride, pl->padding, pl->outWidth, pl->outHeight,
-			                                         (pl->type != NO_POOL) ? slab + cv->poolOffset : NULL, l == nc - 1, ws, wsBytes));
-			continue;
-		}
-		HIP_CALL(fitre_hip_conv_forward(&shape, in, weights + wOffsets[l], bias, slab, ws, wsBytes));
-		/* batch norm, activation and pooling: one pass over the convolution output where the shapes allow, the separate passes
-		 * otherwise; the last layer's output leaves in the linear layers' order: [C][N][a*B+b] -> [N][C][b*A+a] */
-		real *bnOut = slab + cv->batchNormOffset;
-		const int pooled = pl->type != NO_POOL;
-		HIP_CALL((l == nc - 1 ? fitre_hip_bn_act_pool_forward_fc : fitre_hip_bn_act_pool_forward)(
-		    slab, cv->outChannels, n, pooled ? pl->width : cv->outWidth, pooled ? pl->height : cv->outHeight, bnOut,
-		    bnOut + cv->meansOffset, bnOut + cv->variancesOffset, bnOut + cv->runningMeansOffset, bnOut + cv->runningVariancesOffset,
-		    (real)BATCH_NORM_EPSILON, (real)BATCH_NORM_MOMENTUM, forTesting == MODEL_TRAIN, model->actFuns[l], actOut, pl->type, pl->pSize,
-		    pl->stride, pl->padding, pl->outWidth, pl->outHeight, pooled ? slab + cv->poolOffset : NULL, ws, wsBytes));
+		real *bnOut = has_bn(cv) ? slab + cv->batchNormOffset : NULL;
+		/* convolution, batch norm (where the layer has it), activation and pooling in as few passes as the shapes allow; the
+		 * last layer's output leaves in the linear layers' order: [C][N][a*B+b] -> [N][C][b*A+a] */
+		HIP_CALL(fitre_hip_conv_bn_act_pool_forward(
+		    &shape, in, weights + wOffsets[l], bias, slab, bnOut, bnOut ? bnOut + cv->meansOffset : NULL,
+		    bnOut ? bnOut + cv->variancesOffset : NULL, bnOut ? bnOut + cv->runningMeansOffset : NULL,
+		    bnOut ? bnOut + cv->runningVariancesOffset : NULL, (real)BATCH_NORM_EPSILON, (real)BATCH_NORM_MOMENTUM,
+		    forTesting == MODEL_TRAIN, model->actFuns[l], actOut, pl->type, pl->pSize, pl->stride, pl->padding, pl->outWidth,
+		    pl->outHeight, (pl->type != NO_POOL) ? slab + cv->poolOffset : NULL, l == nc - 1, ws, wsBytes));
 	}
 
 	const CONV_LAYER *last = &model->convLayer[nc - 1];

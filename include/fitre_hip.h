@@ -341,6 +341,15 @@ int fitre_hip_conv_forward(const fitre_conv_shape *s, const float *x, const floa
 int fitre_hip_conv_act_pool_forward(const fitre_conv_shape *s, const float *x, const float *w, const float *bias, float *y,
                                     int actFun, float *actOut, int poolType, int ksize, int stride, int padding, int poolA,
                                     int poolB, float *poolOut, int toFc, void *ws, size_t wsBytes);
+/* The same with batch norm (zhat NULL: without).  _workspace: enough for the pass that sums a split product's partials to
+ * take the batch norm's sums as well; with less (fitre_hip_conv_forward_workspace and the other steps' own needs) they are
+ * passes of their own. */
+size_t fitre_hip_conv_bn_act_pool_workspace(const fitre_conv_shape *s, int batchNorm);
+int fitre_hip_conv_bn_act_pool_forward(const fitre_conv_shape *s, const float *x, const float *w, const float *bias, float *y,
+                                       float *zhat, float *mean, float *variance, float *runningMean, float *runningVariance,
+                                       float epsilon, float momentum, int train, int actFun, float *actOut, int poolType,
+                                       int ksize, int stride, int padding, int poolA, int poolB, float *poolOut, int toFc,
+                                       void *ws, size_t wsBytes);
 /* dW[Cout][Cin*k*k] = sum over (n,a,b) of patch(x) * delta.  Replaces im2col + GEMM of
  * functions/cnn_backward.cu:771-783. */
 size_t fitre_hip_conv_weight_grad_workspace(const fitre_conv_shape *s);

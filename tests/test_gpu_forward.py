@@ -173,3 +173,43 @@ def test_thin_convolution_with_activation_and_pool(dev, geom, kind, to_fc, act):
             got = dev.download(po, pooled + 4)
             np.testing.assert_array_equal(got[:-4], dev.download(last, pooled))
             np.testing.assert_array_equal(got[-4:], 7.0)
+
+
+# samples, cin, cout, A, B: one workgroup per channel (4 x 4 and 2 x 2 maps, the cell kernel and the nine-tap one), several
+# segments of a channel, a channel of a multiple of four cells that is no whole number of segments, one that is none
+SPLIT = [(32, 256, 64, 4, 4), (21, 128, 64, 2, 2), (64, 128, 128, 8, 8), (52, 64, 96, 14, 12), (3, 64, 40, 7, 7), (16, 512, 32, 13, 13)]
+
+
+@pytest.mark.parametrize("bn,train", [(True, 1), (True, 0), (False, 1)])
+@pytest.mark.parametrize("kind,to_fc", [(MAX_POOL, 0), (MAX_POOL, 1), (NO_POOL, 0), (NO_POOL, 1)])
+@pytest.mark.parametrize("geom", SPLIT)
+def test_split_convolution_summed_by_the_pass_behind_it(dev, geom, kind, to_fc, bn, train):
+    """fitre_hip_conv_bn_act_pool_forward against fitre_hip_conv_forward and fitre_hip_bn_act_pool_forward(_fc): the same
+    partials summed in the same order, the same bits."""
+    from fitre_amd.structs import fitre_conv_shape
+    n, ci, co, a, b = geom
+    k, s = (2, 2) if a % 2 == 0 and b % 2 == 0 else (3, 2)
+    pa, pb = ((a - k) // s + 1, (b - k) // s + 1) if kind != NO_POOL else (a, b)
+    rng = np.random.default_rng(n + ci * co + a)
+    count, pooled = co * n * a * b, co * n * pa * pb
+    px = dev.upload(rng.standard_normal(ci * n * a * b).astype(np.float32))
+    pw = dev.upload((rng.standard_normal(co * ci * 9) / np.sqrt(ci * 9)).astype(np.float32))
+    pbias = dev.upload(rng.standard_normal(co).astype(np.float32))
+    shape = fitre_conv_shape(n, ci, co, a, b, a, b, 3, 1, 1)
+    nb = 2 * max(hip.fitre_hip_conv_bn_act_pool_workspace(C.byref(shape), 1), 4 * count)
+    ws = dev.alloc(nb)
+    sizes = (count, count, count, pooled, co, co, co, co)
+
+    def passes(whole):
+        y, zhat, act, pool, *stats = bufs = [dev.upload(np.full(size, 0.5, np.float32)) for size in sizes]
+        norm = [zhat, *stats] if bn else [None] * 5
+        rest = (1e-5, 0.9, train, CNN_ACT_SWISH, act, kind, k, s, 0, pa, pb, pool if kind != NO_POOL else None)
+        if whole:
+            ok(hip.fitre_hip_conv_bn_act_pool_forward(C.byref(shape), px, pw, pbias, y, *norm, *rest, to_fc, ws, nb))
+        else:
+            ok(hip.fitre_hip_conv_forward(C.byref(shape), px, pw, pbias, y, ws, nb))
+            ok((hip.fitre_hip_bn_act_pool_forward_fc if to_fc else hip.fitre_hip_bn_act_pool_forward)(y, co, n, a, b, *norm, *rest, ws, nb))
+        return [dev.download(q, size) for q, size in zip(bufs, sizes)]
+
+    for got, want in zip(passes(True), passes(False)):
+        np.testing.assert_array_equal(got, want)
