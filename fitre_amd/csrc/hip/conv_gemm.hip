@@ -589,7 +589,9 @@ int fitre_hip_conv_forward(const fitre_conv_shape *s, const float *x, const floa
 size_t fitre_hip_conv_bn_act_pool_workspace(const fitre_conv_shape *s, int batchNorm)
 {
 	if (!s) return 0;
-	const size_t conv = (fitre_hip_conv_forward_workspace(s) + 255) & ~(size_t)255;
+	size_t conv = fitre_hip_conv_forward_workspace(s);
+	if (quad_forward_eligible(s) && quad_forward_workspace(s) > conv) conv = quad_forward_workspace(s);
+	conv = (conv + 255) & ~(size_t)255;
 	return conv + (batchNorm ? fitre_hip_batch_norm_workspace(s->outChannels, (long)s->samples * s->outA * s->outB) : 0);
 }
 
@@ -615,6 +617,19 @@ int fitre_hip_conv_bn_act_pool_forward(const fitre_conv_shape *s, const float *x
 	const long perChannel = (long)s->samples * s->outA * s->outB;
 	const uintptr_t at = (uintptr_t)y | (uintptr_t)actOut | (uintptr_t)zhat | (uintptr_t)ws;
 	const size_t sums = zhat ? fitre_hip_batch_norm_workspace(s->outChannels, perChannel) : 0;
+	if (quad_forward_eligible(s) && ws && ((at | (uintptr_t)x | (uintptr_t)w) & 15) == 0 && s->outChannels <= 65535 &&
+	    wsBytes >= quad_forward_workspace(s) + sums + 256) {
+		// 2 x 2 maps as a dense product; its partials and, behind them, the batch-norm sums are read by the pass that follows
+		const size_t convBytes = (wsBytes - sums) & ~(size_t)255;
+		int splits = 1;
+		float *partials = nullptr;
+		rc = quad_forward(s, x, w, ws, convBytes, &splits, &partials);
+		if (rc) return rc;
+		const SplitSource src{ partials, splits, (long)s->outChannels * perChannel, bias, y, (double *)((char *)ws + convBytes) };
+		return bn_act_pool_forward_split(toFc != 0, src, s->outChannels, s->samples, s->outA, s->outB, zhat, mean, variance, runningMean,
+		                                 runningVariance, epsilon, momentum, train, actFun, actOut, poolType, ksize, stride, padding, poolA,
+		                                 poolB, poolOut, ws, wsBytes);
+	}
 	if (c3 && ws && (at & 15) == 0 && perChannel % 4 == 0 && s->outChannels <= 65535 && wsBytes >= sums + 4096) {
 		// the batch-norm sums behind the split partials, which the pass that takes them still reads
 		const size_t convBytes = (wsBytes - sums) & ~(size_t)255;

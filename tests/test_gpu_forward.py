@@ -213,3 +213,42 @@ def test_split_convolution_summed_by_the_pass_behind_it(dev, geom, kind, to_fc, 
 
     for got, want in zip(passes(True), passes(False)):
         np.testing.assert_array_equal(got, want)
+
+
+# samples, cin, cout on 2 x 2 maps: the smallest batch of the dense form, ragged samples and channels, an uncut reduction
+@pytest.mark.parametrize("bn,train", [(True, 1), (False, 1)])
+@pytest.mark.parametrize("n,ci,co", [(128, 64, 64), (131, 68, 70), (256, 256, 96), (700, 64, 512)])
+def test_forward_on_two_by_two_maps_as_a_dense_product(dev, n, ci, co, bn, train):
+    """The convolution against float64; normalisation, activation and pool against fitre_hip_bn_act_pool_forward on it."""
+    from fitre_amd.structs import fitre_conv_shape
+    rng = np.random.default_rng(n + ci + co)
+    x = rng.standard_normal((ci, n, 2, 2)).astype(np.float32)
+    w = (rng.standard_normal((co, ci, 3, 3)) / np.sqrt(4 * ci)).astype(np.float32)
+    bias = rng.standard_normal(co).astype(np.float32)
+    px, pw, pbias = dev.upload(x.reshape(-1)), dev.upload(w.reshape(-1)), dev.upload(bias)
+    count, pooled = co * n * 4, co * n
+    shape = fitre_conv_shape(n, ci, co, 2, 2, 2, 2, 3, 1, 1)
+    nb = hip.fitre_hip_conv_bn_act_pool_workspace(C.byref(shape), 1) + 4096
+    ws = dev.alloc(nb)
+    sizes = (count, count, pooled, co, co, co, co)
+
+    def rest(y, call, *head):
+        zhat, act, pool, *stats = bufs = [dev.upload(np.full(size, 0.5, np.float32)) for size in sizes]
+        norm = [zhat, *stats] if bn else [None] * 5
+        tail = (0, ws, nb) if call is hip.fitre_hip_conv_bn_act_pool_forward else (ws, nb)
+        ok(call(*head, *norm, 1e-5, 0.9, train, CNN_ACT_RELU, act, MAX_POOL, 2, 2, 0, 1, 1, pool, *tail))
+        return [dev.download(q, size) for q, size in zip(bufs, sizes)]
+
+    y = dev.upload(np.full(count + 4, 7.0, np.float32))
+    got = rest(y, hip.fitre_hip_conv_bn_act_pool_forward, C.byref(shape), px, pw, pbias, y)
+    out = dev.download(y, count + 4)
+    np.testing.assert_array_equal(out[-4:], 7.0)
+    want = torch.nn.functional.conv2d(torch.from_numpy(x).double().transpose(0, 1), torch.from_numpy(w).double(),
+                                      torch.from_numpy(bias).double(), padding=1).transpose(0, 1).numpy()
+    # a float32 sum of 4 * ci terms of size one over their root, 2^-24 a step
+    assert np.abs(out[:-4] - want.reshape(-1)).max() <= (4 * ci + 16) * 2.0 ** -24 * max(1.0, np.abs(want).max())
+    for a, b in zip(got, rest(y, hip.fitre_hip_bn_act_pool_forward, y, co, n, 2, 2)):
+        if bn:
+            np.testing.assert_allclose(a, b, rtol=1e-5, atol=1e-6)  # more than one segment of a channel from 1025 images on
+        else:
+            np.testing.assert_array_equal(a, b)
