@@ -481,3 +481,15 @@ def test_held_back_reductions_of_small_layers_are_one_launch_with_the_same_bits(
             dev.free(q)
     for shape, px, pd, nw, nbias, nb in data:
         dev.free(px), dev.free(pd)
+
+
+@pytest.mark.parametrize("rows", [1, 17, 64])
+@pytest.mark.parametrize("cols", [1, 63, 239, 240, 241, 256, 257, 1000])
+def test_row_sums_around_the_unrolled_columns(dev, rows, cols):
+    """Sums in double, rounded once: half a unit in the last place, and one more where the order of the sum shows."""
+    m = np.random.default_rng(rows + cols).standard_normal((cols, rows)).astype(np.float32)
+    src, out = dev.upload(m.reshape(-1)), dev.alloc(4 * rows)
+    L.check(hip.fitre_hip_row_sum(src, rows, cols, out))
+    np.testing.assert_allclose(dev.download(out, rows), m.astype(np.float64).sum(0), rtol=2.0 ** -22, atol=1e-12)
+    dev.free(src)
+    dev.free(out)
