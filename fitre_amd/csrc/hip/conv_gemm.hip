@@ -399,6 +399,14 @@ int gemm_ex(int transA, int transB, int M, int N, int K, float alpha, const floa
 	PlainParams br = bk;
 	PlainParams ar{ A, (uint32_t)(aElems * sizeof(float)), lda, J };
 	PlainParams ak = ar;
+	if (!flags && short_product(I, J, R, lane_compute_units(), plan)) {
+		plan = fit_plan(plan, I, J, R, ws, wsBytes);
+		if (plan.splits > 1 && (((uintptr_t)ws) & 3)) return fail(FITRE_E_WORKSPACE, "split-K workspace is misaligned");
+		if (!transB && !transA) return launch_tile<PlainKContig, PlainRowContig, 64, 64, kGemmShortBK>(bk, ar, out, I, J, R, plan, ws, kernelClass, flops);
+		if (!transB && transA) return launch_tile<PlainKContig, PlainKContig, 64, 64, kGemmShortBK>(bk, ak, out, I, J, R, plan, ws, kernelClass, flops);
+		if (transB && !transA) return launch_tile<PlainRowContig, PlainRowContig, 64, 64, kGemmShortBK>(br, ar, out, I, J, R, plan, ws, kernelClass, flops);
+		return launch_tile<PlainRowContig, PlainKContig, 64, 64, kGemmShortBK>(br, ak, out, I, J, R, plan, ws, kernelClass, flops);
+	}
 	if (!transB && !transA) return launch_gemm<PlainKContig, PlainRowContig>(bk, ar, out, I, J, R, plan, ws, wsBytes, kernelClass, flops);
 	if (!transB && transA) return launch_gemm<PlainKContig, PlainKContig>(bk, ak, out, I, J, R, plan, ws, wsBytes, kernelClass, flops);
 	if (transB && !transA) return launch_gemm<PlainRowContig, PlainRowContig>(br, ar, out, I, J, R, plan, ws, wsBytes, kernelClass, flops);

@@ -483,6 +483,37 @@ def test_held_back_reductions_of_small_layers_are_one_launch_with_the_same_bits(
         dev.free(px), dev.free(pd)
 
 
+# Products of less than a chip's worth of 128 x 128 tiles, on 64 x 64 tiles with slices of 32: whole and ragged tiles, one range and several,
+# a last range that is one slice, the smallest reduction, one side at the limit where the narrow tiles stay (64) and above it.
+SHORT_PRODUCTS = [(65, 65, 64), (65, 200, 65), (128, 128, 784), (513, 131, 257), (512, 1000, 784), (784, 512, 1000), (100, 1024, 1040), (64, 500, 300)]
+
+
+@pytest.mark.parametrize("room", [1.0, 0.5, 0.0])
+@pytest.mark.parametrize("M,N,K", SHORT_PRODUCTS)
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_short_products(dev, M, N, K, ta, tb, room):
+    """room: the part of the workspace that is handed over; with less the reduction is cut into fewer ranges, or not at all.
+    |error| <= K 2^-24 sum |a b| for a chain of K fused multiply-adds in float32, whatever its cuts."""
+    rng = np.random.default_rng(M * 7 + N * 3 + K)
+    lda, ldb, ldc = (K if ta else M) + 1, (N if tb else K) + 2, M + 3
+    A = rng.standard_normal((M if ta else K, lda)).astype(np.float32)  # column-major: rows here are columns there
+    B = rng.standard_normal((K if tb else N, ldb)).astype(np.float32)
+    C0 = rng.standard_normal((N, ldc)).astype(np.float32)
+    opA = A[:, :K].T if ta else A[:, :M]      # [K][M]
+    opB = B[:, :N].T if tb else B[:, :K]      # [N][K]
+    want = opB.astype(np.float64) @ opA.astype(np.float64)
+    bound = K * 2.0 ** -24 * (np.abs(opB).astype(np.float64) @ np.abs(opA).astype(np.float64)) + 2.0 ** -23 * np.abs(want)
+    pa, pb, pc = dev.upload(A.reshape(-1)), dev.upload(B.reshape(-1)), dev.upload(C0.reshape(-1))
+    nb = hip.fitre_hip_gemm_workspace(M, N, K)
+    ws = dev.alloc(max(nb, 4))
+    L.check(hip.fitre_hip_gemm(ta, tb, M, N, K, 1.0, pa, lda, pb, ldb, 0.0, pc, ldc, None, ws if room else None, int(nb * room) & ~3))
+    got = dev.download(pc, ldc * N).reshape(N, ldc)
+    assert np.all(np.abs(got[:, :M] - want) <= bound)
+    np.testing.assert_array_equal(got[:, M:], C0[:, M:])
+    for q in (pa, pb, pc, ws):
+        dev.free(q)
+
+
 @pytest.mark.parametrize("rows", [1, 17, 64])
 @pytest.mark.parametrize("cols", [1, 63, 239, 240, 241, 256, 257, 1000])
 def test_row_sums_around_the_unrolled_columns(dev, rows, cols):
