@@ -16,7 +16,8 @@ Prints ONE JSON line: backward images/sec, plus
   roofline      the dominant kernel (largest summed time): algorithmic FLOPs / its average launch
                 duration, measured with HIP events on the library's stream in a second pass of the
                 same K steps (the first, timed pass runs without per-launch events), against the
-                157.3 TFLOP/s fp32-MFMA peak;
+                157.3 TFLOP/s fp32-MFMA peak, or 2516.6 / 6 of the bf16 pipes where a kernel makes every fp32 product from
+                six exact bf16 ones ("/split": fp32 operands, sums and accuracy);
   kernels       the same accounting for every kernel class of the backward pass (time and fraction of its bound;
                 --tables: every figure, the largest launches on their own, and the tables of the other networks, which
                 make the line 20 KB long);
@@ -41,13 +42,14 @@ sys.path.insert(0, ROOT)
 
 PEAK_MFMA_F32_TFLOPS = 157.3
 PEAK_MFMA_F64_TFLOPS = 78.6
+PEAK_MFMA_BF16_TFLOPS = 2516.6
 PEAK_HBM_GBS = 8000.0
 
 KC = dict(conv_dw=0, conv_dx=1, conv_fwd=2, fc_gemm=3, splitk_reduce=4, bn_bwd=5, bn_fwd=6, pool_bwd=7, pool_fwd=8,
           act_bwd=9, act_fwd=10, bias_grad=11, softmax=12, permute=13, blas1=14, pool_act_bwd=15, kfac_factor=16,
           spd_inverse=17)
 MFMA_CLASSES = ("conv_dw", "conv_dx", "conv_fwd", "fc_gemm", "kfac_factor", "spd_inverse")
-TILES = {0: "", 1: "64x64", 2: "64x128", 3: "128x64", 4: "128x128", 5: "96x128", 6: "dense2x2", 7: "cell4x4", 8: "cell8x8", 9: "skinny"}
+TILES = {0: "", 1: "64x64", 2: "64x128", 3: "128x64", 4: "128x128", 5: "96x128", 6: "dense2x2", 7: "cell4x4", 8: "cell8x8", 9: "skinny", 10: "split"}
 
 
 def measured_traffic(kernel):
@@ -119,9 +121,15 @@ def launch_live_fraction(kernel, work, conv_live):
     return max(conv_live.get(round(work), [1.0])), False
 
 
+def matrix_peak(kernel):
+    """TFLOP/s of fp32 work at which the matrix pipes of a kernel are the bound: the split kernels make every fp32 product from
+    six bf16 ones."""
+    return PEAK_MFMA_BF16_TFLOPS / 6 if kernel.endswith("/split") else PEAK_MFMA_F32_TFLOPS
+
+
 def kernel_table(rows, steps, launches=None, conv_live=None, fc_batch=None):
     """Per kernel class (and tile variant): launches per step, average launch duration, achieved rate against the
-    bound of its class (fp32 MFMA for the contraction kernels, HBM for the others); with `launches`, also the
+    bound of its class (matrix_peak for the contraction kernels, HBM for the others); with `launches`, also the
     four largest shapes of each kernel on their own (`largest`: work in FLOP resp. bytes).
     Convolution gradients (conv_live given): the library counts the window-count work 2*M*K*Cout per launch; `frac` is
     by the multiply-adds the kernel EXECUTES (the cell and dense variants leave out the products with the padding, the
@@ -157,7 +165,7 @@ def kernel_table(rows, steps, launches=None, conv_live=None, fc_batch=None):
                                                    for e in big[r["kernel"]]]
             continue
         rate = r["work"] / (r["ms"] * 1e-3) / (1e12 if mfma else 1e9) if r["ms"] > 0 else 0.0
-        peak = PEAK_MFMA_F32_TFLOPS if mfma else PEAK_HBM_GBS
+        peak = matrix_peak(r["kernel"]) if mfma else PEAK_HBM_GBS
         kernels[r["kernel"]] = dict(bound="mfma" if mfma else "hbm", launches_per_step=r["launches"] / steps,
                                     avg_us=round(avg_us, 2), ms_per_step=round(r["ms"] / steps, 4),
                                     achieved=round(rate, 2 if mfma else 1), unit="TFLOP/s" if mfma else "GB/s",
@@ -214,7 +222,7 @@ def largest_launches(launches, keep=4):
         t = ms * 1e-3 / n
         rate = work / t / (1e12 if mfma else 1e9) if t > 0 else 0.0
         out.setdefault(kernel, []).append(dict(work=work, launches=n, avg_us=round(t * 1e6, 2), achieved=round(rate, 2 if mfma else 1),
-                                               frac=round(rate / (PEAK_MFMA_F32_TFLOPS if mfma else PEAK_HBM_GBS), 4)))
+                                               frac=round(rate / (matrix_peak(kernel) if mfma else PEAK_HBM_GBS), 4)))
     return {k: sorted(v, key=lambda e: -e["work"])[:keep] for k, v in out.items()}
 
 
@@ -310,7 +318,7 @@ def gpu_leg(args):
     dom = max(rows, key=lambda r: r["ms"])
     dk = kernels[dom["kernel"]]
     roofline = dict(kernel=dom["kernel"], bound=dk["bound"], achieved=dk["achieved"],
-                    peak=PEAK_MFMA_F32_TFLOPS if dk["bound"] == "mfma" else PEAK_HBM_GBS, unit=dk["unit"],
+                    peak=round(matrix_peak(dom["kernel"]), 1) if dk["bound"] == "mfma" else PEAK_HBM_GBS, unit=dk["unit"],
                     frac=dk["frac"], traffic=None, avg_launch_us=dk["avg_us"],
                     launches_per_step=dk["launches_per_step"])
     for key in ("frac_ninetap", "frac_useful", "work_executed_gflop_per_step", "work_ninetap_gflop_per_step"):
@@ -328,10 +336,13 @@ def gpu_leg(args):
     conv = dict(ms_per_step=round(conv_ms / args.steps, 4), gflop_per_step_ninetap=round(conv_work / args.steps / 1e9, 2),
                 gflop_per_step_executed=round(conv_executed, 2), unit="TFLOP/s")
     conv["achieved"] = round(conv_executed * 1e9 / (conv_ms / args.steps * 1e-3) / 1e12, 2) if conv_ms else 0.0
-    conv["frac"] = round(conv["achieved"] / PEAK_MFMA_F32_TFLOPS, 4)
-    conv["frac_ninetap"] = round(conv_work / (conv_ms * 1e-3) / 1e12 / PEAK_MFMA_F32_TFLOPS, 4) if conv_ms else 0.0
-    conv["note"] = ("frac: multiply-adds the kernels execute; frac_ninetap: the window count 2*M*K*Cout of every layer, which "
-                    "includes products with the zero padding that the cell and dense kernels leave out")
+    # the time every kernel's work takes at the peak of its own pipes
+    at_peak = sum(kernels[r["kernel"]].get("work_executed_gflop_per_step", r["work"] / args.steps / 1e9) / matrix_peak(r["kernel"]) for r in conv_rows)
+    ninetap_at_peak = sum(r["work"] / args.steps / 1e9 / matrix_peak(r["kernel"]) for r in conv_rows)
+    conv["frac"] = round(at_peak / (conv_ms / args.steps), 4) if conv_ms else 0.0
+    conv["frac_ninetap"] = round(ninetap_at_peak / (conv_ms / args.steps), 4) if conv_ms else 0.0
+    conv["note"] = ("frac: multiply-adds the kernels execute at the peak of their own pipes / time; frac_ninetap: the window count "
+                    "2*M*K*Cout of every layer, which includes products with the zero padding that the cell and dense kernels leave out")
     return dict(wall=wall, ms_events=ms_events.value, batch=batch, loss=loss, finite=finite,
                 device=name.value.decode(), compute_units=cus.value, roofline=roofline, kernels=kernels,
                 conv_backward_gemms=conv, kfac_factors=kfac, bandwidth_kernels=bandwidth, forward_ms=round(forward_ms, 4),
@@ -381,7 +392,7 @@ def other_configs_leg(L, dev, steps=10, only=None):
                          launches_per_step=sum(r["launches"] for r in rows) / steps,
                          kernel_ms_per_step=round(sum(r["ms"] for r in rows) / steps, 4),
                          roofline=dict(kernel=dom["kernel"], bound=dk["bound"], achieved=dk["achieved"],
-                                       peak=PEAK_MFMA_F32_TFLOPS if dk["bound"] == "mfma" else PEAK_HBM_GBS,
+                                       peak=round(matrix_peak(dom["kernel"]), 1) if dk["bound"] == "mfma" else PEAK_HBM_GBS,
                                        unit=dk["unit"], frac=dk["frac"], avg_launch_us=dk["avg_us"],
                                        launches_per_step=dk["launches_per_step"]),
                          kernels=kernels)

@@ -5,6 +5,7 @@
 #include "conv_cell.h"
 #include "conv_common.h"
 #include "conv_quad.h"
+#include "conv_split.h"
 #include "conv_thin.h"
 #include "conv_thin_forward.h"
 #include "linear_small.h"
@@ -181,13 +182,6 @@ static size_t c3_pos_workspace(const fitre_conv_shape *s, bool dx, int pairs = 1
 	size_t a = c3_pos_plan(s, dx, device_compute_units(), pairs).wsBytes, b = c3_pos_plan(s, dx, lane_compute_units_min(), pairs).wsBytes;
 	return a > b ? a : b;
 }
-// whether the forward product is cut into as many ranges in the first `less` bytes of a workspace as in all of it
-static bool c3_pos_fits_in(const fitre_conv_shape *s, const void *ws, size_t less, size_t wsBytes)
-{
-	const BlockPlan plan = c3_pos_plan(s, false);
-	const long blocks = s->inChannels / kC3CB, J = (long)s->samples * s->inA * s->inB;
-	return fit_blocks(plan, blocks, s->outChannels, J, ws, less).splits == fit_blocks(plan, blocks, s->outChannels, J, ws, wsBytes).splits;
-}
 static size_t c3_dw_workspace(const fitre_conv_shape *s, int pairs = 1)
 {
 	size_t a = c3_dw_plan(s, device_compute_units(), pairs).wsBytes, b = c3_dw_plan(s, lane_compute_units_min(), pairs).wsBytes;
@@ -268,6 +262,144 @@ static int launch_c3_pos(const fitre_conv_shape *s, const float *src, const floa
 	if (leftSplits) *leftSplits = plan.splits;
 	if (plan.splits > 1 && !leftSplits) launch_splitk_reduce((const float *)ws, plan.splits, I, J, out);
 	return check_launch("conv3x3_pos_kernel");
+}
+
+// ---- forward and input gradient of 3x3 and 5x5 windows on the bf16 pipes (conv_split.h) ------------------------------------
+static bool split_pos_eligible(const fitre_conv_shape *s, bool dx)
+{
+	const int I = dx ? s->inChannels : s->outChannels, cred = dx ? s->outChannels : s->inChannels;
+	return (s->ksize == 3 || s->ksize == 5) && s->stride == 1 && s->padding == s->ksize / 2 && cred % kSplitCB == 0 && I > 16 && cred > 16 &&
+	       conv_split_variant(s->ksize, I, s->inA, s->inB) != nullptr;
+}
+static int split_row_groups(int I) { return I <= 64 ? 2 : (I + 127) / 128 * 4; }
+static size_t split_weights_bytes(const fitre_conv_shape *s, bool dx)
+{
+	const int I = dx ? s->inChannels : s->outChannels, cred = dx ? s->outChannels : s->inChannels;
+	return (size_t)(cred / kSplitCB) * s->ksize * s->ksize * split_row_groups(I) * 192 * sizeof(u32x4);
+}
+static BlockPlan split_pos_plan(const fitre_conv_shape *s, bool dx, int cus = 0, int pairs = 1)
+{
+	if (cus <= 0) cus = lane_compute_units();
+	const long I = dx ? s->inChannels : s->outChannels, J = (long)s->samples * s->inA * s->inB;
+	const long cred = dx ? s->outChannels : s->inChannels;
+	const long it = I <= 64 ? 64 : 128, jt = I <= 64 ? 256 : 128;
+	const long tiles = ((I + it - 1) / it) * ((J + jt - 1) / jt);
+	// measured: 0.55 us a tap and block with a workgroup on every compute unit, two of them share the pipes
+	return plan_blocks(tiles, pairs * cred / kSplitCB, 0.55 * 0.85 * s->ksize * s->ksize, 1, I, J, cus);
+}
+static size_t split_pos_workspace(const fitre_conv_shape *s, bool dx, int pairs = 1)
+{
+	const size_t a = split_pos_plan(s, dx, device_compute_units(), pairs).wsBytes, b = split_pos_plan(s, dx, lane_compute_units_min(), pairs).wsBytes;
+	return (a > b ? a : b) + pairs * split_weights_bytes(s, dx) + 256;
+}
+// bytes of a workspace that are left for partial results beside the split weights, which take its end; 0: no room for those
+static size_t split_pos_room(const fitre_conv_shape *s, bool dx, const void *ws, size_t wsBytes, int pairs, bool prepared)
+{
+	const size_t weights = prepared ? 0 : pairs * split_weights_bytes(s, dx);
+	if (!ws || (((uintptr_t)ws) & 15) || wsBytes < weights + 256) return 0;
+	return (wsBytes - weights) & ~(size_t)255;
+}
+// From how many multiply-adds on: below, the launch that splits the weights (5 us) and a longer start weigh more than the rate.
+// fp32 / split with that launch, us, forward: 128 -> 128 channels, 8 x 8 maps, 40 images (3.8e8) 27.5 / 25.9, 77 (7.3e8) 36.3 /
+// 30.4, 256 (2.4e9) 55 / 47; 16 x 16 maps, 16 images (6e8) 27.1 / 31.5, 77 (2.9e9) 71.5 / 49.6, 256 (9.7e9) 149 / 96; 512 -> 512,
+// 4 x 4, 16 images (6e8) 26.0 / 35.7, 77 (2.9e9) 71 / 52; 5 x 5 windows, 64 -> 64, 15 x 15, 16 images (3.7e8) 29 / 33, 40 (9.2e8)
+// 42 / 39, 256 (5.9e9) 141 / 74.  Products of at most 64 channels have half the workgroups: 64 -> 64, 16 x 16, 128 images (1.2e9)
+// 25.6 / 30.3, 256 (2.4e9) 43 / 37; 32 x 32, 40 images (1.5e9) 46 / 34.  Whole tiles of 4 x 4 maps have the cell form to beat:
+// 256 -> 256, 128 images (1.2e9) 34.3 / 36.4, 256 (2.4e9) 45.4 / 44.5; 512 -> 512, 256 (9.7e9) 123 / 102.
+constexpr double kSplitWork = 7.0e8, kSplitNarrowWork = 1.5e9, kSplitCellWork = 2.0e9;
+static bool split_pos_chosen(const fitre_conv_shape *s, bool dx, const void *ws, size_t wsBytes, int pairs = 1, bool prepared = false)
+{
+	if (!split_pos_eligible(s, dx) || split_pos_room(s, dx, ws, wsBytes, pairs, prepared) == 0) return false;
+	const int I = dx ? s->inChannels : s->outChannels;
+	const double least = cell_pos_eligible(s, dx) ? kSplitCellWork : (s->ksize == 3 && I <= 64 ? kSplitNarrowWork : kSplitWork);
+	return 0.5 * pairs * conv_flops(s) >= least;
+}
+static BlockPlan split_pos_fit(const fitre_conv_shape *s, bool dx, const void *ws, size_t wsBytes, int pairs, bool prepared)
+{
+	const int I = dx ? s->inChannels : s->outChannels, cred = dx ? s->outChannels : s->inChannels;
+	return fit_blocks(split_pos_plan(s, dx, 0, pairs), pairs * cred / kSplitCB, I, (long)s->samples * s->inA * s->inB, ws,
+	                  split_pos_room(s, dx, ws, wsBytes, pairs, prepared));
+}
+
+static int launch_split_weights(const fitre_conv_shape *s, bool dx, const float *w, u32x4 *wp)
+{
+	const int I = dx ? s->inChannels : s->outChannels, cred = dx ? s->outChannels : s->inChannels, groups = split_row_groups(I);
+	const dim3 grid((unsigned)groups, (unsigned)(cred / kSplitCB));
+	if (grid.y > 65535) return fail(FITRE_E_UNSUPPORTED, "split_weights_kernel grid too large");
+	LaunchScope scope(FITRE_KC_PERMUTE, 10.0 * (double)I * cred * s->ksize * s->ksize);
+	if (s->ksize == 3) {
+		if (dx) split_weights_kernel<3, true><<<grid, 256, 0, stream()>>>(w, I, cred, groups, wp);
+		else split_weights_kernel<3, false><<<grid, 256, 0, stream()>>>(w, I, cred, groups, wp);
+	} else {
+		if (dx) split_weights_kernel<5, true><<<grid, 256, 0, stream()>>>(w, I, cred, groups, wp);
+		else split_weights_kernel<5, false><<<grid, 256, 0, stream()>>>(w, I, cred, groups, wp);
+	}
+	return check_launch("split_weights_kernel");
+}
+
+// prepared: weights split beforehand (one pair only; null: split here, into the end of ws).  leftSplits: as in launch_c3_pos.
+static int launch_split_pos(const fitre_conv_shape *s, bool dx, const float *src, const float *w, const float *bias, float *outPtr, void *ws,
+                            size_t wsBytes, const void *prepared, int *leftSplits, const float *src2 = nullptr, const float *w2 = nullptr)
+{
+	const int I = dx ? s->inChannels : s->outChannels, cred = dx ? s->outChannels : s->inChannels;
+	const int J = s->samples * s->inA * s->inB, pairs = src2 ? 2 : 1;
+	const BlockPlan plan = split_pos_fit(s, dx, ws, wsBytes, pairs, prepared != nullptr);
+	const u32x4 *wp = (const u32x4 *)prepared, *wp2 = nullptr;
+	if (!prepared) {
+		u32x4 *made = (u32x4 *)((char *)ws + split_pos_room(s, dx, ws, wsBytes, pairs, false));
+		int rc = launch_split_weights(s, dx, w, made);
+		if (rc) return rc;
+		wp = made;
+		if (src2) {
+			made += split_weights_bytes(s, dx) / sizeof(u32x4);
+			rc = launch_split_weights(s, dx, w2, made);
+			if (rc) return rc;
+			wp2 = made;
+		}
+	}
+	const int P = s->ksize / 2;
+	ConvSplitParams p{};
+	p.src = src, p.w = w, p.wp = wp, p.src2 = src2, p.w2 = w2, p.wp2 = wp2;
+	p.srcBytes = (uint32_t)((size_t)cred * J * sizeof(float));
+	p.I = I, p.cred = cred, p.J = J, p.A = s->inA, p.B = s->inB, p.dx = dx;
+	p.perSplit = plan.perSplit;
+	p.rowGroups = split_row_groups(I);
+	p.before = conv_split_before(P, s->inA, s->inB), p.late = conv_split_late(P, s->inA, s->inB);
+	p.divB = FastDiv((uint32_t)s->inB), p.divA = FastDiv((uint32_t)s->inA);
+	OutParams out{ outPtr, (long)J, 0, bias, nullptr, 1.f, 0.f };
+	OutParams part = out;
+	if (plan.splits > 1) part.C = (float *)ws, part.splitStride = (long)I * J;
+	const ConvSplitVariant &v = *conv_split_variant(s->ksize, I, s->inA, s->inB);
+	const int it = 32 * v.wm, jt = 128 * (4 / v.wm);
+	const dim3 grid((unsigned)((J + jt - 1) / jt), (unsigned)((I + it - 1) / it), (unsigned)plan.splits);
+	if (grid.y > 65535 || grid.z > 65535) return fail(FITRE_E_UNSUPPORTED, "conv_split_kernel grid too large");
+	{
+		LaunchScope scope(dx ? FITRE_KC_CONV_DX : FITRE_KC_CONV_FWD, pairs * conv_flops(s), kTileSplit);
+#define SPLIT_LAUNCH(N) conv_split_kernel<kConvSplitVariants[N].ks, kConvSplitVariants[N].wm, kConvSplitVariants[N].cells, kConvSplitVariants[N].xe><<<grid, kGemmThreads, 0, stream()>>>(p, part)
+		switch (&v - kConvSplitVariants) {
+		case 0: SPLIT_LAUNCH(0); break;
+		case 1: SPLIT_LAUNCH(1); break;
+		case 2: SPLIT_LAUNCH(2); break;
+		case 3: SPLIT_LAUNCH(3); break;
+		case 4: SPLIT_LAUNCH(4); break;
+		default: SPLIT_LAUNCH(5);
+		}
+#undef SPLIT_LAUNCH
+	}
+	if (leftSplits) *leftSplits = plan.splits;
+	if (plan.splits > 1 && !leftSplits) launch_splitk_reduce((const float *)ws, plan.splits, I, J, out);
+	return check_launch("conv_split_kernel");
+}
+
+// whether the forward product takes the same kernel, cut into as many ranges, in the first `less` bytes of a workspace as in all of it
+static bool pos_forward_fits_in(const fitre_conv_shape *s, const void *ws, size_t less, size_t wsBytes)
+{
+	const bool split = split_pos_chosen(s, false, ws, wsBytes);
+	if (split != split_pos_chosen(s, false, ws, less)) return false;
+	if (split) return split_pos_fit(s, false, ws, less, 1, false).splits == split_pos_fit(s, false, ws, wsBytes, 1, false).splits;
+	const BlockPlan plan = c3_pos_plan(s, false);
+	const long blocks = s->inChannels / kC3CB, J = (long)s->samples * s->inA * s->inB;
+	return fit_blocks(plan, blocks, s->outChannels, J, ws, less).splits == fit_blocks(plan, blocks, s->outChannels, J, ws, wsBytes).splits;
 }
 
 // x2 / delta2 (may be null): a second (input, delta) pair whose product is added to the first one's
@@ -577,8 +709,11 @@ extern "C" {
 size_t fitre_hip_conv_forward_workspace(const fitre_conv_shape *s)
 {
 	if (!s) return 0;
-	if (c3_pos_eligible(s, false)) return c3_pos_workspace(s, false);
-	return plan_gemm_workspace(s->outChannels, (long)s->samples * s->outA * s->outB, (long)s->inChannels * s->ksize * s->ksize, false, true);
+	const size_t split = split_pos_eligible(s, false) ? split_pos_workspace(s, false) : 0;
+	const size_t fp32 = c3_pos_eligible(s, false) ? c3_pos_workspace(s, false)
+	                                              : plan_gemm_workspace(s->outChannels, (long)s->samples * s->outA * s->outB,
+	                                                                    (long)s->inChannels * s->ksize * s->ksize, false, true);
+	return split > fp32 ? split : fp32;
 }
 
 int fitre_hip_conv_forward(const fitre_conv_shape *s, const float *x, const float *w, const float *bias, float *y, void *ws,
@@ -588,6 +723,7 @@ int fitre_hip_conv_forward(const fitre_conv_shape *s, const float *x, const floa
 	int rc = check_conv("fitre_hip_conv_forward", s);
 	if (rc) return rc;
 	FITRE_REQUIRE(x && w && y, "fitre_hip_conv_forward: null pointer");
+	if (split_pos_chosen(s, false, ws, wsBytes)) return launch_split_pos(s, false, x, w, bias, y, ws, wsBytes, nullptr, nullptr);
 	if (c3_pos_eligible(s, false)) return launch_c3_pos<false>(s, x, w, bias, y, ws, wsBytes);
 	ThinFwdPlan thin;
 	if (thin_fwd_chosen(s, 0.0, ws, wsBytes, thin)) return launch_thin_forward(s, thin, x, w, bias, y, nullptr);
@@ -632,7 +768,7 @@ int fitre_hip_conv_bn_act_pool_forward(const fitre_conv_shape *s, const float *x
 	FITRE_REQUIRE(!zhat || (mean && variance && runningMean && runningVariance), "fitre_hip_conv_bn_act_pool_forward: null statistics");
 	FITRE_REQUIRE(act_known(actFun), "fitre_hip_conv_bn_act_pool_forward: unknown activation code %d", actFun);
 	FITRE_REQUIRE(poolType == NO_POOL || poolOut, "fitre_hip_conv_bn_act_pool_forward: null pooled output");
-	const bool c3 = c3_pos_eligible(s, false);
+	const bool split = split_pos_chosen(s, false, ws, wsBytes), c3 = split || c3_pos_eligible(s, false);
 	ThinFwdPlan thin;
 	const bool unaligned = (((uintptr_t)y | (uintptr_t)actOut) & 15) != 0; // the engine's steps behind it are launches of their own
 	if (!zhat && !c3 && (poolType == MAX_POOL || poolType == AVG_POOL) && ksize == 2 && stride == 2 && padding == 0 && s->outA % 2 == 0 &&
@@ -665,9 +801,10 @@ int fitre_hip_conv_bn_act_pool_forward(const fitre_conv_shape *s, const float *x
 	}
 	// where the room of the sums would cost the product one of its ranges they are a pass of their own: the same ranges and
 	// the same bits as fitre_hip_conv_forward with this workspace
-	if (c3 && (at & 15) == 0 && perChannel % 4 == 0 && s->outChannels <= 65535 && c3_pos_fits_in(s, ws, convBytes, wsBytes)) {
+	if (c3 && (at & 15) == 0 && perChannel % 4 == 0 && s->outChannels <= 65535 && pos_forward_fits_in(s, ws, convBytes, wsBytes)) {
 		int splits = 1;
-		rc = launch_c3_pos<false>(s, x, w, bias, y, ws, convBytes, &splits);
+		rc = split ? launch_split_pos(s, false, x, w, bias, y, ws, convBytes, nullptr, &splits)
+		           : launch_c3_pos<false>(s, x, w, bias, y, ws, convBytes, &splits);
 		if (rc) return rc;
 		if (splits > 1) {
 			const SplitSource src{ (const float *)ws, splits, (long)s->outChannels * perChannel, bias, y, (double *)((char *)ws + convBytes) };
@@ -769,8 +906,11 @@ size_t fitre_hip_conv_input_grad_workspace(const fitre_conv_shape *s)
 		const size_t q = quad_input_grad_workspace(s), c = c3_pos_eligible(s, true) ? c3_pos_workspace(s, true) : 0;
 		return q > c ? q : c;
 	}
-	if (c3_pos_eligible(s, true)) return c3_pos_workspace(s, true);
-	return plan_gemm_workspace(s->inChannels, (long)s->samples * s->inA * s->inB, (long)s->outChannels * s->ksize * s->ksize, false, true);
+	const size_t split = split_pos_eligible(s, true) ? split_pos_workspace(s, true) : 0;
+	const size_t fp32 = c3_pos_eligible(s, true) ? c3_pos_workspace(s, true)
+	                                             : plan_gemm_workspace(s->inChannels, (long)s->samples * s->inA * s->inB,
+	                                                                   (long)s->outChannels * s->ksize * s->ksize, false, true);
+	return split > fp32 ? split : fp32;
 }
 
 int fitre_hip_conv_input_grad(const fitre_conv_shape *s, const float *delta, const float *w, float *dx, void *ws, size_t wsBytes)
@@ -784,6 +924,7 @@ int fitre_hip_conv_input_grad(const fitre_conv_shape *s, const float *delta, con
 	FITRE_REQUIRE(s->padding < s->ksize, "fitre_hip_conv_input_grad: padding %d >= window %d", s->padding, s->ksize);
 	if (quad_usable(s, ws, wsBytes, quad_input_grad_workspace(s)) && (((((uintptr_t)dx) | ((uintptr_t)delta) | ((uintptr_t)w)) & 15) == 0))
 		return quad_input_grad(s, delta, w, nullptr, dx, ws, wsBytes, nullptr, nullptr);
+	if (split_pos_chosen(s, true, ws, wsBytes)) return launch_split_pos(s, true, delta, w, nullptr, dx, ws, wsBytes, nullptr, nullptr);
 	if (c3_pos_eligible(s, true)) return launch_c3_pos<true>(s, delta, w, nullptr, dx, ws, wsBytes);
 	if (thin_dx_eligible(s)) return launch_thin_dx(s, delta, w, dx);
 	const int I = s->inChannels, J = s->samples * s->inA * s->inB, R = s->outChannels * s->ksize * s->ksize;
@@ -882,7 +1023,8 @@ size_t fitre_hip_conv_pair_workspace(const fitre_conv_shape *s, int kind)
 		const size_t nine = c3_dw_workspace(s, 2), dense = quad_eligible(s) ? quad_weight_grad_workspace(s) : 0;
 		return nine > dense ? nine : dense;
 	}
-	return c3_pos_workspace(s, kind == 1, 2);
+	const size_t fp32 = c3_pos_workspace(s, kind == 1, 2), split = split_pos_eligible(s, kind == 1) ? split_pos_workspace(s, kind == 1, 2) : 0;
+	return split > fp32 ? split : fp32;
 }
 
 int fitre_hip_conv_forward_pair(const fitre_conv_shape *s, const float *x1, const float *w1, const float *x2, const float *w2,
@@ -893,6 +1035,7 @@ int fitre_hip_conv_forward_pair(const fitre_conv_shape *s, const float *x1, cons
 	if (rc) return rc;
 	FITRE_REQUIRE(x1 && w1 && x2 && w2 && y, "fitre_hip_conv_forward_pair: null pointer");
 	if (!c3_pos_eligible(s, false)) return fail(FITRE_E_UNSUPPORTED, "fitre_hip_conv_forward_pair: only 3x3 windows with stride 1 and padding 1");
+	if (split_pos_chosen(s, false, ws, wsBytes, 2)) return launch_split_pos(s, false, x1, w1, bias, y, ws, wsBytes, nullptr, nullptr, x2, w2);
 	return launch_c3_pos<false>(s, x1, w1, bias, y, ws, wsBytes, nullptr, x2, w2);
 }
 
@@ -905,6 +1048,8 @@ int fitre_hip_conv_input_grad_pair(const fitre_conv_shape *s, const float *delta
 	FITRE_REQUIRE(delta1 && w1 && delta2 && w2 && dx, "fitre_hip_conv_input_grad_pair: null pointer");
 	if (s->stride != 1 || !c3_pos_eligible(s, true))
 		return fail(FITRE_E_UNSUPPORTED, "fitre_hip_conv_input_grad_pair: only 3x3 windows with stride 1 and padding 1");
+	if (split_pos_chosen(s, true, ws, wsBytes, 2))
+		return launch_split_pos(s, true, delta1, w1, nullptr, dx, ws, wsBytes, nullptr, nullptr, delta2, w2);
 	return launch_c3_pos<true>(s, delta1, w1, nullptr, dx, ws, wsBytes, nullptr, delta2, w2);
 }
 
@@ -925,7 +1070,8 @@ int fitre_hip_conv_weight_grad_pair(const fitre_conv_shape *s, const float *x1, 
 
 size_t fitre_hip_conv_input_grad_prepared_bytes(const fitre_conv_shape *s)
 {
-	return (s && quad_eligible(s)) ? quad_weff_bytes(s) : 0;
+	if (!s) return 0;
+	return quad_eligible(s) ? quad_weff_bytes(s) : (split_pos_eligible(s, true) ? split_weights_bytes(s, true) : 0);
 }
 
 int fitre_hip_conv_input_grad_prepare(const fitre_conv_shape *s, const float *w, void *prepared, size_t preparedBytes)
@@ -934,11 +1080,12 @@ int fitre_hip_conv_input_grad_prepare(const fitre_conv_shape *s, const float *w,
 	int rc = check_conv("fitre_hip_conv_input_grad_prepare", s);
 	if (rc) return rc;
 	FITRE_REQUIRE(w && prepared, "fitre_hip_conv_input_grad_prepare: null pointer");
-	if (!quad_eligible(s)) return fail(FITRE_E_UNSUPPORTED, "fitre_hip_conv_input_grad_prepare: nothing to prepare for this shape");
-	if (preparedBytes < quad_weff_bytes(s) || (((uintptr_t)prepared) & 15))
+	const size_t need = fitre_hip_conv_input_grad_prepared_bytes(s);
+	if (!need) return fail(FITRE_E_UNSUPPORTED, "fitre_hip_conv_input_grad_prepare: nothing to prepare for this shape");
+	if (preparedBytes < need || (((uintptr_t)prepared) & 15))
 		return fail(FITRE_E_WORKSPACE, "fitre_hip_conv_input_grad_prepare: buffer of %zu bytes is misaligned or smaller than the %zu required",
-		            preparedBytes, quad_weff_bytes(s));
-	return quad_prepare_weights(s, w, (float *)prepared);
+		            preparedBytes, need);
+	return quad_eligible(s) ? quad_prepare_weights(s, w, (float *)prepared) : launch_split_weights(s, true, w, (u32x4 *)prepared);
 }
 
 int fitre_hip_conv_input_grad_split_prepared(const fitre_conv_shape *s, const float *delta, const float *w, const void *prepared,
@@ -966,9 +1113,12 @@ int fitre_hip_conv_input_grad_split_prepared(const fitre_conv_shape *s, const fl
 		}
 		return FITRE_OK;
 	}
-	if (s->stride == 1 && s->padding < s->ksize && c3_pos_eligible(s, true)) {
+	const void *splitWeights = quad_eligible(s) ? nullptr : prepared;
+	const bool split = split_pos_chosen(s, true, ws, wsBytes, 1, splitWeights != nullptr);
+	if (split || (s->stride == 1 && s->padding < s->ksize && c3_pos_eligible(s, true))) {
 		int splits = 1;
-		rc = launch_c3_pos<true>(s, delta, w, nullptr, dx, ws, wsBytes, &splits);
+		rc = split ? launch_split_pos(s, true, delta, w, nullptr, dx, ws, wsBytes, splitWeights, &splits)
+		           : launch_c3_pos<true>(s, delta, w, nullptr, dx, ws, wsBytes, &splits);
 		if (rc) return rc;
 		if (splits > 1) {
 			view->base = (float *)ws;

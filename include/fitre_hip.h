@@ -112,8 +112,8 @@ int fitre_hip_profile_read(int kernelClass, long *launches, double *milliseconds
  * 6 and 7 are the 3x3 convolution kernels that leave out the arithmetic on the padding: 6 = the dense per-image form
  * on 2x2 maps, 7 = the cell form on 4x4 maps, 8 = the cell form of the weight gradient on 8x8 maps (their work is
  * still counted as the nine-tap 2*M*K*Cout); 9 = the weight gradient of a wide linear layer at a batch of at most 64
- * (the whole reduction in registers). */
-#define FITRE_TILE_VARIANTS 10
+ * (the whole reduction in registers); 10 = fp32 products as six bf16 matrix products. */
+#define FITRE_TILE_VARIANTS 11
 int fitre_hip_profile_read_tile(int kernelClass, int tile, long *launches, double *milliseconds, double *work);
 /* The accounted launches one by one, in issue order since the last fitre_hip_profile_enable(1) (at most 65 536
  * are kept): class, tile variant, duration and algorithmic work of launch `index` < *count. */
@@ -433,7 +433,7 @@ int fitre_hip_conv_input_grad_split(const fitre_conv_shape *s, const float *delt
 /* Some shapes multiply by a rearranged copy of the weights (3x3 windows on 2 x 2 maps: the dense per-image form
  * of the convolution, 16/36 of the multiply-adds of the nine-tap form).  The copy depends on the weights only, so
  * a caller can have it made ahead of the chain that needs it, on another lane:
- *   _prepared_bytes  size of the copy, 0 when the shape has none;
+ *   _prepared_bytes  size of the copy, 0 when the shape has none (it does not depend on the number of samples);
  *   _prepare         builds it (stream-ordered);
  *   _split_prepared  fitre_hip_conv_input_grad_split reading it (prepared == NULL: built inside, in ws).
  * No counterpart in the reference, whose weights are reordered per call (dev_backprop_convolution.cu:140-156). */
