@@ -6,6 +6,7 @@
 #include "conv_common.h"
 #include "conv_quad.h"
 #include "conv_split.h"
+#include "conv_split_dw.h"
 #include "conv_thin.h"
 #include "conv_thin_forward.h"
 #include "linear_small.h"
@@ -461,6 +462,123 @@ static int launch_c3_dw(const fitre_conv_shape *s, const float *x, const float *
 	return check_launch("conv3x3_dw_kernel");
 }
 
+// ---- weight gradient of 3x3 and 5x5 windows on the bf16 pipes (conv_split_dw.h) ------------------------------------------------
+struct SplitDwShape {
+	int mode, logGroups; // how a row is cut into groups of eight cells
+	int ob, wo, wc;      // blocks of 32 output channels of a wave; waves along the output and input channels
+	int rowTiles() const { return 32 * ob * wo; }
+	int tiles, stages;   // workgroups of a range; stages of the tap row with the most image rows
+};
+static bool split_dw_shape(const fitre_conv_shape *s, SplitDwShape &d)
+{
+	if ((s->ksize != 3 && s->ksize != 5) || s->stride != 1 || s->padding != s->ksize / 2 || s->inChannels <= 16 || s->outChannels < 32) return false;
+	const int B = s->inB;
+	// a row's last group is filled up with zeros: three quarters of the groups' cells are real at least
+	if (B < 3 || B > 32 || (B == 5 || (B > 8 && B < 12) || (B > 16 && B < 24)) || (B <= 4 && s->ksize != 3)) return false;
+	d.mode = B <= 4 ? kRowsPaired : (B <= 8 ? kRowsWhole : kRowsCut);
+	d.logGroups = B <= 8 ? 0 : (B <= 16 ? 1 : 2);
+	// 5 x 5 windows: ten accumulators a wave leave no room for more than 64 input channels; with at most 64 output channels five
+	// (64 -> 64, 15 x 15, 100 images: 66 us with ten in two waves, 45 with five in four)
+	d.ob = s->ksize == 5 && s->outChannels <= 64 ? 1 : 2;
+	d.wo = s->outChannels <= 64 && d.ob == 2 ? 1 : 2;
+	d.wc = s->inChannels <= 64 || s->ksize == 5 ? 2 : 4;
+	d.tiles = s->ksize * ((s->inChannels + 32 * d.wc - 1) / (32 * d.wc)) * ((s->outChannels + d.rowTiles() - 1) / d.rowTiles());
+	const long rows = (long)s->samples * s->inA, groups = d.mode == kRowsPaired ? (rows + 1) / 2 : rows << d.logGroups;
+	d.stages = (int)((groups + kSplitDwGroups - 1) / kSplitDwGroups);
+	return true;
+}
+static size_t split_dw_range_bytes(const fitre_conv_shape *s) { return sizeof(float) * (size_t)s->outChannels * s->inChannels * s->ksize * s->ksize; }
+static BlockPlan split_dw_plan(const fitre_conv_shape *s, const SplitDwShape &d, int cus = 0, int pairs = 1)
+{
+	if (cus <= 0) cus = weight_grad_units();
+	// measured, us a stage and workgroup with the compute units full
+	const int waves = d.wo * d.wc;
+	const double stageUs = waves == 8 ? 3.8 : (waves == 2 ? 1.1 : (s->ksize == 3 ? 2.05 : (d.ob == 2 ? 2.57 : 1.9)));
+	const int resident = waves == 8 || d.ob == 1 ? 1 : (waves == 4 ? 2 : 3); // from how many on more of them add nothing
+	BlockPlan plan = plan_blocks(d.tiles, (long)pairs * d.stages, 0.85 * stageUs, resident, s->outChannels, (long)s->inChannels * s->ksize * s->ksize, cus);
+	plan.wsBytes = plan.splits * split_dw_range_bytes(s); // an uncut product's partial sums are put in order by the reduction as well
+	return plan;
+}
+static size_t split_dw_workspace(const fitre_conv_shape *s, int pairs = 1)
+{
+	SplitDwShape d;
+	if (!split_dw_shape(s, d)) return 0;
+	size_t need = split_dw_plan(s, d, device_compute_units(), pairs).wsBytes;
+	for (int eighths = 4; eighths <= 8; eighths++) {
+		const size_t c = split_dw_plan(s, d, share_of_units(lane_compute_units_min(), eighths), pairs).wsBytes;
+		need = need > c ? need : c;
+	}
+	return need;
+}
+// From how many multiply-adds on, against the 3 x 3 kernels (whole stages of 64 positions) and the tile engine.  fp32 / split, us,
+// with the reduction: 64 -> 64 channels, 16 x 16 maps, 16 images (1.5e8) 28 / 18; 256 -> 256, 4 x 4, 16 images (1.5e8) 25.5 / 23.3;
+// 512 -> 512, 4 x 4, 4 images (1.5e8, 64 positions) 18.5 / 25; engine: 64 -> 64, 13 x 13, 40 images (2.5e8) 21.3 / 22.2, 128 -> 128,
+// 13 x 13, 16 images (4e8) 29.3 / 29.8, 77 images (1.9e9) 63 / 42; 5 x 5: 64 -> 192, 15 x 15, 4 images (2.8e8) 27.1 / 26.8, 128 ->
+// 128, 8 x 8, 16 images (4.2e8) 29.2 / 29.3, 64 -> 192, 27 x 27, 16 images (3.6e9) 109 / 73.
+constexpr double kSplitDwWork = 1.2e8, kSplitDwEngineWork = 4.5e8;
+constexpr long kSplitDwPositions = 256;
+static bool split_dw_chosen(const fitre_conv_shape *s, const void *ws, size_t wsBytes, int pairs, SplitDwShape &d, BlockPlan &plan)
+{
+	if (!ws || (((uintptr_t)ws) & 3) || !split_dw_shape(s, d)) return false;
+	if (s->ksize == 5 && (s->inChannels <= 32 || s->outChannels <= 32)) return false; // half a tile
+	if ((long)s->samples * s->inA * s->inB < kSplitDwPositions) return false;
+	if (0.5 * pairs * conv_flops(s) < (c3_dw_eligible(s) ? kSplitDwWork : kSplitDwEngineWork)) return false;
+	plan = split_dw_plan(s, d, 0, pairs);
+	// a workspace for less than half of the ranges: longer sums than the fp32 kernels', and a chip that is not full
+	const long fit = (long)(wsBytes / split_dw_range_bytes(s));
+	if (2 * fit < plan.splits) return false;
+	if (fit < plan.splits) {
+		plan.perSplit = (int)((pairs * (long)d.stages + fit - 1) / fit);
+		plan.splits = (int)((pairs * (long)d.stages + plan.perSplit - 1) / plan.perSplit);
+	}
+	return true;
+}
+static int launch_split_dw(const fitre_conv_shape *s, const SplitDwShape &d, const BlockPlan &plan, const float *x, const float *delta, float *dW,
+                           void *ws, const float *x2 = nullptr, const float *delta2 = nullptr)
+{
+	const int J = s->samples * s->inA * s->inB;
+	ConvSplitDwParams p{};
+	p.x = x, p.delta = delta, p.x2 = x2, p.delta2 = delta2;
+	p.xBytes = (uint32_t)((size_t)s->inChannels * J * sizeof(float)), p.deltaBytes = (uint32_t)((size_t)s->outChannels * J * sizeof(float));
+	p.I = s->outChannels, p.cin = s->inChannels, p.J = J, p.A = s->inA, p.B = s->inB, p.samples = s->samples;
+	p.logGroups = d.logGroups, p.stages = d.stages, p.perSplit = plan.perSplit;
+	p.cTiles = (s->inChannels + 32 * d.wc - 1) / (32 * d.wc);
+	p.partial = (float *)ws;
+	for (int i = 0; i < 3; i++) p.divLive[i] = FastDiv((uint32_t)(s->inA > i ? s->inA - i : 1));
+	const dim3 grid((unsigned)(p.cTiles * s->ksize), (unsigned)((s->outChannels + d.rowTiles() - 1) / d.rowTiles()), (unsigned)plan.splits);
+	if (grid.y > 65535 || grid.z > 65535) return fail(FITRE_E_UNSUPPORTED, "conv_split_dw_kernel grid too large");
+	{
+		LaunchScope scope(FITRE_KC_CONV_DW, (x2 ? 2 : 1) * conv_flops(s), kTileSplit);
+#define SPLIT_DW_LAUNCH(KS, M, B_, O, C_) conv_split_dw_kernel<KS, M, B_, O, C_><<<grid, 64 * O * C_, 0, stream()>>>(p)
+#define SPLIT_DW_MODES(O, C_)                                                                                         \
+	{                                                                                                                 \
+		if (d.mode == kRowsPaired) SPLIT_DW_LAUNCH(3, kRowsPaired, 2, O, C_);                                         \
+		else if (d.mode == kRowsWhole) SPLIT_DW_LAUNCH(3, kRowsWhole, 2, O, C_);                                      \
+		else SPLIT_DW_LAUNCH(3, kRowsCut, 2, O, C_);                                                                  \
+	}
+		if (s->ksize == 3) {
+			if (d.wo == 2 && d.wc == 4) SPLIT_DW_MODES(2, 4)
+			else if (d.wo == 2) SPLIT_DW_MODES(2, 2)
+			else if (d.wc == 4) SPLIT_DW_MODES(1, 4)
+			else SPLIT_DW_MODES(1, 2)
+		} else if (d.ob == 2) {
+			if (d.mode == kRowsWhole) SPLIT_DW_LAUNCH(5, kRowsWhole, 2, 2, 2);
+			else SPLIT_DW_LAUNCH(5, kRowsCut, 2, 2, 2);
+		} else {
+			if (d.mode == kRowsWhole) SPLIT_DW_LAUNCH(5, kRowsWhole, 1, 2, 2);
+			else SPLIT_DW_LAUNCH(5, kRowsCut, 1, 2, 2);
+		}
+#undef SPLIT_DW_MODES
+#undef SPLIT_DW_LAUNCH
+	}
+	const int products = s->outChannels * s->inChannels;
+	const dim3 blocks((unsigned)((products + 63) / 64), (unsigned)s->ksize);
+	LaunchScope scope(FITRE_KC_SPLITK_REDUCE, (double)(plan.splits + 1) * split_dw_range_bytes(s));
+	if (s->ksize == 3) split_dw_reduce_kernel<3><<<blocks, 256, 0, stream()>>>((const float *)ws, plan.splits, products, dW);
+	else split_dw_reduce_kernel<5><<<blocks, 256, 0, stream()>>>((const float *)ws, plan.splits, products, dW);
+	return check_launch("conv_split_dw_kernel");
+}
+
 // ---- 3x3 weight gradient with very few input channels (first layer) ----------------------------
 static bool thin_dw_eligible(const fitre_conv_shape *s)
 {
@@ -830,9 +948,8 @@ int fitre_hip_conv_act_pool_forward(const fitre_conv_shape *s, const float *x, c
 }
 
 // ---- weight gradient: I = Cout, J = Cin*k*k, R = positions -------------------
-size_t fitre_hip_conv_weight_grad_workspace(const fitre_conv_shape *s)
+static size_t weight_grad_fp32_workspace(const fitre_conv_shape *s)
 {
-	if (!s) return 0;
 	if (quad_eligible(s)) {
 		const size_t q = quad_weight_grad_workspace(s), c = c3_dw_eligible(s) ? c3_dw_workspace(s) : 0;
 		return q > c ? q : c;
@@ -842,6 +959,13 @@ size_t fitre_hip_conv_weight_grad_workspace(const fitre_conv_shape *s)
 	if (thin_dw_eligible(s) && thin_dw_workspace(s) > general) general = thin_dw_workspace(s);
 	if (thin_dw_general_eligible(s) && thin_dw_general_workspace(s) > general) general = thin_dw_general_workspace(s);
 	return general;
+}
+
+size_t fitre_hip_conv_weight_grad_workspace(const fitre_conv_shape *s)
+{
+	if (!s) return 0;
+	const size_t fp32 = weight_grad_fp32_workspace(s), split = split_dw_workspace(s);
+	return fp32 > split ? fp32 : split;
 }
 
 int fitre_hip_conv_weight_grad_runs_beside(const fitre_conv_shape *s)
@@ -860,6 +984,9 @@ int fitre_hip_conv_weight_grad(const fitre_conv_shape *s, const float *x, const 
 	FITRE_REQUIRE(x && delta && dW, "fitre_hip_conv_weight_grad: null pointer");
 	if (quad_usable(s, ws, wsBytes, quad_weight_grad_workspace(s)) && (((((uintptr_t)x) | ((uintptr_t)delta)) & 15) == 0))
 		return quad_weight_grad(s, x, delta, dW, ws, wsBytes);
+	SplitDwShape split;
+	BlockPlan splitPlan;
+	if (split_dw_chosen(s, ws, wsBytes, 1, split, splitPlan)) return launch_split_dw(s, split, splitPlan, x, delta, dW, ws);
 	if (c3_dw_eligible(s)) return launch_c3_dw(s, x, delta, dW, ws, wsBytes);
 	if (thin_dw_eligible(s) && ws && wsBytes >= thin_dw_workspace(s) && ((((uintptr_t)delta) | ((uintptr_t)ws)) & 15) == 0)
 		return launch_thin_dw(s, x, delta, dW, ws);
@@ -1020,8 +1147,8 @@ size_t fitre_hip_conv_pair_workspace(const fitre_conv_shape *s, int kind)
 {
 	if (!fitre_hip_conv_pair_supported(s, kind)) return 0;
 	if (kind == 2) {
-		const size_t nine = c3_dw_workspace(s, 2), dense = quad_eligible(s) ? quad_weight_grad_workspace(s) : 0;
-		return nine > dense ? nine : dense;
+		const size_t nine = c3_dw_workspace(s, 2), dense = quad_eligible(s) ? quad_weight_grad_workspace(s) : 0, split = split_dw_workspace(s, 2);
+		return nine > dense ? (nine > split ? nine : split) : (dense > split ? dense : split);
 	}
 	const size_t fp32 = c3_pos_workspace(s, kind == 1, 2), split = split_pos_eligible(s, kind == 1) ? split_pos_workspace(s, kind == 1, 2) : 0;
 	return split > fp32 ? split : fp32;
@@ -1065,6 +1192,9 @@ int fitre_hip_conv_weight_grad_pair(const fitre_conv_shape *s, const float *x1, 
 	if (quad_usable(s, ws, wsBytes, quad_weight_grad_workspace(s)) &&
 	    (((((uintptr_t)x1) | ((uintptr_t)delta1) | ((uintptr_t)x2) | ((uintptr_t)delta2)) & 15) == 0))
 		return quad_weight_grad(s, x1, delta1, dW, ws, wsBytes, x2, delta2);
+	SplitDwShape split;
+	BlockPlan splitPlan;
+	if (split_dw_chosen(s, ws, wsBytes, 2, split, splitPlan)) return launch_split_dw(s, split, splitPlan, x1, delta1, dW, ws, x2, delta2);
 	return launch_c3_dw(s, x1, delta1, dW, ws, wsBytes, x2, delta2);
 }
 

@@ -165,3 +165,90 @@ def test_numbers_the_split_does_not_carry(dev, which):
     np.testing.assert_array_equal(got[:, far_off], plain[:, far_off])
     small = source * 2.0**-108
     assert far(conv(dev, case, which, small, w) * 2.0**108, reference(case, which, source, w)) < limit(terms, 0.6)
+
+
+def weight_grad(dev, case, x, d, second=None, ws_bytes=None):
+    n, ci, co, a, b, k = case
+    shape = conv_shape(n, ci, co, a, b, k, 1, k // 2)
+    nb = hip.fitre_hip_conv_pair_workspace(C.byref(shape), 2) if second else hip.fitre_hip_conv_weight_grad_workspace(C.byref(shape))
+    nb = nb if ws_bytes is None else ws_bytes(nb)
+    bufs = [dev.upload(flat(t)) for t in (x, d) + (second or ())] + [dev.alloc(nb), dev.zeros(co * ci * k * k)]
+    ws, out = bufs[-2:]
+    if second:
+        L.check(hip.fitre_hip_conv_weight_grad_pair(C.byref(shape), *bufs[:4], out, ws, nb))
+    else:
+        L.check(hip.fitre_hip_conv_weight_grad(C.byref(shape), *bufs[:2], out, ws, nb))
+    got = dev.download(out, co * ci * k * k).reshape(co, ci, k, k)
+    for q in bufs:
+        dev.free(q)
+    return got
+
+
+def weight_reference(case, x, d):
+    k = case[5]
+    return torch.nn.grad.conv2d_weight(x.double(), (case[2], case[1], k, k), d.double(), padding=k // 2).numpy()
+
+
+# the three ways a row is cut into groups, every arrangement of waves, partial tiles of either kind of channels, and numbers of
+# image rows that are no whole groups or stages
+WEIGHT_CASES = [
+    (75, 256, 272, 4, 4, 3),   # two rows a group
+    (61, 200, 264, 5, 3, 3),   # rows of three cells, an odd number of rows
+    (128, 64, 64, 4, 4, 3),    # 64 x 64 tiles
+    (17, 160, 144, 8, 8, 3),   # a row a group
+    (43, 72, 130, 7, 6, 3),
+    (32, 40, 48, 8, 8, 3),
+    (41, 130, 64, 9, 7, 3),    # 64 x 128 tiles
+    (23, 64, 192, 13, 13, 3),  # two groups a row, the second five cells
+    (9, 100, 70, 16, 16, 3),
+    (5, 96, 128, 12, 32, 3),   # four groups a row
+    (4, 64, 128, 27, 27, 3),
+    (7, 128, 64, 11, 24, 3),   # three of four groups
+    (12, 64, 192, 13, 13, 5),  # 5 x 5 windows
+    (9, 80, 160, 15, 8, 5),
+    (4, 64, 96, 20, 30, 5),
+    (20, 72, 64, 15, 14, 5),   # at most 64 output channels
+    (50, 48, 40, 8, 8, 5),
+    (60, 64, 64, 2, 16, 5),    # fewer image rows than the window
+]
+
+
+@pytest.mark.parametrize("case", WEIGHT_CASES)
+def test_weight_gradient(dev, case):
+    x, _, d = tensors(case)
+    assert far(weight_grad(dev, case, x, d), weight_reference(case, x, d)) < limit(case[0] * case[3] * case[4])
+
+
+def test_weight_gradient_of_a_pair(dev):
+    case = (19, 128, 128, 8, 8, 3)
+    (x, _, d), (x2, _, d2) = tensors(case), tensors(case, 1)
+    got = weight_grad(dev, case, x, d, second=(x2, d2))
+    assert far(got, weight_reference(case, x, d) + weight_reference(case, x2, d2)) < limit(2 * 19 * 64)
+
+
+def test_weight_gradient_in_smaller_workspaces(dev):
+    """Fewer reduction ranges, and (room for less than half of them) the fp32 kernels."""
+    case = (64, 128, 128, 8, 8, 3)
+    x, _, d = tensors(case)
+    want, one = weight_reference(case, x, d), 4 * 128 * 128 * 9
+    for ws_bytes in (lambda nb: nb - one, lambda nb: nb * 3 // 4, lambda nb: 3 * one, lambda nb: 4):
+        assert far(weight_grad(dev, case, x, d, ws_bytes=ws_bytes), want) < limit(64 * 64)
+
+
+@pytest.mark.parametrize("case", [(64, 128, 128, 8, 8, 3), (40, 128, 256, 4, 4, 3), (20, 64, 128, 16, 16, 3), (20, 64, 64, 15, 15, 5)])
+def test_numbers_the_split_does_not_carry_in_a_weight_gradient(dev, case):
+    x, _, d = tensors(case)
+    terms = case[0] * case[3] * case[4]
+    odd, odd_d = x.clone(), d.clone()
+    odd[1, 5, 2, 2], odd[2, 9, 0, 3], odd_d[3, 7, 2, 1] = float("inf"), float(np.finfo(np.float32).max), float("nan")
+    odd_d[2] *= 0.05  # no product with the largest float overflows
+    got, want = weight_grad(dev, case, odd, odd_d), weight_reference(case, odd, odd_d)
+    # (every tap at these cells is inside the image: what is multiplied with padding is not the question here)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(want))
+    np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    huge = np.isfinite(want) & (np.abs(want) > 1e30)
+    rest = np.isfinite(want) & ~huge
+    assert huge.any() and far(got[huge] * 1e-35, want[huge] * 1e-35) < limit(terms)
+    assert far(got[rest], want[rest]) < limit(terms, 0.6)
+    assert far(weight_grad(dev, case, x, d * 2.0**-108) * 2.0**108, weight_reference(case, x, d)) < limit(terms, 0.6)
