@@ -465,7 +465,7 @@ static int launch_c3_dw(const fitre_conv_shape *s, const float *x, const float *
 // ---- weight gradient of 3x3 and 5x5 windows on the bf16 pipes (conv_split_dw.h) ------------------------------------------------
 struct SplitDwShape {
 	int mode, logGroups; // how a row is cut into groups of eight cells
-	int ob, wo, wc;      // blocks of 32 output channels of a wave; waves along the output and input channels
+	int ob, wo;          // blocks of 32 output channels of a wave; waves along them (two along the input channels)
 	int rowTiles() const { return 32 * ob * wo; }
 	int tiles, stages;   // workgroups of a range; stages of the tap row with the most image rows
 };
@@ -477,12 +477,11 @@ static bool split_dw_shape(const fitre_conv_shape *s, SplitDwShape &d)
 	if (B < 3 || B > 32 || (B == 5 || (B > 8 && B < 12) || (B > 16 && B < 24)) || (B <= 4 && s->ksize != 3)) return false;
 	d.mode = B <= 4 ? kRowsPaired : (B <= 8 ? kRowsWhole : kRowsCut);
 	d.logGroups = B <= 8 ? 0 : (B <= 16 ? 1 : 2);
-	// 5 x 5 windows: ten accumulators a wave leave no room for more than 64 input channels; with at most 64 output channels five
-	// (64 -> 64, 15 x 15, 100 images: 66 us with ten in two waves, 45 with five in four)
+	// 5 x 5 windows with at most 64 output channels: 64 -> 64, 15 x 15, 100 images 66 us with ten accumulators in each of two
+	// waves, 45 with five in four
 	d.ob = s->ksize == 5 && s->outChannels <= 64 ? 1 : 2;
 	d.wo = s->outChannels <= 64 && d.ob == 2 ? 1 : 2;
-	d.wc = s->inChannels <= 64 || s->ksize == 5 ? 2 : 4;
-	d.tiles = s->ksize * ((s->inChannels + 32 * d.wc - 1) / (32 * d.wc)) * ((s->outChannels + d.rowTiles() - 1) / d.rowTiles());
+	d.tiles = s->ksize * ((s->inChannels + 63) / 64) * ((s->outChannels + d.rowTiles() - 1) / d.rowTiles());
 	const long rows = (long)s->samples * s->inA, groups = d.mode == kRowsPaired ? (rows + 1) / 2 : rows << d.logGroups;
 	d.stages = (int)((groups + kSplitDwGroups - 1) / kSplitDwGroups);
 	return true;
@@ -492,9 +491,8 @@ static BlockPlan split_dw_plan(const fitre_conv_shape *s, const SplitDwShape &d,
 {
 	if (cus <= 0) cus = weight_grad_units();
 	// measured, us a stage and workgroup with the compute units full
-	const int waves = d.wo * d.wc;
-	const double stageUs = waves == 8 ? 3.8 : (waves == 2 ? 1.1 : (s->ksize == 3 ? 2.05 : (d.ob == 2 ? 2.57 : 1.9)));
-	const int resident = waves == 8 || d.ob == 1 ? 1 : (waves == 4 ? 2 : 3); // from how many on more of them add nothing
+	const double stageUs = d.wo == 1 ? 1.1 : (s->ksize == 3 ? 2.05 : (d.ob == 2 ? 2.57 : 1.9));
+	const int resident = d.wo == 1 ? 3 : (d.ob == 1 ? 1 : 2); // from how many on more of them add nothing
 	BlockPlan plan = plan_blocks(d.tiles, (long)pairs * d.stages, 0.85 * stageUs, resident, s->outChannels, (long)s->inChannels * s->ksize * s->ksize, cus);
 	plan.wsBytes = plan.splits * split_dw_range_bytes(s); // an uncut product's partial sums are put in order by the reduction as well
 	return plan;
@@ -542,31 +540,29 @@ static int launch_split_dw(const fitre_conv_shape *s, const SplitDwShape &d, con
 	p.xBytes = (uint32_t)((size_t)s->inChannels * J * sizeof(float)), p.deltaBytes = (uint32_t)((size_t)s->outChannels * J * sizeof(float));
 	p.I = s->outChannels, p.cin = s->inChannels, p.J = J, p.A = s->inA, p.B = s->inB, p.samples = s->samples;
 	p.logGroups = d.logGroups, p.stages = d.stages, p.perSplit = plan.perSplit;
-	p.cTiles = (s->inChannels + 32 * d.wc - 1) / (32 * d.wc);
+	p.cTiles = (s->inChannels + 63) / 64;
 	p.partial = (float *)ws;
 	for (int i = 0; i < 3; i++) p.divLive[i] = FastDiv((uint32_t)(s->inA > i ? s->inA - i : 1));
 	const dim3 grid((unsigned)(p.cTiles * s->ksize), (unsigned)((s->outChannels + d.rowTiles() - 1) / d.rowTiles()), (unsigned)plan.splits);
 	if (grid.y > 65535 || grid.z > 65535) return fail(FITRE_E_UNSUPPORTED, "conv_split_dw_kernel grid too large");
 	{
 		LaunchScope scope(FITRE_KC_CONV_DW, (x2 ? 2 : 1) * conv_flops(s), kTileSplit);
-#define SPLIT_DW_LAUNCH(KS, M, B_, O, C_) conv_split_dw_kernel<KS, M, B_, O, C_><<<grid, 64 * O * C_, 0, stream()>>>(p)
-#define SPLIT_DW_MODES(O, C_)                                                                                         \
+#define SPLIT_DW_LAUNCH(KS, M, B_, O) conv_split_dw_kernel<KS, M, B_, O, 2><<<grid, 128 * O, 0, stream()>>>(p)
+#define SPLIT_DW_MODES(O)                                                                                             \
 	{                                                                                                                 \
-		if (d.mode == kRowsPaired) SPLIT_DW_LAUNCH(3, kRowsPaired, 2, O, C_);                                         \
-		else if (d.mode == kRowsWhole) SPLIT_DW_LAUNCH(3, kRowsWhole, 2, O, C_);                                      \
-		else SPLIT_DW_LAUNCH(3, kRowsCut, 2, O, C_);                                                                  \
+		if (d.mode == kRowsPaired) SPLIT_DW_LAUNCH(3, kRowsPaired, 2, O);                                             \
+		else if (d.mode == kRowsWhole) SPLIT_DW_LAUNCH(3, kRowsWhole, 2, O);                                          \
+		else SPLIT_DW_LAUNCH(3, kRowsCut, 2, O);                                                                      \
 	}
 		if (s->ksize == 3) {
-			if (d.wo == 2 && d.wc == 4) SPLIT_DW_MODES(2, 4)
-			else if (d.wo == 2) SPLIT_DW_MODES(2, 2)
-			else if (d.wc == 4) SPLIT_DW_MODES(1, 4)
-			else SPLIT_DW_MODES(1, 2)
+			if (d.wo == 2) SPLIT_DW_MODES(2)
+			else SPLIT_DW_MODES(1)
 		} else if (d.ob == 2) {
-			if (d.mode == kRowsWhole) SPLIT_DW_LAUNCH(5, kRowsWhole, 2, 2, 2);
-			else SPLIT_DW_LAUNCH(5, kRowsCut, 2, 2, 2);
+			if (d.mode == kRowsWhole) SPLIT_DW_LAUNCH(5, kRowsWhole, 2, 2);
+			else SPLIT_DW_LAUNCH(5, kRowsCut, 2, 2);
 		} else {
-			if (d.mode == kRowsWhole) SPLIT_DW_LAUNCH(5, kRowsWhole, 1, 2, 2);
-			else SPLIT_DW_LAUNCH(5, kRowsCut, 1, 2, 2);
+			if (d.mode == kRowsWhole) SPLIT_DW_LAUNCH(5, kRowsWhole, 1, 2);
+			else SPLIT_DW_LAUNCH(5, kRowsCut, 1, 2);
 		}
 #undef SPLIT_DW_MODES
 #undef SPLIT_DW_LAUNCH

@@ -72,9 +72,13 @@ __device__ __forceinline__ void split_dw_exact_tile(const ConvSplitDwParams &p, 
 	}
 }
 
-// OB: blocks of 32 output channels of a wave
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Wpass-failed" // three waves a SIMD: what bounds the registers, where LDS has room for two
+// OB: blocks of 32 output channels of a wave.  3 x 3 windows: held to 168 registers where the compiler would take 249 (same time
+// alone: 103 us for 256 -> 256 channels on 8 x 8 maps): two workgroups on a compute unit leave 176 on every SIMD, on which the
+// bandwidth kernels of the layer below run.
 template <int KS, int MODE, int OB, int WO, int WC>
-__global__ void __launch_bounds__(64 * WO *WC, 2)
+__global__ void __launch_bounds__(64 * WO *WC, KS == 3 ? 3 : 2)
 conv_split_dw_kernel(const ConvSplitDwParams p)
 {
 	FITRE_RAISE_MATRIX_WAVE_PRIORITY();
@@ -312,6 +316,8 @@ conv_split_dw_kernel(const ConvSplitDwParams p)
 				if (o < p.I) partial[((size_t)(ta * KS + t) * p.I + o) * p.cin + c] = acc[b][t][v];
 			}
 }
+
+#pragma clang diagnostic pop
 
 // dW[o][c][tap] = sum over the ranges, in order.  64 (o, c) x four phases a workgroup; a phase adds every fourth range, the
 // phases are added in order.  blockIdx.y: tap row.
