@@ -16,15 +16,15 @@ constexpr int kWave = 64;
 void set_error(const char *fmt, ...);
 int fail(int code, const char *fmt, ...);
 hipStream_t stream(); // the selected lane
-// Column-major product C(MxN) = alpha*op(A)*op(B) + beta*C on the tile engine (defined with
-// fitre_hip_gemm).  flags: kGemmMirror = the product is symmetric (M == N, same operand on
+// Column-major product C(MxN) = alpha*op(A)*op(B) + beta*C (+ bias per row) on the bf16 pipes (defined with fitre_hip_gemm).
+int gemm_ex(int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb,
+            float beta, float *C, int ldc, const float *bias, int kernelClass, void *ws, size_t wsBytes);
+// Flags of the products on the fp32 tile engine: kGemmMirror = the product is symmetric (M == N, same operand on
 // both sides): compute the tiles on and above the diagonal and mirror them; kGemmTriK = both
 // operands are zero where the reduction index is below their row / column index.
 // kGemmBLowerTri / kGemmBUpperTri: op(B) (K x N) is zero above / below its diagonal; kGemmALowerTri: op(A) (M x K) is zero
 // above its diagonal -- the reduction skips the zero part (batched products only).
 constexpr int kGemmMirror = 1, kGemmTriK = 2, kGemmBLowerTri = 4, kGemmBUpperTri = 8, kGemmALowerTri = 16;
-int gemm_ex(int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb,
-            float beta, float *C, int ldc, const float *bias, int flags, int kernelClass, void *ws, size_t wsBytes);
 size_t gemm_ex_workspace(int M, int N, int K, int flags);
 // `batch` such products of one shape in one launch (plus one reduction launch when split).  Problem b reads
 // A + b*strideA, B + b*strideB, writes C + b*strideC and keeps its split-K partials in (char *)ws + b*wsStrideBytes;

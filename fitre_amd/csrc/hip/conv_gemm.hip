@@ -308,9 +308,15 @@ static size_t split_pos_room(const fitre_conv_shape *s, bool dx, const void *ws,
 // 25.6 / 30.3, 256 (2.4e9) 43 / 37; 32 x 32, 40 images (1.5e9) 46 / 34.  Whole tiles of 4 x 4 maps have the cell form to beat:
 // 256 -> 256, 128 images (1.2e9) 34.3 / 36.4, 256 (2.4e9) 45.4 / 44.5; 512 -> 512, 256 (9.7e9) 123 / 102.
 constexpr double kSplitWork = 7.0e8, kSplitNarrowWork = 1.5e9, kSplitCellWork = 2.0e9;
+// The gradients only from so many positions on.  A layer with fewer positions than a patch has entries has a weight gradient in the
+// span of its patches; what rounding adds outside of it, the curvature passes multiply by the inverse of the damping.  With these
+// kernels, whose rounding is no larger but another, VGG-11's natural gradient at 32 images (512 positions of 512 channels) moves
+// by 2.8e-4 of its norm, at 64 by 2e-5, at 96 by 1e-5, from 128 images (2048 positions) on by less than 7e-6.
+constexpr long kSplitGradPositions = 2048;
 static bool split_pos_chosen(const fitre_conv_shape *s, bool dx, const void *ws, size_t wsBytes, int pairs = 1, bool prepared = false)
 {
 	if (!split_pos_eligible(s, dx) || split_pos_room(s, dx, ws, wsBytes, pairs, prepared) == 0) return false;
+	if (dx && (long)s->samples * s->inA * s->inB < kSplitGradPositions) return false;
 	const int I = dx ? s->inChannels : s->outChannels;
 	const double least = cell_pos_eligible(s, dx) ? kSplitCellWork : (s->ksize == 3 && I <= 64 ? kSplitNarrowWork : kSplitWork);
 	return 0.5 * pairs * conv_flops(s) >= least;
@@ -509,17 +515,16 @@ static size_t split_dw_workspace(const fitre_conv_shape *s, int pairs = 1)
 	return need;
 }
 // From how many multiply-adds on, against the 3 x 3 kernels (whole stages of 64 positions) and the tile engine.  fp32 / split, us,
-// with the reduction: 64 -> 64 channels, 16 x 16 maps, 16 images (1.5e8) 28 / 18; 256 -> 256, 4 x 4, 16 images (1.5e8) 25.5 / 23.3;
-// 512 -> 512, 4 x 4, 4 images (1.5e8, 64 positions) 18.5 / 25; engine: 64 -> 64, 13 x 13, 40 images (2.5e8) 21.3 / 22.2, 128 -> 128,
+// with the reduction: 64 -> 64 channels, 16 x 16 maps, 16 images (1.5e8) 28 / 18; 128 -> 128, 8 x 8, 40 images (3.8e8) 34 / 27;
+// engine: 64 -> 64, 13 x 13, 40 images (2.5e8) 21.3 / 22.2, 128 -> 128,
 // 13 x 13, 16 images (4e8) 29.3 / 29.8, 77 images (1.9e9) 63 / 42; 5 x 5: 64 -> 192, 15 x 15, 4 images (2.8e8) 27.1 / 26.8, 128 ->
 // 128, 8 x 8, 16 images (4.2e8) 29.2 / 29.3, 64 -> 192, 27 x 27, 16 images (3.6e9) 109 / 73.
 constexpr double kSplitDwWork = 1.2e8, kSplitDwEngineWork = 4.5e8;
-constexpr long kSplitDwPositions = 256;
 static bool split_dw_chosen(const fitre_conv_shape *s, const void *ws, size_t wsBytes, int pairs, SplitDwShape &d, BlockPlan &plan)
 {
 	if (!ws || (((uintptr_t)ws) & 3) || !split_dw_shape(s, d)) return false;
 	if (s->ksize == 5 && (s->inChannels <= 32 || s->outChannels <= 32)) return false; // half a tile
-	if ((long)s->samples * s->inA * s->inB < kSplitDwPositions) return false;
+	if ((long)s->samples * s->inA * s->inB < kSplitGradPositions) return false;
 	if (0.5 * pairs * conv_flops(s) < (c3_dw_eligible(s) ? kSplitDwWork : kSplitDwEngineWork)) return false;
 	plan = split_dw_plan(s, d, 0, pairs);
 	// a workspace for less than half of the ranges: longer sums than the fp32 kernels', and a chip that is not full
@@ -633,7 +638,7 @@ size_t gemm_ex_workspace(int M, int N, int K, int flags)
 }
 
 int gemm_ex(int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb,
-            float beta, float *C, int ldc, const float *bias, int flags, int kernelClass, void *ws, size_t wsBytes)
+            float beta, float *C, int ldc, const float *bias, int kernelClass, void *ws, size_t wsBytes)
 {
 	FITRE_REQUIRE(A && B && C, "fitre_hip_gemm: null pointer");
 	FITRE_REQUIRE(M > 0 && N > 0 && K > 0, "fitre_hip_gemm: non-positive shape %d x %d x %d", M, N, K);
@@ -642,28 +647,17 @@ int gemm_ex(int transA, int transB, int M, int N, int K, float alpha, const floa
 	const size_t aElems = (size_t)lda * (transA ? M : K), bElems = (size_t)ldb * (transB ? K : N);
 	FITRE_REQUIRE(aElems < ((size_t)1 << 30) && bElems < ((size_t)1 << 30), "fitre_hip_gemm: an operand exceeds 2^30 elements");
 	const int I = N, J = M, R = K;
-	GemmPlan plan = plan_gemm(I, J, R, (flags & kGemmMirror) != 0);
-	OutParams out{ C, (long)ldc, 0, nullptr, bias, alpha, beta, (flags & kGemmMirror) ? 1 : 0, (flags & kGemmTriK) ? 1 : 0 };
-	FITRE_REQUIRE(!(flags & kGemmMirror) || M == N, "gemm: a mirrored product must be square");
+	const OutParams out{ C, (long)ldc, 0, nullptr, bias, alpha, beta };
 	const double flops = 2.0 * (double)M * N * K;
 	// engine A(i = n, k): op(B)(k, n).  transB == 0: B[n*ldb + k] (contiguous along k); else B[k*ldb + n]
 	// engine B(j = m, k): op(A)(m, k).  transA == 0: A[k*lda + m] (contiguous along m); else A[m*lda + k]
-	PlainParams bk{ B, (uint32_t)(bElems * sizeof(float)), ldb, I };
-	PlainParams br = bk;
-	PlainParams ar{ A, (uint32_t)(aElems * sizeof(float)), lda, J };
-	PlainParams ak = ar;
-	if (!flags && short_product(I, J, R, lane_compute_units(), plan)) {
-		plan = fit_plan(plan, I, J, R, ws, wsBytes);
-		if (plan.splits > 1 && (((uintptr_t)ws) & 3)) return fail(FITRE_E_WORKSPACE, "split-K workspace is misaligned");
-		if (!transB && !transA) return launch_tile<PlainKContig, PlainRowContig, 64, 64, kGemmShortBK>(bk, ar, out, I, J, R, plan, ws, kernelClass, flops);
-		if (!transB && transA) return launch_tile<PlainKContig, PlainKContig, 64, 64, kGemmShortBK>(bk, ak, out, I, J, R, plan, ws, kernelClass, flops);
-		if (transB && !transA) return launch_tile<PlainRowContig, PlainRowContig, 64, 64, kGemmShortBK>(br, ar, out, I, J, R, plan, ws, kernelClass, flops);
-		return launch_tile<PlainRowContig, PlainKContig, 64, 64, kGemmShortBK>(br, ak, out, I, J, R, plan, ws, kernelClass, flops);
-	}
-	if (!transB && !transA) return launch_gemm<PlainKContig, PlainRowContig>(bk, ar, out, I, J, R, plan, ws, wsBytes, kernelClass, flops);
-	if (!transB && transA) return launch_gemm<PlainKContig, PlainKContig>(bk, ak, out, I, J, R, plan, ws, wsBytes, kernelClass, flops);
-	if (transB && !transA) return launch_gemm<PlainRowContig, PlainRowContig>(br, ar, out, I, J, R, plan, ws, wsBytes, kernelClass, flops);
-	return launch_gemm<PlainRowContig, PlainKContig>(br, ak, out, I, J, R, plan, ws, wsBytes, kernelClass, flops);
+	const PlainParams b{ B, (uint32_t)(bElems * sizeof(float)), ldb, I }, a{ A, (uint32_t)(aElems * sizeof(float)), lda, J };
+	const GemmPlan plan = split_gemm_plan_for(fit_plan(plan_gemm(I, J, R), I, J, R, ws, wsBytes), I, J, R, lane_compute_units());
+	if (plan.splits > 1 && (((uintptr_t)ws) & 3)) return fail(FITRE_E_WORKSPACE, "split-K workspace is misaligned");
+	if (!transB && !transA) return launch_split_gemm<SplitKContig, SplitRowContig>(b, a, out, I, J, R, plan, ws, kernelClass, flops);
+	if (!transB && transA) return launch_split_gemm<SplitKContigMasked, SplitKContig>(b, a, out, I, J, R, plan, ws, kernelClass, flops);
+	if (transB && !transA) return launch_split_gemm<SplitRowContig, SplitRowContig>(b, a, out, I, J, R, plan, ws, kernelClass, flops);
+	return launch_split_gemm<SplitRowContig, SplitKContig>(b, a, out, I, J, R, plan, ws, kernelClass, flops);
 }
 
 
@@ -1294,7 +1288,7 @@ int fitre_hip_gemm(int transA, int transB, int M, int N, int K, float alpha, con
 		                                                                         ldc, bias);
 		return check_launch("small_product_kernel");
 	}
-	return gemm_ex(transA, transB, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, bias, 0, FITRE_KC_FC_GEMM, ws, wsBytes);
+	return gemm_ex(transA, transB, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, bias, FITRE_KC_FC_GEMM, ws, wsBytes);
 }
 
 // ---- backward products of a fully connected layer --------------------------------------------
@@ -1336,7 +1330,7 @@ int fitre_hip_linear_input_grad(int in, int out, int n, const float *W, const fl
 	}
 	float *plain = permute ? staging : result;
 	FITRE_REQUIRE(plain != nullptr && plain != delta, "fitre_hip_linear_input_grad: a product of this size needs the staging buffer");
-	int rc = gemm_ex(1, 0, in, n, out, 1.f, W, out, delta, out, 0.f, plain, in, nullptr, 0, FITRE_KC_FC_GEMM, ws, wsBytes);
+	int rc = gemm_ex(1, 0, in, n, out, 1.f, W, out, delta, out, 0.f, plain, in, nullptr, FITRE_KC_FC_GEMM, ws, wsBytes);
 	if (rc) return rc;
 	if (derivative) {
 		rc = fitre_hip_activation_backward(actBelow, plain, zPre, zPost, plain, (long)in * n);
@@ -1376,7 +1370,7 @@ int fitre_hip_linear_weight_grad(int in, int out, int n, const float *delta, con
 		const int cus = device_compute_units() > 0 ? device_compute_units() : 256;
 		return launch_skinny_dw(in, out, n, delta, zin, dW, db, cus);
 	}
-	int rc = gemm_ex(0, 1, out, in, n, 1.f, delta, out, zin, in, 0.f, dW, out, nullptr, 0, FITRE_KC_FC_GEMM, ws, wsBytes);
+	int rc = gemm_ex(0, 1, out, in, n, 1.f, delta, out, zin, in, 0.f, dW, out, nullptr, FITRE_KC_FC_GEMM, ws, wsBytes);
 	if (rc || !db) return rc;
 	return fitre_hip_row_sum(delta, out, n, db);
 }

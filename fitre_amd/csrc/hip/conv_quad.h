@@ -19,21 +19,9 @@
 // tile stores put a lane's four rows -- the four cells of a map -- into one 16-byte group.
 #pragma once
 #include "conv_common.h"
+#include "split_gemm.h"
 
 namespace fitre {
-
-struct QuadParams {
-	const float *p;
-	uint32_t bytes;  // extent of the tensor
-	int groupStride; // floats between consecutive channels: 4 * samples
-	int rows;
-};
-
-typedef float quad4f __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ quad4f buffer_load4(__amdgpu_buffer_rsrc_t r, uint32_t byteOffset)
-{
-	return __builtin_bit_cast(quad4f, __builtin_amdgcn_raw_buffer_load_b128(r, (int)byteOffset, 0, 0));
-}
 
 // element(row = (c, q), k = n) = p[c * groupStride + 4 * k + q].  A thread moves 16-byte groups: the four rows
 // of one channel at one k; the groups of a channel over the k of a slice are contiguous in memory, and the
@@ -248,14 +236,13 @@ static int quad_launch_tile(const PA &pa, const PB &pb, const OutParams &out, in
 
 template <template <int, int> class OpA, template <int, int> class OpB, class PA, class PB>
 static int quad_launch(const PA &pa, const PB &pb, const OutParams &out, int I, int J, int R, void *ws, size_t wsBytes, int kernelClass,
-                       double flops, int *leftSplits, int mostSplits = 0)
+                       double flops, int *leftSplits)
 {
 	// Both products are small (2 GFLOP at the benchmark's shapes) and latency-bound on the engine's usual plan;
 	// measured sweep (512 x 512 channels, 256 images): 64 x 64 tiles with about four workgroups per compute unit,
 	// deep reduction slices: weight gradient 46 -> 36 us (unsplit, slices of 64), input gradient 43 -> 40 us
 	// (eight splits, slices of 32).
-	const GemmPlan ideal = quad_plan(I, J, R);
-	GemmPlan plan = mostSplits > 0 && mostSplits < ideal.splits ? quad_plan(I, J, R, mostSplits) : ideal;
+	GemmPlan plan = quad_plan(I, J, R);
 	if (plan.splits > 1 && (!ws || wsBytes < plan.wsBytes)) plan = quad_plan(I, J, R, 1); // no room for partials: unsplit
 	if (plan.wsBytes > 0 && (!ws || (((uintptr_t)ws) & 15) || wsBytes < plan.wsBytes))
 		return fail(FITRE_E_WORKSPACE, "split-K workspace of %zu bytes is null, misaligned or smaller than the %zu required", wsBytes,
@@ -312,6 +299,16 @@ static int quad_input_grad(const fitre_conv_shape *s, const float *delta, const 
 // the readers has on such maps, are 1 us longer this way.
 constexpr int kQuadForwardSamples = 128;
 static inline bool quad_forward_eligible(const fitre_conv_shape *s) { return quad_eligible(s) && s->samples >= kQuadForwardSamples; }
+// It runs on the bf16 pipes (split_gemm.h): 512 -> 512 channels, 256 images, 28 -> 18 us beside its consumer.  The two gradients do
+// not.  Where a layer has fewer positions than a patch has entries, as on these maps, the curvature passes multiply the part of a
+// weight gradient that lies outside the span of the patches -- all of it rounding -- by the inverse of the damping: natural
+// gradients of VGG-11 at 256 images moved by 8e-5 of their norm with products as accurate as these, one like the other.
+static inline GemmPlan quad_forward_plan(const fitre_conv_shape *s, int room)
+{
+	const int I = 4 * s->outChannels, J = s->samples, R = 4 * s->inChannels, most = quad_plan(I, J, R).splits;
+	if (room > 0 && room < most) return split_gemm_plan(I, J, R, room, R, device_compute_units());
+	return split_gemm_plan(I, J, R, most, 4L * ((R + most - 1) / most), device_compute_units());
+}
 static inline size_t quad_forward_workspace(const fitre_conv_shape *s)
 {
 	const int I = 4 * s->outChannels;
@@ -340,8 +337,8 @@ static int quad_forward(const fitre_conv_shape *s, const float *x, const float *
 	QuadParams pb{ x, (uint32_t)((size_t)s->inChannels * J * 4 * sizeof(float)), 4 * J, J };
 	OutParams out{ *partials, (long)J, 0, nullptr, nullptr, 1.f, 0.f };
 	out.quadLd = 4L * J;
-	return quad_launch<PlainKContig, QuadKOp>(pa, pb, out, I, J, R, *partials, wsBytes - weffBytes, FITRE_KC_CONV_FWD, conv_flops(s), splits,
-	                                          quad_forward_fits(s, wsBytes));
+	return launch_split_gemm<SplitKContig, SplitQuadK>(pa, pb, out, I, J, R, quad_forward_plan(s, quad_forward_fits(s, wsBytes)), *partials,
+	                                                   FITRE_KC_CONV_FWD, conv_flops(s), splits, 6);
 }
 
 // dW[co][ci][3][3] from x[ci][n][a'b'] and delta[co][n][ab].  ws: [dWeff | split partials].

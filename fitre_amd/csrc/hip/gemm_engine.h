@@ -955,23 +955,6 @@ inline bool deep_slice_plan(long I, long J, long R, bool mirror, int batch, long
 	return true;
 }
 
-// A plain product of less than a chip's worth of 128 x 128 tiles is cut along its reduction into short ranges, each a few slices
-// of sixteen that wait for their loads alone, on a chip that is not full.  The same ranges run on 64 x 64 tiles with slices of
-// thirty-two: four times the workgroups and half the waits, and since a slice reads nothing past its range every sum keeps its
-// order (and its bits).  Gradient and Gauss-Newton product of a 784-512-256-64-... autoencoder on 1000 points, 27 such products:
-// 1041 -> 929 us.  (Fewer, longer ranges were faster still, 847, and further from the 64-bit result, 1.0e-7 against 0.85e-7.)
-// Up to the work where the two meet.  128 x 128 x 16 / 64 x 64 x 32: 1024 x 1024 x 256 (2.7e8 multiply-adds) 25.7 / 21.8 us,
-// 784 x 784 x 784 (4.8e8) 27.7 / 23.9, 784 x 2000 x 512 (8.0e8) 36.0 / 31.6, 512 x 512 x 4000 (1.05e9) 37.1 / 32.1, 512 x
-// 4000 x 512 (1.05e9) 39.5 / 33.8; then 1536 x 1536 x 512 (1.2e9) 45.7 / 45.4, 1024 x 1024 x 2048 (2.1e9) 59.3 / 61.4, 1536 x
-// 1536 x 1000 (2.4e9) 64.2 / 66.3, though 1000 x 3000 x 512 (1.5e9) is 57.8 / 38.9.
-constexpr int kGemmShortBK = 32;
-constexpr double kGemmShortWork = 1.1e9;
-inline bool short_product(long I, long J, long R, long cus, const GemmPlan &plan)
-{
-	return plan.bm == 128 && plan.bn == 128 && R >= 2 * kGemmShortBK && (double)I * J * R <= kGemmShortWork &&
-	       ((I + 127) / 128) * ((J + 127) / 128) < cus;
-}
-
 // ---- batched products of plain operands ------------------------------------------------------------------------
 struct BatchStrides {
 	int batch;

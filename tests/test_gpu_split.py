@@ -75,8 +75,8 @@ def reference(case, which, source, w):
 CASES = [
     (77, 128, 160, 8, 8, 3),   # 160 channels: a partial channel tile; 4928 positions: a partial position tile
     (77, 160, 128, 8, 8, 3),
-    (96, 512, 512, 4, 4, 3),   # many images in a window, split reduction
-    (45, 512, 512, 4, 2, 3),   # rectangular
+    (130, 256, 256, 4, 4, 3),  # many images in a window, split reduction
+    (260, 256, 256, 4, 2, 3),  # rectangular
     (40, 64, 192, 16, 16, 3),  # the input gradient has 64 channels: 256-position tiles
     (21, 64, 128, 32, 32, 3),  # rows of 32
     (7, 128, 144, 27, 64, 3),  # the widest row
@@ -192,24 +192,24 @@ def weight_reference(case, x, d):
 # the three ways a row is cut into groups, every arrangement of waves, partial tiles of either kind of channels, and numbers of
 # image rows that are no whole groups or stages
 WEIGHT_CASES = [
-    (75, 256, 272, 4, 4, 3),   # two rows a group
-    (61, 200, 264, 5, 3, 3),   # rows of three cells, an odd number of rows
+    (130, 256, 272, 4, 4, 3),  # two rows a group
+    (151, 200, 264, 5, 3, 3),  # rows of three cells, an odd number of rows
     (128, 64, 64, 4, 4, 3),    # 64 x 64 tiles
-    (17, 160, 144, 8, 8, 3),   # a row a group
-    (43, 72, 130, 7, 6, 3),
+    (33, 160, 144, 8, 8, 3),   # a row a group
+    (51, 72, 130, 7, 6, 3),
     (32, 40, 48, 8, 8, 3),
     (41, 130, 64, 9, 7, 3),    # 64 x 128 tiles
     (23, 64, 192, 13, 13, 3),  # two groups a row, the second five cells
     (9, 100, 70, 16, 16, 3),
-    (5, 96, 128, 12, 32, 3),   # four groups a row
+    (6, 96, 128, 12, 32, 3),   # four groups a row
     (4, 64, 128, 27, 27, 3),
-    (7, 128, 64, 11, 24, 3),   # three of four groups
-    (12, 64, 192, 13, 13, 5),  # 5 x 5 windows
-    (9, 80, 160, 15, 8, 5),
+    (8, 128, 64, 11, 24, 3),   # three of four groups
+    (13, 64, 192, 13, 13, 5),  # 5 x 5 windows
+    (18, 80, 160, 15, 8, 5),
     (4, 64, 96, 20, 30, 5),
     (20, 72, 64, 15, 14, 5),   # at most 64 output channels
     (50, 48, 40, 8, 8, 5),
-    (60, 64, 64, 2, 16, 5),    # fewer image rows than the window
+    (65, 64, 64, 2, 16, 5),    # fewer image rows than the window
 ]
 
 
@@ -220,10 +220,10 @@ def test_weight_gradient(dev, case):
 
 
 def test_weight_gradient_of_a_pair(dev):
-    case = (19, 128, 128, 8, 8, 3)
+    case = (33, 128, 128, 8, 8, 3)
     (x, _, d), (x2, _, d2) = tensors(case), tensors(case, 1)
     got = weight_grad(dev, case, x, d, second=(x2, d2))
-    assert far(got, weight_reference(case, x, d) + weight_reference(case, x2, d2)) < limit(2 * 19 * 64)
+    assert far(got, weight_reference(case, x, d) + weight_reference(case, x2, d2)) < limit(2 * 33 * 64)
 
 
 def test_weight_gradient_in_smaller_workspaces(dev):
@@ -235,7 +235,7 @@ def test_weight_gradient_in_smaller_workspaces(dev):
         assert far(weight_grad(dev, case, x, d, ws_bytes=ws_bytes), want) < limit(64 * 64)
 
 
-@pytest.mark.parametrize("case", [(64, 128, 128, 8, 8, 3), (40, 128, 256, 4, 4, 3), (20, 64, 128, 16, 16, 3), (20, 64, 64, 15, 15, 5)])
+@pytest.mark.parametrize("case", [(64, 128, 128, 8, 8, 3), (130, 128, 256, 4, 4, 3), (20, 64, 128, 16, 16, 3), (20, 64, 64, 15, 15, 5)])
 def test_numbers_the_split_does_not_carry_in_a_weight_gradient(dev, case):
     x, _, d = tensors(case)
     terms = case[0] * case[3] * case[4]
@@ -252,3 +252,81 @@ def test_numbers_the_split_does_not_carry_in_a_weight_gradient(dev, case):
     assert huge.any() and far(got[huge] * 1e-35, want[huge] * 1e-35) < limit(terms)
     assert far(got[rest], want[rest]) < limit(terms, 0.6)
     assert far(weight_grad(dev, case, x, d * 2.0**-108) * 2.0**108, weight_reference(case, x, d)) < limit(terms, 0.6)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(200, 130, 777), (64, 64, 640), (131, 600, 96)])
+def test_product(dev, M, N, K, ta, tb):
+    """alpha, beta and a bias, and the numbers the split does not carry: in the middle, in a corner, at a ragged end of the
+    reduction, and behind it (where a row of the matrix holds what is not part of the product)."""
+    rng = np.random.default_rng(M + 3 * N + 7 * K + ta + 2 * tb)
+    lda, ldb, ldc = (K if ta else M) + 5, (N if tb else K) + 3, M + 1
+    A = rng.standard_normal((M if ta else K, lda)).astype(np.float32)
+    B = rng.standard_normal((K if tb else N, ldb)).astype(np.float32)
+    C0, bias = rng.standard_normal((N, ldc)).astype(np.float32), rng.standard_normal(M).astype(np.float32)
+    A[:, K if ta else M:] = np.inf
+    B[:, N if tb else K:] = np.nan
+    nb = hip.fitre_hip_gemm_workspace(M, N, K)
+    ws, pbias = dev.alloc(max(nb, 4)), dev.upload(bias)
+
+    def run(a, b):
+        pa, pb, pc = dev.upload(a.reshape(-1)), dev.upload(b.reshape(-1)), dev.upload(C0.reshape(-1))
+        L.check(hip.fitre_hip_gemm(ta, tb, M, N, K, 0.5, pa, lda, pb, ldb, -2.0, pc, ldc, pbias, ws, nb))
+        got = dev.download(pc, ldc * N).reshape(N, ldc)
+        for q in (pa, pb, pc):
+            dev.free(q)
+        return got
+
+    def op(a, b):
+        return (a[:, :K].T if ta else a[:, :M]).astype(np.float64), (b[:, :N].T if tb else b[:, :K]).astype(np.float64)
+
+    opA, opB = op(A, B)
+    rest = bias.astype(np.float64) - 2.0 * C0[:, :M].astype(np.float64)
+    got, want = run(A, B), 0.5 * opB @ opA + rest
+    assert far(got[:, :M], want) < limit(K, 0.6)
+    np.testing.assert_array_equal(got[:, M:], C0[:, M:])
+    odd_a, odd_b = A.copy(), B.copy()
+    opA, opB = op(odd_a, odd_b)
+    views = (odd_a[:, :K].T if ta else odd_a[:, :M]), (odd_b[:, :N].T if tb else odd_b[:, :K])  # [K][M], [N][K] of the copies
+    views[1][:, 3] *= 0.05
+    views[0][3, 7], views[0][K - 1, M - 1], views[1][N - 1, 0] = np.finfo(np.float32).max, np.inf, np.nan
+    with np.errstate(invalid="ignore"):
+        opA, opB = op(odd_a, odd_b)
+        got, want = run(odd_a, odd_b)[:, :M], 0.5 * np.array([[(opB[n] * opA[:, m]).sum() for m in range(M)] for n in range(N)]) + rest
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(want))
+    np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    huge = np.isfinite(want) & (np.abs(want) > 1e30)
+    fine = np.isfinite(want) & ~huge
+    assert far(got[huge] * 1e-35, want[huge] * 1e-35) < limit(K) and far(got[fine], want[fine]) < limit(K, 1.0)
+    for q in (ws, pbias):
+        dev.free(q)
+
+
+@pytest.mark.parametrize("n", [130, 200])
+def test_forward_on_2x2_maps(dev, n):
+    """The dense form of 3 x 3 windows on 2 x 2 maps (through the layer's pass, without normalisation, activation and pool)."""
+    from fitre_amd.structs import CNN_ACT_NONE, NO_POOL
+    ci, co = 96, 132
+    case = (n, ci, co, 2, 2, 3)
+    shape = conv_shape(n, ci, co, 2, 2, 3, 1, 1)
+    x, w, _ = tensors(case)
+    nb, size = hip.fitre_hip_conv_bn_act_pool_workspace(C.byref(shape), 0), co * n * 4
+
+    def run(source):
+        px, pw, ws, y, act = dev.upload(flat(source)), dev.upload(w.numpy().ravel()), dev.alloc(nb), dev.zeros(size), dev.zeros(size)
+        L.check(hip.fitre_hip_conv_bn_act_pool_forward(C.byref(shape), px, pw, None, y, None, None, None, None, None, 1e-5, 0.1, 1, CNN_ACT_NONE,
+                                                       act, NO_POOL, 0, 0, 0, 0, 0, None, 0, ws, nb))
+        got = dev.download(y, size).reshape(co, n, 2, 2)
+        for q in (px, pw, ws, y, act):
+            dev.free(q)
+        return got
+
+    assert far(run(x), reference(case, "fwd", x, w)) < limit(ci * 4)
+    odd = x.clone()
+    odd[5, 3, 1, 0], odd[n - 1, 95, 0, 1] = float("inf"), float("nan")
+    got, want = run(odd), reference(case, "fwd", odd, w)
+    finite = np.isfinite(want)
+    np.testing.assert_array_equal(np.isfinite(got), finite)
+    assert far(got[finite], want[finite]) < limit(ci * 4, 0.6)
+    assert far(run(x * 2.0**-108) * 2.0**108, reference(case, "fwd", x, w)) < limit(ci * 4, 0.6)
