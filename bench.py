@@ -49,7 +49,7 @@ KC = dict(conv_dw=0, conv_dx=1, conv_fwd=2, fc_gemm=3, splitk_reduce=4, bn_bwd=5
           act_bwd=9, act_fwd=10, bias_grad=11, softmax=12, permute=13, blas1=14, pool_act_bwd=15, kfac_factor=16,
           spd_inverse=17)
 MFMA_CLASSES = ("conv_dw", "conv_dx", "conv_fwd", "fc_gemm", "kfac_factor", "spd_inverse")
-TILES = {0: "", 1: "64x64", 2: "64x128", 3: "128x64", 4: "128x128", 5: "96x128", 6: "dense2x2", 7: "cell4x4", 8: "cell8x8", 9: "skinny", 10: "split"}
+TILES = {0: "", 1: "64x64", 2: "64x128", 3: "128x64", 4: "128x128", 5: "96x128", 6: "dense2x2", 7: "cell4x4", 8: "cell8x8", 9: "skinny", 10: "split", 11: "splitcell4x4"}
 
 
 def measured_traffic(kernel):
@@ -108,7 +108,7 @@ def conv_live_fractions(model, batch):
 
 
 # kernel variants that leave out the products with the padding, and the live fraction of the maps they run on
-SKIPS_PADDING = {"/dense2x2": 16 / 36.0, "/cell4x4": 100 / 144.0, "/cell8x8": 484 / 576.0}
+SKIPS_PADDING = {"/dense2x2": 16 / 36.0, "/cell4x4": 100 / 144.0, "/splitcell4x4": 100 / 144.0, "/cell8x8": 484 / 576.0}
 
 
 def launch_live_fraction(kernel, work, conv_live):
@@ -124,7 +124,7 @@ def launch_live_fraction(kernel, work, conv_live):
 def matrix_peak(kernel):
     """TFLOP/s of fp32 work at which the matrix pipes of a kernel are the bound: the split kernels make every fp32 product from
     six bf16 ones."""
-    return PEAK_MFMA_BF16_TFLOPS / 6 if kernel.endswith("/split") else PEAK_MFMA_F32_TFLOPS
+    return PEAK_MFMA_BF16_TFLOPS / 6 if "/split" in kernel else PEAK_MFMA_F32_TFLOPS
 
 
 def kernel_table(rows, steps, launches=None, conv_live=None, fc_batch=None):

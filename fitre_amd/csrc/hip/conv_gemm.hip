@@ -278,11 +278,22 @@ static size_t split_weights_bytes(const fitre_conv_shape *s, bool dx)
 	const int I = dx ? s->inChannels : s->outChannels, cred = dx ? s->outChannels : s->inChannels;
 	return (size_t)(cred / kSplitCB) * s->ksize * s->ksize * split_row_groups(I) * 192 * sizeof(u32x4);
 }
+// 4 x 4 maps in the cell form, where what it leaves out is more than what fills its last tile of 32 images: 512 -> 512 channels,
+// 256 images 80 -> 67 us, 256 -> 512 46 -> 39.  Not for an input gradient on its own: beside a weight gradient (two workgroups
+// and 154 KB of LDS on a compute unit) the window form's 47 KB and 240 registers find room when the first of the two has ended,
+// the cell form's 102 KB when both have, and the chain waits (VGG-11 step 1831 -> 1912 us).
+static bool split_cell_form(const fitre_conv_shape *s, bool dx, int pairs)
+{
+	return !(dx && pairs == 1) && s->ksize == 3 && s->inA == 4 && s->inB == 4 && 100L * ((s->samples + kCellSplitImages - 1) / kCellSplitImages * kCellSplitImages) < 137L * s->samples;
+}
 static BlockPlan split_pos_plan(const fitre_conv_shape *s, bool dx, int cus = 0, int pairs = 1)
 {
 	if (cus <= 0) cus = lane_compute_units();
 	const long I = dx ? s->inChannels : s->outChannels, J = (long)s->samples * s->inA * s->inB;
 	const long cred = dx ? s->outChannels : s->inChannels;
+	if (split_cell_form(s, dx, pairs)) // 150 matrix instructions a wave and block against 216
+		return plan_blocks(((I + kCellSplitRows - 1) / kCellSplitRows) * (((long)s->samples + kCellSplitImages - 1) / kCellSplitImages),
+		                   pairs * cred / kSplitCB, 0.55 * 0.85 * 6.25, 1, I, J, cus);
 	const long it = I <= 64 ? 64 : 128, jt = I <= 64 ? 256 : 128;
 	const long tiles = ((I + it - 1) / it) * ((J + jt - 1) / jt);
 	// measured: 0.55 us a tap and block with a workgroup on every compute unit, two of them share the pipes
@@ -328,18 +339,19 @@ static BlockPlan split_pos_fit(const fitre_conv_shape *s, bool dx, const void *w
 	                  split_pos_room(s, dx, ws, wsBytes, pairs, prepared));
 }
 
-static int launch_split_weights(const fitre_conv_shape *s, bool dx, const float *w, u32x4 *wp)
+// w2 (may be null): a pair's second weights, whose parts follow the first's
+static int launch_split_weights(const fitre_conv_shape *s, bool dx, const float *w, const float *w2, u32x4 *wp)
 {
 	const int I = dx ? s->inChannels : s->outChannels, cred = dx ? s->outChannels : s->inChannels, groups = split_row_groups(I);
-	const dim3 grid((unsigned)groups, (unsigned)(cred / kSplitCB));
+	const dim3 grid((unsigned)groups, (unsigned)(cred / kSplitCB), w2 ? 2u : 1u);
 	if (grid.y > 65535) return fail(FITRE_E_UNSUPPORTED, "split_weights_kernel grid too large");
-	LaunchScope scope(FITRE_KC_PERMUTE, 10.0 * (double)I * cred * s->ksize * s->ksize);
+	LaunchScope scope(FITRE_KC_PERMUTE, (w2 ? 20.0 : 10.0) * (double)I * cred * s->ksize * s->ksize);
 	if (s->ksize == 3) {
-		if (dx) split_weights_kernel<3, true><<<grid, 256, 0, stream()>>>(w, I, cred, groups, wp);
-		else split_weights_kernel<3, false><<<grid, 256, 0, stream()>>>(w, I, cred, groups, wp);
+		if (dx) split_weights_kernel<3, true><<<grid, 256, 0, stream()>>>(w, w2, I, cred, groups, wp);
+		else split_weights_kernel<3, false><<<grid, 256, 0, stream()>>>(w, w2, I, cred, groups, wp);
 	} else {
-		if (dx) split_weights_kernel<5, true><<<grid, 256, 0, stream()>>>(w, I, cred, groups, wp);
-		else split_weights_kernel<5, false><<<grid, 256, 0, stream()>>>(w, I, cred, groups, wp);
+		if (dx) split_weights_kernel<5, true><<<grid, 256, 0, stream()>>>(w, w2, I, cred, groups, wp);
+		else split_weights_kernel<5, false><<<grid, 256, 0, stream()>>>(w, w2, I, cred, groups, wp);
 	}
 	return check_launch("split_weights_kernel");
 }
@@ -354,15 +366,10 @@ static int launch_split_pos(const fitre_conv_shape *s, bool dx, const float *src
 	const u32x4 *wp = (const u32x4 *)prepared, *wp2 = nullptr;
 	if (!prepared) {
 		u32x4 *made = (u32x4 *)((char *)ws + split_pos_room(s, dx, ws, wsBytes, pairs, false));
-		int rc = launch_split_weights(s, dx, w, made);
+		const int rc = launch_split_weights(s, dx, w, w2, made);
 		if (rc) return rc;
 		wp = made;
-		if (src2) {
-			made += split_weights_bytes(s, dx) / sizeof(u32x4);
-			rc = launch_split_weights(s, dx, w2, made);
-			if (rc) return rc;
-			wp2 = made;
-		}
+		if (src2) wp2 = made + split_weights_bytes(s, dx) / sizeof(u32x4);
 	}
 	const int P = s->ksize / 2;
 	ConvSplitParams p{};
@@ -376,6 +383,18 @@ static int launch_split_pos(const fitre_conv_shape *s, bool dx, const float *src
 	OutParams out{ outPtr, (long)J, 0, bias, nullptr, 1.f, 0.f };
 	OutParams part = out;
 	if (plan.splits > 1) part.C = (float *)ws, part.splitStride = (long)I * J;
+	if (split_cell_form(s, dx, pairs) && (((uintptr_t)part.C) & 15) == 0) { // (a plan made for it also fits the window form: the same blocks)
+		const dim3 cells((unsigned)((s->samples + kCellSplitImages - 1) / kCellSplitImages), (unsigned)((I + kCellSplitRows - 1) / kCellSplitRows),
+		                 (unsigned)plan.splits);
+		if (cells.y > 65535 || cells.z > 65535) return fail(FITRE_E_UNSUPPORTED, "conv_split_cell_kernel grid too large");
+		{
+			LaunchScope scope(dx ? FITRE_KC_CONV_DX : FITRE_KC_CONV_FWD, pairs * conv_flops(s), kTileSplitCell);
+			conv_split_cell_kernel<<<cells, kGemmThreads, 0, stream()>>>(p, part);
+		}
+		if (leftSplits) *leftSplits = plan.splits;
+		if (plan.splits > 1 && !leftSplits) launch_splitk_reduce((const float *)ws, plan.splits, I, J, out);
+		return check_launch("conv_split_cell_kernel");
+	}
 	const ConvSplitVariant &v = *conv_split_variant(s->ksize, I, s->inA, s->inB);
 	const int it = 32 * v.wm, jt = 128 * (4 / v.wm);
 	const dim3 grid((unsigned)((J + jt - 1) / jt), (unsigned)((I + it - 1) / it), (unsigned)plan.splits);
@@ -1205,7 +1224,7 @@ int fitre_hip_conv_input_grad_prepare(const fitre_conv_shape *s, const float *w,
 	if (preparedBytes < need || (((uintptr_t)prepared) & 15))
 		return fail(FITRE_E_WORKSPACE, "fitre_hip_conv_input_grad_prepare: buffer of %zu bytes is misaligned or smaller than the %zu required",
 		            preparedBytes, need);
-	return quad_eligible(s) ? quad_prepare_weights(s, w, (float *)prepared) : launch_split_weights(s, true, w, (u32x4 *)prepared);
+	return quad_eligible(s) ? quad_prepare_weights(s, w, (float *)prepared) : launch_split_weights(s, true, w, nullptr, (u32x4 *)prepared);
 }
 
 int fitre_hip_conv_input_grad_split_prepared(const fitre_conv_shape *s, const float *delta, const float *w, const void *prepared,

@@ -36,12 +36,13 @@ struct ConvSplitParams {
 // DX: rows are the layer's input channels, the reduction runs over its output channels, windows are flipped.
 template <int KS, bool DX>
 __global__ void __launch_bounds__(256)
-split_weights_kernel(const float *w, int I, int cred, int rowGroups, u32x4 *wp)
+split_weights_kernel(const float *w, const float *w2, int I, int cred, int rowGroups, u32x4 *wp)
 {
 	constexpr int T = KS * KS, LD = DX ? 32 * T + 1 : kSplitCB * T + 1, ROWS = DX ? kSplitCB : 32;
 	constexpr int SPAN = DX ? 32 * T : kSplitCB * T; // floats in a row, consecutive in memory
 	__shared__ float L[ROWS * LD];
 	const int rb = blockIdx.x, cb = blockIdx.y, i0 = rb * 32, c0 = cb * kSplitCB;
+	if (blockIdx.z) w = w2, wp += (size_t)gridDim.y * T * rowGroups * 192; // a pair's second weights, behind the first
 	const int rowLen = (DX ? I : cred) * T, col0 = (DX ? i0 : c0) * T, row0 = DX ? c0 : i0;
 	const int live = (I - i0 < 32 ? I - i0 : 32) * T; // DX: floats of a row inside the tensor
 	constexpr int N = ROWS * SPAN / 256;
@@ -321,6 +322,155 @@ conv_split_kernel(const ConvSplitParams p, const OutParams out)
 			if (!split && out.biasI) val += out.biasI[i];
 			C[(size_t)i * out.ldc + j] = val;
 		}
+	}
+}
+
+// ---- 4 x 4 maps ------------------------------------------------------------------------------------------------------
+// The columns of a matrix block are one cell of 32 images, so that the 44 of 144 (cell, tap) pairs that reach outside a map are
+// left out: a workgroup owns 32 channels x 32 images, a wave a quadrant of the map and its 25 live pairs.  Quadrants are seen
+// mirrored so that each has the map's corner at local cell (0, 0): what is live is then known at compile time, and only the
+// addresses of cells and taps differ.  The nine source cells of a quadrant stay in registers for a block of sixteen channels;
+// weights stream as above.  One workgroup per compute unit with up to 512 registers a lane.  512 -> 512 channels, 256 images, two
+// ranges: 80 us in the window form, 67 in this.
+constexpr int kCellSplitImages = 32, kCellSplitRows = 32;
+__global__ void __launch_bounds__(kGemmThreads, 1)
+conv_split_cell_kernel(const ConvSplitParams p, const OutParams out)
+{
+	FITRE_RAISE_MATRIX_WAVE_PRIORITY();
+	constexpr int T = 9, LDN = 33, HALF = 16 * LDN, PART = 2 * HALF, BUF = 3 * PART; // 16-byte words: [part][half][cell][image]
+	constexpr int XE = 4, ROW = 20;                                                  // results: floats between two images' maps in LDS
+	static_assert(kCellSplitRows * kCellSplitImages * ROW <= 2 * BUF * 4, "the results fit the buffers");
+	__shared__ u32x4 Bs[2 * BUF];
+
+	const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+	const int khalf = lane >> 5, l32 = lane & 31, qa = wave >> 1, qb = wave & 1;
+	const int n0 = blockIdx.x * kCellSplitImages, i0 = blockIdx.y * kCellSplitRows, j0 = n0 * 16;
+	const int cbHalf = p.cred / kSplitCB, cbTotal = p.src2 ? 2 * cbHalf : cbHalf;
+	const int cbBeg = blockIdx.z * p.perSplit, cbEnd = cbBeg + p.perSplit < cbTotal ? cbBeg + p.perSplit : cbTotal;
+
+	// position tid or tid + 256 of the 512, either half of the channels
+	uint32_t sOff[XE];
+	int sLds[XE];
+#pragma unroll
+	for (int e = 0; e < XE; e++) {
+		const int pos = tid + 256 * (e & 1), half = e >> 1;
+		sOff[e] = j0 + pos < p.J ? 4u * ((uint32_t)(half * 8) * (uint32_t)p.J + (uint32_t)(j0 + pos)) : kOutOfRange;
+		sLds[e] = half * HALF + (pos & 15) * LDN + (pos >> 4);
+	}
+	float sreg[XE][8];
+	v16f acc[4], low[4];
+#pragma unroll
+	for (int c = 0; c < 4; c++)
+#pragma unroll
+		for (int v = 0; v < 16; v++) acc[c][v] = low[c][v] = 0.f;
+	const size_t rowWords = (size_t)blockIdx.y * 192, tapWords = (size_t)p.rowGroups * 192;
+
+#define CELL_LOAD(CB)                                                                                                 \
+	{                                                                                                                 \
+		const bool second_ = (CB) >= cbHalf;                                                                          \
+		const size_t shift_ = (size_t)(((CB) - (second_ ? cbHalf : 0)) * kSplitCB) * p.J;                             \
+		const __amdgpu_buffer_rsrc_t rs_ = make_rsrc((second_ ? p.src2 : p.src) + shift_, p.srcBytes - (uint32_t)(4 * shift_)); \
+		_Pragma("unroll") for (int e = 0; e < XE; e++)                                                                \
+			_Pragma("unroll") for (int q = 0; q < 8; q++)                                                             \
+				sreg[e][q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_, (int)sOff[e], 4 * q * p.J, 0)); \
+	}
+#define CELL_STORE(BUFFER, E)                                                                                         \
+	{                                                                                                                 \
+		u32x4 part_[3];                                                                                               \
+		split_eight(sreg[E], part_);                                                                                  \
+		_Pragma("unroll") for (int s = 0; s < 3; s++) Bs[(BUFFER) * BUF + s * PART + sLds[E]] = part_[s];             \
+	}
+#define CELL_READ(BUFFER)                                                                                             \
+	_Pragma("unroll") for (int r = 0; r < 3; r++)                                                                     \
+		_Pragma("unroll") for (int c = 0; c < 3; c++)                                                                 \
+			_Pragma("unroll") for (int s = 0; s < 3; s++)                                                             \
+				b[r][c][s] = Bs[(BUFFER) * BUF + s * PART + khalf * HALF + ((qa ? 3 - r : r) * 4 + (qb ? 3 - c : c)) * LDN + l32];
+#define CELL_READ_WEIGHTS(SET, BLOCK, TAP)                                                                            \
+	{                                                                                                                 \
+		const int tap_ = (qa ? 2 - (TAP) / 3 : (TAP) / 3) * 3 + (qb ? 2 - (TAP) % 3 : (TAP) % 3);                     \
+		_Pragma("unroll") for (int s = 0; s < 3; s++) a[SET][s] = (BLOCK)[(size_t)tap_ * tapWords + s * 64 + lane];   \
+	}
+#define CELL_PRODUCTS(SUM, PA, PB)                                                                                    \
+	_Pragma("unroll") for (int c = 0; c < 4; c++)                                                                     \
+		if ((c >> 1) + t / 3 >= 1 && (c & 1) + t % 3 >= 1)                                                            \
+			SUM[c] = mfma_bf16(a[t & 1][PA], b[(c >> 1) + t / 3 >= 1 ? (c >> 1) + t / 3 - 1 : 0][(c & 1) + t % 3 >= 1 ? (c & 1) + t % 3 - 1 : 0][PB], SUM[c]);
+
+	u32x4 a[2][3], b[3][3][3];
+	const u32x4 *wBlock = (cbBeg >= cbHalf ? p.wp2 + (size_t)(cbBeg - cbHalf) * T * tapWords : p.wp + (size_t)cbBeg * T * tapWords) + rowWords;
+	CELL_READ_WEIGHTS(0, wBlock, 0);
+	CELL_LOAD(cbBeg);
+#pragma unroll
+	for (int e = 0; e < XE; e++) CELL_STORE(0, e);
+	__syncthreads();
+	for (int cb = cbBeg; cb < cbEnd; cb++) {
+		const int buffer = (cb - cbBeg) & 1;
+		const int nb = cb + 1 < cbEnd ? cb + 1 : cb; // (the last block's is staged once more, and not read)
+		const u32x4 *wNext = (nb >= cbHalf ? p.wp2 + (size_t)(nb - cbHalf) * T * tapWords : p.wp + (size_t)nb * T * tapWords) + rowWords;
+		CELL_READ(buffer);
+#pragma unroll
+		for (int t = 0; t < T; t++) {
+			if (t + 1 < T) CELL_READ_WEIGHTS((t + 1) & 1, wBlock, t + 1) else CELL_READ_WEIGHTS((t + 1) & 1, wNext, 0);
+			if (t == 0) CELL_LOAD(nb);
+			__builtin_amdgcn_sched_barrier(0);
+			if (t >= T - XE) CELL_STORE(buffer ^ 1, t - (T - XE));
+			CELL_PRODUCTS(low, 0, 2);
+			CELL_PRODUCTS(acc, 0, 0);
+			CELL_PRODUCTS(low, 0, 1);
+			CELL_PRODUCTS(low, 1, 1);
+			CELL_PRODUCTS(low, 2, 0);
+			CELL_PRODUCTS(low, 1, 0);
+			if (t >= T - XE) {
+#pragma unroll
+				for (int i = 0; i < 12; i++) {
+					__builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+					__builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+				}
+			}
+			__builtin_amdgcn_sched_barrier(0);
+		}
+#pragma unroll
+		for (int s = 0; s < 3; s++) a[0][s] = a[1][s]; // nine taps: the next block's first fragments are in the other set
+		wBlock = wNext;
+		__syncthreads();
+	}
+#undef CELL_LOAD
+#undef CELL_STORE
+#undef CELL_READ
+#undef CELL_READ_WEIGHTS
+#undef CELL_PRODUCTS
+
+	const bool split = out.splitStride != 0;
+	float *C = out.C + (size_t)blockIdx.z * out.splitStride;
+	bool suspect = false;
+#pragma unroll
+	for (int c = 0; c < 4; c++)
+#pragma unroll
+		for (int v = 0; v < 16; v++) {
+			acc[c][v] += low[c][v];
+			suspect |= split_sum_suspect(acc[c][v]);
+		}
+	if (__syncthreads_or(suspect)) {
+		conv_split_exact_tile<3, kCellSplitRows, kCellSplitImages * 16>(p, out, i0, j0, cbBeg, cbEnd, C);
+		return;
+	}
+	// through LDS, whose maps leave as 16-byte groups along the positions
+	float *R = (float *)Bs;
+#pragma unroll
+	for (int c = 0; c < 4; c++) {
+		const int cell = (qa ? 3 - (c >> 1) : (c >> 1)) * 4 + (qb ? 3 - (c & 1) : (c & 1));
+#pragma unroll
+		for (int v = 0; v < 16; v++) R[((8 * (v / 4) + 4 * khalf + (v % 4)) * kCellSplitImages + l32) * ROW + cell] = acc[c][v];
+	}
+	__syncthreads();
+	for (int e = tid; e < kCellSplitRows * kCellSplitImages * 4; e += kGemmThreads) {
+		const int row = e / (kCellSplitImages * 4), n = e / 4 % kCellSplitImages, quarter = e % 4, i = i0 + row;
+		if (i >= p.I || j0 + n * 16 >= p.J) continue;
+		float4 val = *(const float4 *)&R[(row * kCellSplitImages + n) * ROW + 4 * quarter];
+		if (!split && out.biasI) {
+			const float bias = out.biasI[i];
+			val.x += bias, val.y += bias, val.z += bias, val.w += bias;
+		}
+		*(float4 *)&C[(size_t)i * out.ldc + j0 + n * 16 + 4 * quarter] = val;
 	}
 }
 

@@ -53,7 +53,7 @@ __device__ __forceinline__ v16f mfma_bf16(u32x4 a, u32x4 b, v16f c)
 	return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-constexpr int kTileSplit = 10; // profile variant of these kernels
+constexpr int kTileSplit = 10, kTileSplitCell = 11; // profile variants of these kernels
 
 // a finished sum that the split may not have carried: not finite, or not zero and below 2^-90 (factors of ordinary size
 // beside it then have parts below 2^-133)

@@ -75,7 +75,9 @@ def reference(case, which, source, w):
 CASES = [
     (77, 128, 160, 8, 8, 3),   # 160 channels: a partial channel tile; 4928 positions: a partial position tile
     (77, 160, 128, 8, 8, 3),
-    (130, 256, 256, 4, 4, 3),  # many images in a window, split reduction
+    (130, 256, 256, 4, 4, 3),  # many images in a window, split reduction; forward in the cell form, two images in the last tile
+    (128, 256, 272, 4, 4, 3),  # whole tiles of images, a partial tile of channels
+    (66, 512, 256, 4, 4, 3),   # too little in the last tile of images for the cell form
     (260, 256, 256, 4, 2, 3),  # rectangular
     (40, 64, 192, 16, 16, 3),  # the input gradient has 64 channels: 256-position tiles
     (21, 64, 128, 32, 32, 3),  # rows of 32
@@ -101,13 +103,13 @@ def test_convolution(dev, case, which):
     assert far(conv(dev, case, which, source, w, bias=bias), want) < limit(terms)
 
 
+@pytest.mark.parametrize("case", [(40, 128, 128, 8, 8, 3), (130, 144, 176, 4, 4, 3)])
 @pytest.mark.parametrize("which", ["fwd", "dx"])
-def test_a_pair_of_products(dev, which):
-    case = (40, 128, 128, 8, 8, 3)
+def test_a_pair_of_products(dev, case, which):
     (x, w, d), (x2, w2, d2) = tensors(case), tensors(case, 1)
     s, s2 = (x, x2) if which == "fwd" else (d, d2)
     got = conv(dev, case, which, s, w, second=(s2, w2))
-    assert far(got, reference(case, which, s, w) + reference(case, which, s2, w2)) < limit(2 * 128 * 9)
+    assert far(got, reference(case, which, s, w) + reference(case, which, s2, w2)) < limit(2 * s.shape[1] * 9)
 
 
 def test_smaller_workspaces(dev):
@@ -141,17 +143,16 @@ def test_prepared_weights_give_the_same_bits(dev):
         dev.free(q)
 
 
-@pytest.mark.parametrize("which", ["fwd", "dx"])
-def test_numbers_the_split_does_not_carry(dev, which):
+@pytest.mark.parametrize("case,which", [((80, 128, 128, 8, 8, 3), "fwd"), ((80, 128, 128, 8, 8, 3), "dx"), ((160, 192, 208, 4, 4, 3), "fwd")])
+def test_numbers_the_split_does_not_carry(dev, case, which):
     """Infinities, NaN, the largest floats (which round up to infinity in bf16) and tensors so small that the lower parts of
     their numbers are below the smallest bf16 number: what an fp32 chain gives."""
-    case = (80, 128, 128, 8, 8, 3)
     x, w, d = tensors(case)
     source = x if which == "fwd" else d
-    terms = 128 * 9
+    terms = source.shape[1] * 9
     plain = conv(dev, case, which, source, w)
     odd = source.clone()
-    odd[3, 5, 0, 7], odd[40, 100, 4, 4], odd[79, 127, 7, 7] = float("inf"), float("nan"), float(np.finfo(np.float32).max)
+    odd[3, 5, 0, 3], odd[40, 100, 2, 2], odd[-1, -1, -1, -1] = float("inf"), float("nan"), float(np.finfo(np.float32).max)
     got, want = conv(dev, case, which, odd, w), reference(case, which, odd, w)
     np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
     np.testing.assert_array_equal(np.isinf(got), np.isinf(want))
@@ -161,7 +162,7 @@ def test_numbers_the_split_does_not_carry(dev, which):
     rest = np.isfinite(want) & ~huge
     assert far(got[rest], want[rest]) < limit(terms, 0.6)
     # tiles without such a number keep their bits
-    far_off = slice(8, 30)  # images of tiles of their own (two images a tile)
+    far_off = slice(8, 30) if case[3] == 8 else slice(64, 128)  # images of other tiles (two of 8 x 8, 32 of 4 x 4 a tile)
     np.testing.assert_array_equal(got[:, far_off], plain[:, far_off])
     small = source * 2.0**-108
     assert far(conv(dev, case, which, small, w) * 2.0**108, reference(case, which, source, w)) < limit(terms, 0.6)
