@@ -324,14 +324,18 @@ constexpr double kSplitWork = 7.0e8, kSplitNarrowWork = 1.5e9, kSplitCellWork = 
 // kernels, whose rounding is no larger but another, VGG-11's natural gradient at 32 images (512 positions of 512 channels) moves
 // by 2.8e-4 of its norm, at 64 by 2e-5, at 96 by 1e-5, from 128 images (2048 positions) on by less than 7e-6.
 constexpr long kSplitGradPositions = 2048;
-static bool split_pos_chosen(const fitre_conv_shape *s, bool dx, const void *ws, size_t wsBytes, int pairs = 1, bool prepared = false)
+static bool split_pos_worthwhile(const fitre_conv_shape *s, bool dx, int pairs)
 {
-	if (!split_pos_eligible(s, dx) || split_pos_room(s, dx, ws, wsBytes, pairs, prepared) == 0) return false;
 	if (dx && (long)s->samples * s->inA * s->inB < kSplitGradPositions) return false;
 	const int I = dx ? s->inChannels : s->outChannels;
 	const double least = cell_pos_eligible(s, dx) ? kSplitCellWork : (s->ksize == 3 && I <= 64 ? kSplitNarrowWork : kSplitWork);
 	return 0.5 * pairs * conv_flops(s) >= least;
 }
+static bool split_pos_chosen(const fitre_conv_shape *s, bool dx, const void *ws, size_t wsBytes, int pairs = 1, bool prepared = false)
+{
+	return split_pos_eligible(s, dx) && split_pos_worthwhile(s, dx, pairs) && split_pos_room(s, dx, ws, wsBytes, pairs, prepared) > 0;
+}
+
 static BlockPlan split_pos_fit(const fitre_conv_shape *s, bool dx, const void *ws, size_t wsBytes, int pairs, bool prepared)
 {
 	const int I = dx ? s->inChannels : s->outChannels, cred = dx ? s->outChannels : s->inChannels;
@@ -1210,7 +1214,8 @@ int fitre_hip_conv_weight_grad_pair(const fitre_conv_shape *s, const float *x1, 
 size_t fitre_hip_conv_input_grad_prepared_bytes(const fitre_conv_shape *s)
 {
 	if (!s) return 0;
-	return quad_eligible(s) ? quad_weff_bytes(s) : (split_pos_eligible(s, true) ? split_weights_bytes(s, true) : 0);
+	if (quad_eligible(s)) return quad_weff_bytes(s);
+	return split_pos_eligible(s, true) && split_pos_worthwhile(s, true, 1) ? split_weights_bytes(s, true) : 0;
 }
 
 int fitre_hip_conv_input_grad_prepare(const fitre_conv_shape *s, const float *w, void *prepared, size_t preparedBytes)

@@ -338,6 +338,7 @@ void cnnBackward(CNN_MODEL *model, DEVICE_DATASET *data, real *devPtr, real *z, 
 	void *sideWs = (void *)((char *)bnWs + bnBytes);
 	const size_t sideBytes = backward_side_ws_bytes(model, model->batchSize);
 	char *preparedWs = (char *)sideWs + sideBytes;
+	const char *preparedEnd = preparedWs + backward_prepared_bytes(model, model->batchSize);
 	const void *prepared[MAX_LAYERS] = { NULL };
 	int preparedPending = 0;
 
@@ -361,10 +362,10 @@ void cnnBackward(CNN_MODEL *model, DEVICE_DATASET *data, real *devPtr, real *z, 
 		int any = 0;
 		for (int c = 1; c < nc; c++) {
 			fitre_conv_shape shape = conv_shape(&model->convLayer[c], n);
-			/* the buffers are laid out for the model's batch size; a shape's need does not depend on the batch */
+			/* the buffers are laid out for the model's batch size; a shorter one can take a copy where that takes none */
 			const size_t bytes = fitre_hip_conv_input_grad_prepared_bytes(&shape);
 			prepared[c] = NULL;
-			if (bytes == 0 || !has_bn(&model->convLayer[c - 1])) continue;
+			if (bytes == 0 || bytes > (size_t)(preparedEnd - preparedWs) || !has_bn(&model->convLayer[c - 1])) continue;
 			if (!any) {
 				/* behind whatever the caller has queued on lane 0 (a weight update, say): the copies read the weights */
 				LANE_WAIT(2, 0);
@@ -374,6 +375,7 @@ void cnnBackward(CNN_MODEL *model, DEVICE_DATASET *data, real *devPtr, real *z, 
 			HIP_CALL(fitre_hip_conv_input_grad_prepare(&shape, weights + wOffsets[c], preparedWs, bytes));
 			prepared[c] = preparedWs;
 			preparedWs += (bytes + 255) & ~(size_t)255;
+			if (preparedWs > preparedEnd) preparedWs = (char *)preparedEnd;
 		}
 		if (any) LANE_SELECT(0);
 		preparedPending = any;

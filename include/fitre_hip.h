@@ -432,9 +432,9 @@ typedef struct fitre_split_view {
 int fitre_hip_conv_input_grad_split(const fitre_conv_shape *s, const float *delta, const float *w, float *dx,
                                     void *ws, size_t wsBytes, fitre_split_view *view);
 /* Some shapes multiply by a rearranged copy of the weights (3x3 windows on 2 x 2 maps: the dense per-image form
- * of the convolution, 16/36 of the multiply-adds of the nine-tap form).  The copy depends on the weights only, so
+ * of the convolution, 16/36 of the multiply-adds of the nine-tap form; larger maps: their bf16 parts).  The copy depends on the weights only, so
  * a caller can have it made ahead of the chain that needs it, on another lane:
- *   _prepared_bytes  size of the copy, 0 when the shape has none (it does not depend on the number of samples);
+ *   _prepared_bytes  size of the copy, 0 when the shape has none (it may have none at another number of samples);
  *   _prepare         builds it (stream-ordered);
  *   _split_prepared  fitre_hip_conv_input_grad_split reading it (prepared == NULL: built inside, in ws).
  * No counterpart in the reference, whose weights are reordered per call (dev_backprop_convolution.cu:140-156). */
