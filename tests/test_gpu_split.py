@@ -143,6 +143,19 @@ def test_prepared_weights_give_the_same_bits(dev):
         dev.free(q)
 
 
+@pytest.mark.parametrize("case,copied", [((256, 128, 128, 8, 8, 3), True), ((8, 256, 512, 8, 8, 3), False), ((127, 512, 512, 4, 4, 3), False)])
+def test_copies_are_asked_for_only_where_the_input_gradient_reads_them(dev, case, copied):
+    """Below 2048 positions the fp32 kernels run: no copy, and none is made."""
+    n, ci, co, a, b, _ = case
+    shape = conv_shape(n, ci, co, a, b, 3, 1, 1)
+    assert (hip.fitre_hip_conv_input_grad_prepared_bytes(C.byref(shape)) > 0) == copied
+    w = dev.upload(np.zeros(ci * co * 9, np.float32))
+    room = dev.alloc(6 * ci * 9 * co)
+    assert (hip.fitre_hip_conv_input_grad_prepare(C.byref(shape), w, room, 6 * ci * 9 * co) == 0) == copied
+    dev.free(w)
+    dev.free(room)
+
+
 @pytest.mark.parametrize("case,which", [((80, 128, 128, 8, 8, 3), "fwd"), ((80, 128, 128, 8, 8, 3), "dx"), ((160, 192, 208, 4, 4, 3), "fwd")])
 def test_numbers_the_split_does_not_carry(dev, case, which):
     """Infinities, NaN, the largest floats (which round up to infinity in bf16) and tensors so small that the lower parts of
