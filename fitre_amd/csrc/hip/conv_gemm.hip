@@ -270,6 +270,7 @@ static bool split_pos_eligible(const fitre_conv_shape *s, bool dx)
 {
 	const int I = dx ? s->inChannels : s->outChannels, cred = dx ? s->outChannels : s->inChannels;
 	return (s->ksize == 3 || s->ksize == 5) && s->stride == 1 && s->padding == s->ksize / 2 && cred % kSplitCB == 0 && I > 16 && cred > 16 &&
+	       cred / kSplitCB <= 65535 && I / kCellSplitRows < 65535 && // grids
 	       conv_split_variant(s->ksize, I, s->inA, s->inB) != nullptr;
 }
 static int split_row_groups(int I) { return I <= 64 ? 2 : (I + 127) / 128 * 4; }
@@ -669,6 +670,14 @@ int gemm_ex(int transA, int transB, int M, int N, int K, float alpha, const floa
 	FITRE_REQUIRE(lda >= (transA ? K : M) && ldb >= (transB ? N : K) && ldc >= M, "fitre_hip_gemm: leading dimension too small");
 	const size_t aElems = (size_t)lda * (transA ? M : K), bElems = (size_t)ldb * (transB ? K : N);
 	FITRE_REQUIRE(aElems < ((size_t)1 << 30) && bElems < ((size_t)1 << 30), "fitre_hip_gemm: an operand exceeds 2^30 elements");
+	constexpr int kMostColumns = 65535 * kSplitGemmTile; // of one grid
+	if (N > kMostColumns) { // in two halves, as many as a grid of tiles twice as wide has
+		if (N > 2 * kMostColumns) return fail(FITRE_E_UNSUPPORTED, "fitre_hip_gemm: %d columns", N);
+		const int rc = gemm_ex(transA, transB, M, kMostColumns, K, alpha, A, lda, B, ldb, beta, C, ldc, bias, kernelClass, ws, wsBytes);
+		if (rc) return rc;
+		return gemm_ex(transA, transB, M, N - kMostColumns, K, alpha, A, lda, B + (transB ? (size_t)kMostColumns : (size_t)kMostColumns * ldb), ldb,
+		               beta, C + (size_t)kMostColumns * ldc, ldc, bias, kernelClass, ws, wsBytes);
+	}
 	const int I = N, J = M, R = K;
 	const OutParams out{ C, (long)ldc, 0, nullptr, bias, alpha, beta };
 	const double flops = 2.0 * (double)M * N * K;

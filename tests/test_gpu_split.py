@@ -317,6 +317,22 @@ def test_product(dev, M, N, K, ta, tb):
         dev.free(q)
 
 
+@pytest.mark.parametrize("tb", [0, 1])
+def test_product_of_more_columns_than_a_grid_has(dev, tb):
+    M, N, K = 5, 65535 * 64 + 5, 2
+    rng = np.random.default_rng(tb)
+    A, B = rng.standard_normal((K, M)).astype(np.float32), rng.standard_normal((K, N) if tb else (N, K)).astype(np.float32)
+    nb = hip.fitre_hip_gemm_workspace(M, N, K)
+    pa, pb, pc, ws = dev.upload(A.reshape(-1)), dev.upload(B.reshape(-1)), dev.zeros(M * N), dev.alloc(max(nb, 4))
+    L.check(hip.fitre_hip_gemm(0, tb, M, N, K, 1.0, pa, M, pb, N if tb else K, 0.0, pc, M, None, ws, nb))
+    got = dev.download(pc, M * N).reshape(N, M)
+    for q in (pa, pb, pc, ws):
+        dev.free(q)
+    edge, bound = 65535 * 64, 3 * 2.0**-24  # a sum of two products: each accumulator and their sum are rounded once
+    for cols in (slice(0, 200), slice(edge - 130, N)):
+        assert far(got[cols], (B[:, cols].T if tb else B[cols]).astype(np.float64) @ A.astype(np.float64)) < bound
+
+
 @pytest.mark.parametrize("n", [130, 200])
 def test_forward_on_2x2_maps(dev, n):
     """The dense form of 3 x 3 windows on 2 x 2 maps (through the layer's pass, without normalisation, activation and pool)."""
