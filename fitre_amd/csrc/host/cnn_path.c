@@ -285,7 +285,9 @@ static double backward_conv_work(const CNN_MODEL *model, int n)
  * 256, bytes per thousand FLOP / best share: layer 1 49 / six eighths, layer 2 24 and layer 4 12 / seven or six
  * eighths (equal within the noise), layers 3 and 5 6 and 3 / the whole chip; the pass 1.32 against 1.37 ms.  A pass with
  * few such bytes overall (AlexNet at batch 64: about 400 FLOP per byte against 140) keeps the whole chip for every weight
- * gradient: 2.82 against 3.00 ms with the shares.  The share depends on the network alone, not on whether the lanes are
+ * gradient: 2.82 against 3.00 ms with the shares.  These were fp32 kernels; with the bf16 ones (conv_split_dw.h) the optimum is
+ * flat, forward and backward of VGG-11 at 256 / VGG-16 at 128 images in us, this rule against: the whole chip for all 1823 / 2298,
+ * 1845 / 2280; limits of half as much 1826 / 2296, 1825 / 2311; an eighth less for all 1809 / 2260, 1858 / 2321.  The share depends on the network alone, not on whether the lanes are
  * in use, so that one lane and two give the same bits. */
 static double elementwise_bytes(const CONV_LAYER *l, int n)
 {
