@@ -287,8 +287,8 @@ static double backward_conv_work(const CNN_MODEL *model, int n)
  * few such bytes overall (AlexNet at batch 64: about 400 FLOP per byte against 140) keeps the whole chip for every weight
  * gradient: 2.82 against 3.00 ms with the shares.  These were fp32 kernels; with the bf16 ones (conv_split_dw.h) the optimum is
  * flat, forward and backward of VGG-11 at 256 / VGG-16 at 128 images in us, this rule against: the whole chip for all 1823 / 2298,
- * 1845 / 2280; limits of half as much 1826 / 2296, 1825 / 2311; an eighth less for all 1809 / 2260, 1858 / 2321.  The share depends on the network alone, not on whether the lanes are
- * in use, so that one lane and two give the same bits. */
+ * 1845 / 2280; limits of half as much 1826 / 2296, 1825 / 2311; an eighth less for all 1809 / 2260, 1858 / 2321.  The share
+ * depends on the network alone, not on whether the lanes are in use, so that one lane and two give the same bits. */
 static double elementwise_bytes(const CONV_LAYER *l, int n)
 {
 	return (double)n * l->outHeight * l->outWidth * l->outChannels * (has_bn(l) ? 28.0 : 16.0);
