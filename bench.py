@@ -96,14 +96,21 @@ def live_fraction(layer):
             live(layer.width, layer.outWidth, k, layer.stride, layer.padding)) / float(k * k * layer.outHeight * layer.outWidth)
 
 
+def live_rows(layer):
+    """The same with rows alone: taps whose row lies inside the image, whatever their column."""
+    k = layer.kSize
+    live = sum(1 for o in range(layer.outHeight) for t in range(k) if 0 <= o * layer.stride - layer.padding + t < layer.height)
+    return live / float(k * layer.outHeight)
+
+
 def conv_live_fractions(model, batch):
-    """Algorithmic work 2*M*K*Cout of every convolution layer's gradient launches -> the live_fraction of the layers with
+    """Algorithmic work 2*M*K*Cout of every convolution layer's gradient launches -> (live_fraction, live_rows) of the layers with
     that work (two layers can share it: VGG-11's 256 -> 256 on 8x8 maps and 512 -> 512 on 4x4 maps)."""
     table = {}
     for c in range(model.cLayers):
         l = model.convLayer[c]
         work = 2.0 * batch * l.outHeight * l.outWidth * l.inChannels * l.kSize ** 2 * l.outChannels
-        table.setdefault(round(work), []).append(live_fraction(l))
+        table.setdefault(round(work), []).append((live_fraction(l), live_rows(l)))
     return table
 
 
@@ -112,13 +119,17 @@ SKIPS_PADDING = {"/dense2x2": 16 / 36.0, "/cell4x4": 100 / 144.0, "/splitcell4x4
 
 
 def launch_live_fraction(kernel, work, conv_live):
-    """(live fraction of the layer a launch belongs to, whether its kernel leaves the padding's products out).  Layers
-    of equal work: a variant kernel names its map size; the other kernels run the layers the variants do not take, the
-    larger maps."""
+    """(live fraction of the layer a launch belongs to, fraction of the window count its kernel executes).  Layers of equal
+    work: a variant kernel names its map size; "/split" kernels run them all, so that a launch is taken as their mean (the weight
+    gradient leaves out the rows outside the image); the other kernels run what these do not take, the larger maps."""
     for suffix, frac in SKIPS_PADDING.items():
         if kernel.endswith(suffix):
-            return frac, True
-    return max(conv_live.get(round(work), [1.0])), False
+            return frac, frac
+    layers = conv_live.get(round(work), [(1.0, 1.0)])
+    if kernel.endswith("/split"):
+        live, rows = (sum(l[i] for l in layers) / len(layers) for i in (0, 1))
+        return live, rows if kernel.startswith("conv_dw") else 1.0
+    return max(layers)[0], 1.0
 
 
 def matrix_peak(kernel):
@@ -143,8 +154,8 @@ def kernel_table(rows, steps, launches=None, conv_live=None, fc_batch=None):
         for kernel, cls, work, ms in launches:
             if cls not in ("conv_dw", "conv_dx"):
                 continue
-            live, skips = launch_live_fraction(kernel, work, conv_live)
-            executed[kernel] = executed.get(kernel, 0.0) + work * (live if skips else 1.0)
+            live, done = launch_live_fraction(kernel, work, conv_live)
+            executed[kernel] = executed.get(kernel, 0.0) + work * done
             useful[kernel] = useful.get(kernel, 0.0) + work * live
     for r in rows:
         avg_us = 1e3 * r["ms"] / r["launches"]
