@@ -70,8 +70,10 @@ struct SplitRowContig {
 #pragma unroll
 		for (int e = 0; e < U::UNITS; e++)
 #pragma unroll
-			for (int q = 0; q < 8; q++)
-				off[e][q] = row0 + row < pr.rows ? 4u * (uint32_t)((8 * (groupL + kGemmThreads / ROWS * e) + q) * ld + row0 + row) : kOutOfRange;
+			for (int q = 0; q < 8; q++) { // (a slice of a short reduction may reach past 2^32 bytes: there is no such operand)
+				const unsigned long long at = (unsigned long long)(8 * (groupL + kGemmThreads / ROWS * e) + q) * (unsigned)ld + (unsigned)(row0 + row);
+				off[e][q] = row0 + row < pr.rows && at < (1ull << 30) ? 4u * (uint32_t)at : kOutOfRange;
+			}
 	}
 	__device__ __forceinline__ void load(int k0, int, U &u) const
 	{

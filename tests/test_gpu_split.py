@@ -333,6 +333,26 @@ def test_product_of_more_columns_than_a_grid_has(dev, tb):
         assert far(got[cols], (B[:, cols].T if tb else B[cols]).astype(np.float64) @ A.astype(np.float64)) < bound
 
 
+@pytest.mark.parametrize("ta,tb,M,N", [(0, 0, 36_000_000, 2), (1, 1, 510_000, 130)])
+def test_product_of_a_short_reduction_with_a_large_leading_dimension(dev, ta, tb, M, N):
+    """Two reduction indices 36 million apart: the other thirty of a slice lie past 2^32 bytes, where 32-bit offsets would come
+    back into the tensor; the other operand's rows are followed by numbers that are not part of the product."""
+    K, far_apart, padded = 2, 36_000_000, 40
+    rng = np.random.default_rng(M)
+    A = rng.standard_normal((M, padded) if ta else (K, far_apart)).astype(np.float32)
+    B = rng.standard_normal((K, far_apart) if tb else (N, padded)).astype(np.float32)
+    nb = hip.fitre_hip_gemm_workspace(M, N, K)
+    pa, pb, pc, ws = dev.upload(A.reshape(-1)), dev.upload(B.reshape(-1)), dev.zeros(M * N), dev.alloc(max(nb, 4))
+    L.check(hip.fitre_hip_gemm(ta, tb, M, N, K, 1.0, pa, A.shape[1], pb, B.shape[1], 0.0, pc, M, None, ws, nb))
+    got = dev.download(pc, M * N).reshape(N, M)
+    for q in (pa, pb, pc, ws):
+        dev.free(q)
+    opB = (B[:, :N].T if tb else B[:, :K]).astype(np.float64)
+    for rows in (slice(0, 5000), slice(M - 5000, M)):
+        opA = (A[rows, :K].T if ta else A[:, rows]).astype(np.float64)
+        assert far(got[:, rows], opB @ opA) < 3 * 2.0**-24  # each accumulator and their sum are rounded once
+
+
 @pytest.mark.parametrize("n", [130, 200])
 def test_forward_on_2x2_maps(dev, n):
     """The dense form of 3 x 3 windows on 2 x 2 maps (through the layer's pass, without normalisation, activation and pool)."""
