@@ -318,7 +318,7 @@ conv_split_kernel(const ConvSplitParams p, const OutParams out)
 		for (int v = 0; v < 16; v++) {
 			const int i = i0 + wave / WN * 32 + 8 * (v / 4) + 4 * khalf + (v % 4);
 			if (i >= p.I) continue;
-			float val = acc[tn][v];
+			float val = acc[tn][v] * kSplitSumScale;
 			if (!split && out.biasI) val += out.biasI[i];
 			C[(size_t)i * out.ldc + j] = val;
 		}
@@ -423,7 +423,7 @@ conv_split_cell_kernel(const ConvSplitParams p, const OutParams out)
 #pragma unroll
 				for (int i = 0; i < 12; i++) {
 					__builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-					__builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+					__builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
 				}
 			}
 			__builtin_amdgcn_sched_barrier(0);
@@ -459,7 +459,7 @@ conv_split_cell_kernel(const ConvSplitParams p, const OutParams out)
 	for (int c = 0; c < 4; c++) {
 		const int cell = (qa ? 3 - (c >> 1) : (c >> 1)) * 4 + (qb ? 3 - (c & 1) : (c & 1));
 #pragma unroll
-		for (int v = 0; v < 16; v++) R[((8 * (v / 4) + 4 * khalf + (v % 4)) * kCellSplitImages + l32) * ROW + cell] = acc[c][v];
+		for (int v = 0; v < 16; v++) R[((8 * (v / 4) + 4 * khalf + (v % 4)) * kCellSplitImages + l32) * ROW + cell] = acc[c][v] * kSplitSumScale;
 	}
 	__syncthreads();
 	for (int e = tid; e < kCellSplitRows * kCellSplitImages * 4; e += kGemmThreads) {

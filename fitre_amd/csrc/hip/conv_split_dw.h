@@ -72,13 +72,11 @@ __device__ __forceinline__ void split_dw_exact_tile(const ConvSplitDwParams &p, 
 	}
 }
 
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Wpass-failed" // three waves a SIMD: what bounds the registers, where LDS has room for two
-// OB: blocks of 32 output channels of a wave.  3 x 3 windows: held to 168 registers where the compiler would take 249 (same time
-// alone: 103 us for 256 -> 256 channels on 8 x 8 maps): two workgroups on a compute unit leave 176 on every SIMD, on which the
-// bandwidth kernels of the layer below run.
+// OB: blocks of 32 output channels of a wave.  3 x 3 windows take 193 registers: two workgroups on a compute unit leave 126 on
+// every SIMD, on which the bandwidth kernels of the layer below run.  (Asked for three waves a SIMD the compiler puts the sums
+// into accumulator registers beside 124 others, 220 together: the same time.)
 template <int KS, int MODE, int OB, int WO, int WC>
-__global__ void __launch_bounds__(64 * WO *WC, KS == 3 ? 3 : 2)
+__global__ void __launch_bounds__(64 * WO *WC, 2)
 conv_split_dw_kernel(const ConvSplitDwParams p)
 {
 	FITRE_RAISE_MATRIX_WAVE_PRIORITY();
@@ -222,7 +220,7 @@ conv_split_dw_kernel(const ConvSplitDwParams p)
 	_Pragma("unroll") for (int i = 0; i < (MFMAS); i++)                                                               \
 	{                                                                                                                 \
 		__builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                                            \
-		__builtin_amdgcn_sched_group_barrier(0x002, 7, 0);                                                            \
+		__builtin_amdgcn_sched_group_barrier(0x002, 9, 0);                                                            \
 	}
 
 	SPLIT_DW_LOAD(stBeg);
@@ -313,11 +311,9 @@ conv_split_dw_kernel(const ConvSplitDwParams p)
 #pragma unroll
 			for (int v = 0; v < 16; v++) {
 				const int o = o0 + wo * 32 * OB + b * 32 + 8 * (v / 4) + 4 * khalf + (v % 4);
-				if (o < p.I) partial[((size_t)(ta * KS + t) * p.I + o) * p.cin + c] = acc[b][t][v];
+				if (o < p.I) partial[((size_t)(ta * KS + t) * p.I + o) * p.cin + c] = acc[b][t][v] * kSplitSumScale;
 			}
 }
-
-#pragma clang diagnostic pop
 
 // dW[o][c][tap] = sum over the ranges, in order.  64 (o, c) x four phases a workgroup; a phase adds every fourth range, the
 // phases are added in order.  blockIdx.y: tap row.

@@ -229,7 +229,7 @@ split_gemm_kernel(const typename OpA::Params pa, const typename OpB::Params pb, 
 	opA.load(kbeg + 2 * BK, kend, ua[0]);
 	opB.load(kbeg + 2 * BK, kend, ub[0]);
 	__syncthreads();
-	constexpr int STEPS = BK / 16, MFMAS = STEPS * TM * TN * 6, VECTOR = (OpA::U::UNITS + OpB::U::UNITS) * 46;
+	constexpr int STEPS = BK / 16, MFMAS = STEPS * TM * TN * 6, VECTOR = (OpA::U::UNITS + OpB::U::UNITS) * 54;
 #define SPLIT_GEMM_PRODUCTS(SUM, PA, PB)                                                                              \
 	_Pragma("unroll") for (int tm = 0; tm < TM; tm++)                                                                 \
 		_Pragma("unroll") for (int tn = 0; tn < TN; tn++) SUM[tm][tn] = mfma_bf16(a[step][tm][PA], b[step][tn][PB], SUM[tm][tn]);
@@ -306,7 +306,7 @@ split_gemm_kernel(const typename OpA::Params pa, const typename OpB::Params pb, 
 #pragma unroll
 			for (int v = 0; v < 16; v++) {
 				const int i = i0 + wm * (BM / 2) + tm * 32 + 8 * (v / 4) + 4 * khalf + (v % 4);
-				if (i < I) split_gemm_store(out, C, i, j, acc[tm][tn][v]);
+				if (i < I) split_gemm_store(out, C, i, j, acc[tm][tn][v] * kSplitSumScale);
 			}
 		}
 }

@@ -353,30 +353,74 @@ def test_product_of_a_short_reduction_with_a_large_leading_dimension(dev, ta, tb
         assert far(got[:, rows], opB @ opA) < 3 * 2.0**-24  # each accumulator and their sum are rounded once
 
 
-@pytest.mark.parametrize("n", [130, 200])
-def test_forward_on_2x2_maps(dev, n):
+def forward_2x2(dev, case, x, w):
     """The dense form of 3 x 3 windows on 2 x 2 maps (through the layer's pass, without normalisation, activation and pool)."""
     from fitre_amd.structs import CNN_ACT_NONE, NO_POOL
+    n, ci, co = case[:3]
+    shape = conv_shape(n, ci, co, 2, 2, 3, 1, 1)
+    nb, size = hip.fitre_hip_conv_bn_act_pool_workspace(C.byref(shape), 0), co * n * 4
+    px, pw, ws, y, act = dev.upload(flat(x)), dev.upload(w.numpy().ravel()), dev.alloc(nb), dev.zeros(size), dev.zeros(size)
+    L.check(hip.fitre_hip_conv_bn_act_pool_forward(C.byref(shape), px, pw, None, y, None, None, None, None, None, 1e-5, 0.1, 1, CNN_ACT_NONE,
+                                                   act, NO_POOL, 0, 0, 0, 0, 0, None, 0, ws, nb))
+    got = dev.download(y, size).reshape(co, n, 2, 2)
+    for q in (px, pw, ws, y, act):
+        dev.free(q)
+    return got
+
+
+@pytest.mark.parametrize("n", [130, 200])
+def test_forward_on_2x2_maps(dev, n):
     ci, co = 96, 132
     case = (n, ci, co, 2, 2, 3)
-    shape = conv_shape(n, ci, co, 2, 2, 3, 1, 1)
     x, w, _ = tensors(case)
-    nb, size = hip.fitre_hip_conv_bn_act_pool_workspace(C.byref(shape), 0), co * n * 4
-
-    def run(source):
-        px, pw, ws, y, act = dev.upload(flat(source)), dev.upload(w.numpy().ravel()), dev.alloc(nb), dev.zeros(size), dev.zeros(size)
-        L.check(hip.fitre_hip_conv_bn_act_pool_forward(C.byref(shape), px, pw, None, y, None, None, None, None, None, 1e-5, 0.1, 1, CNN_ACT_NONE,
-                                                       act, NO_POOL, 0, 0, 0, 0, 0, None, 0, ws, nb))
-        got = dev.download(y, size).reshape(co, n, 2, 2)
-        for q in (px, pw, ws, y, act):
-            dev.free(q)
-        return got
-
-    assert far(run(x), reference(case, "fwd", x, w)) < limit(ci * 4)
+    assert far(forward_2x2(dev, case, x, w), reference(case, "fwd", x, w)) < limit(ci * 4)
     odd = x.clone()
     odd[5, 3, 1, 0], odd[n - 1, 95, 0, 1] = float("inf"), float("nan")
-    got, want = run(odd), reference(case, "fwd", odd, w)
+    got, want = forward_2x2(dev, case, odd, w), reference(case, "fwd", odd, w)
     finite = np.isfinite(want)
     np.testing.assert_array_equal(np.isfinite(got), finite)
     assert far(got[finite], want[finite]) < limit(ci * 4, 0.6)
-    assert far(run(x * 2.0**-108) * 2.0**108, reference(case, "fwd", x, w)) < limit(ci * 4, 0.6)
+    assert far(forward_2x2(dev, case, x * 2.0**-108, w) * 2.0**108, reference(case, "fwd", x, w)) < limit(ci * 4, 0.6)
+
+
+def product(dev, a, b):
+    (K, M), N = a.shape, b.shape[0]
+    nb = hip.fitre_hip_gemm_workspace(M, N, K)
+    pa, pb, pc, ws = dev.upload(a.numpy().ravel()), dev.upload(b.numpy().ravel()), dev.zeros(M * N), dev.alloc(max(nb, 4))
+    L.check(hip.fitre_hip_gemm(0, 0, M, N, K, 1.0, pa, M, pb, K, 0.0, pc, M, None, ws, nb))
+    got = dev.download(pc, M * N).reshape(N, M)
+    for q in (pa, pb, pc, ws):
+        dev.free(q)
+    return got
+
+
+def one_of_each(kernel):
+    """(factors, run(dev, factors), float64 result, terms of a sum) of a product on one of the kernels."""
+    if kernel == "product":
+        g = torch.Generator().manual_seed(1)
+        factors = torch.randn(777, 200, generator=g), torch.randn(130, 777, generator=g)
+        return factors, product, lambda a, b: (b.double() @ a.double()).numpy(), 777
+    case = {"forward": (80, 128, 128, 8, 8, 3), "input gradient": (80, 128, 128, 8, 8, 3), "cell": (159, 192, 208, 4, 4, 3), "2x2": (130, 96, 132, 2, 2, 3),
+            "weight gradient": (64, 128, 128, 8, 8, 3), "weight gradient 5x5": (20, 64, 64, 15, 15, 5)}[kernel]
+    x, w, d = tensors(case)
+    if kernel.startswith("weight"):
+        return (x, d), lambda dev, x, d: weight_grad(dev, case, x, d), lambda x, d: weight_reference(case, x, d), case[0] * case[3] * case[4]
+    which = "dx" if kernel == "input gradient" else "fwd"
+    run = (lambda dev, s, w: forward_2x2(dev, case, s, w)) if kernel == "2x2" else (lambda dev, s, w: conv(dev, case, which, s, w))
+    return (d if which == "dx" else x, w), run, lambda s, w: reference(case, which, s, w), case[1] * case[5] ** 2
+
+
+@pytest.mark.parametrize("kernel", ["forward", "input gradient", "cell", "2x2", "weight gradient", "weight gradient 5x5", "product"])
+def test_small_numbers(dev, kernel):
+    """Factors of any size are carried, subnormal ones too: a power of two in front of a tensor changes no bit, a factor without its
+    lower parts is not hidden by a large one beside it, and what is below the smallest normal result is rounded, not dropped."""
+    (a, b), run, want, terms = one_of_each(kernel)
+    plain = run(dev, a, b)
+    np.testing.assert_array_equal(run(dev, a * 2.0**-100, b), plain * np.float32(2.0**-100))
+    np.testing.assert_array_equal(run(dev, a, b * 2.0**-100), plain * np.float32(2.0**-100))
+    for first, second in ((-124, 60), (-138, 100), (60, -124), (100, -138)):
+        fa, fb = a * 2.0**first, b * 2.0**second  # from 2^-127 on rounded to the numbers there are
+        back = 2.0 ** -(first + second)
+        assert far(run(dev, fa, fb).astype(np.float64) * back, want(fa, fb) * back) < limit(terms)
+    tiny = run(dev, a * 2.0**-70, b * 2.0**-70).astype(np.float64) - want(a * 2.0**-70, b * 2.0**-70)
+    assert np.abs(tiny).max() < (terms / 16 + 1) * 2.0**-150  # every range of the reduction is rounded once, the shortest has sixteen terms
