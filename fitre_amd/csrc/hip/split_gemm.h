@@ -91,8 +91,8 @@ struct SplitRowContig {
 	static __device__ __forceinline__ float at(const Params &pr, int i, int k) { return pr.p[(size_t)k * pr.ld + i]; }
 };
 
-// element(row, k) = p[row * ld + k].  MASK: what lies behind kend is made zero; one operand of a product is enough (a number
-// there times the other's zero is zero, or not finite and then found in the sum).
+// element(row, k) = p[row * ld + k].  MASK: what lies behind kend is made zero.  One operand of a product is enough where the other's
+// rows follow each other: a number of the matrix times zero is zero, or not finite and then found in the sum.
 template <int ROWS, int BK, bool MASK>
 struct SplitKContigT {
 	typedef SplitUnits<ROWS, BK> U;

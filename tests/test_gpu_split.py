@@ -353,6 +353,26 @@ def test_product_of_a_short_reduction_with_a_large_leading_dimension(dev, ta, tb
         assert far(got[:, rows], opB @ opA) < 3 * 2.0**-24  # each accumulator and their sum are rounded once
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (1, 1)])
+def test_product_of_padded_matrices(dev, ta, tb):
+    """What lies between the rows of a matrix has no part in a sum, nor in how it is computed: the same bits whatever it is."""
+    M, N, K = 200, 130, 777
+    rng = np.random.default_rng(ta + 2 * tb)
+    A = rng.standard_normal((M, K + 7) if ta else (K, M + 7)).astype(np.float32)
+    B = rng.standard_normal((K, N + 7) if tb else (N, K + 7)).astype(np.float32)
+    nb = hip.fitre_hip_gemm_workspace(M, N, K)
+    got = []
+    for between in (0.0, np.nan, np.inf):
+        A[:, -7:] = B[:, -7:] = between
+        pa, pb, pc, ws = dev.upload(A.reshape(-1)), dev.upload(B.reshape(-1)), dev.zeros(M * N), dev.alloc(max(nb, 4))
+        L.check(hip.fitre_hip_gemm(ta, tb, M, N, K, 1.0, pa, A.shape[1], pb, B.shape[1], 0.0, pc, M, None, ws, nb))
+        got.append(dev.download(pc, M * N))
+        for q in (pa, pb, pc, ws):
+            dev.free(q)
+    np.testing.assert_array_equal(got[0], got[1])
+    np.testing.assert_array_equal(got[0], got[2])
+
+
 def forward_2x2(dev, case, x, w):
     """The dense form of 3 x 3 windows on 2 x 2 maps (through the layer's pass, without normalisation, activation and pool)."""
     from fitre_amd.structs import CNN_ACT_NONE, NO_POOL
