@@ -42,9 +42,10 @@ template <int KS, int MODE, int OT, int CT, int WAVES>
 __device__ __forceinline__ void split_dw_exact_tile(const ConvSplitDwParams &p, int o0, int c0, int ta, int stBeg, int stEnd, float *partial)
 {
 	constexpr int P = KS / 2;
+	static_assert(CT % 64 == 0, "whole groups of 64 (input channel, tap)");
 	const int lane = threadIdx.x & 63, off = ta - P, a0 = off < 0 ? -off : 0, live = p.A - (off < 0 ? -off : off);
 	const int rows = p.samples * live;
-	for (int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); g < OT / 8 * (CT * KS / 32); g += WAVES) {
+	for (int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); g < OT / 8 * (CT * KS / 64); g += WAVES) {
 		const int oBase = o0 + g % (OT / 8) * 8, e = g / (OT / 8) * 64 + lane;
 		const int c = c0 + e % CT, tb = e / CT;
 		if (oBase >= p.I) continue;
