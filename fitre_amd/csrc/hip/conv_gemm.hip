@@ -123,9 +123,11 @@ static BlockPlan fit_blocks(BlockPlan p, long nBlocks, long I, long J, const voi
 	return p;
 }
 
+// a workspace query comes with any numbers; those of the position kernels divide by a map's cells
+static bool is_map(const fitre_conv_shape *s) { return s->inA > 0 && s->inB > 0 && (long)s->inA * s->inB <= 1 << 30; }
 static bool c3_geometry(const fitre_conv_shape *s)
 {
-	return s->ksize == 3 && s->stride == 1 && s->padding == 1 && s->inB <= 64 && s->outA == s->inA && s->outB == s->inB;
+	return is_map(s) && s->ksize == 3 && s->stride == 1 && s->padding == 1 && s->inB <= 64 && s->outA == s->inA && s->outB == s->inB;
 }
 // forward: reduce over Cin; input gradient: reduce over Cout
 static bool c3_pos_eligible(const fitre_conv_shape *s, bool dx)
@@ -269,7 +271,7 @@ static int launch_c3_pos(const fitre_conv_shape *s, const float *src, const floa
 static bool split_pos_eligible(const fitre_conv_shape *s, bool dx)
 {
 	const int I = dx ? s->inChannels : s->outChannels, cred = dx ? s->outChannels : s->inChannels;
-	return (s->ksize == 3 || s->ksize == 5) && s->stride == 1 && s->padding == s->ksize / 2 && cred % kSplitCB == 0 && I > 16 && cred > 16 &&
+	return is_map(s) && (s->ksize == 3 || s->ksize == 5) && s->stride == 1 && s->padding == s->ksize / 2 && cred % kSplitCB == 0 && I > 16 && cred > 16 &&
 	       cred / kSplitCB <= 65535 && I / kCellSplitRows < 65535 && // grids
 	       conv_split_variant(s->ksize, I, s->inA, s->inB) != nullptr;
 }

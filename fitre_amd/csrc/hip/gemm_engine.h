@@ -852,6 +852,7 @@ inline GemmPlan plan_gemm(long I, long J, long R, bool mirror = false, int cus =
 // Workspace that covers the plan of every lane (a size query does not know the lane of the launch).
 inline size_t plan_gemm_workspace(long I, long J, long R, bool mirror = false, bool rows96 = false)
 {
+	if (I <= 0 || J <= 0 || R <= 0) return 0; // of a shape that is none
 	size_t a = plan_gemm(I, J, R, mirror, device_compute_units(), rows96).wsBytes;
 	size_t b = plan_gemm(I, J, R, mirror, lane_compute_units_min(), rows96).wsBytes;
 	return a > b ? a : b;
