@@ -1,7 +1,10 @@
 """fp32 products on the bf16 matrix pipes (fitre_amd/csrc/hip/split_bf16.h): convolutions large enough to take them, against
 float64.  A sum of K normal terms in fp32 multiply-adds is off by a random walk of K roundings, measured at 0.3 sqrt(K) 2^-24 of
-its norm; these kernels round less often (0.1), and a product that drops one of its six parts is off by 2^-17 or more."""
+its norm; these kernels round less often (0.1), and a product that drops one of its six parts is off by 2^-17 or more.
+
+Every call is made under the launch accounting, which says whether the kernel that the case is written for was the one that ran."""
 import ctypes as C
+from contextlib import contextmanager
 
 import numpy as np
 import pytest
@@ -32,11 +35,37 @@ def tensors(case, seed=0):
     return x, w, d
 
 
+CONV_DW, CONV_DX, CONV_FWD, FC_GEMM = 0, 1, 2, 3  # kernel classes and tile variants of include/fitre_hip.h
+FP32, SPLIT, CELL = "fp32", 10, 11
+
+
+@contextmanager
+def taken(kernel_class, tile, launches=1):
+    """The launches of a class made inside are of this variant (FP32: none of either split one)."""
+    count, ms, work = C.c_long(), C.c_double(), C.c_double()
+    L.check(hip.fitre_hip_profile_enable(1))
+    try:
+        yield
+        made = {}
+        for t in (SPLIT, CELL):
+            L.check(hip.fitre_hip_profile_read_tile(kernel_class, t, C.byref(count), C.byref(ms), C.byref(work)))
+            made[t] = count.value
+    finally:
+        L.check(hip.fitre_hip_profile_enable(0))
+    assert made == {t: launches * (t == tile) for t in (SPLIT, CELL)}
+
+
+def form(case, which, second=None):
+    """The window form, or the cell form on 4 x 4 maps that fill its tiles of 32 images (no input gradient on its own)."""
+    n, cell = case[0], case[3:] == (4, 4, 3) and (which == "fwd" or second)
+    return CELL if cell and 100 * (-(-n // 32) * 32) < 137 * n else SPLIT
+
+
 def flat(t):  # the library's order of a tensor [N][C][A][B]
     return t.transpose(0, 1).contiguous().numpy().ravel()
 
 
-def conv(dev, case, which, source, w, second=None, bias=None, ws_bytes=None):
+def conv(dev, case, which, source, w, second=None, bias=None, ws_bytes=None, tile=None):
     n, ci, co, a, b, k = case
     shape = conv_shape(n, ci, co, a, b, k, 1, k // 2)
     out_channels = co if which == "fwd" else ci
@@ -50,15 +79,16 @@ def conv(dev, case, which, source, w, second=None, bias=None, ws_bytes=None):
     if second:
         p2, w2 = dev.upload(flat(second[0])), dev.upload(second[1].numpy().ravel())
         bufs += [p2, w2]
-    if which == "fwd":
-        pb = dev.upload(bias.numpy()) if bias is not None else None
-        if pb:
-            bufs.append(pb)
-        L.check(hip.fitre_hip_conv_forward_pair(C.byref(shape), ps, pw, p2, w2, pb, out, ws, nb) if second else
-                hip.fitre_hip_conv_forward(C.byref(shape), ps, pw, pb, out, ws, nb))
-    else:
-        L.check(hip.fitre_hip_conv_input_grad_pair(C.byref(shape), ps, pw, p2, w2, out, ws, nb) if second else
-                hip.fitre_hip_conv_input_grad(C.byref(shape), ps, pw, out, ws, nb))
+    pb = dev.upload(bias.numpy()) if bias is not None else None
+    if pb:
+        bufs.append(pb)
+    with taken(CONV_FWD if which == "fwd" else CONV_DX, tile or form(case, which, second)):
+        if which == "fwd":
+            L.check(hip.fitre_hip_conv_forward_pair(C.byref(shape), ps, pw, p2, w2, pb, out, ws, nb) if second else
+                    hip.fitre_hip_conv_forward(C.byref(shape), ps, pw, pb, out, ws, nb))
+        else:
+            L.check(hip.fitre_hip_conv_input_grad_pair(C.byref(shape), ps, pw, p2, w2, out, ws, nb) if second else
+                    hip.fitre_hip_conv_input_grad(C.byref(shape), ps, pw, out, ws, nb))
     got = dev.download(out, out_channels * n * a * b).reshape(out_channels, n, a, b)
     for q in bufs:
         dev.free(q)
@@ -76,22 +106,23 @@ CASES = [
     (77, 128, 160, 8, 8, 3),   # 160 channels: a partial channel tile; 4928 positions: a partial position tile
     (77, 160, 128, 8, 8, 3),
     (130, 256, 256, 4, 4, 3),  # many images in a window, split reduction; forward in the cell form, two images in the last tile
-    (128, 256, 272, 4, 4, 3),  # whole tiles of images, a partial tile of channels
-    (66, 512, 256, 4, 4, 3),   # too little in the last tile of images for the cell form
+    (224, 256, 272, 4, 4, 3),  # whole tiles of images, a partial tile of channels
+    (132, 512, 256, 4, 4, 3),
     (260, 256, 256, 4, 2, 3),  # rectangular
-    (40, 64, 192, 16, 16, 3),  # the input gradient has 64 channels: 256-position tiles
+    (56, 64, 192, 16, 16, 3),  # the input gradient has 64 channels: 256-position tiles
     (21, 64, 128, 32, 32, 3),  # rows of 32
     (7, 128, 144, 27, 64, 3),  # the widest row
-    (150, 48, 272, 13, 5, 3),  # odd extents
-    (40, 32, 48, 40, 24, 3),   # at most 64 channels each way
+    (200, 48, 272, 13, 5, 3),  # odd extents
+    (115, 32, 48, 40, 24, 3),  # at most 64 channels each way
     (40, 64, 192, 13, 13, 5),  # 5 x 5 windows
     (11, 64, 192, 27, 27, 5),
     (30, 96, 80, 9, 14, 5),
 ]
 
 
-@pytest.mark.parametrize("which", ["fwd", "dx"])
-@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("case,which", [(case, which) for case in CASES for which in ("fwd", "dx")] + [
+    ((66, 512, 256, 4, 4, 3), "fwd"),  # too little in the last tile of images for the cell form
+])
 def test_convolution(dev, case, which):
     x, w, d = tensors(case)
     source = x if which == "fwd" else d
@@ -118,8 +149,9 @@ def test_smaller_workspaces(dev):
     x, w, _ = tensors(case)
     want = reference(case, "fwd", x, w)
     weights = 6 * 9 * 256 * 256
-    for ws_bytes in (lambda nb: nb, lambda nb: weights + 2 * 4 * 256 * 40 * 64 + 600, lambda nb: weights + 256, lambda nb: weights):
-        assert far(conv(dev, case, "fwd", x, w, ws_bytes=ws_bytes), want) < limit(256 * 9)
+    for ws_bytes, tile in ((lambda nb: nb, SPLIT), (lambda nb: weights + 2 * 4 * 256 * 40 * 64 + 600, SPLIT), (lambda nb: weights + 256, SPLIT),
+                           (lambda nb: weights, FP32)):
+        assert far(conv(dev, case, "fwd", x, w, ws_bytes=ws_bytes, tile=tile), want) < limit(256 * 9)
 
 
 def test_prepared_weights_give_the_same_bits(dev):
@@ -133,11 +165,13 @@ def test_prepared_weights_give_the_same_bits(dev):
     nb = prepared_bytes + 256  # no room for partial results: one range
     pd, pw, ws, out, prepared = dev.upload(flat(d)), dev.upload(w.numpy().ravel()), dev.alloc(nb), dev.zeros(ci * n * a * b), dev.alloc(prepared_bytes)
     view = fitre_split_view()
-    L.check(hip.fitre_hip_conv_input_grad_split(C.byref(shape), pd, pw, out, ws, nb, C.byref(view)))
+    with taken(CONV_DX, SPLIT):
+        L.check(hip.fitre_hip_conv_input_grad_split(C.byref(shape), pd, pw, out, ws, nb, C.byref(view)))
     assert view.splits == 1
     first = dev.download(out, ci * n * a * b)
     L.check(hip.fitre_hip_conv_input_grad_prepare(C.byref(shape), pw, prepared, prepared_bytes))
-    L.check(hip.fitre_hip_conv_input_grad_split_prepared(C.byref(shape), pd, pw, prepared, out, ws, nb, C.byref(view)))
+    with taken(CONV_DX, SPLIT):
+        L.check(hip.fitre_hip_conv_input_grad_split_prepared(C.byref(shape), pd, pw, prepared, out, ws, nb, C.byref(view)))
     np.testing.assert_array_equal(dev.download(out, ci * n * a * b), first)
     for q in (pd, pw, ws, out, prepared):
         dev.free(q)
@@ -156,7 +190,7 @@ def test_copies_are_asked_for_only_where_the_input_gradient_reads_them(dev, case
     dev.free(room)
 
 
-@pytest.mark.parametrize("case,which", [((80, 128, 128, 8, 8, 3), "fwd"), ((80, 128, 128, 8, 8, 3), "dx"), ((160, 192, 208, 4, 4, 3), "fwd")])
+@pytest.mark.parametrize("case,which", [((80, 128, 128, 8, 8, 3), "fwd"), ((80, 128, 128, 8, 8, 3), "dx"), ((159, 192, 208, 4, 4, 3), "fwd")])
 def test_numbers_the_split_does_not_carry(dev, case, which):
     """Infinities, NaN, the largest floats (which round up to infinity in bf16) and tensors so small that the lower parts of
     their numbers are below the smallest bf16 number: what an fp32 chain gives."""
@@ -181,17 +215,18 @@ def test_numbers_the_split_does_not_carry(dev, case, which):
     assert far(conv(dev, case, which, small, w) * 2.0**108, reference(case, which, source, w)) < limit(terms, 0.6)
 
 
-def weight_grad(dev, case, x, d, second=None, ws_bytes=None):
+def weight_grad(dev, case, x, d, second=None, ws_bytes=None, tile=SPLIT):
     n, ci, co, a, b, k = case
     shape = conv_shape(n, ci, co, a, b, k, 1, k // 2)
     nb = hip.fitre_hip_conv_pair_workspace(C.byref(shape), 2) if second else hip.fitre_hip_conv_weight_grad_workspace(C.byref(shape))
     nb = nb if ws_bytes is None else ws_bytes(nb)
     bufs = [dev.upload(flat(t)) for t in (x, d) + (second or ())] + [dev.alloc(nb), dev.zeros(co * ci * k * k)]
     ws, out = bufs[-2:]
-    if second:
-        L.check(hip.fitre_hip_conv_weight_grad_pair(C.byref(shape), *bufs[:4], out, ws, nb))
-    else:
-        L.check(hip.fitre_hip_conv_weight_grad(C.byref(shape), *bufs[:2], out, ws, nb))
+    with taken(CONV_DW, tile):
+        if second:
+            L.check(hip.fitre_hip_conv_weight_grad_pair(C.byref(shape), *bufs[:4], out, ws, nb))
+        else:
+            L.check(hip.fitre_hip_conv_weight_grad(C.byref(shape), *bufs[:2], out, ws, nb))
     got = dev.download(out, co * ci * k * k).reshape(co, ci, k, k)
     for q in bufs:
         dev.free(q)
@@ -203,27 +238,32 @@ def weight_reference(case, x, d):
     return torch.nn.grad.conv2d_weight(x.double(), (case[2], case[1], k, k), d.double(), padding=k // 2).numpy()
 
 
-# the three ways a row is cut into groups, every arrangement of waves, partial tiles of either kind of channels, and numbers of
-# image rows that are no whole groups or stages
+# the three ways a row is cut into groups, every arrangement of waves with each, partial tiles of either kind of channels, and
+# numbers of image rows that are no whole groups or stages
 WEIGHT_CASES = [
     (130, 256, 272, 4, 4, 3),  # two rows a group
     (151, 200, 264, 5, 3, 3),  # rows of three cells, an odd number of rows
-    (128, 64, 64, 4, 4, 3),    # 64 x 64 tiles
+    (256, 64, 64, 4, 4, 3),    # 64 x 64 tiles
     (33, 160, 144, 8, 8, 3),   # a row a group
-    (51, 72, 130, 7, 6, 3),
-    (32, 40, 48, 8, 8, 3),
-    (41, 130, 64, 9, 7, 3),    # 64 x 128 tiles
-    (23, 64, 192, 13, 13, 3),  # two groups a row, the second five cells
+    (130, 72, 130, 7, 6, 3),
+    (512, 72, 130, 1, 8, 3),   # one image row: two of three tap rows are outside
+    (112, 40, 48, 8, 8, 3),    # 64 x 64 tiles
+    (97, 130, 64, 9, 7, 3),
+    (25, 64, 192, 13, 13, 3),  # two groups a row, the second five cells
     (9, 100, 70, 16, 16, 3),
+    (10, 96, 64, 16, 16, 3),   # 64 x 64 tiles
     (6, 96, 128, 12, 32, 3),   # four groups a row
-    (4, 64, 128, 27, 27, 3),
-    (8, 128, 64, 11, 24, 3),   # three of four groups
+    (9, 64, 128, 27, 27, 3),
+    (8, 128, 64, 11, 24, 3),   # three of four groups, 64 x 64 tiles
     (13, 64, 192, 13, 13, 5),  # 5 x 5 windows
     (18, 80, 160, 15, 8, 5),
-    (4, 64, 96, 20, 30, 5),
+    (5, 64, 96, 20, 30, 5),
+    (5, 64, 192, 27, 27, 5),
     (20, 72, 64, 15, 14, 5),   # at most 64 output channels
-    (50, 48, 40, 8, 8, 5),
-    (65, 64, 64, 2, 16, 5),    # fewer image rows than the window
+    (150, 48, 40, 8, 8, 5),
+    (5, 96, 64, 27, 27, 5),
+    (140, 64, 64, 2, 16, 5),   # fewer image rows than the window
+    (280, 64, 64, 1, 16, 5),
 ]
 
 
@@ -245,8 +285,8 @@ def test_weight_gradient_in_smaller_workspaces(dev):
     case = (64, 128, 128, 8, 8, 3)
     x, _, d = tensors(case)
     want, one = weight_reference(case, x, d), 4 * 128 * 128 * 9
-    for ws_bytes in (lambda nb: nb - one, lambda nb: nb * 3 // 4, lambda nb: 3 * one, lambda nb: 4):
-        assert far(weight_grad(dev, case, x, d, ws_bytes=ws_bytes), want) < limit(64 * 64)
+    for ws_bytes, tile in ((lambda nb: nb - one, SPLIT), (lambda nb: nb * 3 // 4, SPLIT), (lambda nb: 3 * one, FP32), (lambda nb: 4, FP32)):
+        assert far(weight_grad(dev, case, x, d, ws_bytes=ws_bytes, tile=tile), want) < limit(64 * 64)
 
 
 @pytest.mark.parametrize("case", [(64, 128, 128, 8, 8, 3), (130, 128, 256, 4, 4, 3), (20, 64, 128, 16, 16, 3), (20, 64, 64, 15, 15, 5)])
@@ -269,7 +309,7 @@ def test_numbers_the_split_does_not_carry_in_a_weight_gradient(dev, case):
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
-@pytest.mark.parametrize("M,N,K", [(200, 130, 777), (64, 64, 640), (131, 600, 96)])
+@pytest.mark.parametrize("M,N,K", [(200, 130, 777), (64, 64, 2560), (131, 600, 520)])
 def test_product(dev, M, N, K, ta, tb):
     """alpha, beta and a bias, and the numbers the split does not carry: in the middle, in a corner, at a ragged end of the
     reduction, and behind it (where a row of the matrix holds what is not part of the product)."""
@@ -285,7 +325,8 @@ def test_product(dev, M, N, K, ta, tb):
 
     def run(a, b):
         pa, pb, pc = dev.upload(a.reshape(-1)), dev.upload(b.reshape(-1)), dev.upload(C0.reshape(-1))
-        L.check(hip.fitre_hip_gemm(ta, tb, M, N, K, 0.5, pa, lda, pb, ldb, -2.0, pc, ldc, pbias, ws, nb))
+        with taken(FC_GEMM, SPLIT):
+            L.check(hip.fitre_hip_gemm(ta, tb, M, N, K, 0.5, pa, lda, pb, ldb, -2.0, pc, ldc, pbias, ws, nb))
         got = dev.download(pc, ldc * N).reshape(N, ldc)
         for q in (pa, pb, pc):
             dev.free(q)
@@ -319,12 +360,13 @@ def test_product(dev, M, N, K, ta, tb):
 
 @pytest.mark.parametrize("tb", [0, 1])
 def test_product_of_more_columns_than_a_grid_has(dev, tb):
-    M, N, K = 5, 65535 * 64 + 5, 2
+    M, N, K = 16, 65535 * 64 + 5, 2
     rng = np.random.default_rng(tb)
     A, B = rng.standard_normal((K, M)).astype(np.float32), rng.standard_normal((K, N) if tb else (N, K)).astype(np.float32)
     nb = hip.fitre_hip_gemm_workspace(M, N, K)
     pa, pb, pc, ws = dev.upload(A.reshape(-1)), dev.upload(B.reshape(-1)), dev.zeros(M * N), dev.alloc(max(nb, 4))
-    L.check(hip.fitre_hip_gemm(0, tb, M, N, K, 1.0, pa, M, pb, N if tb else K, 0.0, pc, M, None, ws, nb))
+    with taken(FC_GEMM, SPLIT, launches=2):
+        L.check(hip.fitre_hip_gemm(0, tb, M, N, K, 1.0, pa, M, pb, N if tb else K, 0.0, pc, M, None, ws, nb))
     got = dev.download(pc, M * N).reshape(N, M)
     for q in (pa, pb, pc, ws):
         dev.free(q)
@@ -343,7 +385,8 @@ def test_product_of_a_short_reduction_with_a_large_leading_dimension(dev, ta, tb
     B = rng.standard_normal((K, far_apart) if tb else (N, padded)).astype(np.float32)
     nb = hip.fitre_hip_gemm_workspace(M, N, K)
     pa, pb, pc, ws = dev.upload(A.reshape(-1)), dev.upload(B.reshape(-1)), dev.zeros(M * N), dev.alloc(max(nb, 4))
-    L.check(hip.fitre_hip_gemm(ta, tb, M, N, K, 1.0, pa, A.shape[1], pb, B.shape[1], 0.0, pc, M, None, ws, nb))
+    with taken(FC_GEMM, SPLIT):
+        L.check(hip.fitre_hip_gemm(ta, tb, M, N, K, 1.0, pa, A.shape[1], pb, B.shape[1], 0.0, pc, M, None, ws, nb))
     got = dev.download(pc, M * N).reshape(N, M)
     for q in (pa, pb, pc, ws):
         dev.free(q)
@@ -365,7 +408,8 @@ def test_product_of_padded_matrices(dev, ta, tb):
     for between in (0.0, np.nan, np.inf):
         A[:, -7:] = B[:, -7:] = between
         pa, pb, pc, ws = dev.upload(A.reshape(-1)), dev.upload(B.reshape(-1)), dev.zeros(M * N), dev.alloc(max(nb, 4))
-        L.check(hip.fitre_hip_gemm(ta, tb, M, N, K, 1.0, pa, A.shape[1], pb, B.shape[1], 0.0, pc, M, None, ws, nb))
+        with taken(FC_GEMM, SPLIT):
+            L.check(hip.fitre_hip_gemm(ta, tb, M, N, K, 1.0, pa, A.shape[1], pb, B.shape[1], 0.0, pc, M, None, ws, nb))
         got.append(dev.download(pc, M * N))
         for q in (pa, pb, pc, ws):
             dev.free(q)
@@ -407,7 +451,8 @@ def product(dev, a, b):
     (K, M), N = a.shape, b.shape[0]
     nb = hip.fitre_hip_gemm_workspace(M, N, K)
     pa, pb, pc, ws = dev.upload(a.numpy().ravel()), dev.upload(b.numpy().ravel()), dev.zeros(M * N), dev.alloc(max(nb, 4))
-    L.check(hip.fitre_hip_gemm(0, 0, M, N, K, 1.0, pa, M, pb, K, 0.0, pc, M, None, ws, nb))
+    with taken(FC_GEMM, SPLIT):
+        L.check(hip.fitre_hip_gemm(0, 0, M, N, K, 1.0, pa, M, pb, K, 0.0, pc, M, None, ws, nb))
     got = dev.download(pc, M * N).reshape(N, M)
     for q in (pa, pb, pc, ws):
         dev.free(q)
