@@ -666,7 +666,9 @@ int gemm_ex(int transA, int transB, int M, int N, int K, float alpha, const floa
 	const double flops = 2.0 * (double)M * N * K;
 	// engine A(i = n, k): op(B)(k, n).  transB == 0: B[n*ldb + k] (contiguous along k); else B[k*ldb + n]
 	// engine B(j = m, k): op(A)(m, k).  transA == 0: A[k*lda + m] (contiguous along m); else A[m*lda + k]
-	const PlainParams b{ B, (uint32_t)(bElems * sizeof(float)), ldb, I }, a{ A, (uint32_t)(aElems * sizeof(float)), lda, J };
+	// an operand ends with its last number: what would pad its last row need not be there, and the loads of a slice reach past a row
+	const size_t aEnd = aElems - (size_t)(lda - (transA ? K : M)), bEnd = bElems - (size_t)(ldb - (transB ? N : K));
+	const PlainParams b{ B, (uint32_t)(bEnd * sizeof(float)), ldb, I }, a{ A, (uint32_t)(aEnd * sizeof(float)), lda, J };
 	const GemmPlan plan = split_gemm_plan_for(fit_plan(plan_gemm(I, J, R), I, J, R, ws, wsBytes), I, J, R, lane_compute_units());
 	if (plan.splits > 1 && (((uintptr_t)ws) & 3)) return fail(FITRE_E_WORKSPACE, "split-K workspace is misaligned");
 	// Numbers between two rows are not the product's and need not be finite: masked, so that they do not send its tiles to the fp32

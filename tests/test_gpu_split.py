@@ -417,6 +417,32 @@ def test_product_of_padded_matrices(dev, ta, tb):
     np.testing.assert_array_equal(got[0], got[2])
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("K", [777, 640])
+def test_product_of_parts_of_larger_matrices(dev, ta, tb, K):
+    """Columns cut out of larger matrices: the last one ends with its last number, at the end of the memory there is."""
+    M, N, room = 330, 270, 1 << 20
+    rng = np.random.default_rng(K + ta + 2 * tb)
+    ends, views = [], []
+    for rows, cols in ((M, K) if ta else (K, M)), ((K, N) if tb else (N, K)):
+        ld = cols + 150
+        whole = np.full(room, np.nan, np.float32)
+        first = room - ((rows - 1) * ld + cols)
+        part = np.lib.stride_tricks.as_strided(whole[first:], (rows, cols), (4 * ld, 4))
+        part[:] = rng.standard_normal((rows, cols))
+        ends.append((dev.upload(whole), first, ld))
+        views.append(part.astype(np.float64))
+    (pa, fa, lda), (pb, fb, ldb) = ends
+    nb = hip.fitre_hip_gemm_workspace(M, N, K)
+    pc, ws = dev.zeros(M * N), dev.alloc(max(nb, 4))
+    with taken(FC_GEMM, SPLIT):
+        L.check(hip.fitre_hip_gemm(ta, tb, M, N, K, 1.0, C.c_void_p(pa.value + 4 * fa), lda, C.c_void_p(pb.value + 4 * fb), ldb, 0.0, pc, M, None, ws, nb))
+    got = dev.download(pc, M * N).reshape(N, M)
+    for q in (pa, pb, pc, ws):
+        dev.free(q)
+    assert far(got, (views[1].T if tb else views[1]) @ (views[0].T if ta else views[0])) < limit(K)
+
+
 def forward_2x2(dev, case, x, w):
     """The dense form of 3 x 3 windows on 2 x 2 maps (through the layer's pass, without normalisation, activation and pool)."""
     from fitre_amd.structs import CNN_ACT_NONE, NO_POOL
