@@ -478,10 +478,9 @@ static int launch_c3_dw(const fitre_conv_shape *s, const float *x, const float *
 // ---- weight gradient of 3x3 and 5x5 windows on the bf16 pipes (conv_split_dw.h) ------------------------------------------------
 struct SplitDwShape {
 	int mode, logGroups; // how a row is cut into groups of eight cells
-	int ob, wo;          // blocks of 32 output channels of a wave; waves along them (two along the input channels)
-	int rowTiles() const { return 32 * ob * wo; }
 	int tiles, stages;   // workgroups of a range; stages of the tap row with the most image rows
 };
+static int split_dw_tiles(int channels) { return (channels + kSplitDwTile - 1) / kSplitDwTile; }
 static bool split_dw_shape(const fitre_conv_shape *s, SplitDwShape &d)
 {
 	if ((s->ksize != 3 && s->ksize != 5) || s->stride != 1 || s->padding != s->ksize / 2 || s->inChannels <= 16 || s->outChannels < 32) return false;
@@ -490,11 +489,7 @@ static bool split_dw_shape(const fitre_conv_shape *s, SplitDwShape &d)
 	if (B < 3 || B > 32 || (B == 5 || (B > 8 && B < 12) || (B > 16 && B < 24)) || (B <= 4 && s->ksize != 3)) return false;
 	d.mode = B <= 4 ? kRowsPaired : (B <= 8 ? kRowsWhole : kRowsCut);
 	d.logGroups = B <= 8 ? 0 : (B <= 16 ? 1 : 2);
-	// 5 x 5 windows with at most 64 output channels: 64 -> 64, 15 x 15, 100 images 66 us with ten accumulators in each of two
-	// waves, 45 with five in four
-	d.ob = s->ksize == 5 && s->outChannels <= 64 ? 1 : 2;
-	d.wo = s->outChannels <= 64 && d.ob == 2 ? 1 : 2;
-	d.tiles = s->ksize * ((s->inChannels + 63) / 64) * ((s->outChannels + d.rowTiles() - 1) / d.rowTiles());
+	d.tiles = s->ksize * split_dw_tiles(s->inChannels) * split_dw_tiles(s->outChannels);
 	const long rows = (long)s->samples * s->inA, groups = d.mode == kRowsPaired ? (rows + 1) / 2 : rows << d.logGroups;
 	d.stages = (int)((groups + kSplitDwGroups - 1) / kSplitDwGroups);
 	return true;
@@ -503,9 +498,10 @@ static size_t split_dw_range_bytes(const fitre_conv_shape *s) { return sizeof(fl
 static BlockPlan split_dw_plan(const fitre_conv_shape *s, const SplitDwShape &d, int cus = 0, int pairs = 1)
 {
 	if (cus <= 0) cus = weight_grad_units();
-	// measured, us a stage and workgroup with the compute units full
-	const double stageUs = d.wo == 1 ? 1.1 : (s->ksize == 3 ? 2.05 : (d.ob == 2 ? 2.57 : 1.9));
-	const int resident = d.wo == 1 ? 3 : (d.ob == 1 ? 1 : 2); // from how many on more of them add nothing
+	// measured, us a stage and workgroup with two on every compute unit, behind the first 6: 3 x 3 0.98 to 1.1 from 13 stages on, 5 x 5
+	// 1.5 to 1.7
+	const double stageUs = s->ksize == 3 ? 1.03 : 1.55;
+	const int resident = 2; // from how many on more of them add nothing
 	BlockPlan plan = plan_blocks(d.tiles, (long)pairs * d.stages, 0.85 * stageUs, resident, s->outChannels, (long)s->inChannels * s->ksize * s->ksize, cus);
 	plan.wsBytes = plan.splits * split_dw_range_bytes(s); // an uncut product's partial sums are put in order by the reduction as well
 	return plan;
@@ -552,31 +548,19 @@ static int launch_split_dw(const fitre_conv_shape *s, const SplitDwShape &d, con
 	p.xBytes = (uint32_t)((size_t)s->inChannels * J * sizeof(float)), p.deltaBytes = (uint32_t)((size_t)s->outChannels * J * sizeof(float));
 	p.I = s->outChannels, p.cin = s->inChannels, p.J = J, p.A = s->inA, p.B = s->inB, p.samples = s->samples;
 	p.logGroups = d.logGroups, p.stages = d.stages, p.perSplit = plan.perSplit;
-	p.cTiles = (s->inChannels + 63) / 64;
+	p.cTiles = split_dw_tiles(s->inChannels);
 	p.partial = (float *)ws;
 	for (int i = 0; i < 3; i++) p.divLive[i] = FastDiv((uint32_t)(s->inA > i ? s->inA - i : 1));
-	const dim3 grid((unsigned)(p.cTiles * s->ksize), (unsigned)((s->outChannels + d.rowTiles() - 1) / d.rowTiles()), (unsigned)plan.splits);
+	const dim3 grid((unsigned)(p.cTiles * s->ksize), (unsigned)split_dw_tiles(s->outChannels), (unsigned)plan.splits);
 	if (grid.y > 65535 || grid.z > 65535) return fail(FITRE_E_UNSUPPORTED, "conv_split_dw_kernel grid too large");
 	{
 		LaunchScope scope(FITRE_KC_CONV_DW, (x2 ? 2 : 1) * conv_flops(s), kTileSplit);
-#define SPLIT_DW_LAUNCH(KS, M, B_, O) conv_split_dw_kernel<KS, M, B_, O, 2><<<grid, 128 * O, 0, stream()>>>(p)
-#define SPLIT_DW_MODES(O)                                                                                             \
-	{                                                                                                                 \
-		if (d.mode == kRowsPaired) SPLIT_DW_LAUNCH(3, kRowsPaired, 2, O);                                             \
-		else if (d.mode == kRowsWhole) SPLIT_DW_LAUNCH(3, kRowsWhole, 2, O);                                          \
-		else SPLIT_DW_LAUNCH(3, kRowsCut, 2, O);                                                                      \
-	}
-		if (s->ksize == 3) {
-			if (d.wo == 2) SPLIT_DW_MODES(2)
-			else SPLIT_DW_MODES(1)
-		} else if (d.ob == 2) {
-			if (d.mode == kRowsWhole) SPLIT_DW_LAUNCH(5, kRowsWhole, 2, 2);
-			else SPLIT_DW_LAUNCH(5, kRowsCut, 2, 2);
-		} else {
-			if (d.mode == kRowsWhole) SPLIT_DW_LAUNCH(5, kRowsWhole, 1, 2);
-			else SPLIT_DW_LAUNCH(5, kRowsCut, 1, 2);
-		}
-#undef SPLIT_DW_MODES
+#define SPLIT_DW_LAUNCH(KS, M) conv_split_dw_kernel<KS, M><<<grid, kGemmThreads, 0, stream()>>>(p)
+		if (s->ksize == 5 && d.mode == kRowsWhole) SPLIT_DW_LAUNCH(5, kRowsWhole);
+		else if (s->ksize == 5) SPLIT_DW_LAUNCH(5, kRowsCut);
+		else if (d.mode == kRowsPaired) SPLIT_DW_LAUNCH(3, kRowsPaired);
+		else if (d.mode == kRowsWhole) SPLIT_DW_LAUNCH(3, kRowsWhole);
+		else SPLIT_DW_LAUNCH(3, kRowsCut);
 #undef SPLIT_DW_LAUNCH
 	}
 	const int products = s->outChannels * s->inChannels;

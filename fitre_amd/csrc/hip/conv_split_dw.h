@@ -2,13 +2,22 @@
 //
 //     dW[o][c][ta][tb] = sum_m delta[o][m] * x[c][m + (ta-P)*B + (tb-P)]
 //
-// A workgroup takes ONE tap row ta, 32 * OB * WO output and 32 * WC input channels and a range of the reduction; a wave
-// 32 * OB x 32 channels and the KS taps of the row.  The reduction runs over the image rows at which the tap row is inside the image (the
+// A workgroup takes ONE tap row ta, 64 output and 64 input channels and a range of the reduction; a wave 32 x 32 channels and the
+// KS taps of the row.  The reduction runs over the image rows at which the tap row is inside the image (the
 // others are never touched), in groups of eight consecutive cells of a row -- or of two rows of maps at most four cells wide --
 // the short last group of a row filled up with zeros.  Groups of delta and, ta - P rows away, of x are split while they are
 // staged: LDS [part][group][channel][8 cells] holds the matrix fragments as they are read.  The fragment of tap tb is the
 // group's word moved by tb - P cells: a funnel shift with the last (first) two cells of the group before (behind) it, which are
 // zero at the end of a row.  Stages of four groups, double buffered.
+//
+// The five small products have accumulators of their own.  Added to the large ones, each of the six would round the whole sum, also
+// where there is next to nothing to add, and gradients are full of that: 256 -> 256 channels, 8 x 8 maps, 256 images, inputs
+// behind a ReLU, error against 64 bits with one accumulator / two / on the fp32 pipe 4.3e-7 / 1.4e-7 / 3.7e-7, and with one error
+// in fifty not zero 1.2e-7 / 4.0e-8 / 6.4e-8; weight gradients of VGG-11's layers on 8 x 8 and 4 x 4 maps at 256 images 4.5e-7 to
+// 5.8e-7 / 2.3e-7 to 3.8e-7 / 4.0e-7 to 5.5e-7.  What is left is the pipe's own: it adds eight products at a time and cuts each off below
+// the last place of the largest, towards zero.  Where the errors of a channel are a few large ones of one sign among many small
+// ones of the other, all of the small ones lose the same way: its second layer 1.6e-6, nearly all of it one number a
+// channel, against 6.4e-7 on the fp32 pipe.
 //
 // Partial sums leave as [range][tap][o][c], whole rows of c; split_dw_reduce_kernel adds the ranges in double, in order.
 #pragma once
@@ -18,6 +27,7 @@
 namespace fitre {
 
 constexpr int kSplitDwGroups = 4; // groups per stage: two bf16 MFMA steps
+constexpr int kSplitDwTile = 64;  // output and input channels of a workgroup
 
 // how a row is cut into groups
 constexpr int kRowsPaired = 0; // B <= 4: two rows a group
@@ -38,10 +48,10 @@ struct ConvSplitDwParams {
 };
 
 // the tile by fp32 multiply-adds: eight output channels x 64 (input channel, tap) a wave at a time
-template <int KS, int MODE, int OT, int CT, int WAVES>
+template <int KS, int MODE>
 __device__ __forceinline__ void split_dw_exact_tile(const ConvSplitDwParams &p, int o0, int c0, int ta, int stBeg, int stEnd, float *partial)
 {
-	constexpr int P = KS / 2;
+	constexpr int P = KS / 2, OT = kSplitDwTile, CT = kSplitDwTile, G = kSplitDwGroups, WAVES = kGemmThreads / 64;
 	static_assert(CT % 64 == 0, "whole groups of 64 (input channel, tap)");
 	const int lane = threadIdx.x & 63, off = ta - P, a0 = off < 0 ? -off : 0, live = p.A - (off < 0 ? -off : off);
 	const int rows = p.samples * live;
@@ -56,8 +66,8 @@ __device__ __forceinline__ void split_dw_exact_tile(const ConvSplitDwParams &p, 
 		for (int st = stBeg; st < stEnd; st++) {
 			const bool second = st >= p.stages;
 			const float *x = (second ? p.x2 : p.x) + (size_t)(mine ? c : 0) * p.J, *d = second ? p.delta2 : p.delta;
-			const int q0 = (st - (second ? p.stages : 0)) * kSplitDwGroups;
-			for (int k = 0; k < kSplitDwGroups * 8; k++) {
+			const int q0 = (st - (second ? p.stages : 0)) * G;
+			for (int k = 0; k < G * 8; k++) {
 				const int q = q0 + k / 8, cell = k % 8;
 				const int r = MODE == kRowsPaired ? 2 * q + cell / 4 : (MODE == kRowsWhole ? q : q >> p.logGroups);
 				const int b = MODE == kRowsPaired ? cell % 4 : (MODE == kRowsWhole ? cell : (q & ((1 << p.logGroups) - 1)) * 8 + cell);
@@ -73,23 +83,26 @@ __device__ __forceinline__ void split_dw_exact_tile(const ConvSplitDwParams &p, 
 	}
 }
 
-// OB: blocks of 32 output channels of a wave.  3 x 3 windows take 193 registers: two workgroups on a compute unit leave 126 on
-// every SIMD, on which the bandwidth kernels of the layer below run.  (Asked for three waves a SIMD the compiler puts the sums
-// into accumulator registers beside 124 others, 220 together: the same time.)
-template <int KS, int MODE, int OB, int WO, int WC>
-__global__ void __launch_bounds__(64 * WO *WC, 2)
+// 3 x 3 windows take at most 180 registers, 5 x 5 ones 243: two workgroups find room on a compute unit and leave 144 of a SIMD's 512,
+// or 16, to the bandwidth kernels of the layer below.  Whole passes, us, this tile against 128 output channels in eight waves with
+// stages of eight groups, one workgroup on a compute unit: VGG-11 b256 1655 / 1700, VGG-16 b128 1900 / 1960, AlexNet b64 2730 /
+// 2870.  Alone the larger tile is the faster one (256 -> 256 channels, 8 x 8 maps, 256 images, with the reduction 110 / 99 us;
+// 64 -> 192, 27 x 27, 5 x 5 windows, 64 images 163 / 185), but nothing of the chain starts beside it before all of it has ended.
+// Held to 168 registers for three workgroups: 1706 / 1998 / 2836.
+template <int KS, int MODE>
+__global__ void __launch_bounds__(kGemmThreads, 2)
 conv_split_dw_kernel(const ConvSplitDwParams p)
 {
 	FITRE_RAISE_MATRIX_WAVE_PRIORITY();
-	constexpr int P = KS / 2, T = 64 * WO * WC, OT = 32 * OB * WO, CT = 32 * WC, G = kSplitDwGroups;
+	constexpr int P = KS / 2, T = kGemmThreads, OT = kSplitDwTile, CT = kSplitDwTile, G = kSplitDwGroups;
 	constexpr int DLD = OT + 4, XLD = CT + 4; // 16-byte words a group; four spare ones spread the stores of the groups over the banks
 	constexpr int DPART = G * DLD, XPART = G * XLD;
-	constexpr int DE = OT * G / T, XE = CT * G / T;
+	static_assert(G == 4 && OT * G == T && CT * G == T, "two steps a stage; a thread stages one group of either");
 	__shared__ u32x4 Ds[2][3 * DPART], Xs[2][3 * XPART];
 
 	const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 	const int khalf = lane >> 5, l32 = lane & 31;
-	const int wo = wave % WO, wc = wave / WO;
+	const int wo = wave & 1, wc = wave >> 1;
 	// an XCD takes consecutive (range, tile) indices: workgroups that read the same positions share its L2
 	int bx, by, bz;
 	{
@@ -113,28 +126,18 @@ conv_split_dw_kernel(const ConvSplitDwParams p)
 	// this thread's group of a stage, and the channels whose groups it stages
 	const int qs = tid % G, g = MODE == kRowsCut ? qs & ((1 << p.logGroups) - 1) : 0;
 	const int valid = p.B - 8 * g; // cells of its group that are inside the row (kRowsPaired: of each of its two)
-	uint32_t dRow[DE], xRow[XE];
-#pragma unroll
-	for (int e = 0; e < DE; e++) {
-		const int row = o0 + tid / G + T / G * e;
-		dRow[e] = row < p.I ? 4u * (uint32_t)row * (uint32_t)p.J : kGroupOutOfRange;
-	}
-#pragma unroll
-	for (int e = 0; e < XE; e++) {
-		const int row = c0 + tid / G + T / G * e;
-		xRow[e] = row < p.cin ? 4u * (uint32_t)row * (uint32_t)p.J : kGroupOutOfRange;
-	}
+	const int dRow = o0 + tid / G, xRow = c0 + tid / G;
+	const uint32_t dOff = dRow < p.I ? 4u * (uint32_t)dRow * (uint32_t)p.J : kGroupOutOfRange;
+	const uint32_t xOff = xRow < p.cin ? 4u * (uint32_t)xRow * (uint32_t)p.J : kGroupOutOfRange;
 	const int dLds = qs * DLD + tid / G, xLds = qs * XLD + tid / G;
 	for (int i = tid; i < 3 * XPART; i += T) Xs[0][i] = Xs[1][i] = u32x4{ 0, 0, 0, 0 }; // the spare words are what lies past a row's end
 
-	u32x4 dreg[DE][2], xreg[XE][2];
-	v16f acc[OB][KS];
+	u32x4 dreg[2], xreg[2];
+	v16f acc[KS], low[KS]; // the large products, and the five small ones
 #pragma unroll
-	for (int b = 0; b < OB; b++)
+	for (int t = 0; t < KS; t++)
 #pragma unroll
-		for (int t = 0; t < KS; t++)
-#pragma unroll
-			for (int v = 0; v < 16; v++) acc[b][t][v] = 0.f;
+		for (int v = 0; v < 16; v++) acc[t][v] = low[t][v] = 0.f;
 
 #define SPLIT_DW_ROW(R, OFFSET)                                                                                       \
 	{                                                                                                                 \
@@ -154,18 +157,11 @@ conv_split_dw_kernel(const ConvSplitDwParams p)
 		const bool in0_ = r_ < rows, in1_ = MODE == kRowsPaired ? r_ + 1 < rows : in0_;                               \
 		if constexpr (MODE == kRowsPaired) SPLIT_DW_ROW(r_ + 1, at1_);                                                \
 		const int shift_ = 4 * off * p.B;                                                                             \
-		_Pragma("unroll") for (int e = 0; e < DE; e++)                                                                \
-		{                                                                                                             \
-			const bool row_ = dRow[e] != kGroupOutOfRange;                                                            \
-			dreg[e][0] = __builtin_amdgcn_raw_buffer_load_b128(dRs_, (int)((row_ & in0_) ? dRow[e] + at0_ : kGroupOutOfRange), 0, 0); \
-			dreg[e][1] = __builtin_amdgcn_raw_buffer_load_b128(dRs_, (int)((row_ & in1_) ? dRow[e] + at1_ : kGroupOutOfRange), 0, 0); \
-		}                                                                                                             \
-		_Pragma("unroll") for (int e = 0; e < XE; e++)                                                                \
-		{                                                                                                             \
-			const bool row_ = xRow[e] != kGroupOutOfRange;                                                            \
-			xreg[e][0] = __builtin_amdgcn_raw_buffer_load_b128(xRs_, (int)((row_ & in0_) ? xRow[e] + at0_ + shift_ : kGroupOutOfRange), 0, 0); \
-			xreg[e][1] = __builtin_amdgcn_raw_buffer_load_b128(xRs_, (int)((row_ & in1_) ? xRow[e] + at1_ + shift_ : kGroupOutOfRange), 0, 0); \
-		}                                                                                                             \
+		const bool dIn_ = dOff != kGroupOutOfRange, xIn_ = xOff != kGroupOutOfRange;                                    \
+		dreg[0] = __builtin_amdgcn_raw_buffer_load_b128(dRs_, (int)((dIn_ & in0_) ? dOff + at0_ : kGroupOutOfRange), 0, 0); \
+		dreg[1] = __builtin_amdgcn_raw_buffer_load_b128(dRs_, (int)((dIn_ & in1_) ? dOff + at1_ : kGroupOutOfRange), 0, 0); \
+		xreg[0] = __builtin_amdgcn_raw_buffer_load_b128(xRs_, (int)((xIn_ & in0_) ? xOff + at0_ + shift_ : kGroupOutOfRange), 0, 0); \
+		xreg[1] = __builtin_amdgcn_raw_buffer_load_b128(xRs_, (int)((xIn_ & in1_) ? xOff + at1_ + shift_ : kGroupOutOfRange), 0, 0); \
 	}
 #define SPLIT_DW_STORE_ONE(REG, LDS, PARTWORDS)                                                                       \
 	{                                                                                                                 \
@@ -179,11 +175,10 @@ conv_split_dw_kernel(const ConvSplitDwParams p)
 		split_eight(v_, part_);                                                                                       \
 		_Pragma("unroll") for (int s = 0; s < 3; s++) (LDS)[s * (PARTWORDS)] = part_[s];                              \
 	}
-#define SPLIT_DW_STORE_DELTA(BUFFER, E) SPLIT_DW_STORE_ONE(dreg[E], &Ds[BUFFER][dLds + T / G * (E)], DPART)
-#define SPLIT_DW_STORE_X(BUFFER, E) SPLIT_DW_STORE_ONE(xreg[E], &Xs[BUFFER][xLds + T / G * (E)], XPART)
-// fragments of a step: part S of delta (two blocks of 32 channels); part S of x and the cells beside it
-#define SPLIT_DW_READ_A(TO, BUFFER, STEP, S)                                                                          \
-	_Pragma("unroll") for (int b = 0; b < OB; b++) TO[b] = Ds[BUFFER][(S) * DPART + (2 * (STEP) + khalf) * DLD + wo * 32 * OB + b * 32 + l32];
+#define SPLIT_DW_STORE_DELTA(BUFFER) SPLIT_DW_STORE_ONE(dreg, &Ds[BUFFER][dLds], DPART)
+#define SPLIT_DW_STORE_X(BUFFER) SPLIT_DW_STORE_ONE(xreg, &Xs[BUFFER][xLds], XPART)
+// fragments of a step: part S of delta; part S of x and the cells beside it
+#define SPLIT_DW_READ_A(TO, BUFFER, STEP, S) TO = Ds[BUFFER][(S) * DPART + (2 * (STEP) + khalf) * DLD + wo * 32 + l32]
 #define SPLIT_DW_READ_X(BUFFER, STEP, S)                                                                              \
 	{                                                                                                                 \
 		const u32x4 *xw_ = &Xs[BUFFER][(2 * (STEP) + khalf) * XLD + wc * 32 + l32 + (S) * XPART];                     \
@@ -213,9 +208,8 @@ conv_split_dw_kernel(const ConvSplitDwParams p)
 			else if (by_ == 1) f[t][1] &= 0x0000ffffu;                                                                \
 		}                                                                                                             \
 	}
-#define SPLIT_DW_PRODUCTS(A)                                                                                          \
-	_Pragma("unroll") for (int b = 0; b < OB; b++)                                                                    \
-		_Pragma("unroll") for (int t = 0; t < KS; t++) acc[b][t] = mfma_bf16(A[b], f[t], acc[b][t]);
+#define SPLIT_DW_PRODUCTS(SUM, A)                                                                                     \
+	_Pragma("unroll") for (int t = 0; t < KS; t++) SUM[t] = mfma_bf16(A, f[t], SUM[t]);
 // vector instructions of the staging between the matrix instructions
 #define SPLIT_DW_MIX(MFMAS)                                                                                           \
 	_Pragma("unroll") for (int i = 0; i < (MFMAS); i++)                                                               \
@@ -226,18 +220,15 @@ conv_split_dw_kernel(const ConvSplitDwParams p)
 
 	SPLIT_DW_LOAD(stBeg);
 	__syncthreads(); // the zeros are in place
-#pragma unroll
-	for (int e = 0; e < DE; e++) SPLIT_DW_STORE_DELTA(0, e);
-#pragma unroll
-	for (int e = 0; e < XE; e++) SPLIT_DW_STORE_X(0, e);
+	SPLIT_DW_STORE_DELTA(0);
+	SPLIT_DW_STORE_X(0);
 	if (stBeg + 1 < stEnd) SPLIT_DW_LOAD(stBeg + 1);
 	__syncthreads();
 
 	// A phase multiplies one part of x with the parts of delta it is kept with, while the next phase's part of either is read.
-	// The next stage is split and stored during the second step's first two phases and the one after it requested behind
-	// them; the barrier comes before the last phase, whose operands are in registers, so that the next stage's first
-	// fragments are read under it.
-	u32x4 d0[2][OB], d1[OB], d2[OB], word, f[KS];
+	// The next stage is split and stored during the first step's last phase and the second's second, and the one after it requested
+	// behind them; the barrier comes before the last phase, whose operands are in registers, so that the next stage's first fragments are read under it.
+	u32x4 d0[2], d1, d2, word, f[KS];
 	uint32_t last = 0, first = 0; // two cells of the group before, two of the one behind: zero at the end of a row
 	SPLIT_DW_READ_A(d0[0], 0, 0, 0);
 	SPLIT_DW_READ_X(0, 0, 2);
@@ -249,23 +240,15 @@ conv_split_dw_kernel(const ConvSplitDwParams p)
 			SPLIT_DW_TAPS();
 			SPLIT_DW_READ_A(d1, buffer, step, 1);
 			SPLIT_DW_READ_X(buffer, step, 1);
-			if (ends) {
-#pragma unroll
-				for (int e = 0; e < XE; e++) SPLIT_DW_STORE_X(buffer ^ 1, e);
-			}
-			SPLIT_DW_PRODUCTS(d0[step & 1]);
-			if (ends) SPLIT_DW_MIX(OB * KS);
+			SPLIT_DW_PRODUCTS(low, d0[step & 1]);
 			__builtin_amdgcn_sched_barrier(0);
 			SPLIT_DW_TAPS();
 			SPLIT_DW_READ_A(d2, buffer, step, 2);
 			SPLIT_DW_READ_X(buffer, step, 0);
-			if (ends) {
-#pragma unroll
-				for (int e = 0; e < DE; e++) SPLIT_DW_STORE_DELTA(buffer ^ 1, e);
-			}
-			SPLIT_DW_PRODUCTS(d1);
-			SPLIT_DW_PRODUCTS(d0[step & 1]);
-			if (ends) SPLIT_DW_MIX(2 * OB * KS);
+			if (ends) SPLIT_DW_STORE_DELTA(buffer ^ 1);
+			SPLIT_DW_PRODUCTS(low, d1);
+			SPLIT_DW_PRODUCTS(low, d0[step & 1]);
+			if (ends) SPLIT_DW_MIX(2 * KS);
 			__builtin_amdgcn_sched_barrier(0);
 			SPLIT_DW_TAPS();
 			if (ends) {
@@ -274,9 +257,11 @@ conv_split_dw_kernel(const ConvSplitDwParams p)
 			}
 			SPLIT_DW_READ_A(d0[(step + 1) & 1], ends ? buffer ^ 1 : buffer, ends ? 0 : step + 1, 0);
 			SPLIT_DW_READ_X(ends ? buffer ^ 1 : buffer, ends ? 0 : step + 1, 2);
-			SPLIT_DW_PRODUCTS(d2);
-			SPLIT_DW_PRODUCTS(d1);
-			SPLIT_DW_PRODUCTS(d0[step & 1]);
+			if (!ends) SPLIT_DW_STORE_X(buffer ^ 1);
+			SPLIT_DW_PRODUCTS(low, d2);
+			SPLIT_DW_PRODUCTS(low, d1);
+			SPLIT_DW_PRODUCTS(acc, d0[step & 1]);
+			if (!ends) SPLIT_DW_MIX(3 * KS);
 			__builtin_amdgcn_sched_barrier(0);
 		}
 	}
@@ -294,26 +279,25 @@ conv_split_dw_kernel(const ConvSplitDwParams p)
 	float *partial = p.partial + (size_t)bz * KS * KS * p.I * p.cin;
 	bool suspect = false;
 #pragma unroll
-	for (int b = 0; b < OB; b++)
+	for (int t = 0; t < KS; t++)
 #pragma unroll
-		for (int t = 0; t < KS; t++)
-#pragma unroll
-			for (int v = 0; v < 16; v++) suspect |= split_sum_suspect(acc[b][t][v]);
+		for (int v = 0; v < 16; v++) {
+			acc[t][v] += low[t][v];
+			suspect |= split_sum_suspect(acc[t][v]);
+		}
 	if (__syncthreads_or(suspect)) {
-		split_dw_exact_tile<KS, MODE, OT, CT, WO * WC>(p, o0, c0, ta, stBeg, stEnd, partial);
+		split_dw_exact_tile<KS, MODE>(p, o0, c0, ta, stBeg, stEnd, partial);
 		return;
 	}
 	const int c = c0 + wc * 32 + l32;
 	if (c >= p.cin) return;
 #pragma unroll
-	for (int b = 0; b < OB; b++)
+	for (int t = 0; t < KS; t++)
 #pragma unroll
-		for (int t = 0; t < KS; t++)
-#pragma unroll
-			for (int v = 0; v < 16; v++) {
-				const int o = o0 + wo * 32 * OB + b * 32 + 8 * (v / 4) + 4 * khalf + (v % 4);
-				if (o < p.I) partial[((size_t)(ta * KS + t) * p.I + o) * p.cin + c] = acc[b][t][v] * kSplitSumScale;
-			}
+		for (int v = 0; v < 16; v++) {
+			const int o = o0 + wo * 32 + 8 * (v / 4) + 4 * khalf + (v % 4);
+			if (o < p.I) partial[((size_t)(ta * KS + t) * p.I + o) * p.cin + c] = acc[t][v] * kSplitSumScale;
+		}
 }
 
 // dW[o][c][tap] = sum over the ranges, in order.  64 (o, c) x four phases a workgroup; a phase adds every fourth range, the
