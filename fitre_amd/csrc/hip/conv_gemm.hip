@@ -628,6 +628,19 @@ size_t gemm_ex_workspace(int M, int N, int K, int flags)
 	return plan_gemm_workspace(N, M, K, (flags & kGemmMirror) != 0);
 }
 
+// Products bound by what they write stay on the fp32 engine, whose larger tiles take less to begin with.  fp32 / split, us: half a
+// slice of reduction indices 8192 x 8192 x 8 84 / 96 (4096 x 4096 x 8 30 / 29; 8192 x 8192 x 17 102 / 97); both operands
+// row-contiguous, which takes 202 registers in place of 146 and so two workgroups on a compute unit in place of three, 3000 x 3000 x
+// 48 26 / 29 (x 96 35 / 32), 6227 x 5916 x 128 116 / 127, 8192 x 8192 x 192 265 / 271 (x 256 at 6227 x 5916 192 / 199; 1500 x 1500 x 64 19 /
+// 13); results of few rows or columns, of which a tile is mostly nothing, 400 000 x 20 x 48 38 / 44 (x 96 58 / 50, x 40 27 / 26),
+// row-contiguous 400 000 x 20 x 256 130 / 148.
+static bool fp32_product(bool rowContiguous, int I, int J, int R)
+{
+	const bool thin = I <= 32 || J <= 32, large = (double)I * J >= 3.0e7;
+	if ((thin && R <= 64) || (large && R <= 16)) return true;
+	return rowContiguous && ((R <= 64 && (double)I * J >= 8.0e6) || (thin && R <= 256) || (large && R <= 192));
+}
+
 int gemm_ex(int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb,
             float beta, float *C, int ldc, const float *bias, int kernelClass, void *ws, size_t wsBytes)
 {
@@ -653,6 +666,13 @@ int gemm_ex(int transA, int transB, int M, int N, int K, float alpha, const floa
 	// an operand ends with its last number: what would pad its last row need not be there, and the loads of a slice reach past a row
 	const size_t aEnd = aElems - (size_t)(lda - (transA ? K : M)), bEnd = bElems - (size_t)(ldb - (transB ? N : K));
 	const PlainParams b{ B, (uint32_t)(bEnd * sizeof(float)), ldb, I }, a{ A, (uint32_t)(aEnd * sizeof(float)), lda, J };
+	if (fp32_product(transB && !transA, I, J, R)) {
+		const GemmPlan fp32 = plan_gemm(I, J, R);
+		if (!transB && !transA) return launch_gemm<PlainKContig, PlainRowContig>(b, a, out, I, J, R, fp32, ws, wsBytes, kernelClass, flops);
+		if (!transB && transA) return launch_gemm<PlainKContig, PlainKContig>(b, a, out, I, J, R, fp32, ws, wsBytes, kernelClass, flops);
+		if (transB && !transA) return launch_gemm<PlainRowContig, PlainRowContig>(b, a, out, I, J, R, fp32, ws, wsBytes, kernelClass, flops);
+		return launch_gemm<PlainRowContig, PlainKContig>(b, a, out, I, J, R, fp32, ws, wsBytes, kernelClass, flops);
+	}
 	const GemmPlan plan = split_gemm_plan_for(fit_plan(plan_gemm(I, J, R), I, J, R, ws, wsBytes), I, J, R, lane_compute_units());
 	if (plan.splits > 1 && (((uintptr_t)ws) & 3)) return fail(FITRE_E_WORKSPACE, "split-K workspace is misaligned");
 	// Numbers between two rows are not the product's and need not be finite: masked, so that they do not send its tiles to the fp32

@@ -368,42 +368,69 @@ def test_product(dev, M, N, K, ta, tb):
         dev.free(q)
 
 
-@pytest.mark.parametrize("tb", [0, 1])
-def test_product_of_more_columns_than_a_grid_has(dev, tb):
-    M, N, K = 16, 65535 * 64 + 5, 2
-    rng = np.random.default_rng(tb)
-    A, B = rng.standard_normal((K, M)).astype(np.float32), rng.standard_normal((K, N) if tb else (N, K)).astype(np.float32)
+@pytest.mark.parametrize("ta,tb,M,N,K,tile", [
+    (0, 0, 32, 140_001, 64, FP32), (1, 0, 140_001, 32, 64, FP32), (1, 1, 32, 140_001, 64, FP32), (0, 0, 33, 140_001, 64, SPLIT),
+    (1, 0, 32, 140_001, 65, SPLIT), (0, 1, 31, 140_001, 256, FP32), (0, 1, 31, 140_001, 257, SPLIT), (0, 1, 3001, 2999, 64, FP32),
+    (0, 1, 3001, 2999, 65, SPLIT), (0, 1, 6000, 5001, 192, FP32), (0, 1, 6000, 5001, 193, SPLIT), (0, 0, 6000, 5001, 16, FP32),
+    (1, 1, 6000, 5001, 17, SPLIT), (1, 0, 6000, 5001, 16, FP32)])
+def test_products_bound_by_what_they_write(dev, ta, tb, M, N, K, tile):
+    """Both sides of the lines up to which the fp32 engine has them."""
+    rng = np.random.default_rng(M + N + K)
+    A, B = rng.standard_normal((M, K) if ta else (K, M)).astype(np.float32), rng.standard_normal((K, N) if tb else (N, K)).astype(np.float32)
     nb = hip.fitre_hip_gemm_workspace(M, N, K)
     pa, pb, pc, ws = dev.upload(A.reshape(-1)), dev.upload(B.reshape(-1)), dev.zeros(M * N), dev.alloc(max(nb, 4))
-    with taken(FC_GEMM, SPLIT, launches=2):
-        L.check(hip.fitre_hip_gemm(0, tb, M, N, K, 1.0, pa, M, pb, N if tb else K, 0.0, pc, M, None, ws, nb))
-    got = dev.download(pc, M * N).reshape(N, M)
-    for q in (pa, pb, pc, ws):
-        dev.free(q)
-    edge, bound = 65535 * 64, 3 * 2.0**-24  # a sum of two products: each accumulator and their sum are rounded once
-    for cols in (slice(0, 200), slice(edge - 130, N)):
-        assert far(got[cols], (B[:, cols].T if tb else B[cols]).astype(np.float64) @ A.astype(np.float64)) < bound
-
-
-@pytest.mark.parametrize("ta,tb,M,N", [(0, 0, 36_000_000, 2), (1, 1, 510_000, 130)])
-def test_product_of_a_short_reduction_with_a_large_leading_dimension(dev, ta, tb, M, N):
-    """Two reduction indices 36 million apart: the other thirty of a slice lie past 2^32 bytes, where 32-bit offsets would come
-    back into the tensor; the other operand's rows are followed by numbers that are not part of the product."""
-    K, far_apart, padded = 2, 36_000_000, 40
-    rng = np.random.default_rng(M)
-    A = rng.standard_normal((M, padded) if ta else (K, far_apart)).astype(np.float32)
-    B = rng.standard_normal((K, far_apart) if tb else (N, padded)).astype(np.float32)
-    nb = hip.fitre_hip_gemm_workspace(M, N, K)
-    pa, pb, pc, ws = dev.upload(A.reshape(-1)), dev.upload(B.reshape(-1)), dev.zeros(M * N), dev.alloc(max(nb, 4))
-    with taken(FC_GEMM, SPLIT):
+    with taken(FC_GEMM, tile):
         L.check(hip.fitre_hip_gemm(ta, tb, M, N, K, 1.0, pa, A.shape[1], pb, B.shape[1], 0.0, pc, M, None, ws, nb))
     got = dev.download(pc, M * N).reshape(N, M)
     for q in (pa, pb, pc, ws):
         dev.free(q)
-    opB = (B[:, :N].T if tb else B[:, :K]).astype(np.float64)
-    for rows in (slice(0, 5000), slice(M - 5000, M)):
-        opA = (A[rows, :K].T if ta else A[:, rows]).astype(np.float64)
-        assert far(got[:, rows], opB @ opA) < 3 * 2.0**-24  # each accumulator and their sum are rounded once
+    opA, opB = (A.T if ta else A).astype(np.float64), (B.T if tb else B).astype(np.float64)
+    for cols in (slice(0, 100), slice(N - 100, N)):
+        assert far(got[cols], opB[cols] @ opA) < limit(K) + 2.0**-24
+
+
+@pytest.mark.parametrize("tb,K,split", [(0, 17, 2), (1, 2, 1)])
+def test_product_of_more_columns_than_a_grid_has(dev, tb, K, split):
+    """In two launches; a large result of two terms a sum is one of the fp32 engine's."""
+    M, N = 33, 65535 * 64 + 37
+    rng = np.random.default_rng(tb)
+    A, B = rng.standard_normal((K, M)).astype(np.float32), rng.standard_normal((K, N) if tb else (N, K)).astype(np.float32)
+    nb = hip.fitre_hip_gemm_workspace(M, N, K)
+    pa, pb, pc, ws = dev.upload(A.reshape(-1)), dev.upload(B.reshape(-1)), dev.zeros(M * N), dev.alloc(max(nb, 4))
+    with taken(FC_GEMM, SPLIT, launches=split):
+        L.check(hip.fitre_hip_gemm(0, tb, M, N, K, 1.0, pa, M, pb, N if tb else K, 0.0, pc, M, None, ws, nb))
+    got = dev.download(pc, M * N).reshape(N, M)
+    for q in (pa, pb, pc, ws):
+        dev.free(q)
+    edge = 65535 * 64
+    for cols in (slice(0, 200), slice(edge - 130, N)):
+        assert far(got[cols], (B[:, cols].T if tb else B[cols]).astype(np.float64) @ A.astype(np.float64)) < 3 * 2.0**-24  # few roundings
+
+
+@pytest.mark.parametrize("ta,tb,M,N", [(0, 0, 2000, 4000), (1, 1, 4000, 2000)])
+def test_product_of_a_short_reduction_with_a_large_leading_dimension(dev, ta, tb, M, N):
+    """Seventeen reduction indices 35 million apart: the other fifteen of a slice lie past 2^32 bytes, where 32-bit offsets would come
+    back into the first row; the other operand's rows are followed by numbers that are not part of the product."""
+    K, far_apart, padded = 17, 35_000_000, 40
+    rng = np.random.default_rng(M)
+    near = rng.standard_normal((M if ta else N, padded)).astype(np.float32)
+    rows = rng.standard_normal((K, N if tb else M)).astype(np.float32)
+    first = np.ones(far_apart, np.float32)  # (and what follows the first row's numbers)
+    first[:rows.shape[1]] = rows[0]
+    apart = dev.zeros(K * far_apart)
+    for k in range(K):
+        row = first if k == 0 else rows[k]
+        L.check(hip.fitre_hip_copy_h2d(C.c_void_p(apart.value + 4 * k * far_apart), row.ctypes.data_as(C.c_void_p), row.nbytes))
+    nb = hip.fitre_hip_gemm_workspace(M, N, K)
+    other, pc, ws = dev.upload(near.reshape(-1)), dev.zeros(M * N), dev.alloc(max(nb, 4))
+    pa, lda, pb, ldb = (other, padded, apart, far_apart) if ta else (apart, far_apart, other, padded)
+    with taken(FC_GEMM, SPLIT):
+        L.check(hip.fitre_hip_gemm(ta, tb, M, N, K, 1.0, pa, lda, pb, ldb, 0.0, pc, M, None, ws, nb))
+    got = dev.download(pc, M * N).reshape(N, M)
+    for q in (apart, other, pc, ws):
+        dev.free(q)
+    a, b = (near[:, :K].T, rows.T) if ta else (rows, near[:, :K])
+    assert far(got, b.astype(np.float64) @ a.astype(np.float64)) < 3 * 2.0**-24  # each accumulator and their sum are rounded a few times
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (1, 1)])
