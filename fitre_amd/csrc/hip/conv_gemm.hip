@@ -303,10 +303,14 @@ static size_t split_pos_room(const fitre_conv_shape *s, bool dx, const void *ws,
 // 25.6 / 30.3, 256 (2.4e9) 43 / 37; 32 x 32, 40 images (1.5e9) 46 / 34.  Whole tiles of 4 x 4 maps have the cell form to beat:
 // 256 -> 256, 128 images (1.2e9) 34.3 / 36.4, 256 (2.4e9) 45.4 / 44.5; 512 -> 512, 256 (9.7e9) 123 / 102.
 constexpr double kSplitWork = 7.0e8, kSplitNarrowWork = 1.5e9, kSplitCellWork = 2.0e9;
-// The gradients only from so many positions on.  A layer with fewer positions than a patch has entries has a weight gradient in the
-// span of its patches; what rounding adds outside of it, the curvature passes multiply by the inverse of the damping.  With these
-// kernels, whose rounding is no larger but another, VGG-11's natural gradient at 32 images (512 positions of 512 channels) moves
-// by 2.8e-4 of its norm, at 64 by 2e-5, at 96 by 1e-5, from 128 images (2048 positions) on by less than 7e-6.
+// The gradients only from so many positions on: below, results stay those of the fp32 kernels.  The line is one network's and no
+// bound of an error.  A layer with fewer positions than a patch has entries (4608 with 512 channels) has a weight gradient in the span of
+// its patches; what rounding adds outside of it, the curvature passes multiply by the inverse of the damping, so that a natural
+// gradient shows which kernels its gradients came from.  VGG-11, moved by both gradients / by input gradients alone at 32 images
+// (512 positions of 512 channels) 2.3e-4 / 0 of its norm, at 64 1.7e-5 / 1.1e-5, at 96 8e-6 / 5e-6; from 128 images (2048 positions), where
+// the split kernels run, by 5e-6 or less.  That is the error of either side: what an exact weight gradient would change in the natural
+// gradients of those two layers is 2.0e-4 and 2.1e-4 with the fp32 kernels, 1.0e-4 and 2.0e-4 with these at 32 images, 1.5e-5 and 1.7e-5 /
+// 0.8e-5 and 1.0e-5 at 64, 4e-6 and 6e-6 / 2e-6 and 4e-6 at 128.  Products of linear layers have no such line.
 constexpr long kSplitGradPositions = 2048;
 static bool split_pos_worthwhile(const fitre_conv_shape *s, bool dx, int pairs)
 {

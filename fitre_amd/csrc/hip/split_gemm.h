@@ -343,8 +343,9 @@ inline GemmPlan split_gemm_plan(long I, long J, long R, long mostSplits, long lo
 	return best;
 }
 
-// The plan in the place of an fp32 one: no more ranges (its workspace), and none more than four times as long.  A sum of K terms is
-// off by 0.1 sqrt(K) 2^-24 of its norm here and by 0.3 sqrt(K) 2^-24 there, so that its error is no larger.
+// The plan in the place of an fp32 one: no more ranges (its workspace), and none more than four times as long.  A sum of K terms
+// of either sign is off by 0.1 sqrt(K) 2^-24 of its norm here and by 0.3 sqrt(K) 2^-24 there, so that its error is no larger (of one
+// sign: split_bf16.h).
 inline GemmPlan split_gemm_plan_for(const GemmPlan &fp32, long I, long J, long R, long cus)
 {
 	return split_gemm_plan(I, J, R, fp32.splits, 4L * fp32.kChunk, cus);
