@@ -193,6 +193,23 @@ __device__ __forceinline__ float act_derivative(int actFun, float zi, float zo)
 	}
 }
 
+// d f'(x), as fitre_hip_activation_backward evaluates it
+__device__ __forceinline__ float act_backward_value(int actFun, float d, float zi, float zo)
+{
+	switch (actFun) {
+	case ACT_LOGISTIC: return d * zo * (1.f - zo);
+	case ACT_TANH: return d * ((1.f + zo) * (1.f - zo));
+	case CNN_ACT_SOFTPLUS: return d * (1.f / (1.f + expf(-zi)));
+	case CNN_ACT_SWISH: {
+		float t = 1.f / (1.f + expf(-zi));
+		return d * (zo + t * (1.f - zo));
+	}
+	case CNN_ACT_RELU: return zo > 0.f ? d : 0.f;
+	case CNN_ACT_ELU: return zo < 0.f ? d * (zo + 1.f) : d;
+	default: return d;
+	}
+}
+
 // the activation functions, as fitre_hip_activation_forward evaluates them
 __device__ __forceinline__ float act_forward_value(int actFun, float x)
 {

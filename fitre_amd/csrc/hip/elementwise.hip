@@ -183,6 +183,16 @@ void elementwise_release()
 	g_partials = nullptr, g_host_result = nullptr;
 }
 
+// the sums of `count` pairs of doubles, to host memory the device writes
+__global__ void __launch_bounds__(256) head_sums_kernel(const double *pairs, long count, float *result)
+{
+	__shared__ double lds[2][4];
+	double a = 0.0, b = 0.0;
+	for (long i = threadIdx.x; i < count; i += 256) a += pairs[2 * i], b += pairs[2 * i + 1];
+	a = block_sum<256>(a, lds[0]), b = block_sum<256>(b, lds[1]);
+	if (threadIdx.x == 0) result[0] = (float)a, result[1] = (float)b;
+}
+
 static int ensure_reduce_buffers()
 {
 	if (g_partials) return FITRE_OK;
@@ -557,6 +567,22 @@ int fitre_hip_activation_rop_backward(int actFun, const float *rdelta, const flo
 	LaunchScope scope(FITRE_KC_ACT_BWD, 24.0 * (double)n);
 	activation_rop_backward_kernel<<<blocks_for(n, 1024, 8192), 256, 0, stream()>>>(actFun, rdelta, delta, z_in, z_out, rz_in, out, n);
 	return check_launch("activation_rop_backward_kernel");
+}
+
+int fitre_hip_dense_head_sums(const double *headSums, long tiles, float *first, float *second)
+{
+	EW_CHECK("fitre_hip_dense_head_sums", headSums && tiles > 0 && first && second);
+	int rc = ensure_reduce_buffers();
+	if (rc) return rc;
+	{
+		LaunchScope scope(FITRE_KC_BLAS1, 16.0 * (double)tiles);
+		head_sums_kernel<<<1, 256, 0, stream()>>>(headSums, tiles, g_host_result);
+		rc = check_launch("head_sums_kernel");
+		if (rc) return rc;
+	}
+	FITRE_HIP_TRY(hipStreamSynchronize(stream()));
+	*first = g_host_result[0], *second = g_host_result[1];
+	return FITRE_OK;
 }
 
 int fitre_hip_fc_rop_backward(int actFun, const float *z, const float *rdz, const float *rx, const float *dx, float *out, long n)

@@ -37,22 +37,6 @@ struct SmallGemmParams {
 	float *partial;  // [range][N * M results, then M row sums] (no epilogue: small_gemm_reduce_kernel applies alpha and stores)
 };
 
-__device__ __forceinline__ float act_backward_value(int actFun, float d, float zi, float zo)
-{
-	switch (actFun) {
-	case ACT_LOGISTIC: return d * zo * (1.f - zo);
-	case ACT_TANH: return d * ((1.f + zo) * (1.f - zo));
-	case CNN_ACT_SOFTPLUS: return d * (1.f / (1.f + expf(-zi)));
-	case CNN_ACT_SWISH: {
-		float t = 1.f / (1.f + expf(-zi));
-		return d * (zo + t * (1.f - zo));
-	}
-	case CNN_ACT_RELU: return zo > 0.f ? d : 0.f;
-	case CNN_ACT_ELU: return zo < 0.f ? d * (zo + 1.f) : d;
-	default: return d;
-	}
-}
-
 // one workgroup's block (bx, by) of the result over reduction range bz
 __device__ __forceinline__ void small_gemm_block(const SmallGemmParams &p, const int bx, const int by, const int bz)
 {

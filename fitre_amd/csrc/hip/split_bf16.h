@@ -66,6 +66,15 @@ __device__ __forceinline__ v16f mfma_bf16(u32x4 a, u32x4 b, v16f c)
 	return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
+typedef float quad4f __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ quad4f buffer_load4(__amdgpu_buffer_rsrc_t r, uint32_t byteOffset)
+{
+	return __builtin_bit_cast(quad4f, __builtin_amdgcn_raw_buffer_load_b128(r, (int)byteOffset, 0, 0));
+}
+
+// an offset that stays out of range with a few words added to it
+constexpr uint32_t kSplitNowhere = 0xFFFFFF00u;
+
 constexpr int kTileSplit = 10, kTileSplitCell = 11; // profile variants of these kernels
 
 // a sum that the split may not have carried: not finite

@@ -18,15 +18,6 @@ struct QuadParams {
 	int rows;
 };
 
-typedef float quad4f __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ quad4f buffer_load4(__amdgpu_buffer_rsrc_t r, uint32_t byteOffset)
-{
-	return __builtin_bit_cast(quad4f, __builtin_amdgcn_raw_buffer_load_b128(r, (int)byteOffset, 0, 0));
-}
-
-// an offset that stays out of range with a few words added to it
-constexpr uint32_t kSplitNowhere = 0xFFFFFF00u;
-
 // ROWS x BK of an operand: UNITS groups of eight indices of a row per thread
 template <int ROWS, int BK>
 struct SplitUnits {

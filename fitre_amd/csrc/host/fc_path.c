@@ -99,6 +99,8 @@ static size_t largest_layer(const NN_MODEL *model)
 	return m;
 }
 
+static real *align_reals(real *p) { return (real *)(((size_t)p + 255) & ~(size_t)255); }
+
 /* workspace (bytes) of the products of a pass over `points` columns */
 static size_t product_ws_bytes(const NN_MODEL *model, int points, int backward)
 {
@@ -114,6 +116,35 @@ static size_t product_ws_bytes(const NN_MODEL *model, int points, int backward)
 	return (need + 255) & ~(size_t)255;
 }
 
+/* W z + b and its derivatives as one launch per layer (fitre_hip_dense_products): networks whose activations give their own
+ * derivative and whose products are within a few rounds of the chip. */
+static int fused_activation(int act) { return act == ACT_LOGISTIC || act == ACT_TANH || act == ACT_LINEAR; }
+
+static int fused_layers(const NN_MODEL *model, int points, int hidden, int backward)
+{
+	for (int i = 0; i < model->numLayers; i++) {
+		if (i < hidden && !fused_activation(model->actFuns[i])) return 0;
+		const int in = model->layerSizes[i], out = model->layerSizes[i + 1];
+		if (!fitre_hip_dense_product_fits(0, 0, out, points, in)) return 0;
+		if (backward && !(fitre_hip_dense_product_fits(0, 1, out, in, points) && fitre_hip_dense_product_fits(1, 0, in, points, out))) return 0;
+	}
+	return 1;
+}
+
+static fitre_dense_product dense(int transA, int transB, int M, int N, int K, const real *A, const real *B, real *C)
+{
+	fitre_dense_product p = { 0 };
+	p.transA = transA, p.transB = transB, p.M = M, p.N = N, p.K = K, p.A = A, p.B = B, p.C = C;
+	p.alpha = 1.f;
+	return p;
+}
+
+/* the weight gradients of a pass depend on nothing but what it left behind: eight to a launch */
+static void dense_all(const fitre_dense_product *p, int count)
+{
+	for (int at = 0; at < count; at += 8) HIP_CALL(fitre_hip_dense_products(p + at, count - at < 8 ? count - at : 8));
+}
+
 long nnForwardMemRequired(NN_MODEL *model, int points)
 {
 	/* [terms of the output head | product workspace] */
@@ -126,8 +157,6 @@ long nnGradientMemRequired(NN_MODEL *model, int points)
 	return (long)largest_layer(model) * points + 2L * points + nnForwardMemRequired(model, points) +
 	       (long)(product_ws_bytes(model, points, 1) / sizeof(real)) + 256;
 }
-
-static real *align_reals(real *p) { return (real *)(((size_t)p + 255) & ~(size_t)255); }
 
 static void layer_forward(int actFunction, const real *W, int wRows, int wCols, const real *b, const real *z, int zRows,
                           int zCols, real *output, int extendedCopy, void *ws, size_t wsBytes)
@@ -153,10 +182,25 @@ void applyLayerActivation(int actFunction, real *W, int wRows, int wCols, real *
 	HIP_CALL(fitre_hip_sync());
 }
 
-void nnForwardPass(NN_MODEL *model, DEVICE_DATASET *data, real *weights, real *z, real *errTerm, real *logLikelihood,
-                   real *modelError, real *hostPtr, real *devPtr, DATASET_SIZE isGradient, DATA_TYPE dataType)
+/* sums of a head's terms that are still on the device (tiles == 0: none) */
+typedef struct head_terms {
+	double *sums;
+	long tiles;
+	int points, mse;
+} HEAD_TERMS;
+
+static void finish_head(const HEAD_TERMS *head, real *logLikelihood, real *modelError)
 {
-	(void)hostPtr;
+	real ll = 0, squares = 0;
+	if (!head->tiles) return;
+	HIP_CALL(fitre_hip_dense_head_sums(head->sums, head->tiles, &ll, &squares));
+	*logLikelihood = ll * (real)(-1.0 / (double)head->points);
+	*modelError = head->mse ? squares / (real)head->points : 0;
+}
+
+static HEAD_TERMS forward_pass(NN_MODEL *model, DEVICE_DATASET *data, real *weights, real *z, real *errTerm, real *logLikelihood,
+                               real *modelError, real *devPtr, DATASET_SIZE isGradient, DATA_TYPE dataType)
+{
 	const int numLayers = model->numLayers;
 	const int *layerSizes = model->layerSizes;
 	const int *zOffsets = (isGradient == FULL_DATASET) ? model->zOffsets : model->sZOffsets;
@@ -179,6 +223,25 @@ void nnForwardPass(NN_MODEL *model, DEVICE_DATASET *data, real *weights, real *z
 	real *terms = devPtr;
 	void *ws = align_reals(terms + numElements);
 	const size_t wsBytes = product_ws_bytes(model, numCols, 0);
+
+	HEAD_TERMS terms_left = { NULL, 0, numColsTarget, model->type == MODEL_TYPE_MSE };
+	const int last = model->actFuns[numLayers - 1];
+	if ((last == ACT_LINEAR || last == ACT_LOGISTIC) && numCols == numColsTarget && fused_layers(model, numCols, numLayers, 0)) {
+		for (int i = 0; i < numLayers; i++) {
+			const int out = layerSizes[i + 1];
+			fitre_dense_product p = dense(0, 0, out, numCols, layerSizes[i], weights + wOffsets[i], (i == 0) ? dataset : z + zOffsets[i],
+			                              z + zOffsets[i + 1]);
+			p.bias = weights + bOffsets[i], p.act = model->actFuns[i], p.then = FITRE_DENSE_ACTIVATE;
+			if (i == numLayers - 1) {
+				p.then = (last == ACT_LINEAR) ? FITRE_DENSE_LINEAR_HEAD : FITRE_DENSE_LOGISTIC_HEAD;
+				p.d = target, p.also = errTerm;
+				terms_left.sums = p.headSums = (double *)align_reals(terms); /* 16 bytes a tile of 64 x 32 results or more */
+				terms_left.tiles = fitre_hip_dense_product_tiles(out, numCols);
+			}
+			HIP_CALL(fitre_hip_dense_products(&p, 1));
+		}
+		return terms_left;
+	}
 
 	for (int i = 0; i < numLayers; i++) {
 		const real *in = (i == 0) ? dataset : z + zOffsets[i];
@@ -217,6 +280,15 @@ void nnForwardPass(NN_MODEL *model, DEVICE_DATASET *data, real *weights, real *z
 		*modelError = mse / (real)numColsTarget;
 	}
 	HIP_CALL(fitre_hip_sync());
+	return terms_left;
+}
+
+void nnForwardPass(NN_MODEL *model, DEVICE_DATASET *data, real *weights, real *z, real *errTerm, real *logLikelihood,
+                   real *modelError, real *hostPtr, real *devPtr, DATASET_SIZE isGradient, DATA_TYPE dataType)
+{
+	(void)hostPtr;
+	const HEAD_TERMS head = forward_pass(model, data, weights, z, errTerm, logLikelihood, modelError, devPtr, isGradient, dataType);
+	finish_head(&head, logLikelihood, modelError); /* waits for the device, as the pass does that leaves no terms */
 }
 
 void evaluateModel(NN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, real *weights, real *logLikelihood,
@@ -252,8 +324,30 @@ void computeGradient(NN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratc
 	const int *rZOffsets = (isGradient == SAMPLED_DATASET) ? model->sRZOffsets : model->rZOffsets;
 	const int *bOffsets = model->bOffsets, *wOffsets = model->wOffsets;
 
-	nnForwardPass(model, data, weights, z, errorTerm, logLikelihood, modelError, scratch->nextHostPtr, nextDevPtr, isGradient,
-	              TRAIN_DATA);
+	const int fused = fused_layers(model, n, numLayers - 1, 1);
+	real *const topError = fused ? dx + rZOffsets[numLayers - 1] : errorTerm; /* the fused sweep works in the dx slots */
+	const HEAD_TERMS head = forward_pass(model, data, weights, z, topError, logLikelihood, modelError, nextDevPtr, isGradient, TRAIN_DATA);
+	if (fused) {
+		fitre_dense_product grads[MAX_LAYERS];
+		int count = 0;
+		for (int i = numLayers - 1; i >= 0; i--) {
+			const int out = layerSizes[i + 1], in = layerSizes[i];
+			/* dW = err * z_i', db = sum(err, 2), both scaled; err = f'(z_i) .* W_i' * err, one layer down */
+			fitre_dense_product *p = &grads[count++];
+			*p = dense(0, 1, out, in, n, dx + rZOffsets[i], (i == 0) ? dataset : z + zOffsets[i], dW + wOffsets[i]);
+			p->alpha = (real)(-1.0 / (double)n), p->rowSums = dW + bOffsets[i];
+			if (i > 0) {
+				fitre_dense_product q = dense(1, 0, in, n, out, weights + wOffsets[i], dx + rZOffsets[i], dx + rZOffsets[i - 1]);
+				q.then = FITRE_DENSE_DERIVATIVE, q.act = model->actFuns[i - 1], q.z = z + zOffsets[i];
+				HIP_CALL(fitre_hip_dense_products(&q, 1));
+			}
+		}
+		dense_all(grads, count);
+		finish_head(&head, logLikelihood, modelError);
+		HIP_CALL(fitre_hip_sync());
+		return;
+	}
+	finish_head(&head, logLikelihood, modelError);
 	void *ws = align_reals(nextDevPtr + nnForwardMemRequired(model, n));
 	const size_t wsBytes = product_ws_bytes(model, n, 1);
 
@@ -337,6 +431,48 @@ static void nn_rop(NN_MODEL *model, DEVICE_DATASET *data, real *z, real *dx, rea
 	real *tmp = oneVector + 2L * data->features;
 	void *ws = align_reals(tmp + (long)largest_layer(model) * n);
 	const real *VW = vec;
+
+	if (fused_layers(model, n, numLayers - 1, 1)) {
+		fitre_dense_product grads[MAX_LAYERS];
+		int count = 0;
+		for (int i = 0; i < numLayers; i++) {
+			const int out = layerSizes[i + 1], act = model->actFuns[i];
+			/* Rx = VW z + Vb + W Rz;  Rz = f'(.) Rx;  Rdx = -Rz at the top */
+			fitre_dense_product p = dense(0, 0, out, n, layerSizes[i], VW + wOffsets[i], (i == 0) ? trainX : z + zOffsets[i], Rz + zOffsets[i + 1]);
+			if (i > 0) p.A2 = weights + wOffsets[i], p.B2 = Rz + zOffsets[i];
+			p.bias = VW + bOffsets[i];
+			if (!gaussNewton) p.raw = Rx + zOffsets[i + 1];
+			if (i == numLayers - 1 && act == ACT_SOFTMAX) {
+				p.C = Rx + zOffsets[i + 1], p.raw = NULL;
+				HIP_CALL(fitre_hip_dense_products(&p, 1));
+				HIP_CALL(fitre_hip_column_softmax_rop(z + zOffsets[i + 1], p.C, out, n, Rz + zOffsets[i + 1]));
+				HIP_CALL(fitre_hip_copy_d2d(Rdx + rZOffsets[i], Rz + zOffsets[i + 1], sizeof(real) * (size_t)out * n));
+				HIP_CALL(fitre_hip_scal(out * n, -1.f, Rdx + rZOffsets[i]));
+				continue;
+			}
+			p.then = FITRE_DENSE_DERIVATIVE, p.act = act, p.z = z + zOffsets[i + 1];
+			if (i == numLayers - 1) p.also = Rdx + rZOffsets[i];
+			HIP_CALL(fitre_hip_dense_products(&p, 1));
+		}
+		for (int i = numLayers - 1; i >= 0; i--) {
+			const int out = layerSizes[i + 1], in = layerSizes[i];
+			/* RdW_i = Rdx_i z_i' (+ dx_i Rz_i', zero for the first layer); Rdb_i = sum(Rdx_i, 2) */
+			fitre_dense_product *p = &grads[count++];
+			*p = dense(0, 1, out, in, n, Rdx + rZOffsets[i], (i == 0) ? trainX : z + zOffsets[i], RdW + wOffsets[i]);
+			if (!gaussNewton && i > 0) p->A2 = dx + rZOffsets[i], p->B2 = Rz + zOffsets[i];
+			p->alpha = (real)(-1.0 / (double)n), p->rowSums = RdW + bOffsets[i];
+			if (i > 0) { /* Rdz_i as below, and what the layer under it makes of it */
+				fitre_dense_product q = dense(1, 0, in, n, out, weights + wOffsets[i], Rdx + rZOffsets[i], Rdx + rZOffsets[i - 1]);
+				if (!gaussNewton || i == numLayers - 1) q.A2 = VW + wOffsets[i], q.B2 = dx + rZOffsets[i];
+				q.then = FITRE_DENSE_ROP_BACKWARD, q.act = model->actFuns[i - 1], q.z = z + zOffsets[i];
+				if (!gaussNewton) q.x = Rx + zOffsets[i], q.d = dx + rZOffsets[i - 1];
+				HIP_CALL(fitre_hip_dense_products(&q, 1));
+			}
+		}
+		dense_all(grads, count);
+		HIP_CALL(fitre_hip_sync());
+		return;
+	}
 
 	HIP_CALL(fitre_hip_memset(RdW, 0, sizeof(real) * (size_t)model->pSize));
 

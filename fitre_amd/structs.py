@@ -158,3 +158,13 @@ class fitre_fc_tail_layer(C.Structure):
     """One layer of fitre_hip_fc_tail_backward (include/fitre_hip.h)."""
     _fields_ = [("in_", C.c_int), ("out", C.c_int), ("act", C.c_int), ("W", C.c_void_p), ("zPre", C.c_void_p),
                 ("zPost", C.c_void_p), ("zin", C.c_void_p), ("slot", C.c_void_p), ("dW", C.c_void_p), ("db", C.c_void_p)]
+
+
+FITRE_DENSE_STORE, FITRE_DENSE_ACTIVATE, FITRE_DENSE_DERIVATIVE, FITRE_DENSE_ROP_BACKWARD, FITRE_DENSE_LOGISTIC_HEAD, FITRE_DENSE_LINEAR_HEAD = range(6)
+
+
+class fitre_dense_product(C.Structure):
+    """A product of fitre_hip_dense_products and the step behind it (include/fitre_hip.h)."""
+    _fields_ = ([(n, C.c_int) for n in ("transA", "transB", "M", "N", "K")] + [(n, C.c_void_p) for n in ("A", "B", "A2", "B2")] +
+                [("alpha", C.c_float), ("bias", C.c_void_p), ("then", C.c_int), ("act", C.c_int)] +
+                [(n, C.c_void_p) for n in ("C", "raw", "also", "z", "x", "d", "headSums", "rowSums")])

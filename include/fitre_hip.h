@@ -453,6 +453,42 @@ int fitre_hip_gemm(int transA, int transB, int M, int N, int K, float alpha, con
                    const float *B, int ldb, float beta, float *C, int ldc, const float *bias, void *ws,
                    size_t wsBytes);
 
+/* A product of the fully connected family and the step behind it in one launch, and several independent ones (at most eight,
+ * transposed alike) in one launch: v(MxN) = alpha * (op(A)*op(B) + op(A2)*op(B2)) + bias per row, column-major with tight leading
+ * dimensions, A2 / B2 (like A / B) and bias may be NULL; not both operands transposed.  Then, M x N like C throughout:
+ *   STORE         C = v
+ *   ACTIVATE      C = f(v), f = act
+ *   DERIVATIVE    C = f'(.) .* v, by the activation's output z (functions/eval_gradient.cu: activations whose derivative it gives)
+ *   ROP_BACKWARD  C = f'(z) .* v + x .* g(z) .* d (fitre_hip_fc_rop_backward; x NULL: the first term)
+ *   LOGISTIC_HEAD C = f(v), also = d - C, the sums of the log-likelihood terms of logits v and targets d and of (d - C)^2
+ *   LINEAR_HEAD   C = v, also = 2 (d - v), both sums of (d - v)^2
+ * raw (may be NULL): v is stored too.  also: of no head, where not NULL, -C.  headSums: fitre_hip_dense_product_tiles
+ * pairs of doubles (B not transposed, one product a call), which fitre_hip_dense_head_sums adds and returns (it waits for the lane).  rowSums (may be NULL): alpha times the
+ * sums of A's rows (A not transposed), the first pair's.  Needs no workspace. */
+enum {
+	FITRE_DENSE_STORE = 0,
+	FITRE_DENSE_ACTIVATE = 1,
+	FITRE_DENSE_DERIVATIVE = 2,
+	FITRE_DENSE_ROP_BACKWARD = 3,
+	FITRE_DENSE_LOGISTIC_HEAD = 4,
+	FITRE_DENSE_LINEAR_HEAD = 5
+};
+typedef struct fitre_dense_product {
+	int transA, transB, M, N, K;
+	const float *A, *B, *A2, *B2;
+	float alpha;
+	const float *bias;
+	int then, act;
+	float *C, *raw, *also;
+	const float *z, *x, *d;
+	double *headSums;
+	float *rowSums;
+} fitre_dense_product;
+int fitre_hip_dense_product_fits(int transA, int transB, int M, int N, int K); /* this way is the shorter one */
+long fitre_hip_dense_product_tiles(int M, int N);
+int fitre_hip_dense_products(const fitre_dense_product *p, int count);
+int fitre_hip_dense_head_sums(const double *headSums, long tiles, float *first, float *second);
+
 /* Backward products of one fully connected layer, W out x in column-major, delta out x n, one launch each
  * where the layer is small (fitre_hip_linear_is_small), the plain sequence of steps otherwise.
  *   input gradient (functions/cnn_backward.cu:250-254 followed by the activation step of the layer below,
