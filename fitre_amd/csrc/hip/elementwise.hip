@@ -173,8 +173,8 @@ __global__ void __launch_bounds__(256) reduce_stage2(const double *partial, int 
 }
 
 constexpr int kRedBlocks = 1024;
-static double *g_partials = nullptr; // kRedBlocks doubles + 1 float result slot
-static float *g_host_result = nullptr;
+static double *g_partials = nullptr;     // kRedBlocks doubles
+static float *g_host_result = nullptr;   // pinned: the last kernel of a reduction writes it, and no copy follows
 
 void elementwise_release()
 {
@@ -196,7 +196,7 @@ __global__ void __launch_bounds__(256) head_sums_kernel(const double *pairs, lon
 static int ensure_reduce_buffers()
 {
 	if (g_partials) return FITRE_OK;
-	FITRE_HIP_TRY(hipMalloc((void **)&g_partials, (kRedBlocks + 2) * sizeof(double)));
+	FITRE_HIP_TRY(hipMalloc((void **)&g_partials, kRedBlocks * sizeof(double)));
 	FITRE_HIP_TRY(hipHostMalloc((void **)&g_host_result, 64, hipHostMallocDefault));
 	return FITRE_OK;
 }
@@ -215,12 +215,10 @@ static int scalar_reduce(const char *name, int n, const float *x, const float *y
 	{
 		LaunchScope scope(FITRE_KC_BLAS1, 4.0 * n * (OP == RED_DOT ? 2 : 1));
 		unsigned blocks = blocks_for(n, 256 * 8, kRedBlocks);
-		float *devResult = (float *)(g_partials + kRedBlocks);
 		reduce_stage1<OP><<<blocks, 256, 0, stream()>>>(x, y, n, g_partials);
-		reduce_stage2<OP><<<1, 256, 0, stream()>>>(g_partials, (int)blocks, devResult);
+		reduce_stage2<OP><<<1, 256, 0, stream()>>>(g_partials, (int)blocks, g_host_result);
 		rc = check_launch(name);
 		if (rc) return rc;
-		FITRE_HIP_TRY(hipMemcpyAsync(g_host_result, devResult, sizeof(float), hipMemcpyDeviceToHost, stream()));
 	}
 	FITRE_HIP_TRY(hipStreamSynchronize(stream()));
 	*result = *g_host_result;

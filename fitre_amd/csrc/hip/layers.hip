@@ -1662,12 +1662,40 @@ __global__ void __launch_bounds__(256) mean_kernel(const float *x, int n, float 
 	double acc = 0.0;
 	for (int i = threadIdx.x; i < n; i += 256) acc += (double)x[i];
 	double t = block_sum<256>(acc, lds);
-	if (threadIdx.x == 0) out[0] = (float)(t / (double)n);
+	if (threadIdx.x == 0) out[0] = (float)(t / (double)n); // may be host memory
 }
 
 static float *g_nll = nullptr;
 static int g_nll_rows = 0;
 static float *g_loss_host = nullptr;
+
+static int loss_room(int rows)
+{
+	if (rows > g_nll_rows) {
+		FITRE_HIP_TRY(hipDeviceSynchronize()); // the buffer is shared by every lane
+		if (g_nll) FITRE_HIP_TRY(hipFree(g_nll));
+		g_nll = nullptr;
+		g_nll_rows = 0;
+		int cap = rows < 4096 ? 4096 : rows;
+		FITRE_HIP_TRY(hipMalloc((void **)&g_nll, sizeof(float) * (size_t)cap));
+		g_nll_rows = cap;
+	}
+	if (!g_loss_host) FITRE_HIP_TRY(hipHostMalloc((void **)&g_loss_host, 64, hipHostMallocDefault));
+	return FITRE_OK;
+}
+float *loss_terms(int rows) { return loss_room(rows) == FITRE_OK ? g_nll : nullptr; }
+int loss_mean(int rows, float *lossHost)
+{
+	{
+		LaunchScope scope(FITRE_KC_SOFTMAX, 4.0 * rows);
+		mean_kernel<<<1, 256, 0, stream()>>>(g_nll, rows, g_loss_host); // pinned memory the device writes: no copy behind it
+		const int rc = check_launch("mean_kernel");
+		if (rc) return rc;
+	}
+	FITRE_HIP_TRY(hipStreamSynchronize(stream()));
+	*lossHost = *g_loss_host;
+	return FITRE_OK;
+}
 
 void layers_release()
 {
@@ -2253,27 +2281,15 @@ int fitre_hip_softmax_cross_entropy(const float *logits, const float *target, in
 	FITRE_NEED_INIT();
 	FITRE_REQUIRE(logits && target && probs && lossHost, "fitre_hip_softmax_cross_entropy: null pointer");
 	FITRE_REQUIRE(rows > 0 && classes > 0, "fitre_hip_softmax_cross_entropy: non-positive shape (%d x %d)", rows, classes);
-	if (rows > g_nll_rows) {
-		FITRE_HIP_TRY(hipDeviceSynchronize()); // the buffer is shared by every lane
-		if (g_nll) FITRE_HIP_TRY(hipFree(g_nll));
-		g_nll = nullptr;
-		g_nll_rows = 0;
-		int cap = rows < 4096 ? 4096 : rows;
-		FITRE_HIP_TRY(hipMalloc((void **)&g_nll, sizeof(float) * ((size_t)cap + 16)));
-		g_nll_rows = cap;
-	}
-	if (!g_loss_host) FITRE_HIP_TRY(hipHostMalloc((void **)&g_loss_host, 64, hipHostMallocDefault));
+	float *nll = loss_terms(rows);
+	if (!nll) return FITRE_E_DEVICE;
 	{
 		LaunchScope scope(FITRE_KC_SOFTMAX, 4.0 * rows * classes * 2);
-		softmax_ce_kernel<<<blocks_for(rows, 4), 256, 0, stream()>>>(logits, target, rows, classes, probs, errors, g_nll);
-		mean_kernel<<<1, 256, 0, stream()>>>(g_nll, rows, g_nll + g_nll_rows);
+		softmax_ce_kernel<<<blocks_for(rows, 4), 256, 0, stream()>>>(logits, target, rows, classes, probs, errors, nll);
 		int rc = check_launch("softmax_ce_kernel");
 		if (rc) return rc;
 	}
-	FITRE_HIP_TRY(hipMemcpyAsync(g_loss_host, g_nll + g_nll_rows, sizeof(float), hipMemcpyDeviceToHost, stream()));
-	FITRE_HIP_TRY(hipStreamSynchronize(stream()));
-	*lossHost = *g_loss_host;
-	return FITRE_OK;
+	return loss_mean(rows, lossHost);
 }
 
 int fitre_hip_cross_entropy_rop_error(const float *rz, const float *probs, int rows, int classes, float *rError)
