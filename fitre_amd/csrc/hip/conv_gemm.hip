@@ -9,6 +9,7 @@
 #include "conv_split_dw.h"
 #include "conv_thin.h"
 #include "conv_thin_forward.h"
+#include "thin_net.h"
 #include "linear_small.h"
 #include "linear_tail.h"
 #include "linear_forward.h"
@@ -1408,6 +1409,49 @@ int fitre_hip_linear_weight_grad(int in, int out, int n, const float *delta, con
 	int rc = gemm_ex(0, 1, out, in, n, 1.f, delta, out, zin, in, 0.f, dW, out, nullptr, FITRE_KC_FC_GEMM, ws, wsBytes);
 	if (rc || !db) return rc;
 	return fitre_hip_row_sum(delta, out, n, db);
+}
+
+// ---- forward pass of a whole small network ----------------------------------------------------
+int fitre_hip_thin_net_forward_fits(int convs, const fitre_thin_net_layer *c, int linears, const fitre_fc_forward_layer *l, int n, int classes)
+{
+	NetParams p{};
+	int words;
+	return c && (linears == 0 || l) && net_fits(n) && net_plan(convs, c, linears, l, n, classes, p, words);
+}
+int fitre_hip_thin_net_forward(int convs, const fitre_thin_net_layer *c, int linears, const fitre_fc_forward_layer *l, int n, const float *x,
+                               const float *target, int classes, float *probs, float *errors, float *lossHost)
+{
+	FITRE_NEED_INIT();
+	FITRE_REQUIRE(c && x && target && probs && lossHost && (linears == 0 || l), "fitre_hip_thin_net_forward: null pointer");
+	NetParams p{};
+	int words;
+	FITRE_REQUIRE(net_plan(convs, c, linears, l, n, classes, p, words), "fitre_hip_thin_net_forward: this network does not fit one launch");
+	double work = 0.0;
+	for (int i = 0; i < convs; i++) {
+		FITRE_REQUIRE(c[i].w && c[i].y && c[i].actOut && c[i].poolOut, "fitre_hip_thin_net_forward: null pointer");
+		FITRE_REQUIRE(act_known(c[i].act), "fitre_hip_thin_net_forward: unknown activation code %d", c[i].act);
+		NetConv &q = p.c[i];
+		q.w = c[i].w, q.bias = c[i].bias, q.y = c[i].y, q.actOut = c[i].actOut, q.poolOut = c[i].poolOut, q.act = c[i].act, q.average = c[i].average != 0;
+		work += conv_flops(&c[i].shape);
+	}
+	for (int f = 0; f < linears; f++) {
+		FITRE_REQUIRE(l[f].W && l[f].pre && l[f].post, "fitre_hip_thin_net_forward: null pointer");
+		FITRE_REQUIRE(act_known(l[f].act), "fitre_hip_thin_net_forward: unknown activation code %d", l[f].act);
+		int logWidth = 0;
+		while ((1 << logWidth) < l[f].out) logWidth++;
+		p.l[f] = NetLinear{ l[f].in, l[f].out, l[f].act, logWidth, l[f].W, l[f].bias, l[f].pre, l[f].post };
+		work += 2.0 * l[f].in * l[f].out * n;
+	}
+	p.x = x, p.target = target, p.probs = probs, p.errors = errors;
+	p.nll = loss_terms(n);
+	if (!p.nll) return FITRE_E_DEVICE;
+	{
+		LaunchScope scope(FITRE_KC_CONV_FWD, work, 0);
+		thin_net_forward_kernel<<<(unsigned)n, kNetThreads, sizeof(float) * (size_t)words, stream()>>>(p);
+		const int rc = check_launch("thin_net_forward_kernel");
+		if (rc) return rc;
+	}
+	return loss_mean(n, lossHost);
 }
 
 // ---- forward pass of a run of small layers ----------------------------------------------------

@@ -23,9 +23,6 @@ constexpr int kThinMaxChannels = 16; // accumulators a thread holds
 constexpr int kThinLdsFloats = 12288; // 48 KB of staging per workgroup
 
 struct ThinConvParams {
-	const float *x;     // [Cin][N][inA][inB]   (weight gradient)
-	const float *delta; // [Cout][N][outA][outB]
-	const float *w;     // [Cout][Cin][k][k]     (input gradient)
 	int cin, cout, samples, inA, inB, outA, outB, ksize, stride, pad;
 	int imagesPerGroup;
 	int ciPerGroup; // input gradient: input channels per workgroup
@@ -37,6 +34,20 @@ struct ThinConvParams {
 	FastDiv divPBx;          // weight gradient: row length of the bordered input
 	FastDiv divXPlane[2], divDPos[2]; // weight gradient: bordered input plane / positions of a full band [0] and of an image's last band [1]
 };
+
+__device__ __forceinline__ void thin_store_row(float *out, const float *v, int store, int left)
+{
+	if (store == 4) {
+		*reinterpret_cast<float4 *>(out) = make_float4(v[0], v[1], v[2], v[3]);
+	} else if (store == 2) {
+		*reinterpret_cast<float2 *>(out) = make_float2(v[0], v[1]);
+		if (left > 2) *reinterpret_cast<float2 *>(out + 2) = make_float2(v[2], v[3]);
+	} else {
+#pragma unroll
+		for (int j = 0; j < 4; j++)
+			if (j < left) out[j] = v[j];
+	}
+}
 
 // ---- input gradient (stride 1): dx[ci][n][a][b] = sum_co sum_taps W[co][ci][ta][tb] * delta[co][n][a - ta + p][b - tb + p]
 // One workgroup per (image, group of input channels).  The image's delta (all output channels) sits in LDS with a
@@ -63,6 +74,36 @@ struct ThinPoolFold {
 	int actFun;
 };
 
+// the gradients of two neighbouring windows of the map below, whose two rows of four cells are r0, r1 (behind the activation) and i0,
+// i1 (before it)
+__device__ __forceinline__ void thin_fold_windows(const ThinPoolFold &fold, float left, float right, float4 r0, float4 r1, float4 i0, float4 i1, size_t at, int bigB)
+{
+	float4 g0 = make_float4(0.f, 0.f, 0.f, 0.f), g1 = g0;
+	int arg = scan2x2(r0.x, r0.y, r1.x, r1.y);
+	if (arg == 0) g0.x = left;
+	else if (arg == 1) g0.y = left;
+	else if (arg == 2) g1.x = left;
+	else if (arg == 3) g1.y = left;
+	arg = scan2x2(r0.z, r0.w, r1.z, r1.w);
+	if (arg == 0) g0.z = right;
+	else if (arg == 1) g0.w = right;
+	else if (arg == 2) g1.z = right;
+	else if (arg == 3) g1.w = right;
+	if (fold.dxPool) {
+		*reinterpret_cast<float4 *>(fold.dxPool + at) = g0;
+		*reinterpret_cast<float4 *>(fold.dxPool + at + bigB) = g1;
+	}
+	g0.x *= act_derivative(fold.actFun, i0.x, r0.x);
+	g0.y *= act_derivative(fold.actFun, i0.y, r0.y);
+	g0.z *= act_derivative(fold.actFun, i0.z, r0.z);
+	g0.w *= act_derivative(fold.actFun, i0.w, r0.w);
+	g1.x *= act_derivative(fold.actFun, i1.x, r1.x);
+	g1.y *= act_derivative(fold.actFun, i1.y, r1.y);
+	g1.z *= act_derivative(fold.actFun, i1.z, r1.z);
+	g1.w *= act_derivative(fold.actFun, i1.w, r1.w);
+	*reinterpret_cast<float4 *>(fold.dxAct + at) = g0;
+	*reinterpret_cast<float4 *>(fold.dxAct + at + bigB) = g1;
+}
 template <int KS, bool FOLD>
 __global__ void __launch_bounds__(256)
 thin_input_grad_kernel(const ThinConvParams p, const float *__restrict__ w, const float *__restrict__ delta, float *__restrict__ dx,
@@ -170,34 +211,7 @@ thin_input_grad_kernel(const ThinConvParams p, const float *__restrict__ w, cons
 #pragma unroll
 				for (int h = 0; h < 2; h++) {
 					if (b0 + 2 * h >= p.inB) continue;
-					const float4 r0 = zo[h][0], r1 = zo[h][1];
-					float4 g0 = make_float4(0.f, 0.f, 0.f, 0.f), g1 = g0;
-					int arg = scan2x2(r0.x, r0.y, r1.x, r1.y);
-					if (arg == 0) g0.x = acc[2 * h];
-					else if (arg == 1) g0.y = acc[2 * h];
-					else if (arg == 2) g1.x = acc[2 * h];
-					else if (arg == 3) g1.y = acc[2 * h];
-					arg = scan2x2(r0.z, r0.w, r1.z, r1.w);
-					if (arg == 0) g0.z = acc[2 * h + 1];
-					else if (arg == 1) g0.w = acc[2 * h + 1];
-					else if (arg == 2) g1.z = acc[2 * h + 1];
-					else if (arg == 3) g1.w = acc[2 * h + 1];
-					const size_t at = below + 4 * h;
-					if (fold.dxPool) {
-						*reinterpret_cast<float4 *>(fold.dxPool + at) = g0;
-						*reinterpret_cast<float4 *>(fold.dxPool + at + bigB) = g1;
-					}
-					const float4 i0 = zi[h][0], i1 = zi[h][1];
-					g0.x *= act_derivative(fold.actFun, i0.x, r0.x);
-					g0.y *= act_derivative(fold.actFun, i0.y, r0.y);
-					g0.z *= act_derivative(fold.actFun, i0.z, r0.z);
-					g0.w *= act_derivative(fold.actFun, i0.w, r0.w);
-					g1.x *= act_derivative(fold.actFun, i1.x, r1.x);
-					g1.y *= act_derivative(fold.actFun, i1.y, r1.y);
-					g1.z *= act_derivative(fold.actFun, i1.z, r1.z);
-					g1.w *= act_derivative(fold.actFun, i1.w, r1.w);
-					*reinterpret_cast<float4 *>(fold.dxAct + at) = g0;
-					*reinterpret_cast<float4 *>(fold.dxAct + at + bigB) = g1;
+					thin_fold_windows(fold, acc[2 * h], acc[2 * h + 1], zo[h][0], zo[h][1], zi[h][0], zi[h][1], below + 4 * h, bigB);
 				}
 			}
 		}
@@ -396,7 +410,6 @@ static inline int thin_dw_row_words(const fitre_conv_shape *s)
 static inline ThinConvParams thin_params(const fitre_conv_shape *s)
 {
 	ThinConvParams p;
-	p.x = p.delta = p.w = nullptr;
 	p.cin = s->inChannels, p.cout = s->outChannels, p.samples = s->samples;
 	p.inA = s->inA, p.inB = s->inB, p.outA = s->outA, p.outB = s->outB;
 	p.ksize = s->ksize, p.stride = s->stride, p.pad = s->padding;

@@ -12,7 +12,7 @@
 // Measured, a whole forward and backward pass, before and after: LeNet with batch norm at batch 1024 488 -> 362 us, without at
 // batch 128 176 -> 149, with average pools at batch 16 175 -> 145.
 #pragma once
-#include "conv_thin.h"
+#include "conv_thin_matrix.h"
 
 namespace fitre {
 
@@ -32,20 +32,6 @@ struct ThinFwdParams {
 	bool average, toFc;
 	float *actOut, *poolOut;
 };
-
-__device__ __forceinline__ void thin_store_row(float *out, const float *v, int store, int left)
-{
-	if (store == 4) {
-		*reinterpret_cast<float4 *>(out) = make_float4(v[0], v[1], v[2], v[3]);
-	} else if (store == 2) {
-		*reinterpret_cast<float2 *>(out) = make_float2(v[0], v[1]);
-		if (left > 2) *reinterpret_cast<float2 *>(out + 2) = make_float2(v[2], v[3]);
-	} else {
-#pragma unroll
-		for (int j = 0; j < 4; j++)
-			if (j < left) out[j] = v[j];
-	}
-}
 
 // Words of a bordered image below which a workgroup's images are staged together.  Of the time one by one, 1 to 1024 images:
 // 0.2 at 96 words, 0.35 at 288, 0.7 at 768, 0.83 to 0.87 at 1152; 0.94 to 1.05 at 1296, 1.0 to 1.04 at 1680 and 1.0 to 1.06
@@ -280,6 +266,17 @@ static int launch_thin_forward(const fitre_conv_shape *s, const ThinFwdPlan &pla
 	const dim3 grid((unsigned)plan.groupsX, (unsigned)plan.groupsY);
 	const size_t lds = sizeof(float) * (size_t)p.images * imageFloats;
 	LaunchScope scope(FITRE_KC_CONV_FWD, conv_flops(s), 0);
+	ThinMatPlan m;
+	if (s->outChannels >= kThinMatLeastRows && thin_mat_plan(s, fold != nullptr, m)) {
+		m.p.src = x, m.p.w = w, m.p.bias = bias, m.p.out = y, m.p.store = p.store;
+		if (fold) {
+			m.p.act = fold->act, m.p.average = fold->average, m.p.toFc = fold->toFc, m.p.actOut = fold->actOut, m.p.poolOut = fold->poolOut;
+			launch_thin_matrix<true>(m);
+		} else {
+			launch_thin_matrix<false>(m);
+		}
+		return check_launch("thin_matrix_kernel");
+	}
 	auto launch = [&](auto kernel) { kernel<<<grid, 256, lds, stream()>>>(p, x, w); };
 	auto pick = [&](auto ks) {
 		constexpr int KS = decltype(ks)::value;

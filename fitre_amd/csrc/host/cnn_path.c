@@ -181,6 +181,45 @@ long cnnBackwardMemRequired(CNN_MODEL *model)
 	return (long)((backward_ws_bytes(model, model->batchSize) + sizeof(real) - 1) / sizeof(real));
 }
 
+/* the linear layers from l up as the fused forward launches see them */
+static int forward_rest(const CNN_MODEL *model, const real *weights, real *z, int n, int l, fitre_fc_forward_layer *rest)
+{
+	const int nc = model->cLayers, left = model->lLayers - l;
+	for (int k = 0; k < left && left <= 4; k++) {
+		const FC_LAYER *g = &model->fcLayer[l + k];
+		real *post = z + model->zOffsets[l + k + 1 + nc];
+		fitre_fc_forward_layer t = { g->in, g->out, g->actFun, weights + model->wOffsets[l + k + nc],
+			                         (model->bias == 0) ? NULL : weights + model->bOffsets[l + k + nc], post + (long)g->out * n, post };
+		rest[k] = t;
+	}
+	return left;
+}
+
+/* a network of few channels without batch norm (LeNet): every layer, softmax and loss in one launch; 0 where it is none */
+static int forward_in_one_launch(const CNN_MODEL *model, const DEVICE_DATASET *data, real *z, real *probs, real *errors, int n, real *loss)
+{
+	fitre_thin_net_layer conv[3];
+	fitre_fc_forward_layer rest[4];
+	const int nc = model->cLayers;
+	if (nc > 3 || model->lLayers > 4) return 0;
+	for (int l = 0; l < nc; l++) {
+		const CONV_LAYER *cv = &model->convLayer[l];
+		const POOL_LAYER *pl = &model->poolLayer[l];
+		real *slab = z + model->zOffsets[l + 1];
+		if (has_bn(cv) || (pl->type != MAX_POOL && pl->type != AVG_POOL) || pl->pSize != 2 || pl->stride != 2 || pl->padding != 0 ||
+		    pl->outWidth * 2 != cv->outWidth || pl->outHeight * 2 != cv->outHeight || cv->outputOffset != cv->poolOffset)
+			return 0;
+		fitre_thin_net_layer t = { conv_shape(cv, n), model->actFuns[l], pl->type == AVG_POOL, data->weights + model->wOffsets[l],
+			                       (model->bias == 0) ? NULL : data->weights + model->bOffsets[l], slab, slab + cv->activationOffset,
+			                       slab + cv->poolOffset };
+		conv[l] = t;
+	}
+	forward_rest(model, data->weights, z, n, 0, rest);
+	if (!fitre_hip_thin_net_forward_fits(nc, conv, model->lLayers, rest, n, data->numClasses)) return 0;
+	HIP_CALL(fitre_hip_thin_net_forward(nc, conv, model->lLayers, rest, n, data->currentBatch, data->sampledTrainY, data->numClasses, probs, errors, loss));
+	return 1;
+}
+
 real cnnForward(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, real *z, real *probs, real *errors,
                 int s, int curBatchSize, EVAL_TYPE forTesting)
 {
@@ -201,6 +240,11 @@ real cnnForward(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, r
 		exit(-1);
 	}
 
+	real loss = 0;
+	if (forward_in_one_launch(model, data, z, probs, errors, n, &loss)) {
+		HIP_CALL(fitre_hip_sync());
+		return loss;
+	}
 	for (int l = 0; l < nc; l++) {
 		const CONV_LAYER *cv = &model->convLayer[l];
 		const POOL_LAYER *pl = &model->poolLayer[l];
@@ -231,14 +275,7 @@ real cnnForward(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, r
 		/* the layers from here up in one launch, where they are small enough (LeNet's three, VGG's one, the upper two of the
 		 * CIFAR AlexNet) */
 		fitre_fc_forward_layer rest[4];
-		const int left = model->lLayers - l;
-		for (int k = 0; k < left && left <= 4; k++) {
-			const FC_LAYER *g = &model->fcLayer[l + k];
-			real *post = z + zOffsets[l + k + 1 + nc];
-			fitre_fc_forward_layer t = { g->in, g->out, g->actFun, weights + wOffsets[l + k + nc],
-				                         (model->bias == 0) ? NULL : weights + bOffsets[l + k + nc], post + (long)g->out * n, post };
-			rest[k] = t;
-		}
+		const int left = forward_rest(model, weights, z, n, l, rest);
 		if (left <= 4 && fitre_hip_fc_tail_forward_fits(left, rest, n)) {
 			HIP_CALL(fitre_hip_fc_tail_forward(left, rest, n, z + zOffsets[l + nc] + outputOffset));
 			break;
@@ -254,7 +291,6 @@ real cnnForward(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, r
 	}
 
 	const real *logits = (model->lLayers == 0) ? feat : z + zOffsets[model->lLayers + nc];
-	real loss = 0;
 	HIP_CALL(fitre_hip_softmax_cross_entropy(logits, data->sampledTrainY, n, data->numClasses, probs, errors, &loss));
 	HIP_CALL(fitre_hip_sync());
 	return loss;

@@ -168,3 +168,8 @@ class fitre_dense_product(C.Structure):
     _fields_ = ([(n, C.c_int) for n in ("transA", "transB", "M", "N", "K")] + [(n, C.c_void_p) for n in ("A", "B", "A2", "B2")] +
                 [("alpha", C.c_float), ("bias", C.c_void_p), ("then", C.c_int), ("act", C.c_int)] +
                 [(n, C.c_void_p) for n in ("C", "raw", "also", "z", "x", "d", "headSums", "rowSums")])
+
+
+class fitre_thin_net_layer(C.Structure):
+    """A convolution layer of fitre_hip_thin_net_forward (include/fitre_hip.h)."""
+    _fields_ = [("shape", fitre_conv_shape), ("act", C.c_int), ("average", C.c_int)] + [(n, C.c_void_p) for n in ("w", "bias", "y", "actOut", "poolOut")]

@@ -525,6 +525,21 @@ typedef struct fitre_fc_forward_layer {
 int fitre_hip_fc_tail_forward_fits(int layers, const fitre_fc_forward_layer *l, int n);
 int fitre_hip_fc_tail_forward(int layers, const fitre_fc_forward_layer *l, int n, const float *x);
 
+/* The forward pass of a whole small network in one launch (functions/cnn_forward.cu:49-383): one to three convolutions (windows of 3
+ * or 5, stride 1, at most sixteen channels, even maps) with an activation and a 2 x 2 / stride 2 pool behind each, none to four
+ * linear layers as in fitre_hip_fc_tail_forward, softmax, loss errors (may be NULL) and the mean loss, which is waited for.  The
+ * tensors are those the steps of their own leave; the last pool's output is in the linear layers' order.  _fits: the network
+ * is one of these, and this way is the shorter one. */
+typedef struct fitre_thin_net_layer {
+	fitre_conv_shape shape;
+	int act, average; /* average != 0: average pool, else max pool */
+	const float *w, *bias;
+	float *y, *actOut, *poolOut;
+} fitre_thin_net_layer;
+int fitre_hip_thin_net_forward_fits(int convs, const fitre_thin_net_layer *c, int linears, const fitre_fc_forward_layer *l, int n, int classes);
+int fitre_hip_thin_net_forward(int convs, const fitre_thin_net_layer *c, int linears, const fitre_fc_forward_layer *l, int n, const float *x,
+                               const float *target, int classes, float *probs, float *errors, float *lossHost);
+
 /* The backward products of a whole tail of small fully connected layers (layers[0] the lowest) in two launches (three
  * when the batch is above 512): every layer's delta (after its activation derivative) into its slot, dW = delta * zin',
  * db = delta * 1, and the lowest layer's input gradient W' * delta into `features` -- in a convolution layer's layout
