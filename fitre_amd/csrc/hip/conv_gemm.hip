@@ -349,6 +349,14 @@ static int launch_split_weights(const fitre_conv_shape *s, bool dx, const float 
 	return check_launch("split_weights_kernel");
 }
 
+template <bool DX>
+static void launch_split_weights_batch(int ksize, const SplitWeightsBatch &b)
+{
+	const unsigned blocks = (unsigned)b.first[b.count];
+	if (ksize == 3) split_weights_batch_kernel<3, DX><<<blocks, 256, 0, stream()>>>(b);
+	else split_weights_batch_kernel<5, DX><<<blocks, 256, 0, stream()>>>(b);
+}
+
 // prepared: weights split beforehand (one pair only; null: split here, into the end of ws).  leftSplits: as in launch_c3_pos.
 static int launch_split_pos(const fitre_conv_shape *s, bool dx, const float *src, const float *w, const float *bias, float *outPtr, void *ws,
                             size_t wsBytes, const void *prepared, int *leftSplits, const float *src2 = nullptr, const float *w2 = nullptr)
@@ -411,11 +419,11 @@ static int launch_split_pos(const fitre_conv_shape *s, bool dx, const float *src
 }
 
 // whether the forward product takes the same kernel, cut into as many ranges, in the first `less` bytes of a workspace as in all of it
-static bool pos_forward_fits_in(const fitre_conv_shape *s, const void *ws, size_t less, size_t wsBytes)
+static bool pos_forward_fits_in(const fitre_conv_shape *s, const void *ws, size_t less, size_t wsBytes, bool prepared)
 {
-	const bool split = split_pos_chosen(s, false, ws, wsBytes);
-	if (split != split_pos_chosen(s, false, ws, less)) return false;
-	if (split) return split_pos_fit(s, false, ws, less, 1, false).splits == split_pos_fit(s, false, ws, wsBytes, 1, false).splits;
+	const bool split = split_pos_chosen(s, false, ws, wsBytes, 1, prepared);
+	if (split != split_pos_chosen(s, false, ws, less, 1, prepared)) return false;
+	if (split) return split_pos_fit(s, false, ws, less, 1, prepared).splits == split_pos_fit(s, false, ws, wsBytes, 1, prepared).splits;
 	const BlockPlan plan = c3_pos_plan(s, false);
 	const long blocks = s->inChannels / kC3CB, J = (long)s->samples * s->inA * s->inB;
 	return fit_blocks(plan, blocks, s->outChannels, J, ws, less).splits == fit_blocks(plan, blocks, s->outChannels, J, ws, wsBytes).splits;
@@ -904,6 +912,15 @@ int fitre_hip_conv_bn_act_pool_forward(const fitre_conv_shape *s, const float *x
                                        float momentum, int train, int actFun, float *actOut, int poolType, int ksize, int stride, int padding,
                                        int poolA, int poolB, float *poolOut, int toFc, void *ws, size_t wsBytes)
 {
+	return fitre_hip_conv_bn_act_pool_forward_prepared(s, x, w, nullptr, bias, y, zhat, mean, variance, runningMean, runningVariance, epsilon, momentum,
+	                                                   train, actFun, actOut, poolType, ksize, stride, padding, poolA, poolB, poolOut, toFc, ws, wsBytes);
+}
+
+int fitre_hip_conv_bn_act_pool_forward_prepared(const fitre_conv_shape *s, const float *x, const float *w, const void *prepared, const float *bias,
+                                                float *y, float *zhat, float *mean, float *variance, float *runningMean, float *runningVariance,
+                                                float epsilon, float momentum, int train, int actFun, float *actOut, int poolType, int ksize,
+                                                int stride, int padding, int poolA, int poolB, float *poolOut, int toFc, void *ws, size_t wsBytes)
+{
 	FITRE_NEED_INIT();
 	int rc = check_conv("fitre_hip_conv_bn_act_pool_forward", s);
 	if (rc) return rc;
@@ -911,7 +928,10 @@ int fitre_hip_conv_bn_act_pool_forward(const fitre_conv_shape *s, const float *x
 	FITRE_REQUIRE(!zhat || (mean && variance && runningMean && runningVariance), "fitre_hip_conv_bn_act_pool_forward: null statistics");
 	FITRE_REQUIRE(act_known(actFun), "fitre_hip_conv_bn_act_pool_forward: unknown activation code %d", actFun);
 	FITRE_REQUIRE(poolType == NO_POOL || poolOut, "fitre_hip_conv_bn_act_pool_forward: null pooled output");
-	const bool split = split_pos_chosen(s, false, ws, wsBytes), c3 = split || c3_pos_eligible(s, false);
+	FITRE_REQUIRE((((uintptr_t)prepared) & 15) == 0, "fitre_hip_conv_bn_act_pool_forward: misaligned weight copy");
+	const bool quad = quad_forward_eligible(s);
+	const void *splitWeights = quad ? nullptr : prepared; // (a layer in the dense form that its workspace does not hold makes its own)
+	const bool split = split_pos_chosen(s, false, ws, wsBytes, 1, splitWeights != nullptr), c3 = split || c3_pos_eligible(s, false);
 	ThinFwdPlan thin;
 	const bool unaligned = (((uintptr_t)y | (uintptr_t)actOut) & 15) != 0; // the engine's steps behind it are launches of their own
 	if (!zhat && !c3 && (poolType == MAX_POOL || poolType == AVG_POOL) && ksize == 2 && stride == 2 && padding == 0 && s->outA % 2 == 0 &&
@@ -930,12 +950,12 @@ int fitre_hip_conv_bn_act_pool_forward(const fitre_conv_shape *s, const float *x
 	// fitre_hip_conv_bn_act_pool_workspace lays it out
 	const size_t sums = zhat ? fitre_hip_batch_norm_workspace(s->outChannels, perChannel) : 0;
 	const size_t convBytes = ws && wsBytes > sums ? (wsBytes - sums) & ~(size_t)255 : 0;
-	if (quad_forward_eligible(s) && ((at | (uintptr_t)x | (uintptr_t)w) & 15) == 0 && s->outChannels <= 65535 &&
+	if (quad && ((at | (uintptr_t)x | (uintptr_t)w) & 15) == 0 && s->outChannels <= 65535 &&
 	    quad_forward_fits(s, convBytes) > 0) {
 		// 2 x 2 maps as a dense product; its partials and, behind them, the batch-norm sums are read by the pass that follows
 		int splits = 1;
 		float *partials = nullptr;
-		rc = quad_forward(s, x, w, ws, convBytes, &splits, &partials);
+		rc = quad_forward(s, x, w, prepared, ws, convBytes, &splits, &partials);
 		if (rc) return rc;
 		const SplitSource src{ partials, splits, (long)s->outChannels * perChannel, bias, y, (double *)((char *)ws + convBytes) };
 		return bn_act_pool_forward_split(toFc != 0, src, s->outChannels, s->samples, s->outA, s->outB, zhat, mean, variance, runningMean,
@@ -944,9 +964,10 @@ int fitre_hip_conv_bn_act_pool_forward(const fitre_conv_shape *s, const float *x
 	}
 	// where the room of the sums would cost the product one of its ranges they are a pass of their own: the same ranges and
 	// the same bits as fitre_hip_conv_forward with this workspace
-	if (c3 && (at & 15) == 0 && perChannel % 4 == 0 && s->outChannels <= 65535 && pos_forward_fits_in(s, ws, convBytes, wsBytes)) {
+	if (c3 && (at & 15) == 0 && perChannel % 4 == 0 && s->outChannels <= 65535 &&
+	    pos_forward_fits_in(s, ws, convBytes, wsBytes, splitWeights != nullptr)) {
 		int splits = 1;
-		rc = split ? launch_split_pos(s, false, x, w, bias, y, ws, convBytes, nullptr, &splits)
+		rc = split ? launch_split_pos(s, false, x, w, bias, y, ws, convBytes, splitWeights, &splits)
 		           : launch_c3_pos<false>(s, x, w, bias, y, ws, convBytes, &splits);
 		if (rc) return rc;
 		if (splits > 1) {
@@ -1244,6 +1265,61 @@ int fitre_hip_conv_input_grad_prepare(const fitre_conv_shape *s, const float *w,
 	return quad_eligible(s) ? quad_prepare_weights(s, w, (float *)prepared) : launch_split_weights(s, true, w, nullptr, (u32x4 *)prepared);
 }
 
+size_t fitre_hip_conv_forward_prepared_bytes(const fitre_conv_shape *s)
+{
+	if (!s) return 0;
+	if (quad_forward_eligible(s)) return quad_weff_bytes(s);
+	return split_pos_eligible(s, false) && split_pos_worthwhile(s, false, 1) ? split_weights_bytes(s, false) : 0;
+}
+
+int fitre_hip_conv_prepare_weights(int count, const fitre_conv_shape *s, const float *const *w, void *const *prepared, int inputGrad)
+{
+	FITRE_NEED_INIT();
+	FITRE_REQUIRE(count >= 0 && (count == 0 || (s && w && prepared)), "fitre_hip_conv_prepare_weights: null pointer");
+	SplitWeightsBatch split[2] = {}; // windows of 3, of 5
+	QuadBatch quad = {};
+	double splitBytes = 0.0, quadBytes = 0.0;
+	int widest = 0;
+	auto flush = [&](int which) { // 0, 1: split weights, 2: dense forms
+		if (which < 2 && split[which].count) {
+			LaunchScope scope(FITRE_KC_PERMUTE, splitBytes);
+			if (inputGrad) launch_split_weights_batch<true>(which ? 5 : 3, split[which]);
+			else launch_split_weights_batch<false>(which ? 5 : 3, split[which]);
+			split[which].count = 0, splitBytes = 0.0;
+		} else if (which == 2 && quad.count) {
+			LaunchScope scope(FITRE_KC_PERMUTE, quadBytes);
+			quad_weff_batch_kernel<<<dim3((unsigned)((widest + 255) / 256), (unsigned)quad.first[quad.count]), 256, 0, stream()>>>(quad);
+			quad.count = 0, quadBytes = 0.0, widest = 0;
+		}
+	};
+	for (int i = 0; i < count; i++) {
+		const int rc = check_conv("fitre_hip_conv_prepare_weights", &s[i]);
+		if (rc) return rc;
+		FITRE_REQUIRE(w[i] && prepared[i] && (((uintptr_t)prepared[i]) & 15) == 0, "fitre_hip_conv_prepare_weights: null or misaligned pointer");
+		const size_t bytes = inputGrad ? fitre_hip_conv_input_grad_prepared_bytes(&s[i]) : fitre_hip_conv_forward_prepared_bytes(&s[i]);
+		if (!bytes) return fail(FITRE_E_UNSUPPORTED, "fitre_hip_conv_prepare_weights: nothing to prepare for layer %d", i);
+		if (inputGrad ? quad_eligible(&s[i]) : quad_forward_eligible(&s[i])) {
+			if (quad.count == kQuadBatch || (quad.count && quad.first[quad.count] + s[i].outChannels > 65535)) flush(2);
+			FITRE_REQUIRE(s[i].outChannels <= 65535, "fitre_hip_conv_prepare_weights: %d output channels", s[i].outChannels);
+			const int m = quad.count++;
+			quad.first[m + 1] = quad.first[m] + s[i].outChannels;
+			quad.cin[m] = s[i].inChannels, quad.w[m] = w[i], quad.weff[m] = (float *)prepared[i];
+			if (s[i].inChannels > widest) widest = s[i].inChannels;
+			quadBytes += 4.0 * 25.0 * (double)s[i].inChannels * s[i].outChannels;
+		} else {
+			const int which = s[i].ksize == 3 ? 0 : 1;
+			SplitWeightsBatch &b = split[which];
+			if (b.count == kSplitWeightsBatch) flush(which);
+			const int m = b.count++, I = inputGrad ? s[i].inChannels : s[i].outChannels, cred = inputGrad ? s[i].outChannels : s[i].inChannels;
+			b.I[m] = I, b.cred[m] = cred, b.rowGroups[m] = split_row_groups(I), b.w[m] = w[i], b.wp[m] = (u32x4 *)prepared[i];
+			b.first[m + 1] = b.first[m] + b.rowGroups[m] * (cred / kSplitCB);
+			splitBytes += (double)bytes * 10.0 / 6.0;
+		}
+	}
+	for (int which = 0; which < 3; which++) flush(which);
+	return check_launch("split_weights_batch_kernel");
+}
+
 int fitre_hip_conv_input_grad_split_prepared(const fitre_conv_shape *s, const float *delta, const float *w, const void *prepared,
                                              float *dx, void *ws, size_t wsBytes, fitre_split_view *view)
 {
@@ -1422,7 +1498,7 @@ int fitre_hip_thin_net_forward(int convs, const fitre_thin_net_layer *c, int lin
                                const float *target, int classes, float *probs, float *errors, float *lossHost)
 {
 	FITRE_NEED_INIT();
-	FITRE_REQUIRE(c && x && target && probs && lossHost && (linears == 0 || l), "fitre_hip_thin_net_forward: null pointer");
+	FITRE_REQUIRE(c && x && target && probs && (linears == 0 || l), "fitre_hip_thin_net_forward: null pointer");
 	NetParams p{};
 	int words;
 	FITRE_REQUIRE(net_plan(convs, c, linears, l, n, classes, p, words), "fitre_hip_thin_net_forward: this network does not fit one launch");

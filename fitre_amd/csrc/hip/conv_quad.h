@@ -118,9 +118,8 @@ __host__ __device__ inline int quad_tap(int ab, int apbp)
 }
 
 // Weff[(co, ab)][(ci, a'b')] from W[co][ci][3][3]: one thread per (co, ci), lanes along ci
-__global__ void __launch_bounds__(256) quad_weff_build_kernel(const float *w, int cin, int cout, float *weff)
+__device__ __forceinline__ void quad_weff_build(const float *w, int cin, int ci, int co, float *weff)
 {
-	const int ci = blockIdx.x * blockDim.x + threadIdx.x, co = blockIdx.y;
 	if (ci >= cin) return;
 	float t[9];
 	const float *src = w + ((size_t)co * cin + ci) * 9;
@@ -131,6 +130,25 @@ __global__ void __launch_bounds__(256) quad_weff_build_kernel(const float *w, in
 		float4 v = make_float4(t[quad_tap(ab, 0)], t[quad_tap(ab, 1)], t[quad_tap(ab, 2)], t[quad_tap(ab, 3)]);
 		*reinterpret_cast<float4 *>(weff + ((size_t)(co * 4 + ab) * cin + ci) * 4) = v;
 	}
+}
+__global__ void __launch_bounds__(256) quad_weff_build_kernel(const float *w, int cin, int cout, float *weff)
+{
+	quad_weff_build(w, cin, blockIdx.x * blockDim.x + threadIdx.x, blockIdx.y, weff);
+}
+// several layers' (blockIdx.y: output channels of one after the other)
+constexpr int kQuadBatch = 8;
+struct QuadBatch {
+	int count;
+	int first[kQuadBatch + 1]; // output channels of the layers before
+	int cin[kQuadBatch];
+	const float *w[kQuadBatch];
+	float *weff[kQuadBatch];
+};
+__global__ void __launch_bounds__(256) quad_weff_batch_kernel(const QuadBatch b)
+{
+	int m = 0;
+	while (m + 1 < b.count && (int)blockIdx.y >= b.first[m + 1]) m++;
+	quad_weff_build(b.w[m], b.cin[m], blockIdx.x * blockDim.x + threadIdx.x, (int)blockIdx.y - b.first[m], b.weff[m]);
 }
 
 // dW[co][ci][3][3] from dWeff[(co, ab)][(ci, a'b')]: the entries of one tap are added in the order of ab
@@ -326,14 +344,18 @@ static inline int quad_forward_fits(const fitre_conv_shape *s, size_t wsBytes)
 	const long fit = wsBytes > weffBytes ? (long)((wsBytes - weffBytes) / one) : 0;
 	return (int)(fit >= ideal ? ideal : (2 * fit >= ideal ? fit : 0));
 }
-static int quad_forward(const fitre_conv_shape *s, const float *x, const float *w, void *ws, size_t wsBytes, int *splits, float **partials)
+// prepared: the dense form made beforehand (null: in ws)
+static int quad_forward(const fitre_conv_shape *s, const float *x, const float *w, const void *prepared, void *ws, size_t wsBytes, int *splits, float **partials)
 {
 	const int I = 4 * s->outChannels, J = s->samples, R = 4 * s->inChannels;
 	const size_t weffBytes = quad_weff_bytes(s);
-	int rc = quad_prepare_weights(s, w, (float *)ws);
-	if (rc) return rc;
+	if (!prepared) {
+		const int rc = quad_prepare_weights(s, w, (float *)ws);
+		if (rc) return rc;
+		prepared = ws;
+	}
 	*partials = (float *)((char *)ws + weffBytes);
-	PlainParams pa{ (const float *)ws, (uint32_t)weffBytes, R, I };
+	PlainParams pa{ (const float *)prepared, (uint32_t)weffBytes, R, I };
 	QuadParams pb{ x, (uint32_t)((size_t)s->inChannels * J * 4 * sizeof(float)), 4 * J, J };
 	OutParams out{ *partials, (long)J, 0, nullptr, nullptr, 1.f, 0.f };
 	out.quadLd = 4L * J;

@@ -35,14 +35,12 @@ struct ConvSplitParams {
 // [channel block][tap][32 rows][part][half of the channels][row][8 channels] of bf16; rows past I are zero.  A workgroup makes one (channel block, 32 rows): its floats go through LDS, read in memory order.
 // DX: rows are the layer's input channels, the reduction runs over its output channels, windows are flipped.
 template <int KS, bool DX>
-__global__ void __launch_bounds__(256)
-split_weights_kernel(const float *w, const float *w2, int I, int cred, int rowGroups, u32x4 *wp)
+__device__ __forceinline__ void split_weights_block(const float *w, int I, int cred, int rowGroups, u32x4 *wp, int rb, int cb)
 {
 	constexpr int T = KS * KS, LD = DX ? 32 * T + 1 : kSplitCB * T + 1, ROWS = DX ? kSplitCB : 32;
 	constexpr int SPAN = DX ? 32 * T : kSplitCB * T; // floats in a row, consecutive in memory
 	__shared__ float L[ROWS * LD];
-	const int rb = blockIdx.x, cb = blockIdx.y, i0 = rb * 32, c0 = cb * kSplitCB;
-	if (blockIdx.z) w = w2, wp += (size_t)gridDim.y * T * rowGroups * 192; // a pair's second weights, behind the first
+	const int i0 = rb * 32, c0 = cb * kSplitCB;
 	const int rowLen = (DX ? I : cred) * T, col0 = (DX ? i0 : c0) * T, row0 = DX ? c0 : i0;
 	const int live = (I - i0 < 32 ? I - i0 : 32) * T; // DX: floats of a row inside the tensor
 	constexpr int N = ROWS * SPAN / 256;
@@ -72,6 +70,33 @@ split_weights_kernel(const float *w, const float *w2, int I, int cred, int rowGr
 #pragma unroll
 		for (int s = 0; s < 3; s++) dst[s * 64] = part[s];
 	}
+}
+
+// one layer's; blockIdx.z: a pair's second weights, whose parts follow the first's
+template <int KS, bool DX>
+__global__ void __launch_bounds__(256)
+split_weights_kernel(const float *w, const float *w2, int I, int cred, int rowGroups, u32x4 *wp)
+{
+	if (blockIdx.z) w = w2, wp += (size_t)gridDim.y * KS * KS * rowGroups * 192;
+	split_weights_block<KS, DX>(w, I, cred, rowGroups, wp, blockIdx.x, blockIdx.y);
+}
+
+// several layers': a pass has the copies of all of them made at once, beside its first steps
+constexpr int kSplitWeightsBatch = 16;
+struct SplitWeightsBatch {
+	int count;
+	int first[kSplitWeightsBatch + 1]; // blocks of the layers before
+	int I[kSplitWeightsBatch], cred[kSplitWeightsBatch], rowGroups[kSplitWeightsBatch];
+	const float *w[kSplitWeightsBatch];
+	u32x4 *wp[kSplitWeightsBatch];
+};
+template <int KS, bool DX>
+__global__ void __launch_bounds__(256) split_weights_batch_kernel(const SplitWeightsBatch b)
+{
+	int m = 0;
+	while (m + 1 < b.count && (int)blockIdx.x >= b.first[m + 1]) m++;
+	const int block = (int)blockIdx.x - b.first[m], groups = b.rowGroups[m], cb = block / groups;
+	split_weights_block<KS, DX>(b.w[m], b.I[m], b.cred[m], groups, b.wp[m], block - cb * groups, cb);
 }
 
 // ---- the product --------------------------------------------------------------------------------------------------

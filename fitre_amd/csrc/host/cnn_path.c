@@ -9,6 +9,7 @@
  * working buffers of the backward pass.
  */
 #include <stdio.h>
+#include <stdint.h>
 #include <stdlib.h>
 #include "fitre_cnn.h"
 #include "fitre_hip.h"
@@ -171,9 +172,49 @@ int fitreBackwardUnsupportedLayer(const CNN_MODEL *model)
 	return 0;
 }
 
+/* weight copies of the forward convolutions, one buffer per layer that has one, behind the workspace */
+static size_t forward_prepared_bytes(const CNN_MODEL *model, int batch)
+{
+	size_t need = 0;
+	for (int i = 1; i < model->cLayers; i++) {
+		fitre_conv_shape s = conv_shape(&model->convLayer[i], batch);
+		need += (fitre_hip_conv_forward_prepared_bytes(&s) + 255) & ~(size_t)255;
+	}
+	return need;
+}
+
 long cnnForwardMemRequired(CNN_MODEL *model)
 {
-	return (long)((forward_ws_bytes(model, model->batchSize) + sizeof(real) - 1) / sizeof(real));
+	const size_t need = ((forward_ws_bytes(model, model->batchSize) + 255) & ~(size_t)255) + forward_prepared_bytes(model, model->batchSize);
+	return (long)((need + sizeof(real) - 1) / sizeof(real));
+}
+
+/* Queues the copies of every layer that has one on the selected lane, two launches whatever the number of layers (one by one they were
+ * 5 to 8 us each, and their launches held up the pass behind them: VGG-11 at 256 images 1688 -> 1633 us, VGG-16 at 128 1999 -> 1899
+ * with both passes' copies made so), and returns how many there are.  make == 0: they are there, and only found again.  The buffers are
+ * laid out for the model's batch size; a layer of a shorter one that finds no room makes its own.  (The forward pass's on
+ * lane 2, beside its first layer: no shorter, as both are bound by memory there, and AlexNet at 64 images 1 % longer.) */
+static int prepare_weights(const CNN_MODEL *model, const real *weights, int n, int inputGrad, char *at, const char *end, const void **prepared, int make)
+{
+	fitre_conv_shape shapes[MAX_LAYERS];
+	const real *w[MAX_LAYERS];
+	void *to[MAX_LAYERS];
+	int count = 0;
+	at += -(uintptr_t)at & 15;
+	if (at > end) at = (char *)end;
+	for (int c = 1; c < model->cLayers; c++) {
+		fitre_conv_shape shape = conv_shape(&model->convLayer[c], n);
+		const size_t bytes = inputGrad ? fitre_hip_conv_input_grad_prepared_bytes(&shape) : fitre_hip_conv_forward_prepared_bytes(&shape);
+		prepared[c] = NULL;
+		if (bytes == 0 || bytes > (size_t)(end - at) || (inputGrad && !has_bn(&model->convLayer[c - 1]))) continue;
+		shapes[count] = shape, w[count] = weights + model->wOffsets[c], to[count] = at;
+		prepared[c] = at;
+		count++;
+		at += (bytes + 255) & ~(size_t)255;
+		if (at > end) at = (char *)end;
+	}
+	if (count && make) HIP_CALL(fitre_hip_conv_prepare_weights(count, shapes, w, to, inputGrad));
+	return count;
 }
 
 long cnnBackwardMemRequired(CNN_MODEL *model)
@@ -228,7 +269,7 @@ real cnnForward(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, r
 	const real *weights = data->weights;
 	const int nc = model->cLayers, n = curBatchSize;
 	void *ws = (void *)scratch->nextDevPtr;
-	const size_t wsBytes = sizeof(real) * (size_t)cnnForwardMemRequired(model);
+	const size_t wsBytes = (forward_ws_bytes(model, model->batchSize) + 255) & ~(size_t)255;
 
 	if (forTesting != MODEL_TRAIN && forTesting != MODEL_TRAIN_ACCURACY && forTesting != MODEL_TEST_ACCURACY) {
 		fprintf(stderr, "Unknown EVAL_TYPE... \n\n");
@@ -245,6 +286,8 @@ real cnnForward(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, r
 		HIP_CALL(fitre_hip_sync());
 		return loss;
 	}
+	const void *prepared[MAX_LAYERS] = { NULL };
+	prepare_weights(model, weights, n, 0, (char *)ws + wsBytes, (char *)ws + sizeof(real) * (size_t)cnnForwardMemRequired(model), prepared, 1);
 	for (int l = 0; l < nc; l++) {
 		const CONV_LAYER *cv = &model->convLayer[l];
 		const POOL_LAYER *pl = &model->poolLayer[l];
@@ -257,8 +300,8 @@ real cnnForward(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, r
 		real *bnOut = has_bn(cv) ? slab + cv->batchNormOffset : NULL;
 		/* convolution, batch norm (where the layer has it), activation and pooling in as few passes as the shapes allow; the
 		 * last layer's output leaves in the linear layers' order: [C][N][a*B+b] -> [N][C][b*A+a] */
-		HIP_CALL(fitre_hip_conv_bn_act_pool_forward(
-		    &shape, in, weights + wOffsets[l], bias, slab, bnOut, bnOut ? bnOut + cv->meansOffset : NULL,
+		HIP_CALL(fitre_hip_conv_bn_act_pool_forward_prepared(
+		    &shape, in, weights + wOffsets[l], prepared[l], bias, slab, bnOut, bnOut ? bnOut + cv->meansOffset : NULL,
 		    bnOut ? bnOut + cv->variancesOffset : NULL, bnOut ? bnOut + cv->runningMeansOffset : NULL,
 		    bnOut ? bnOut + cv->runningVariancesOffset : NULL, (real)BATCH_NORM_EPSILON, (real)BATCH_NORM_MOMENTUM,
 		    forTesting == MODEL_TRAIN, model->actFuns[l], actOut, pl->type, pl->pSize, pl->stride, pl->padding, pl->outWidth,
@@ -375,7 +418,7 @@ void cnnBackward(CNN_MODEL *model, DEVICE_DATASET *data, real *devPtr, real *z, 
 	const size_t bnBytes = backward_bn_ws_bytes(model, model->batchSize);
 	void *sideWs = (void *)((char *)bnWs + bnBytes);
 	const size_t sideBytes = backward_side_ws_bytes(model, model->batchSize);
-	char *preparedWs = (char *)sideWs + sideBytes;
+	char *const preparedWs = (char *)sideWs + sideBytes;
 	const char *preparedEnd = preparedWs + backward_prepared_bytes(model, model->batchSize);
 	const void *prepared[MAX_LAYERS] = { NULL };
 	int preparedPending = 0;
@@ -396,27 +439,11 @@ void cnnBackward(CNN_MODEL *model, DEVICE_DATASET *data, real *devPtr, real *z, 
 
 	/* Weight copies of the layers whose input gradient reads one: they depend on the weights only, so lane 2 makes
 	 * them while the chain works through the linear layers. */
-	{
-		int any = 0;
-		for (int c = 1; c < nc; c++) {
-			fitre_conv_shape shape = conv_shape(&model->convLayer[c], n);
-			/* the buffers are laid out for the model's batch size; a shorter one can take a copy where that takes none */
-			const size_t bytes = fitre_hip_conv_input_grad_prepared_bytes(&shape);
-			prepared[c] = NULL;
-			if (bytes == 0 || bytes > (size_t)(preparedEnd - preparedWs) || !has_bn(&model->convLayer[c - 1])) continue;
-			if (!any) {
-				/* behind whatever the caller has queued on lane 0 (a weight update, say): the copies read the weights */
-				LANE_WAIT(2, 0);
-				LANE_SELECT(2);
-			}
-			any = 1;
-			HIP_CALL(fitre_hip_conv_input_grad_prepare(&shape, weights + wOffsets[c], preparedWs, bytes));
-			prepared[c] = preparedWs;
-			preparedWs += (bytes + 255) & ~(size_t)255;
-			if (preparedWs > preparedEnd) preparedWs = (char *)preparedEnd;
-		}
-		if (any) LANE_SELECT(0);
-		preparedPending = any;
+	if (preparedWs < preparedEnd) {
+		LANE_WAIT(2, 0);
+		LANE_SELECT(2);
+		preparedPending = prepare_weights(model, weights, n, 1, preparedWs, preparedEnd, prepared, 1);
+		LANE_SELECT(0);
 	}
 
 	/* Linear layers, top down.  The delta of a layer (after its activation derivative) is written once, into the

@@ -358,6 +358,12 @@ int fitre_hip_conv_bn_act_pool_forward(const fitre_conv_shape *s, const float *x
                                        float epsilon, float momentum, int train, int actFun, float *actOut, int poolType,
                                        int ksize, int stride, int padding, int poolA, int poolB, float *poolOut, int toFc,
                                        void *ws, size_t wsBytes);
+/* with the weight copy of fitre_hip_conv_forward_prepared_bytes (prepared NULL: made inside, in ws) */
+int fitre_hip_conv_bn_act_pool_forward_prepared(const fitre_conv_shape *s, const float *x, const float *w, const void *prepared,
+                                                const float *bias, float *y, float *zhat, float *mean, float *variance, float *runningMean,
+                                                float *runningVariance, float epsilon, float momentum, int train, int actFun, float *actOut,
+                                                int poolType, int ksize, int stride, int padding, int poolA, int poolB, float *poolOut, int toFc,
+                                                void *ws, size_t wsBytes);
 /* dW[Cout][Cin*k*k] = sum over (n,a,b) of patch(x) * delta.  Replaces im2col + GEMM of
  * functions/cnn_backward.cu:771-783. */
 size_t fitre_hip_conv_weight_grad_workspace(const fitre_conv_shape *s);
@@ -440,6 +446,10 @@ int fitre_hip_conv_input_grad_split(const fitre_conv_shape *s, const float *delt
  * No counterpart in the reference, whose weights are reordered per call (dev_backprop_convolution.cu:140-156). */
 size_t fitre_hip_conv_input_grad_prepared_bytes(const fitre_conv_shape *s);
 int fitre_hip_conv_input_grad_prepare(const fitre_conv_shape *s, const float *w, void *prepared, size_t preparedBytes);
+/* The same for forward convolutions that are called with what follows them, and the copies of several layers at once (inputGrad != 0:
+ * the input gradients', else the forward convolutions'), in as few launches as there are kinds of copies. */
+size_t fitre_hip_conv_forward_prepared_bytes(const fitre_conv_shape *s);
+int fitre_hip_conv_prepare_weights(int count, const fitre_conv_shape *s, const float *const *w, void *const *prepared, int inputGrad);
 int fitre_hip_conv_input_grad_split_prepared(const fitre_conv_shape *s, const float *delta, const float *w,
                                              const void *prepared, float *dx, void *ws, size_t wsBytes,
                                              fitre_split_view *view);

@@ -1,0 +1,74 @@
+"""Weight copies made for several layers at once: the bits of the steps they replace."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from fitre_amd import lib as L
+from fitre_amd.structs import CNN_ACT_RELU, MAX_POOL, NO_POOL, fitre_conv_shape
+
+pytestmark = pytest.mark.gpu
+hip = L.hip
+
+
+def ok(rc):
+    assert rc == 0, hip.fitre_hip_last_error().decode()
+
+
+# samples, channels in and out, map, window: both windows, ragged groups of channels, the cell form, the dense form
+LAYERS = [(96, 64, 130, 13, 3), (64, 64, 192, 15, 5), (300, 256, 512, 4, 3), (130, 512, 64, 2, 3), (128, 96, 300, 8, 3), (132, 64, 68, 2, 3)]
+
+
+def layer(n, ci, co, a, k):
+    return fitre_conv_shape(n, ci, co, a, a, a, a, k, 1, k // 2)
+
+
+@pytest.mark.parametrize("grad", [0, 1])
+def test_copies_of_several_layers(dev, grad):
+    """One call for all of them leaves in every buffer what a call for the layer alone does."""
+    shapes = [layer(*g) for g in LAYERS]
+    query = hip.fitre_hip_conv_input_grad_prepared_bytes if grad else hip.fitre_hip_conv_forward_prepared_bytes
+    shapes = [s for s in shapes if query(C.byref(s))] * 5  # more than one launch holds
+    assert len(shapes) > 16
+    rng = np.random.default_rng(1)
+    w = [dev.upload(rng.standard_normal(s.inChannels * s.outChannels * s.ksize ** 2).astype(np.float32)) for s in shapes]
+    size = [query(C.byref(s)) for s in shapes]
+    one, all_ = ([dev.upload(np.full(b // 4 + 4, 7, np.float32)) for b in size] for _ in range(2))
+    for s, a, o in zip(shapes, w, one):
+        ok(hip.fitre_hip_conv_prepare_weights(1, C.byref(s), C.byref(C.c_void_p(a.value)), C.byref(C.c_void_p(o.value)), grad))
+        if grad:
+            ok(hip.fitre_hip_conv_input_grad_prepare(C.byref(s), a, o, query(C.byref(s))))
+    n = len(shapes)
+    ok(hip.fitre_hip_conv_prepare_weights(n, (fitre_conv_shape * n)(*shapes), (C.c_void_p * n)(*[a.value for a in w]),
+                                          (C.c_void_p * n)(*[a.value for a in all_]), grad))
+    for b, x, y in zip(size, one, all_):
+        got = dev.download(y, b // 4 + 4).view(np.uint32)
+        np.testing.assert_array_equal(got, dev.download(x, b // 4 + 4).view(np.uint32))
+        assert (got[-4:].view(np.float32) == 7).all()
+    bad = layer(1, 3, 3, 5, 3)
+    assert hip.fitre_hip_conv_prepare_weights(1, C.byref(bad), C.byref(C.c_void_p(w[0].value)), C.byref(C.c_void_p(one[0].value)), grad) != 0
+
+
+@pytest.mark.parametrize("geom", LAYERS)
+def test_forward_with_a_copy(dev, geom):
+    """The same bits with the copy made beforehand as with the one made inside."""
+    s = layer(*geom)
+    n, ci, co, a, k = geom
+    rng = np.random.default_rng(n)
+    x, w = dev.upload(rng.standard_normal(ci * n * a * a).astype(np.float32)), dev.upload(rng.standard_normal(co * ci * k * k).astype(np.float32))
+    bias, count, bytes_ = dev.upload(rng.standard_normal(co).astype(np.float32)), co * n * a * a, hip.fitre_hip_conv_forward_prepared_bytes(C.byref(s))
+    assert bytes_ > 0
+    copy = dev.alloc(bytes_)
+    ok(hip.fitre_hip_conv_prepare_weights(1, C.byref(s), C.byref(C.c_void_p(w.value)), C.byref(C.c_void_p(copy.value)), 0))
+    nb = hip.fitre_hip_conv_bn_act_pool_workspace(C.byref(s), 1)
+    ws = dev.alloc(nb)
+    pool = (MAX_POOL, 2, 2, 0, a // 2, a // 2) if a % 2 == 0 else (NO_POOL, 0, 0, 0, a, a)
+    results = []
+    for prepared in (None, copy):
+        bufs = [dev.zeros(count), dev.zeros(count), dev.zeros(co), dev.zeros(co), dev.zeros(co), dev.zeros(co), dev.zeros(count), dev.zeros(count)]
+        y, zhat, mean, var, rmean, rvar, act, top = bufs
+        ok(hip.fitre_hip_conv_bn_act_pool_forward_prepared(C.byref(s), x, w, prepared, bias, y, zhat, mean, var, rmean, rvar, 1e-5, 0.9, 1, CNN_ACT_RELU, act,
+                                                           *pool, top if pool[0] != NO_POOL else None, 0, ws, nb))
+        results.append([dev.download(b, m) for b, m in zip(bufs, (count, count, co, co, co, co, count, count))])
+    for u, v in zip(*results):
+        np.testing.assert_array_equal(u, v)
