@@ -1665,9 +1665,29 @@ __global__ void __launch_bounds__(256) mean_kernel(const float *x, int n, float 
 	if (threadIdx.x == 0) out[0] = (float)(t / (double)n); // may be host memory
 }
 
+// totals[0] += rows * mean: what a caller that adds up batches would do with the mean, without its wait
+__global__ void __launch_bounds__(256) mean_add_kernel(const float *x, int n, float *totals)
+{
+	__shared__ double lds[4];
+	double acc = 0.0;
+	for (int i = threadIdx.x; i < n; i += 256) acc += (double)x[i];
+	const double t = block_sum<256>(acc, lds);
+	if (threadIdx.x == 0) totals[0] = __fadd_rn(totals[0], __fmul_rn((float)(t / (double)n), (float)n));
+}
+// totals[1] += sum of squares (of hits, each zero or one), which is left in totals[2]
+__global__ void __launch_bounds__(256) hits_add_kernel(const float *x, int n, float *totals)
+{
+	__shared__ double lds[4];
+	double acc = 0.0;
+	for (int i = threadIdx.x; i < n; i += 256) acc += (double)x[i] * (double)x[i];
+	const double t = block_sum<256>(acc, lds);
+	if (threadIdx.x == 0) totals[2] = (float)t, totals[1] = __fadd_rn(totals[1], (float)t);
+}
+
 static float *g_nll = nullptr;
 static int g_nll_rows = 0;
-static float *g_loss_host = nullptr;
+static float *g_loss_host = nullptr; // pinned: a batch's loss, and from kTotals on the totals of a sweep
+constexpr int kTotals = 8;
 
 static int loss_room(int rows)
 {
@@ -1686,6 +1706,11 @@ static int loss_room(int rows)
 float *loss_terms(int rows) { return loss_room(rows) == FITRE_OK ? g_nll : nullptr; }
 int loss_mean(int rows, float *lossHost)
 {
+	if (!lossHost) {
+		LaunchScope scope(FITRE_KC_SOFTMAX, 4.0 * rows);
+		mean_add_kernel<<<1, 256, 0, stream()>>>(g_nll, rows, g_loss_host + kTotals);
+		return check_launch("mean_add_kernel");
+	}
 	{
 		LaunchScope scope(FITRE_KC_SOFTMAX, 4.0 * rows);
 		mean_kernel<<<1, 256, 0, stream()>>>(g_nll, rows, g_loss_host); // pinned memory the device writes: no copy behind it
@@ -2114,6 +2139,21 @@ int fitre::bn_act_pool_forward_split(bool toFc, const SplitSource &split, int ch
 	                           momentum, train, actFun, actOut, poolType, ksize, stride, padding, outA, outB, poolOut, ws, wsBytes);
 }
 
+static int softmax_cross_entropy(const float *logits, const float *target, int rows, int classes, float *probs, float *errors, float *lossHost)
+{
+	FITRE_REQUIRE(logits && target && probs, "fitre_hip_softmax_cross_entropy: null pointer");
+	FITRE_REQUIRE(rows > 0 && classes > 0, "fitre_hip_softmax_cross_entropy: non-positive shape (%d x %d)", rows, classes);
+	float *nll = loss_terms(rows);
+	if (!nll) return FITRE_E_DEVICE;
+	{
+		LaunchScope scope(FITRE_KC_SOFTMAX, 4.0 * rows * classes * 2);
+		softmax_ce_kernel<<<blocks_for(rows, 4), 256, 0, stream()>>>(logits, target, rows, classes, probs, errors, nll);
+		int rc = check_launch("softmax_ce_kernel");
+		if (rc) return rc;
+	}
+	return loss_mean(rows, lossHost);
+}
+
 extern "C" {
 
 int fitre_hip_bn_act_pool_forward(const float *in, int channels, int samples, int inA, int inB, float *zhat, float *mean,
@@ -2279,17 +2319,44 @@ int fitre_hip_softmax_cross_entropy(const float *logits, const float *target, in
                                     float *errors, float *lossHost)
 {
 	FITRE_NEED_INIT();
-	FITRE_REQUIRE(logits && target && probs && lossHost, "fitre_hip_softmax_cross_entropy: null pointer");
-	FITRE_REQUIRE(rows > 0 && classes > 0, "fitre_hip_softmax_cross_entropy: non-positive shape (%d x %d)", rows, classes);
-	float *nll = loss_terms(rows);
-	if (!nll) return FITRE_E_DEVICE;
-	{
-		LaunchScope scope(FITRE_KC_SOFTMAX, 4.0 * rows * classes * 2);
-		softmax_ce_kernel<<<blocks_for(rows, 4), 256, 0, stream()>>>(logits, target, rows, classes, probs, errors, nll);
-		int rc = check_launch("softmax_ce_kernel");
-		if (rc) return rc;
-	}
-	return loss_mean(rows, lossHost);
+	FITRE_REQUIRE(lossHost, "fitre_hip_softmax_cross_entropy: null pointer");
+	return softmax_cross_entropy(logits, target, rows, classes, probs, errors, lossHost);
+}
+
+int fitre_hip_softmax_cross_entropy_add(const float *logits, const float *target, int rows, int classes, float *probs, float *errors)
+{
+	FITRE_NEED_INIT();
+	return softmax_cross_entropy(logits, target, rows, classes, probs, errors, nullptr);
+}
+
+int fitre_hip_totals_begin(void)
+{
+	FITRE_NEED_INIT();
+	const int rc = loss_room(1);
+	if (rc) return rc;
+	FITRE_HIP_TRY(hipStreamSynchronize(stream())); // nothing adds to them any more
+	for (int i = 0; i < 3; i++) g_loss_host[kTotals + i] = 0.f;
+	return FITRE_OK;
+}
+
+int fitre_hip_totals_end(float *loss, float *hits, float *lastHits)
+{
+	FITRE_NEED_INIT();
+	FITRE_REQUIRE(loss && hits && g_loss_host, "fitre_hip_totals_end: null pointer or no fitre_hip_totals_begin before it");
+	FITRE_HIP_TRY(hipStreamSynchronize(stream()));
+	*loss = g_loss_host[kTotals], *hits = g_loss_host[kTotals + 1];
+	if (lastHits) *lastHits = g_loss_host[kTotals + 2];
+	return FITRE_OK;
+}
+
+int fitre_hip_accuracy_add(const float *probs, const float *target, int rows, int classes, float *hits)
+{
+	const int rc = fitre_hip_accuracy_hits(probs, target, rows, classes, hits);
+	if (rc) return rc;
+	FITRE_REQUIRE(g_loss_host, "fitre_hip_accuracy_add: no fitre_hip_totals_begin before it");
+	LaunchScope scope(FITRE_KC_BLAS1, 4.0 * rows);
+	hits_add_kernel<<<1, 256, 0, stream()>>>(hits, rows, g_loss_host + kTotals);
+	return check_launch("hits_add_kernel");
 }
 
 int fitre_hip_cross_entropy_rop_error(const float *rz, const float *probs, int rows, int classes, float *rError)

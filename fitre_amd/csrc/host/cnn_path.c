@@ -13,6 +13,7 @@
 #include <stdlib.h>
 #include "fitre_cnn.h"
 #include "fitre_hip.h"
+#include "sweep.h"
 
 #define HIP_CALL(expr)                                                                               \
 	do {                                                                                             \
@@ -261,10 +262,10 @@ static int forward_in_one_launch(const CNN_MODEL *model, const DEVICE_DATASET *d
 	return 1;
 }
 
-real cnnForward(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, real *z, real *probs, real *errors,
-                int s, int curBatchSize, EVAL_TYPE forTesting)
+/* loss NULL: added to the totals of a sweep, and nothing is waited for */
+static void forward_pass(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, real *z, real *probs, real *errors, int curBatchSize,
+                         EVAL_TYPE forTesting, int sameWeights, real *loss)
 {
-	(void)s;
 	const int *wOffsets = model->wOffsets, *bOffsets = model->bOffsets, *zOffsets = model->zOffsets;
 	const real *weights = data->weights;
 	const int nc = model->cLayers, n = curBatchSize;
@@ -281,13 +282,9 @@ real cnnForward(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, r
 		exit(-1);
 	}
 
-	real loss = 0;
-	if (forward_in_one_launch(model, data, z, probs, errors, n, &loss)) {
-		HIP_CALL(fitre_hip_sync());
-		return loss;
-	}
+	if (forward_in_one_launch(model, data, z, probs, errors, n, loss)) return;
 	const void *prepared[MAX_LAYERS] = { NULL };
-	prepare_weights(model, weights, n, 0, (char *)ws + wsBytes, (char *)ws + sizeof(real) * (size_t)cnnForwardMemRequired(model), prepared, 1);
+	prepare_weights(model, weights, n, 0, (char *)ws + wsBytes, (char *)ws + sizeof(real) * (size_t)cnnForwardMemRequired(model), prepared, !sameWeights);
 	for (int l = 0; l < nc; l++) {
 		const CONV_LAYER *cv = &model->convLayer[l];
 		const POOL_LAYER *pl = &model->poolLayer[l];
@@ -334,9 +331,24 @@ real cnnForward(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, r
 	}
 
 	const real *logits = (model->lLayers == 0) ? feat : z + zOffsets[model->lLayers + nc];
-	HIP_CALL(fitre_hip_softmax_cross_entropy(logits, data->sampledTrainY, n, data->numClasses, probs, errors, &loss));
+	if (loss) HIP_CALL(fitre_hip_softmax_cross_entropy(logits, data->sampledTrainY, n, data->numClasses, probs, errors, loss));
+	else HIP_CALL(fitre_hip_softmax_cross_entropy_add(logits, data->sampledTrainY, n, data->numClasses, probs, errors));
+}
+
+real cnnForward(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, real *z, real *probs, real *errors,
+                int s, int curBatchSize, EVAL_TYPE forTesting)
+{
+	(void)s;
+	real loss = 0;
+	forward_pass(model, data, scratch, z, probs, errors, curBatchSize, forTesting, 0, &loss);
 	HIP_CALL(fitre_hip_sync());
 	return loss;
+}
+
+void fitre_forward_batch(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratch, real *z, real *probs, real *errors, int n, EVAL_TYPE mode,
+                         int sameWeights)
+{
+	forward_pass(model, data, scratch, z, probs, errors, n, mode, sameWeights, NULL);
 }
 
 /* Multiply-adds of the convolution layers' two gradient products: what decides whether a pass is long enough for

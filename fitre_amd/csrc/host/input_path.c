@@ -6,6 +6,7 @@
 
 #include "fitre_cnn.h"
 #include "fitre_hip.h"
+#include "sweep.h"
 #include "fitre_input.h"
 #include "fitre_shim.h"
 
@@ -79,11 +80,8 @@ void normalizeCIFAR10(real *input, int samples, int channels, int height, int wi
 	HIP_CALL(fitre_hip_sync());
 }
 
-void augmentData(CNN_MODEL *model, DEVICE_DATASET *data, int offset, int currentBatchSize, real *devPtr, real *hostPtr,
-                 int enableDA, DATASET_TYPE datasetType)
+static void augment_queued(CNN_MODEL *model, DEVICE_DATASET *data, int currentBatchSize, real *devPtr, int enableDA, DATASET_TYPE datasetType)
 {
-	(void)offset;
-	(void)hostPtr;
 	const CONV_LAYER *c = &model->convLayer[0];
 	const int channels = c->inChannels, height = c->height, width = c->width, samples = currentBatchSize;
 	real *first = data->sampledTrainX;
@@ -103,8 +101,16 @@ void augmentData(CNN_MODEL *model, DEVICE_DATASET *data, int offset, int current
 	}
 	HIP_CALL(fitre_hip_augment_batch(first, 1, samples, channels, height, width, cropUniforms, 4, 0.f, flipUniforms, mean, std,
 	                                 255.f, second));
-	HIP_CALL(fitre_hip_sync());
 	data->currentBatch = second;
+}
+
+void augmentData(CNN_MODEL *model, DEVICE_DATASET *data, int offset, int currentBatchSize, real *devPtr, real *hostPtr,
+                 int enableDA, DATASET_TYPE datasetType)
+{
+	(void)offset;
+	(void)hostPtr;
+	augment_queued(model, data, currentBatchSize, devPtr, enableDA, datasetType);
+	HIP_CALL(fitre_hip_sync());
 }
 
 /* rows indices[offset + i] (indices == NULL: offset + i) of the host set, gathered in a staging buffer and sent
@@ -148,11 +154,14 @@ static void generalization_sweep(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH
                                  EVAL_TYPE mode, int dropShortTail, real *likelihood, real *accuracy)
 {
 	real hits = 0;
-	int curIdx = 0, curBatchSize = model->batchSize;
-	real *nextDevPtr = scratch->nextDevPtr, *nextHostPtr = scratch->nextHostPtr, *nextPageLckPtr = scratch->nextPageLckPtr;
+	int curIdx = 0, curBatchSize = model->batchSize, before = 0;
+	real *nextDevPtr = scratch->nextDevPtr, *nextPageLckPtr = scratch->nextPageLckPtr;
 	*likelihood = 0;
 	*accuracy = 0;
 	if (curBatchSize > setSize) curBatchSize = setSize;
+	/* queued batch behind batch: losses and hits add up on the device, the weights' copies are made once, and only the sums are waited
+	 * for (four batches of 256 images of VGG-11: 16 waits less) */
+	HIP_CALL(fitre_hip_totals_begin());
 	while (curIdx < setSize && curBatchSize > 0) {
 		if (hostSet != NULL) {
 			select_host_rows(hostSet, data->sampledTrainX, data->sampledTrainY, curBatchSize, NULL, curIdx, NULL);
@@ -161,12 +170,12 @@ static void generalization_sweep(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH
 			                            sizeof(real) * (size_t)data->features * curBatchSize));
 			HIP_CALL(fitre_hip_copy_d2d(data->sampledTrainY, setY + curIdx, sizeof(real) * (size_t)curBatchSize));
 		}
-		augmentData(model, data, curIdx, curBatchSize, nextDevPtr, nextHostPtr, 0, data->datasetType);
-		real batchLikelihood = cnnForward(model, data, scratch, z, probs, errors, curIdx, curBatchSize, mode);
-		*likelihood += batchLikelihood * curBatchSize;
-		computeAccuracy(probs, hostSet != NULL ? data->sampledTrainY : (real *)(setY + curIdx), curBatchSize, data->numClasses,
-		                nextDevPtr, nextPageLckPtr);
-		hits += *nextPageLckPtr;
+		augment_queued(model, data, curBatchSize, nextDevPtr, 0, data->datasetType);
+		fitre_forward_batch(model, data, scratch, z, probs, errors, curBatchSize, mode, before == curBatchSize);
+		before = curBatchSize;
+		/* the hits go where the forward pass had its partial sums */
+		HIP_CALL(fitre_hip_accuracy_add(probs, hostSet != NULL ? data->sampledTrainY : (real *)(setY + curIdx), curBatchSize, data->numClasses,
+		                                nextDevPtr));
 		curIdx += curBatchSize;
 		if (curIdx + model->batchSize < setSize) {
 			curBatchSize = model->batchSize;
@@ -175,6 +184,7 @@ static void generalization_sweep(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH
 			if (dropShortTail) break;
 		}
 	}
+	HIP_CALL(fitre_hip_totals_end(likelihood, &hits, nextPageLckPtr));
 	*accuracy = hits * (real)100. / (real)setSize;
 	*likelihood /= (real)setSize;
 }

@@ -303,6 +303,14 @@ int fitre_hip_row_sum(const float *mat, int rows, int cols, float *out);
  * written to host memory, complete on return.  errors may be NULL. */
 int fitre_hip_softmax_cross_entropy(const float *logits, const float *target, int rows, int classes,
                                     float *probs, float *errors, float *lossHost);
+/* A sweep over batches without a wait in between (functions/cnn_accuracy.cu:61-174 adds up on the host): _begin sets the totals to
+ * zero, _cross_entropy_add adds rows times the batch's loss, _accuracy_add the hits (written to `hits`, rows floats, too), in the
+ * order they are queued and in the arithmetic of a host that adds floats; _end waits and returns them, and the last batch's
+ * hits where asked for.  One sweep at a time. */
+int fitre_hip_totals_begin(void);
+int fitre_hip_softmax_cross_entropy_add(const float *logits, const float *target, int rows, int classes, float *probs, float *errors);
+int fitre_hip_accuracy_add(const float *probs, const float *target, int rows, int classes, float *hits);
+int fitre_hip_totals_end(float *loss, float *hits, float *lastHits);
 /* errors = (probs - onehot)/rows only (computeCrossEntropyError, :231-245) */
 int fitre_hip_cross_entropy_error(const float *probs, const float *target, int rows, int classes,
                                   float *errors);
@@ -537,8 +545,8 @@ int fitre_hip_fc_tail_forward(int layers, const fitre_fc_forward_layer *l, int n
 
 /* The forward pass of a whole small network in one launch (functions/cnn_forward.cu:49-383): one to three convolutions (windows of 3
  * or 5, stride 1, at most sixteen channels, even maps) with an activation and a 2 x 2 / stride 2 pool behind each, none to four
- * linear layers as in fitre_hip_fc_tail_forward, softmax, loss errors (may be NULL) and the mean loss, which is waited for.  The
- * tensors are those the steps of their own leave; the last pool's output is in the linear layers' order.  _fits: the network
+ * linear layers as in fitre_hip_fc_tail_forward, softmax, loss errors (may be NULL) and the mean loss, which is waited for (lossHost NULL:
+ * added to the totals below).  The tensors are those the steps of their own leave; the last pool's output is in the linear layers' order.  _fits: the network
  * is one of these, and this way is the shorter one. */
 typedef struct fitre_thin_net_layer {
 	fitre_conv_shape shape;

@@ -1,4 +1,4 @@
-"""Weight copies made for several layers at once: the bits of the steps they replace."""
+"""Weight copies made for several layers at once, and a sweep without waits: the bits of the steps they replace."""
 import ctypes as C
 
 import numpy as np
@@ -72,3 +72,27 @@ def test_forward_with_a_copy(dev, geom):
         results.append([dev.download(b, m) for b, m in zip(bufs, (count, count, co, co, co, co, count, count))])
     for u, v in zip(*results):
         np.testing.assert_array_equal(u, v)
+
+
+def test_totals_of_a_sweep(dev):
+    """Losses and hits added on the device are those a host adds up in floats, batch by batch."""
+    rng = np.random.default_rng(3)
+    loss, hits, last = (C.c_float() for _ in range(3))
+    want_loss, want_hits = np.float32(0), np.float32(0)
+    ok(hip.fitre_hip_totals_begin())
+    for rows, classes in ((256, 10), (1, 10), (77, 3), (1000, 65)):
+        logits, labels = dev.upload(rng.standard_normal((rows, classes)).astype(np.float32)), dev.upload(rng.integers(1, classes + 1, rows).astype(np.float32))
+        probs, errors, h, dot = dev.zeros(rows * classes), dev.zeros(rows * classes), dev.zeros(rows), C.c_float()
+        ok(hip.fitre_hip_softmax_cross_entropy_add(logits, labels, rows, classes, probs, errors))
+        ok(hip.fitre_hip_accuracy_add(probs, labels, rows, classes, h))
+        one = C.c_float()
+        ok(hip.fitre_hip_softmax_cross_entropy(logits, labels, rows, classes, probs, errors, C.byref(one)))
+        ok(hip.fitre_hip_accuracy_hits(probs, labels, rows, classes, h))
+        ok(hip.fitre_hip_dot(rows, h, h, C.byref(dot)))
+        want_loss = np.float32(want_loss + np.float32(np.float32(one.value) * np.float32(rows)))
+        want_hits = np.float32(want_hits + np.float32(dot.value))
+    ok(hip.fitre_hip_totals_end(C.byref(loss), C.byref(hits), C.byref(last)))
+    assert (loss.value, hits.value, last.value) == (want_loss, want_hits, dot.value)
+    ok(hip.fitre_hip_totals_begin())
+    ok(hip.fitre_hip_totals_end(C.byref(loss), C.byref(hits), None))
+    assert (loss.value, hits.value) == (0, 0)
