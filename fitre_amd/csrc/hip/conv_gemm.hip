@@ -1127,6 +1127,15 @@ int fitre_hip_thin_reduce_defer(int on)
 		if (rc) return rc;
 	}
 	g_thin_reduce_deferred = (on != 0);
+	if (!on) g_thin_dw_deferred = false;
+	return FITRE_OK;
+}
+
+int fitre_hip_weight_grads_defer(void)
+{
+	const int rc = fitre_hip_thin_reduce_defer(1);
+	if (rc) return rc;
+	g_thin_dw_deferred = true;
 	return FITRE_OK;
 }
 
@@ -1727,7 +1736,12 @@ static int fc_tail_run(int layers, const fitre_fc_tail_layer *l, int n, const fl
 			part += (size_t)nRanges * ((size_t)q.M * q.N + q.M);
 		}
 	}
-	{
+	if (g_thin_dw_deferred && !ranges) { // held back with the convolutions' weight gradients
+		const int rc = g_thin_dw.linear.count ? thin_reduce_flush() : FITRE_OK;
+		if (rc) return rc;
+		g_thin_dw.linear = b;
+		g_thin_dw_flops += chainFlops;
+	} else {
 		LaunchScope scope(FITRE_KC_FC_GEMM, chainFlops, 0);
 		small_gemm_batch_kernel<<<(unsigned)b.first[layers], 256, 0, stream()>>>(b);
 	}

@@ -37,16 +37,20 @@ struct SmallGemmParams {
 	float *partial;  // [range][N * M results, then M row sums] (no epilogue: small_gemm_reduce_kernel applies alpha and stores)
 };
 
-// one workgroup's block (bx, by) of the result over reduction range bz
-__device__ __forceinline__ void small_gemm_block(const SmallGemmParams &p, const int bx, const int by, const int bz)
+constexpr int kSmallLdsFloats = 2 * kSmallDepth * (kSmallTile + 1);
+// one workgroup's block (bx, by) of the result over reduction range bz; lds: kSmallLdsFloats.  ROWS: both operands run along the result
+// (sAm == 1, sBn == 1)
+template <bool ROWS>
+__device__ __forceinline__ void small_gemm_block(const SmallGemmParams &p, const int bx, const int by, const int bz, float *lds)
 {
-	__shared__ float As[kSmallDepth][kSmallTile + 1]; // [k][m]
-	__shared__ float Bs[kSmallDepth][kSmallTile + 1]; // [k][n]
+	float(*As)[kSmallTile + 1] = reinterpret_cast<float(*)[kSmallTile + 1]>(lds); // [k][m]
+	float(*Bs)[kSmallTile + 1] = As + kSmallDepth;                               // [k][n]
 	const int tid = threadIdx.x;
 	const int m0 = bx * kSmallTile, n0 = by * kSmallTile;
 	const int tm = tid & 15, tn = tid >> 4;
 	// loads run along whichever index is contiguous in memory; all of a block's loads are in flight together
-	const bool aAlongM = p.sAm == 1, bAlongN = p.sBn == 1;
+	const bool aAlongM = ROWS || p.sAm == 1, bAlongN = ROWS || p.sBn == 1;
+	const long sAm = ROWS ? 1 : p.sAm, sBn = ROWS ? 1 : p.sBn;
 	constexpr int kPer = kSmallDepth * kSmallTile / 256; // elements of each operand a thread loads per block
 	float acc00 = 0.f, acc01 = 0.f, acc10 = 0.f, acc11 = 0.f, rs0 = 0.f, rs1 = 0.f;
 	const bool sums = p.rowSums != nullptr && by == 0 && tn == 0;
@@ -60,9 +64,9 @@ __device__ __forceinline__ void small_gemm_block(const SmallGemmParams &p, const
 			const int am = aAlongM ? (e & 31) : e / kSmallDepth, ak = aAlongM ? (e >> 5) : e % kSmallDepth;
 			const int bn = bAlongN ? (e & 31) : e / kSmallDepth, bk = bAlongN ? (e >> 5) : e % kSmallDepth;
 			const bool aok = (m0 + am < p.M) & (k0 + ak < kEnd), bok = (n0 + bn < p.N) & (k0 + bk < kEnd);
-			av[i] = aok ? p.A[(long)(m0 + am) * p.sAm + (long)(k0 + ak) * p.sAk] : 0.f;
-			bv[i] = bok ? p.B[(long)(k0 + bk) * p.sBk + (long)(n0 + bn) * p.sBn] : 0.f;
-			if (p.copyB != nullptr && bx == 0 && bok) p.copyB[(long)(k0 + bk) * p.sBk + (long)(n0 + bn) * p.sBn] = bv[i];
+			av[i] = aok ? p.A[(long)(m0 + am) * sAm + (long)(k0 + ak) * p.sAk] : 0.f;
+			bv[i] = bok ? p.B[(long)(k0 + bk) * p.sBk + (long)(n0 + bn) * sBn] : 0.f;
+			if (p.copyB != nullptr && bx == 0 && bok) p.copyB[(long)(k0 + bk) * p.sBk + (long)(n0 + bn) * sBn] = bv[i];
 		}
 		__syncthreads(); // the previous block's readers are done
 #pragma unroll
@@ -129,10 +133,11 @@ __device__ __forceinline__ void small_gemm_block(const SmallGemmParams &p, const
 
 __global__ void __launch_bounds__(256) small_gemm_kernel(const SmallGemmParams p)
 {
-	small_gemm_block(p, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z);
+	__shared__ float lds[kSmallLdsFloats];
+	small_gemm_block<false>(p, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, lds);
 }
 
-// several independent products as one launch: the blocks of product j are blockIdx.x in [first[j], first[j + 1])
+// several independent products of operands that run along the result as one launch: the blocks of product j are blockIdx.x in [first[j], first[j + 1])
 constexpr int kSmallBatch = 4;
 struct SmallGemmBatch {
 	int count;
@@ -140,14 +145,18 @@ struct SmallGemmBatch {
 	int gridX[kSmallBatch], gridY[kSmallBatch];
 	SmallGemmParams p[kSmallBatch];
 };
-__global__ void __launch_bounds__(256) small_gemm_batch_kernel(const SmallGemmBatch b)
+__device__ __forceinline__ void small_gemm_batch_block(const SmallGemmBatch &b, const int block, float *lds)
 {
-	const int block = (int)blockIdx.x;
 	int j = 0;
 	while (j + 1 < b.count && block >= b.first[j + 1]) j++;
 	const int local = block - b.first[j];
 	const int bx = local % b.gridX[j], rest = local / b.gridX[j];
-	small_gemm_block(b.p[j], bx, rest % b.gridY[j], rest / b.gridY[j]);
+	small_gemm_block<true>(b.p[j], bx, rest % b.gridY[j], rest / b.gridY[j], lds);
+}
+__global__ void __launch_bounds__(256) small_gemm_batch_kernel(const SmallGemmBatch b)
+{
+	__shared__ float lds[kSmallLdsFloats];
+	small_gemm_batch_block(b, (int)blockIdx.x, lds);
 }
 
 // the second launch of a batch whose reductions were cut into ranges: every product's sums in range order, in double

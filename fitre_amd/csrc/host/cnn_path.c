@@ -470,6 +470,8 @@ void cnnBackward(CNN_MODEL *model, DEVICE_DATASET *data, real *devPtr, real *z, 
 	feature_extent(model, &extA, &extB);
 	fitre_fc_tail_layer tail[4];
 	const int fusedTail = tail_shapes(model, n, tail);
+	/* a pass on one lane: the weight gradients of small layers, the linear ones' too, wait for one launch at its end */
+	if (!lanes) HIP_CALL(fitre_hip_weight_grads_defer());
 	int tailFoldedPool = 0;
 	if (fusedTail) {
 		/* small layers (LeNet's 400-120-84-10): the whole tail in two launches on the chain's lane -- every delta into its

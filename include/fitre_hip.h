@@ -397,6 +397,10 @@ int fitre_hip_conv_weight_grad(const fitre_conv_shape *s, const float *x, const 
 size_t fitre_hip_thin_reduce_bytes(const fitre_conv_shape *s);
 int fitre_hip_thin_reduce_defer(int on);
 int fitre_hip_thin_reduce_flush(void);
+/* fitre_hip_thin_reduce_defer(1), and the products in front of those launches are held back with them, as are the weight gradients of
+ * fitre_hip_fc_tail_backward (where they need no second launch): all in one launch in front of the reductions' one.  The inputs and
+ * deltas of such calls must stay untouched until then, too. */
+int fitre_hip_weight_grads_defer(void);
 size_t fitre_hip_conv_weight_bias_grad_workspace(const fitre_conv_shape *s);
 int fitre_hip_conv_weight_bias_grad(const fitre_conv_shape *s, const float *x, const float *delta, float *dW,
                                     float *db, void *ws, size_t wsBytes);

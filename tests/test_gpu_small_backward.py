@@ -1,4 +1,4 @@
-"""Backward pass of small layers: input gradients whose waves share output channels."""
+"""Backward pass of small layers: input gradients whose waves share output channels, weight gradients made together."""
 import ctypes as C
 
 import numpy as np
@@ -7,7 +7,7 @@ import torch
 import torch.nn.functional as F
 
 from fitre_amd import lib as L
-from fitre_amd.structs import fitre_conv_shape
+from fitre_amd.structs import CNN_ACT_NONE, fitre_conv_shape, fitre_fc_tail_layer
 
 pytestmark = pytest.mark.gpu
 hip = L.hip
@@ -34,3 +34,44 @@ def test_input_gradient(dev, n, ci, co, a, k, pad):
     assert (got[-4:] == 7).all()
     # one rounding per term and sum: error at most (terms + 3) u times the terms' sizes
     assert (abs(got[:-4] - want) <= (co * k * k + 3) * 2.0**-24 * 1.01 * size).all()
+
+
+@pytest.mark.parametrize("n", [1, 13, 512, 700])
+def test_weight_gradients_together(dev, n):
+    """Held back with the linear layers' above and made in one launch (a fifth layer makes the first four's): the bits of the calls alone,
+    and nothing written before."""
+    rng = np.random.default_rng(n)
+    up = lambda size: dev.upload(rng.standard_normal(size).astype(np.float32))
+    full = lambda size: dev.upload(np.full(size, 7, np.float32))
+    shapes = [fitre_conv_shape(n, ci, co, a, b, a + 2 * p - k + 1, b + 2 * p - k + 1, k, 1, p)
+              for ci, co, a, b, k, p in [(3, 6, 32, 32, 5, 0), (6, 16, 14, 14, 5, 0), (2, 1, 7, 12, 3, 1), (1, 8, 9, 9, 5, 2), (4, 9, 10, 11, 3, 0)]]
+    convs = [(s, up(s.inChannels * n * s.inA * s.inB), up(s.outChannels * n * s.outA * s.outB)) for s in shapes]
+    dims = [(65, 33), (33, 31), (31, 2)]
+    W, zin, top = [up(i * o) for i, o in dims], [up(n * i) for i, _ in dims], up(2 * n)
+
+    def run(held):
+        bufs, outs = [], []
+        tail = (fitre_fc_tail_layer * 3)()
+        for t, (i, o) in enumerate(dims):
+            slot, dW, db = full(n * o), full(i * o), full(o)
+            tail[t] = fitre_fc_tail_layer(i, o, CNN_ACT_NONE, W[t].value, None, None, zin[t].value, slot.value, dW.value, db.value)
+            outs += [(dW, i * o), (db, o)]
+            bufs.append(slot)
+        if held:
+            ok(hip.fitre_hip_weight_grads_defer())
+        nb = hip.fitre_hip_fc_tail_workspace(3, tail, n)
+        ok(hip.fitre_hip_fc_tail_backward(3, tail, n, top, 0, 0, full(n * 65), dev.alloc(max(nb, 4)), nb))
+        for s, x, d in convs:
+            assert hip.fitre_hip_thin_reduce_bytes(C.byref(s)) > 0
+            nb = max(hip.fitre_hip_conv_weight_bias_grad_workspace(C.byref(s)), hip.fitre_hip_thin_reduce_bytes(C.byref(s)))
+            size = s.outChannels * s.inChannels * s.ksize**2
+            dW, db = full(size), full(s.outChannels)
+            ok(hip.fitre_hip_conv_weight_bias_grad(C.byref(s), x, d, dW, db, dev.alloc(nb), nb))
+            outs += [(dW, size), (db, s.outChannels)]
+        if held:
+            assert all((dev.download(*o) == 7).all() for o in outs[-2:])
+            ok(hip.fitre_hip_thin_reduce_defer(0))
+        return [dev.download(*o).view(np.uint32) for o in outs]
+
+    for alone, together in zip(run(False), run(True)):
+        np.testing.assert_array_equal(together, alone)
