@@ -104,9 +104,9 @@ int layers_device_setup(int device);
 // Shutdown hooks of the files that keep device buffers between calls (loss scratch, reduction partials, patch
 // decode tables): free them and forget their sizes, so that a later fitre_hip_init -- possibly on another device --
 // starts clean.  Called by fitre_hip_shutdown after every lane has drained.
-// Loss terms of a batch on the device (room for `rows`; null: no memory), and their mean, which is waited for (lossHost null: added to
+// Where a batch's loss terms go (room for `rows`; null: no memory), and their mean, which is waited for (lossHost null: added to
 // the totals of a sweep instead, times the rows).
-float *loss_terms(int rows);
+float *loss_terms(int rows, const float *lossHost);
 int loss_mean(int rows, float *lossHost);
 void layers_release();
 void elementwise_release();

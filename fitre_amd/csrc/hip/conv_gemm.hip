@@ -1528,7 +1528,7 @@ int fitre_hip_thin_net_forward(int convs, const fitre_thin_net_layer *c, int lin
 		work += 2.0 * l[f].in * l[f].out * n;
 	}
 	p.x = x, p.target = target, p.probs = probs, p.errors = errors;
-	p.nll = loss_terms(n);
+	p.nll = loss_terms(n, lossHost);
 	if (!p.nll) return FITRE_E_DEVICE;
 	{
 		LaunchScope scope(FITRE_KC_CONV_FWD, work, 0);

@@ -96,3 +96,17 @@ def test_totals_of_a_sweep(dev):
     ok(hip.fitre_hip_totals_begin())
     ok(hip.fitre_hip_totals_end(C.byref(loss), C.byref(hits), None))
     assert (loss.value, hits.value) == (0, 0)
+
+
+@pytest.mark.parametrize("rows", [1, 77, 1024, 1025, 5000])
+def test_mean_loss(dev, rows):
+    """Up to 1024 rows the host takes the mean of the terms, above a kernel does; labels out of range add nothing."""
+    rng = np.random.default_rng(rows)
+    logits, labels = rng.standard_normal((rows, 10)).astype(np.float32), rng.integers(0, 13, rows)
+    labels[-1] = 10
+    loss, probs = C.c_float(), dev.zeros(rows * 10)
+    ok(hip.fitre_hip_softmax_cross_entropy(dev.upload(logits), dev.upload(labels.astype(np.float32)), rows, 10, probs, dev.zeros(rows * 10), C.byref(loss)))
+    p = dev.download(probs, rows * 10).reshape(rows, 10).astype(np.float64)
+    kept = (labels >= 1) & (labels <= 10)
+    want = -np.log(p[kept, labels[kept] - 1]).sum() / rows
+    assert abs(loss.value - want) <= 4 * 2.0**-23 * want  # a logarithm's last place and one rounding of the mean
