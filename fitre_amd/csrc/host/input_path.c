@@ -184,7 +184,7 @@ static void generalization_sweep(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH
 			if (dropShortTail) break;
 		}
 	}
-	HIP_CALL(fitre_hip_totals_end(likelihood, &hits, nextPageLckPtr));
+	HIP_CALL(fitre_hip_totals_end(likelihood, &hits, before ? nextPageLckPtr : NULL));
 	*accuracy = hits * (real)100. / (real)setSize;
 	*likelihood /= (real)setSize;
 }
