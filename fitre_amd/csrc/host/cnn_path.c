@@ -487,14 +487,14 @@ void cnnBackward(CNN_MODEL *model, DEVICE_DATASET *data, real *devPtr, real *z, 
 			tail[f].db = (model->bias != 0) ? gradient + bOffsets[f + nc] : NULL;
 		}
 		const POOL_LAYER *pl = &model->poolLayer[nc - 1];
-		if (!has_bn(last) && pl->type == MAX_POOL && pl->pSize == 2 && pl->stride == 2 && pl->padding == 0 && pl->width == 2 * extA &&
+		if (!has_bn(last) && (pl->type == MAX_POOL || pl->type == AVG_POOL) && pl->pSize == 2 && pl->stride == 2 && pl->padding == 0 && pl->width == 2 * extA &&
 		    pl->height == 2 * extB && pl->outWidth == extA && pl->outHeight == extB) {
 			/* the top convolution layer's pool and activation steps ride on the launch that produces their delta */
 			const real *slabT = z + zOffsets[nc];
 			real *dslabT = dx + zOffsets[nc];
-			HIP_CALL(fitre_hip_fc_tail_backward_pool_act(model->lLayers, tail, n, delta, extA, extB, features, model->actFuns[nc - 1], slabT,
-			                                             slabT + last->activationOffset, dslabT, dslabT + last->activationOffset, sideWs,
-			                                             sideBytes));
+			HIP_CALL(fitre_hip_fc_tail_backward_pool_type_act(model->lLayers, tail, n, delta, extA, extB, features, pl->type, model->actFuns[nc - 1],
+			                                                  slabT, slabT + last->activationOffset, dslabT, dslabT + last->activationOffset,
+			                                                  sideWs, sideBytes));
 			tailFoldedPool = 1;
 		} else {
 			HIP_CALL(fitre_hip_fc_tail_backward(model->lLayers, tail, n, delta, extA, extB, features, sideWs, sideBytes));
@@ -615,14 +615,14 @@ void cnnBackward(CNN_MODEL *model, DEVICE_DATASET *data, real *devPtr, real *z, 
 			} else {
 				const CONV_LAYER *lb = &model->convLayer[c - 1];
 				const POOL_LAYER *pb = &model->poolLayer[c - 1];
-				if (pb->type == MAX_POOL && pb->pSize == 2 && pb->stride == 2 && pb->padding == 0 && pb->width == 2 * shape.inA &&
+				if ((pb->type == MAX_POOL || pb->type == AVG_POOL) && pb->pSize == 2 && pb->stride == 2 && pb->padding == 0 && pb->width == 2 * shape.inA &&
 				    pb->height == 2 * shape.inB && pb->outWidth == shape.inA && pb->outHeight == shape.inB &&
 				    fitre_hip_conv_input_grad_folds_pool(&shape)) {
 					const real *slabB = z + zOffsets[c];
 					real *dslabB = dx + zOffsets[c];
-					HIP_CALL(fitre_hip_conv_input_grad_pool_act(&shape, cur, weights + wOffsets[c], delta, model->actFuns[c - 1], slabB,
-					                                            slabB + lb->activationOffset, dslabB, dslabB + lb->activationOffset, ws,
-					                                            wsBytes));
+					HIP_CALL(fitre_hip_conv_input_grad_pool_type_act(&shape, cur, weights + wOffsets[c], delta, pb->type, model->actFuns[c - 1],
+					                                                 slabB, slabB + lb->activationOffset, dslabB,
+					                                                 dslabB + lb->activationOffset, ws, wsBytes));
 					poolFolded = 1;
 				} else {
 					HIP_CALL(fitre_hip_conv_input_grad(&shape, cur, weights + wOffsets[c], delta, ws, wsBytes));

@@ -419,6 +419,10 @@ int fitre_hip_conv_input_grad_folds_pool(const fitre_conv_shape *s);
 int fitre_hip_conv_input_grad_pool_act(const fitre_conv_shape *s, const float *delta, const float *w, float *dx, int actFun,
                                        const float *z_in, const float *z_act, float *dxPool, float *dxAct, void *ws,
                                        size_t wsBytes);
+/* ... behind a pool of that type, MAX_POOL or AVG_POOL */
+int fitre_hip_conv_input_grad_pool_type_act(const fitre_conv_shape *s, const float *delta, const float *w, float *dx, int poolType, int actFun,
+                                            const float *z_in, const float *z_act, float *dxPool, float *dxAct, void *ws,
+                                            size_t wsBytes);
 /* Sums of two products of one shape in one launch, for the R operator of the Hessian-vector product
  * (functions/cnn_hv_forward.cu, cnn_hv_backward.cu: every convolution there is a sum of two):
  *   forward_pair:      y  = conv(x1, w1) + conv(x2, w2) + bias
@@ -592,6 +596,10 @@ int fitre_hip_fc_tail_backward(int layers, const fitre_fc_tail_layer *l, int n, 
 int fitre_hip_fc_tail_backward_pool_act(int layers, const fitre_fc_tail_layer *l, int n, const float *delta, int extA,
                                         int extB, float *features, int actFun, const float *z_in, const float *z_act,
                                         float *dxPool, float *dxAct, void *ws, size_t wsBytes);
+/* ... behind a pool of that type, MAX_POOL or AVG_POOL */
+int fitre_hip_fc_tail_backward_pool_type_act(int layers, const fitre_fc_tail_layer *l, int n, const float *delta, int extA,
+                                             int extB, float *features, int poolType, int actFun, const float *z_in, const float *z_act,
+                                             float *dxPool, float *dxAct, void *ws, size_t wsBytes);
 
 /* ---- Kronecker factors of the KFAC curvature approximation --------------------------------------
  * Each factor is a dense symmetric matrix, written in full (row-major == column-major).  The

@@ -1,4 +1,4 @@
-"""Backward pass of small layers: input gradients whose waves share output channels, weight gradients made together."""
+"""Backward pass of small layers: input gradients whose waves share output channels or go on through a pool, weight gradients made together."""
 import ctypes as C
 
 import numpy as np
@@ -7,7 +7,7 @@ import torch
 import torch.nn.functional as F
 
 from fitre_amd import lib as L
-from fitre_amd.structs import CNN_ACT_NONE, fitre_conv_shape, fitre_fc_tail_layer
+from fitre_amd.structs import ACT_TANH, AVG_POOL, CNN_ACT_NONE, CNN_ACT_RELU, CNN_ACT_SWISH, MAX_POOL, fitre_conv_shape, fitre_fc_tail_layer
 
 pytestmark = pytest.mark.gpu
 hip = L.hip
@@ -75,3 +75,43 @@ def test_weight_gradients_together(dev, n):
 
     for alone, together in zip(run(False), run(True)):
         np.testing.assert_array_equal(together, alone)
+
+
+@pytest.mark.parametrize("pool", [MAX_POOL, AVG_POOL])
+@pytest.mark.parametrize("act", [CNN_ACT_NONE, CNN_ACT_RELU, CNN_ACT_SWISH, ACT_TANH])
+@pytest.mark.parametrize("n,ci,co,a,b,k", [(16, 6, 16, 14, 14, 5), (3, 5, 7, 6, 10, 3), (130, 2, 3, 5, 7, 3)])
+def test_through_a_pool(dev, n, ci, co, a, b, k, act, pool):
+    """An input gradient and a linear tail's delta taken on through the pool and activation below: the bits of the steps of their own."""
+    s = fitre_conv_shape(n, ci, co, a, b, a - k + 1, b - k + 1, k, 1, 0)
+    rng = np.random.default_rng(n + act)
+    up = lambda size: dev.upload(rng.standard_normal(size).astype(np.float32))
+    full = lambda size: dev.upload(np.full(size, 7, np.float32))
+    cells = ci * n * a * b
+    d, w, zi, za = up(co * n * s.outA * s.outB), up(co * ci * k * k), up(4 * cells), up(4 * cells)
+    nb = hip.fitre_hip_conv_input_grad_workspace(C.byref(s))
+    ws = dev.alloc(max(nb, 4))
+    got, want = [[full(cells), full(4 * cells), full(4 * cells)] for _ in range(2)]
+    ok(hip.fitre_hip_conv_input_grad_pool_type_act(C.byref(s), d, w, got[0], pool, act, zi, za, got[1], got[2], ws, nb))
+    ok(hip.fitre_hip_conv_input_grad(C.byref(s), d, w, want[0], ws, nb))
+    behind = lambda t: ok(hip.fitre_hip_pool_act_backward(pool, act, t[0], zi, za, ci, n, 2 * a, 2 * b, 2, 2, 0, a, b, t[1], t[2]))
+    behind(want)
+
+    dims, tops = [(ci * a * b, 30), (30, 4)], up(4 * n)
+    W, zin = [up(i * o) for i, o in dims], [up(n * i) for i, _ in dims]
+
+    def tail(call):
+        layers = (fitre_fc_tail_layer * 2)(*[fitre_fc_tail_layer(i, o, CNN_ACT_NONE, W[t].value, None, None, zin[t].value, full(n * o).value, full(i * o).value,
+                                                                 full(o).value) for t, (i, o) in enumerate(dims)])
+        size = hip.fitre_hip_fc_tail_workspace(2, layers, n)
+        ok(call(layers, dev.alloc(max(size, 4)), size))
+
+    if hip.fitre_hip_fc_tail_fits(2, (fitre_fc_tail_layer * 2)(*[fitre_fc_tail_layer(i, o, CNN_ACT_NONE) for i, o in dims]), n):
+        x, y = [[full(cells), full(4 * cells), full(4 * cells)] for _ in range(2)]
+        tail(lambda l, v, size: hip.fitre_hip_fc_tail_backward_pool_type_act(2, l, n, tops, a, b, x[0], pool, act, zi, za, x[1], x[2], v, size))
+        tail(lambda l, v, size: hip.fitre_hip_fc_tail_backward(2, l, n, tops, a, b, y[0], v, size))
+        behind(y)
+        got, want = got + x, want + y
+    for i, (u, v) in enumerate(zip(got, want)):
+        size = 4 * cells if i % 3 else cells
+        np.testing.assert_array_equal(dev.download(u, size), dev.download(v, size))
+    assert hip.fitre_hip_conv_input_grad_pool_type_act(C.byref(s), d, w, got[0], 77, act, zi, za, got[1], got[2], ws, nb) != 0
