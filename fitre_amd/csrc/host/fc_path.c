@@ -226,7 +226,9 @@ static HEAD_TERMS forward_pass(NN_MODEL *model, DEVICE_DATASET *data, real *weig
 
 	HEAD_TERMS terms_left = { NULL, 0, numColsTarget, model->type == MODEL_TYPE_MSE };
 	const int last = model->actFuns[numLayers - 1];
-	if ((last == ACT_LINEAR || last == ACT_LOGISTIC) && numCols == numColsTarget && fused_layers(model, numCols, numLayers, 0)) {
+	/* points of more features than the first layer reads lie further apart than the fused products take them */
+	if ((last == ACT_LINEAR || last == ACT_LOGISTIC) && numRows == layerSizes[0] && numCols == numColsTarget &&
+	    fused_layers(model, numCols, numLayers, 0)) {
 		for (int i = 0; i < numLayers; i++) {
 			const int out = layerSizes[i + 1];
 			fitre_dense_product p = dense(0, 0, out, numCols, layerSizes[i], weights + wOffsets[i], (i == 0) ? dataset : z + zOffsets[i],

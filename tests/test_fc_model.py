@@ -258,6 +258,23 @@ def test_gpu_gradient_against_oracle(dev, oracle64, name, n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("more", [0, 3])
+@pytest.mark.parametrize("name", ["autoencoder_logistic", "regression_linear", "classifier_softmax"])
+def test_gpu_evaluation_of_points_with_more_features_than_the_first_layer_reads(dev, oracle64, name, more):
+    """data->features is how far the points are apart; the first layer reads the first layerSizes[0] of them."""
+    n, rng = 23, np.random.default_rng(more)
+    m, w, x, y = make_data(name, n, rng)
+    w32, x32, y32 = w.astype(np.float32), x.astype(np.float32), y.astype(np.float32)
+    data, scratch, pw = device_setup(dev, m, w32, np.concatenate([x32, rng.standard_normal((n, more))], 1).astype(np.float32), y32, n)
+    data.features = m.layerSizes[0] + more
+    ll, merr = C.c_float(), C.c_float()
+    oll, omerr = oracle64.nn_forward(m, w32, x32.reshape(-1), y32.reshape(-1), n, n)[:2]
+    for kind in (TRAIN_DATA, TEST_DATA):
+        L.cnn.evaluateModel(C.byref(m), C.byref(data), C.byref(scratch), pw, C.byref(ll), C.byref(merr), FULL_DATASET, kind)
+        assert abs(ll.value - oll) < TOL * max(1, abs(oll)) and abs(merr.value - omerr) < TOL * max(1, abs(omerr))
+
+
+@pytest.mark.gpu
 def test_gpu_sampled_dataset_uses_the_input_as_target(dev, oracle64):
     name, n = "autoencoder_logistic", 64
     rng = np.random.default_rng(3)
