@@ -28,6 +28,7 @@ void conv_gemm_release()
 		if (g_ktables[i]) (void)hipFree(g_ktables[i]);
 		g_ktables[i] = nullptr, g_ktable_caps[i] = 0;
 	}
+	thin_held_forget();
 }
 
 // bn = tile extent along the positions, which fixes how the waves stride through a slice

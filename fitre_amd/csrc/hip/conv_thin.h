@@ -577,6 +577,14 @@ static bool g_thin_dw_deferred = false;
 static ThinDwBatch g_thin_dw = {};
 static size_t g_thin_dw_lds = 0;
 static double g_thin_dw_flops = 0.0;
+// work held back is of the device and the buffers it was queued for: a shutdown drops it, and with it the request to hold more
+static void thin_held_forget()
+{
+	g_thin_reduce_deferred = g_thin_dw_deferred = false;
+	g_thin_reduce.jobs = g_thin_dw.jobs = g_thin_dw.blocks = g_thin_dw.linear.count = 0;
+	g_thin_reduce_bytes = g_thin_dw_flops = 0.0;
+	g_thin_dw_lds = 0;
+}
 static int thin_dw_flush()
 {
 	ThinDwBatch &b = g_thin_dw;

@@ -115,3 +115,40 @@ def test_through_a_pool(dev, n, ci, co, a, b, k, act, pool):
         size = 4 * cells if i % 3 else cells
         np.testing.assert_array_equal(dev.download(u, size), dev.download(v, size))
     assert hip.fitre_hip_conv_input_grad_pool_type_act(C.byref(s), d, w, got[0], 77, act, zi, za, got[1], got[2], ws, nb) != 0
+
+
+def test_work_held_back_ends_with_the_device_layer(dev):
+    """Neither what was held back before a shutdown nor the request to hold more reaches the layer that is set up after it."""
+    n, ci, co = 13, 6, 16
+    s = fitre_conv_shape(n, ci, co, 14, 14, 10, 10, 5, 1, 0)
+    rng = np.random.default_rng(4)
+    x, d = (dev.upload(rng.standard_normal(size).astype(np.float32)) for size in (ci * n * 196, co * n * 100))
+    dims, size = [(65, 33), (33, 4)], co * ci * 25
+    W, zin = [dev.zeros(i * o) for i, o in dims], [dev.zeros(n * i) for i, _ in dims]
+    dW, db, nb = dev.zeros(size), dev.zeros(co), hip.fitre_hip_conv_weight_bias_grad_workspace(C.byref(s))
+    ws = dev.alloc(nb)
+    tail = (fitre_fc_tail_layer * 2)(*[fitre_fc_tail_layer(i, o, CNN_ACT_NONE, W[t].value, None, None, zin[t].value, dev.zeros(n * o).value,
+                                                           dev.zeros(i * o).value, dev.zeros(o).value) for t, (i, o) in enumerate(dims)])
+    tail_nb = hip.fitre_hip_fc_tail_workspace(2, tail, n)
+    grads = lambda: ok(hip.fitre_hip_conv_weight_bias_grad(C.byref(s), x, d, dW, db, ws, nb))
+
+    def made():  # weight gradients and reductions of partial sums; the linear products are in the first
+        out = []
+        for kernel_class in (0, 3, 4):
+            count, ms, work = C.c_long(), C.c_double(), C.c_double()
+            ok(hip.fitre_hip_profile_read(kernel_class, C.byref(count), C.byref(ms), C.byref(work)))
+            out.append(count.value)
+        return out
+
+    ok(hip.fitre_hip_weight_grads_defer())
+    ok(hip.fitre_hip_fc_tail_backward(2, tail, n, dev.zeros(4 * n), 0, 0, dev.zeros(n * 65), dev.alloc(max(tail_nb, 4)), tail_nb))
+    grads()
+    ok(hip.fitre_hip_shutdown())
+    ok(hip.fitre_hip_init(0))
+    ok(hip.fitre_hip_profile_enable(1))
+    ok(hip.fitre_hip_thin_reduce_flush())
+    assert made() == [0, 0, 0]
+    grads()
+    assert made() == [1, 0, 1]
+    ok(hip.fitre_hip_profile_enable(0))
+    assert dev.download(dW, size).any()
