@@ -194,8 +194,10 @@ long cnnForwardMemRequired(CNN_MODEL *model)
  * 5 to 8 us each, and their launches held up the pass behind them: VGG-11 at 256 images 1688 -> 1633 us, VGG-16 at 128 1999 -> 1899
  * with both passes' copies made so), and returns how many there are.  make == 0: they are there, and only found again.  The buffers are
  * laid out for the model's batch size; a layer of a shorter one that finds no room makes its own.  (The forward pass's on
- * lane 2, beside its first layer: no shorter, as both are bound by memory there, and AlexNet at 64 images 1 % longer.) */
-static int prepare_weights(const CNN_MODEL *model, const real *weights, int n, int inputGrad, char *at, const char *end, const void **prepared, int make)
+ * lane 2, beside its first layer: no shorter, as both are bound by memory there, and AlexNet at 64 images 1 % longer.)  lane != 0: on that
+ * lane, behind whatever the caller has queued on lane 0 (a weight update, say); nothing is ordered where there is no copy to make. */
+static int prepare_weights(const CNN_MODEL *model, const real *weights, int n, int inputGrad, char *at, const char *end, const void **prepared, int make,
+                           int lane)
 {
 	fitre_conv_shape shapes[MAX_LAYERS];
 	const real *w[MAX_LAYERS];
@@ -214,7 +216,14 @@ static int prepare_weights(const CNN_MODEL *model, const real *weights, int n, i
 		at += (bytes + 255) & ~(size_t)255;
 		if (at > end) at = (char *)end;
 	}
-	if (count && make) HIP_CALL(fitre_hip_conv_prepare_weights(count, shapes, w, to, inputGrad));
+	if (count && make) {
+		if (lane) {
+			HIP_CALL(fitre_hip_lane_wait(lane, 0));
+			HIP_CALL(fitre_hip_lane_select(lane));
+		}
+		HIP_CALL(fitre_hip_conv_prepare_weights(count, shapes, w, to, inputGrad));
+		if (lane) HIP_CALL(fitre_hip_lane_select(0));
+	}
 	return count;
 }
 
@@ -284,7 +293,7 @@ static void forward_pass(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *s
 
 	if (forward_in_one_launch(model, data, z, probs, errors, n, loss)) return;
 	const void *prepared[MAX_LAYERS] = { NULL };
-	prepare_weights(model, weights, n, 0, (char *)ws + wsBytes, (char *)ws + sizeof(real) * (size_t)cnnForwardMemRequired(model), prepared, !sameWeights);
+	prepare_weights(model, weights, n, 0, (char *)ws + wsBytes, (char *)ws + sizeof(real) * (size_t)cnnForwardMemRequired(model), prepared, !sameWeights, 0);
 	for (int l = 0; l < nc; l++) {
 		const CONV_LAYER *cv = &model->convLayer[l];
 		const POOL_LAYER *pl = &model->poolLayer[l];
@@ -451,12 +460,7 @@ void cnnBackward(CNN_MODEL *model, DEVICE_DATASET *data, real *devPtr, real *z, 
 
 	/* Weight copies of the layers whose input gradient reads one: they depend on the weights only, so lane 2 makes
 	 * them while the chain works through the linear layers. */
-	if (preparedWs < preparedEnd) {
-		LANE_WAIT(2, 0);
-		LANE_SELECT(2);
-		preparedPending = prepare_weights(model, weights, n, 1, preparedWs, preparedEnd, prepared, 1);
-		LANE_SELECT(0);
-	}
+	preparedPending = prepare_weights(model, weights, n, 1, preparedWs, preparedEnd, prepared, 1, lanes ? 2 : 0);
 
 	/* Linear layers, top down.  The delta of a layer (after its activation derivative) is written once, into the
 	 * layer's dx slot -- the snapshot the Hessian-vector product and the KFAC factors read -- and everything that
