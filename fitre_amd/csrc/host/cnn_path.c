@@ -59,9 +59,10 @@ static void feature_extent(const CNN_MODEL *model, int *extA, int *extB)
 	}
 }
 
+/* A sweep writes a batch's hits, a real an image, to the front of this (input_path.c) while the weight copies behind it are kept. */
 static size_t forward_ws_bytes(const CNN_MODEL *model, int batch)
 {
-	size_t need = 256;
+	size_t need = max_sz(256, sizeof(real) * (size_t)batch);
 	for (int i = 0; i < model->cLayers; i++) {
 		const CONV_LAYER *c = &model->convLayer[i];
 		fitre_conv_shape s = conv_shape(c, batch);

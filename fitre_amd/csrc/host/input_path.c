@@ -173,7 +173,7 @@ static void generalization_sweep(CNN_MODEL *model, DEVICE_DATASET *data, SCRATCH
 		augment_queued(model, data, curBatchSize, nextDevPtr, 0, data->datasetType);
 		fitre_forward_batch(model, data, scratch, z, probs, errors, curBatchSize, mode, before == curBatchSize);
 		before = curBatchSize;
-		/* the hits go where the forward pass had its partial sums */
+		/* the hits go where the forward pass had its partial sums, in front of the copies (forward_ws_bytes holds them) */
 		HIP_CALL(fitre_hip_accuracy_add(probs, hostSet != NULL ? data->sampledTrainY : (real *)(setY + curIdx), curBatchSize, data->numClasses,
 		                                nextDevPtr));
 		curIdx += curBatchSize;

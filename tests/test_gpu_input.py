@@ -192,3 +192,55 @@ def test_generalization_error_sweeps(dev, oracle64):
     for q in (setX, setY, sampledX, sampledY):
         dev.free(q)
     gm.release()
+
+
+def test_sweep_keeps_the_weight_copies_of_a_pass_between_its_batches(dev):
+    """Two full batches of VGG-11 and a short one: losses and hits of forward passes one by one, which make their own copies; the same
+    after the weights have changed."""
+    from fitre_amd.structs import MODEL_TEST_ACCURACY
+    from helpers import GpuModel, build_vgg11, conv_shape, he_weights
+    rng = np.random.default_rng(12)
+    batch, size, feats = 128, 300, 3072
+    model = build_vgg11(batch)
+    layers = [conv_shape(batch, c.inChannels, c.outChannels, c.height, c.width, c.kSize, c.stride, c.padding) for c in model.convLayer[:model.cLayers]]
+    assert sum(hip.fitre_hip_conv_forward_prepared_bytes(C.byref(s)) > 0 for s in layers) >= 5
+    gm = GpuModel(dev, model, he_weights(model, rng, 0.1).astype(np.float32), rng.standard_normal(batch * feats).astype(np.float32),
+                  rng.integers(1, 11, batch).astype(np.float32), batch)
+    data, images = gm.data, (rng.standard_normal((size, 8)) @ rng.standard_normal((8, feats)) * 20 + 128).clip(0, 255).round()
+    setX, setY = dev.upload(images.astype(np.float32).reshape(-1)), dev.upload(rng.integers(1, 11, size).astype(np.float32))
+    for _ in range(5):
+        gm.forward()  # running statistics
+    both, labels = dev.zeros(2 * batch * feats), dev.zeros(batch)
+    data.testSetX, data.testSetY, data.testSizeX, data.datasetType = setX.value, setY.value, size, CIFAR10
+    data.sampledTrainX, data.sampledTrainY = both.value, labels.value
+    pinned = (C.c_float * 4)()
+    gm.scratch.nextPageLckPtr = C.cast(pinned, C.c_void_p).value
+    args = C.byref(model), C.byref(data), C.byref(gm.scratch)
+
+    def one_by_one():
+        loss, hits = np.float32(0), np.float32(0)
+        for at_ in range(0, size, batch):
+            n = min(batch, size - at_)
+            ok(hip.fitre_hip_copy_d2d(both, at(setX, feats * at_), 4 * feats * n))
+            ok(hip.fitre_hip_copy_d2d(labels, at(setY, at_), 4 * n))
+            L.cnn.augmentData(args[0], args[1], at_, n, gm.scratch.nextDevPtr, None, 0, CIFAR10)
+            mean = L.cnn.cnnForward(*args, gm.z, gm.probs, gm.errors, at_, n, MODEL_TEST_ACCURACY)
+            L.cnn.computeAccuracy(gm.probs, labels, n, 10, gm.scratch.nextDevPtr, pinned)
+            loss, hits = np.float32(loss + np.float32(np.float32(mean) * np.float32(n))), np.float32(hits + np.float32(pinned[0]))
+        return loss / np.float32(size), hits * np.float32(100) / np.float32(size), gm.get("probs")
+
+    seen = []
+    for change in (1.0, 0.5):
+        ok(hip.fitre_hip_scal(model.pSize, change, gm.w))
+        like, acc = C.c_float(), C.c_float()
+        L.cnn.computeTestGeneralizationErrors(*args, gm.z, gm.probs, gm.errors, C.byref(like), C.byref(acc))
+        probs = gm.get("probs")
+        loss, hits, alone = one_by_one()
+        assert abs(like.value - loss) <= 4 * 2.0**-24 * loss  # a rounding of each batch's mean, which a kernel takes here and the host there
+        assert acc.value == hits and pinned[0] <= size % batch
+        np.testing.assert_array_equal(probs, alone)
+        seen.append(like.value)
+    assert abs(seen[0] - seen[1]) > 1e-3 * seen[0]
+    for q in (setX, setY, both, labels):
+        dev.free(q)
+    gm.release()

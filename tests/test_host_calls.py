@@ -72,3 +72,22 @@ L.cnn.cnnBackward(C.byref(m), C.byref(data), p(1), p(2), p(3), p(4), p(5), p(6),
     else:
         assert not copies and not any("2" in c[1:] for c in calls if c[0] in ("wait", "lane"))
         assert ["lane", "1"] in calls  # on two lanes
+
+
+def test_hits_of_a_sweep_stay_clear_of_the_weight_copies(noting):
+    """Two batches of 100 images and one of 50, the copies of the first kept for the second, with layers that need no workspace of their own."""
+    calls = noting("""
+m, data, scratch, p = build_vgg11(100), S.DEVICE_DATASET(), S.SCRATCH_AREA(), lambda i: C.c_void_p(i << 34)
+data.testSizeX, data.features, data.numClasses, data.datasetType = 250, 3072, 10, S.CIFAR10
+scratch.nextDevPtr, scratch.nextPageLckPtr = 1 << 34, 2 << 34
+loss, accuracy = C.c_float(), C.c_float()
+L.cnn.computeTestGeneralizationErrors(C.byref(m), C.byref(data), C.byref(scratch), p(3), p(4), p(5), C.byref(loss), C.byref(accuracy))
+print("room", 4 * L.cnn.cnnForwardMemRequired(C.byref(m)))
+""")
+    room = int(calls[-1][1])
+    assert [c[0] for c in calls if c[0] in ("copies", "hits")] == ["copies", "hits", "hits", "copies", "hits"]
+    copies = [int(w) for c in calls if c[0] == "copies" for w in c[2:]]
+    assert len(copies) == 14 and all(c[1] == "0" for c in calls if c[0] == "copies")
+    hits = [(int(c[1]), int(c[2])) for c in calls if c[0] == "hits"]
+    assert [rows for _, rows in hits] == [100, 100, 50]
+    assert all(at + 4 * rows <= min(copies) and at >= 1 << 34 for at, rows in hits) and max(copies) + 256 <= (1 << 34) + room
