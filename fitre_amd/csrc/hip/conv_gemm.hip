@@ -1295,14 +1295,14 @@ int fitre_hip_conv_prepare_weights(int count, const fitre_conv_shape *s, const f
 	FITRE_REQUIRE(count >= 0 && (count == 0 || (s && w && prepared)), "fitre_hip_conv_prepare_weights: null pointer");
 	SplitWeightsBatch split[2] = {}; // windows of 3, of 5
 	QuadBatch quad = {};
-	double splitBytes = 0.0, quadBytes = 0.0;
+	double splitBytes[2] = {}, quadBytes = 0.0;
 	int widest = 0;
 	auto flush = [&](int which) { // 0, 1: split weights, 2: dense forms
 		if (which < 2 && split[which].count) {
-			LaunchScope scope(FITRE_KC_PERMUTE, splitBytes);
+			LaunchScope scope(FITRE_KC_PERMUTE, splitBytes[which]);
 			if (inputGrad) launch_split_weights_batch<true>(which ? 5 : 3, split[which]);
 			else launch_split_weights_batch<false>(which ? 5 : 3, split[which]);
-			split[which].count = 0, splitBytes = 0.0;
+			split[which].count = 0, splitBytes[which] = 0.0;
 		} else if (which == 2 && quad.count) {
 			LaunchScope scope(FITRE_KC_PERMUTE, quadBytes);
 			quad_weff_batch_kernel<<<dim3((unsigned)((widest + 255) / 256), (unsigned)quad.first[quad.count]), 256, 0, stream()>>>(quad);
@@ -1330,7 +1330,7 @@ int fitre_hip_conv_prepare_weights(int count, const fitre_conv_shape *s, const f
 			const int m = b.count++, I = inputGrad ? s[i].inChannels : s[i].outChannels, cred = inputGrad ? s[i].outChannels : s[i].inChannels;
 			b.I[m] = I, b.cred[m] = cred, b.rowGroups[m] = split_row_groups(I), b.w[m] = w[i], b.wp[m] = (u32x4 *)prepared[i];
 			b.first[m + 1] = b.first[m] + b.rowGroups[m] * (cred / kSplitCB);
-			splitBytes += (double)bytes * 10.0 / 6.0;
+			splitBytes[which] += (double)bytes * 10.0 / 6.0;
 		}
 	}
 	for (int which = 0; which < 3; which++) flush(which);

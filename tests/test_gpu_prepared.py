@@ -49,6 +49,32 @@ def test_copies_of_several_layers(dev, grad):
     assert hip.fitre_hip_conv_prepare_weights(1, C.byref(bad), C.byref(C.c_void_p(w[0].value)), C.byref(C.c_void_p(one[0].value)), grad) != 0
 
 
+def test_accounted_bytes_of_several_layers_copies(dev):
+    """A launch's bytes are those of its own layers: both windows and, behind them, the dense form."""
+    shapes = [layer(*LAYERS[i]) for i in (0, 1, 4, 5)]
+    buf = lambda words: C.c_void_p(dev.zeros(words).value)
+    w = [buf(s.inChannels * s.outChannels * s.ksize ** 2) for s in shapes]
+    to = [buf(hip.fitre_hip_conv_forward_prepared_bytes(C.byref(s)) // 4 + 1) for s in shapes]
+
+    def accounted(which):
+        n = len(which)
+        ok(hip.fitre_hip_profile_enable(1))
+        ok(hip.fitre_hip_conv_prepare_weights(n, (fitre_conv_shape * n)(*[shapes[i] for i in which]), (C.c_void_p * n)(*[w[i].value for i in which]),
+                                              (C.c_void_p * n)(*[to[i].value for i in which]), 0))
+        count, kind, tile, ms, work = C.c_long(), C.c_int(), C.c_int(), C.c_double(), C.c_double()
+        ok(hip.fitre_hip_profile_launch_count(C.byref(count)))
+        out = []
+        for i in range(count.value):
+            ok(hip.fitre_hip_profile_read_launch(i, C.byref(kind), C.byref(tile), C.byref(ms), C.byref(work)))
+            out.append(work.value)
+        ok(hip.fitre_hip_profile_enable(0))
+        return out
+
+    (three,), (five,), (eight,), (dense,) = (accounted([i]) for i in range(4))
+    assert min(three, five, eight, dense) > 0
+    assert accounted([0, 1, 2, 3]) == [three + eight, five, dense]
+
+
 @pytest.mark.parametrize("geom", LAYERS)
 def test_forward_with_a_copy(dev, geom):
     """The same bits with the copy made beforehand as with the one made inside."""
