@@ -7,7 +7,7 @@
 // words of a bordered row (two 16-byte reads for a 5-wide window) feed up to 8 * 5 * COG multiply-adds whose other
 // operand, the weight, is uniform over the wave and comes through scalar loads.  The patch is also what a 2 x 2 pool needs:
 // two pooled cells, so the activation and the pool (and the linear layers' order of the last layer's output) come from
-// registers instead of three further launches.  Rows of LDS are as long as the border needs or a little longer, where that
+// registers instead of three further launches.  From nine output channels on the plan launches conv_thin_matrix.h.  Rows of LDS are as long as the border needs or a little longer, where that
 // spreads sixteen neighbouring lanes' 16-byte reads over the banks.
 // Measured, a whole forward and backward pass, before and after: LeNet with batch norm at batch 1024 488 -> 362 us, without at
 // batch 128 176 -> 149, with average pools at batch 16 175 -> 145.
@@ -181,7 +181,7 @@ struct ThinFwdPlan {
 };
 // false: not for this kernel.  Up to sixteen channels on either side (alexnet's 3 -> 96 and VGG's 3 -> 64 first layers are the
 // tile engine's).  Layer on the engine / here, 128 images: 24 -> 24 channels 33 / 35 us, 32 -> 32 36 / 60 (14 x 14 maps), so
-// sixteen in is where the engine's rows fill; with three in, 32 x 32 maps, 5 x 5 windows 3 -> 16 30 / 15, 3 -> 32 36 / 22,
+// sixteen in is where the engine's rows fill; with three in, 32 x 32 maps, 5 x 5 windows 3 -> 16 22 / 12, 3 -> 32 36 / 22,
 // 3 -> 64 41 / 35, so sixteen out is on the safe side.
 static inline bool thin_fwd_plan(const fitre_conv_shape *s, ThinFwdPlan &p)
 {
@@ -203,9 +203,10 @@ static inline bool thin_fwd_plan(const fitre_conv_shape *s, ThinFwdPlan &p)
 	p.chunks = (items + 63) / 64, p.chunk = (items + p.chunks - 1) / p.chunks;
 	// channels of a wave: one until every SIMD has two waves (a wave is a serial chain of cin * k^2 * 8 multiply-adds a
 	// channel), then two, and four where they divide the channels and every SIMD has sixteen, for half the LDS reads.  One /
-	// two / four, 5 x 5 windows: 16 -> 16 on 14 x 14 maps 23 / 28 / 44 us at 128 images, 76 / 57 / 69 at 1024, 342 / 324 / 319 at
-	// 8192; 6 -> 16 12.3 / 15.1 / 23.2 at 128, 24.7 / 22.2 / 25.2 at 1024, 102 / 99 / 98 at 8192; 3 -> 6 on 32 x 32, all a
-	// little better with one, 10.9 / 11.7 / 17.0 at 128, 30.1 / 31.3 / 34.5 at 1024.
+	// two / four, 5 x 5 windows: 8 -> 8 on 14 x 14 maps 15.2 / 18.5 / 25.4 us at 128 images, 30.2 / 26.2 / 37.4 at 2048, 83 / 78 / 98
+	// at 8192; on 32 x 32 44.3 / 41.7 / 37.7 at 512, 137 / 129 / 130 at 2048; 3 -> 6 on 32 x 32 9.0 / 9.2 / 12.1 at 128, 26.9 / 26.4 /
+	// 28.8 at 1024.  The line of four was drawn at sixteen channels (342 / 324 / 319 at 8192), which the matrix form takes now;
+	// at four and eight it is the better one in few places on either side of that line.
 	const int cus = device_compute_units();
 	const long waves1 = (long)p.groupsX * p.chunks * s->outChannels;
 	p.cog = waves1 <= 8L * cus ? 1 : 2;
@@ -218,8 +219,9 @@ static inline bool thin_fwd_plan(const fitre_conv_shape *s, ThinFwdPlan &p)
 	return true;
 }
 // Microseconds of such a launch while the chip has room: loads of eight words a thread to stage the images, then the taps of
-// a wave's channels one after the other.  Fitted to 2365 launches (windows of 3 and 5, 1 to 16 channels in, 4 to 16 out, maps
-// of 5 to 28, 1 to 1024 images): 0.5 us off on average, 2.1 at most.
+// a wave's channels one after the other.  Fitted to 2365 launches of the vector kernel (windows of 3 and 5, 1 to 16 channels in, 4
+// to 16 out, maps of 5 to 28, 1 to 1024 images): 0.5 us off on average, 2.1 at most.  The matrix form, which runs from nine channels out
+// on, takes less (16 -> 16 channels on 14 x 14 maps 21.6 / 14.0 us at 32 images, 29.0 / 15.0 at 256).
 static inline double thin_fwd_us(const fitre_conv_shape *s, const ThinFwdPlan &p)
 {
 	const int loads = p.imageFloats < kThinFwdSmallImage ? (p.images * p.imageFloats + 2047) / 2048 : p.images * ((p.imageFloats + 2047) / 2048);
@@ -229,11 +231,12 @@ static inline double thin_fwd_us(const fitre_conv_shape *s, const ThinFwdPlan &p
 }
 // Where the kernel is the shorter way.  Two chains compete at a small batch: its own, and the tile engine's, which a plan that is
 // cut over its reduction makes shorter (such an estimate holds within a fifth; an uncut plan takes 1.7 times its estimate).
-// 5 x 5 windows on 14 x 14 maps, engine / kernel: 6 -> 16 channels 19.7 / 11.1 us at 32 images, 20.0 / 11.6 at 256; 8 -> 10
-// 13.1 / 13.6 at 8, 22.7 / 13.8 at 32; 16 -> 16 14.4 / 21.6 at 32, 38.2 / 29.0 at 256.  Of 2520 such layers the choice is
-// wrong by more than 3 % for 29, by a quarter at most.  sparedUs: launches behind the engine's that the kernel's epilogue makes
-// unnecessary.  A workspace that does not hold the engine's ranges leaves it the long chain (16 -> 16 channels, 32 images: 14.4 us
-// cut, 38 uncut, 21.4 here).
+// 5 x 5 windows on 14 x 14 maps, engine / kernel: 6 -> 8 channels 18.5 / 10.7 us at 32 images, 18.8 / 11.5 at 256; 8 -> 8
+// 15.3 / 15.1 at 8, 13.6 / 15.1 at 32; 16 -> 8 13.9 / 21.4 at 32, 37.2 / 21.7 at 256.  Of 400 layers of four to eight channels out, as
+// above, the choice is wrong by more than 3 % for ten, by 9 % at most.  Of 400 of nine to sixteen, whose estimate is too long, none
+// comes here wrongly, but 65 stay on the engine that are shorter here (8 -> 10 at 8 images 13.8 / 8.6, 16 -> 16 at 32 14.3 / 14.0;
+// 2.7 times at most).  sparedUs: launches behind the engine's that the kernel's epilogue makes unnecessary.  A workspace that does not
+// hold the engine's ranges leaves it the long chain (16 -> 16 channels, 32 images: 14.3 us cut, 38 uncut, 14.0 here).
 constexpr double kThinFwdFoldUs = 3.0;
 static inline bool thin_fwd_chosen(const fitre_conv_shape *s, double sparedUs, const void *ws, size_t wsBytes, ThinFwdPlan &plan)
 {
@@ -265,9 +268,10 @@ static int launch_thin_forward(const fitre_conv_shape *s, const ThinFwdPlan &pla
 	p.store = (s->outB % 4 == 0 && (at & 15) == 0) ? 4 : ((s->outB % 2 == 0 && (at & 7) == 0) ? 2 : 1);
 	const dim3 grid((unsigned)plan.groupsX, (unsigned)plan.groupsY);
 	const size_t lds = sizeof(float) * (size_t)p.images * imageFloats;
-	LaunchScope scope(FITRE_KC_CONV_FWD, conv_flops(s), 0);
 	ThinMatPlan m;
-	if (s->outChannels >= kThinMatLeastRows && thin_mat_plan(s, fold != nullptr, m)) {
+	const bool matrix = s->outChannels >= kThinMatLeastRows && thin_mat_plan(s, fold != nullptr, m);
+	LaunchScope scope(FITRE_KC_CONV_FWD, conv_flops(s), matrix ? kTileThinMatrix : 0);
+	if (matrix) {
 		m.p.src = x, m.p.w = w, m.p.bias = bias, m.p.out = y, m.p.store = p.store;
 		if (fold) {
 			m.p.act = fold->act, m.p.average = fold->average, m.p.toFc = fold->toFc, m.p.actOut = fold->actOut, m.p.poolOut = fold->poolOut;

@@ -19,6 +19,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ v4f mfma_f32_16(float a, float b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 constexpr int kThinMatLeastRows = 9;
+constexpr int kTileThinMatrix = 12; // profile variant
 constexpr int kThinMatRows = 16, kThinMatPitch = 17; // rows of a product; words between two reduction indices of the weights in LDS
 constexpr int kThinMatWaves = 4, kThinMatThreads = 64 * kThinMatWaves;
 

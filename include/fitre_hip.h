@@ -113,8 +113,8 @@ int fitre_hip_profile_read(int kernelClass, long *launches, double *milliseconds
  * on 2x2 maps, 7 = the cell form on 4x4 maps, 8 = the cell form of the weight gradient on 8x8 maps (their work is
  * still counted as the nine-tap 2*M*K*Cout); 9 = the weight gradient of a wide linear layer at a batch of at most 64
  * (the whole reduction in registers); 10 = fp32 products as six bf16 matrix products, 11 = the
- * same in the cell form on 4x4 maps. */
-#define FITRE_TILE_VARIANTS 12
+ * same in the cell form on 4x4 maps; 12 = the forward convolution of nine to sixteen channels on the fp32 matrix pipes. */
+#define FITRE_TILE_VARIANTS 13
 int fitre_hip_profile_read_tile(int kernelClass, int tile, long *launches, double *milliseconds, double *work);
 /* The accounted launches one by one, in issue order since the last fitre_hip_profile_enable(1) (at most 65 536
  * are kept): class, tile variant, duration and algorithmic work of launch `index` < *count. */

@@ -255,7 +255,7 @@ def test_forward_on_two_by_two_maps_as_a_dense_product(dev, n, ci, co, bn, train
             np.testing.assert_array_equal(a, b)
 
 
-CONV_FWD, SPLITK_REDUCE, DENSE_2X2 = 2, 4, 6  # classes and the tile variant of include/fitre_hip.h
+CONV_FWD, SPLITK_REDUCE, DENSE_2X2, THIN_MATRIX = 2, 4, 6, 12  # classes and tile variants of include/fitre_hip.h
 
 
 def launches(kernel_class, tile=None):
@@ -397,7 +397,7 @@ def test_room_for_the_permutation_is_asked_for_where_it_is_used_and_before_anyth
     (1, 3, 6, 32, 32, 5, 0, 1), (64, 3, 5, 5, 5, 5, 0, 0),
     (64, 1, 4, 7, 7, 5, 0, 1), (257, 6, 16, 7, 7, 5, 0, 1), (33, 12, 9, 6, 7, 3, 1, 1), (1000, 1, 3, 4, 4, 3, 0, 1)])
 def test_few_channels_take_the_shorter_of_two_chains(dev, n, ci, co, a, b, k, pad, thin):
-    """Which kernel ran (the vector one has no tile), and its result."""
+    """Which kernel ran (the vector one has no tile, and from nine channels on it is the matrix form), and its result."""
     from fitre_amd.structs import fitre_conv_shape
     rng = np.random.default_rng(n + ci + co)
     x = rng.standard_normal((ci, n, a, b)).astype(np.float32)
@@ -408,7 +408,7 @@ def test_few_channels_take_the_shorter_of_two_chains(dev, n, ci, co, a, b, k, pa
     y, ws = dev.upload(np.full(count + 4, 7.0, np.float32)), dev.alloc(nb)
     ok(hip.fitre_hip_profile_enable(1))
     ok(hip.fitre_hip_conv_forward(C.byref(shape), dev.upload(x.reshape(-1)), dev.upload(w.reshape(-1)), None, y, ws, nb))
-    assert launches(CONV_FWD, 0) == thin and launches(CONV_FWD) == 1
+    assert launches(CONV_FWD, 0 if co < 9 else THIN_MATRIX) == thin and launches(CONV_FWD) == 1
     ok(hip.fitre_hip_profile_enable(0))
     got = dev.download(y, count + 4)
     np.testing.assert_array_equal(got[-4:], 7.0)
@@ -467,7 +467,7 @@ def test_dense_form_against_float64(dev, n, ci, co):
 
 
 # geometry of THIN, and the channels that a wave of the vector kernel takes: two with an odd number of them, four, in both windows
-VARIANTS = [((210, 2, 5, 36, 36, 5, 0), 2), ((210, 2, 7, 34, 34, 3, 0), 2), ((512, 1, 16, 36, 36, 5, 0), 4), ((512, 1, 16, 34, 34, 3, 0), 4),
+VARIANTS = [((210, 2, 5, 36, 36, 5, 0), 2), ((210, 2, 7, 34, 34, 3, 0), 2), ((1024, 1, 8, 36, 36, 5, 0), 4), ((1024, 1, 8, 34, 34, 3, 0), 4),
             ((1025, 1, 8, 34, 33, 3, 0), 4)]
 
 
@@ -482,6 +482,16 @@ def test_channel_groups_of_the_vector_kernel(dev, geom, channels, kind, to_fc):
     ok(hip.fitre_hip_profile_enable(1))
     test_thin_convolution_with_activation_and_pool(dev, geom, kind, to_fc, CNN_ACT_SWISH)
     assert launches(CONV_FWD, 0) == 2 and launches(CONV_FWD) == 2  # with and without a bias
+    ok(hip.fitre_hip_profile_enable(0))
+
+
+# nine and sixteen channels, bands of an image and several images a workgroup, both windows
+@pytest.mark.parametrize("kind,to_fc", [(MAX_POOL, 1), (NO_POOL, 0)])
+@pytest.mark.parametrize("geom", [(512, 1, 16, 36, 36, 5, 0), (512, 1, 16, 34, 34, 3, 0), (4, 3, 9, 28, 20, 5, 2), (1025, 12, 9, 6, 8, 3, 1), (2100, 6, 16, 14, 14, 5, 0)])
+def test_matrix_form_of_nine_to_sixteen_channels(dev, geom, kind, to_fc):
+    ok(hip.fitre_hip_profile_enable(1))
+    test_thin_convolution_with_activation_and_pool(dev, geom, kind, to_fc, CNN_ACT_SWISH)
+    assert launches(CONV_FWD, THIN_MATRIX) == 2 and launches(CONV_FWD) == 2  # with and without a bias
     ok(hip.fitre_hip_profile_enable(0))
 
 
@@ -506,7 +516,7 @@ def test_few_channels_on_unaligned_tensors_need_no_workspace(dev):
 
 
 def test_few_channels_without_room_for_the_engines_ranges(dev):
-    """The vector kernel, whose time needs no workspace, where the tile engine would have to run uncut."""
+    """The kernel of few channels, whose time needs no workspace, where the tile engine would have to run uncut."""
     from fitre_amd.structs import fitre_conv_shape
     shape = fitre_conv_shape(8, 16, 16, 14, 14, 10, 10, 5, 1, 0)
     nb = hip.fitre_hip_conv_forward_workspace(C.byref(shape))
@@ -514,5 +524,5 @@ def test_few_channels_without_room_for_the_engines_ranges(dev):
     for room, thin in ((nb, 0), (nb // 4, 1), (0, 1)):
         ok(hip.fitre_hip_profile_enable(1))
         ok(hip.fitre_hip_conv_forward(C.byref(shape), x, w, None, y, ws if room else None, room))
-        assert launches(CONV_FWD, 0) == thin and launches(CONV_FWD) == 1
+        assert launches(CONV_FWD, THIN_MATRIX) == thin and launches(CONV_FWD) == 1
         ok(hip.fitre_hip_profile_enable(0))
