@@ -211,6 +211,18 @@ def test_oracle_offsets_follow_the_reference_arithmetic(oracle64):
 
 
 # ------------------------------------------------------------------------------------------ GPU
+POINTS = [11, 300, 4096, 4097]  # up to 4096 each product and what follows it are one launch, above the general products run
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(CASES))
+def test_gpu_line_between_fused_and_general_products(dev, name):
+    sizes = CASES[name][0]
+    for n in POINTS:
+        for i, o in zip(sizes, sizes[1:]):
+            assert L.hip.fitre_hip_dense_product_fits(0, 1, o, i, n) == (n <= 4096) and L.hip.fitre_hip_dense_product_fits(0, 0, o, n, i)
+
+
 def device_setup(dev, m, w, x, y, n, sampled=False):
     data = DEVICE_DATASET()
     px, py, pw = dev.upload(x.reshape(-1)), dev.upload(y.reshape(-1)), dev.upload(w)
@@ -229,7 +241,7 @@ def device_setup(dev, m, w, x, y, n, sampled=False):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", list(CASES))
-@pytest.mark.parametrize("n", [11, 300])
+@pytest.mark.parametrize("n", POINTS)
 def test_gpu_gradient_against_oracle(dev, oracle64, name, n):
     rng = np.random.default_rng(sum(map(ord, name)) + n)
     m, w, x, y = make_data(name, n, rng)
@@ -308,7 +320,7 @@ def test_gpu_apply_layer_activation_keeps_the_pre_activation_copy(dev, oracle64)
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", HV_CASES)
-@pytest.mark.parametrize("n", [11, 300])
+@pytest.mark.parametrize("n", POINTS)
 def test_gpu_hessian_vector_products_against_oracle(dev, oracle64, name, n):
     """hessianVec and gaussNewtonHessianVec after computeGradient at the same point, result at the head of the arena."""
     rng = np.random.default_rng(sum(map(ord, name)) + 7 * n)

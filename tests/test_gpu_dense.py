@@ -14,8 +14,10 @@ hip = L.hip
 TOL = 2e-6  # of the largest result, which bounds the activations and derivatives behind it too
 
 # (M, N, K): around the tile of 64 rows x 32 (or 64) columns, the step of 16 and the eight waves of a workgroup; a grid past
-# the compute units, whose tiles are twice as wide; rows that are no whole 16-byte groups
-SHAPES = [(1, 1, 1), (63, 31, 15), (64, 32, 16), (65, 33, 17), (66, 64, 127), (64, 65, 128), (130, 100, 129), (33, 17, 784), (784, 1000, 40), (1001, 999, 33)]
+# the compute units, whose tiles are twice as wide; rows that are no whole 16-byte groups; the longest reduction the family brings, twice that
+# with a second pair
+SHAPES = [(1, 1, 1), (63, 31, 15), (64, 32, 16), (65, 33, 17), (66, 64, 127), (64, 65, 128), (130, 100, 129), (33, 17, 784), (784, 1000, 40), (1001, 999, 33), (70, 40, 4095),
+          (65, 33, 4096)]
 
 
 def ok(rc):
