@@ -191,12 +191,14 @@ long cnnForwardMemRequired(CNN_MODEL *model)
 	return (long)((need + sizeof(real) - 1) / sizeof(real));
 }
 
-/* Queues the copies of every layer that has one on the selected lane, two launches whatever the number of layers (one by one they were
- * 5 to 8 us each, and their launches held up the pass behind them: VGG-11 at 256 images 1688 -> 1633 us, VGG-16 at 128 1999 -> 1899
- * with both passes' copies made so), and returns how many there are.  make == 0: they are there, and only found again.  The buffers are
- * laid out for the model's batch size; a layer of a shorter one that finds no room makes its own.  (The forward pass's on
- * lane 2, beside its first layer: no shorter, as both are bound by memory there, and AlexNet at 64 images 1 % longer.)  lane != 0: on that
- * lane, behind whatever the caller has queued on lane 0 (a weight update, say); nothing is ordered where there is no copy to make. */
+/* Queues the copies of every layer that has one and returns how many there are: a launch for each kind of copy (windows of 3 and of 5,
+ * sixteen layers to a launch; the dense form of 2 x 2 maps, eight).  One by one they were 5 to 8 us each, and their launches held up the
+ * pass behind them.  Forward pass with its copies together / each in front of its layer, us: VGG-11 593 / 605 at 256 images, 322 /
+ * 344 at 77, VGG-16 707 / 741 at 128, AlexNet, which has four, 969 / 974 at 64 and 338 / 346 at 8.  make == 0: they are there, and
+ * only found again.  The buffers are laid out for the model's batch size; a layer of a shorter one that finds no room makes its own.
+ * lane != 0: on that lane, behind whatever the caller has queued on lane 0 (a weight update, say); nothing is ordered where there is
+ * no copy to make.  (The forward pass's on lane 2, beside its first layer, were no shorter, as both are bound by memory there, and
+ * AlexNet at 64 images 1 % longer.) */
 static int prepare_weights(const CNN_MODEL *model, const real *weights, int n, int inputGrad, char *at, const char *end, const void **prepared, int make,
                            int lane)
 {

@@ -554,8 +554,8 @@ int fitre_hip_fc_tail_forward(int layers, const fitre_fc_forward_layer *l, int n
 /* The forward pass of a whole small network in one launch (functions/cnn_forward.cu:49-383): one to three convolutions (windows of 3
  * or 5, stride 1, at most sixteen channels, even maps) with an activation and a 2 x 2 / stride 2 pool behind each, none to four
  * linear layers as in fitre_hip_fc_tail_forward, softmax, loss errors (may be NULL) and the mean loss, which is waited for (lossHost NULL:
- * added to the totals below).  The tensors are those the steps of their own leave; the last pool's output is in the linear layers' order.  _fits: the network
- * is one of these, and this way is the shorter one. */
+ * added to the totals of fitre_hip_totals_begin).  The tensors are those the steps of their own leave; the last pool's output is in
+ * the linear layers' order.  _fits: the network is one of these, and this way is the shorter one. */
 typedef struct fitre_thin_net_layer {
 	fitre_conv_shape shape;
 	int act, average; /* average != 0: average pool, else max pool */
