@@ -326,7 +326,8 @@ void computeGradient(NN_MODEL *model, DEVICE_DATASET *data, SCRATCH_AREA *scratc
 	const int *rZOffsets = (isGradient == SAMPLED_DATASET) ? model->sRZOffsets : model->rZOffsets;
 	const int *bOffsets = model->bOffsets, *wOffsets = model->wOffsets;
 
-	const int fused = fused_layers(model, n, numLayers - 1, 1);
+	/* (a data set of other than one target a point has its error term where it has room, in scratch) */
+	const int fused = (isGradient == SAMPLED_DATASET || data->trainSizeX == data->trainSizeY) && fused_layers(model, n, numLayers - 1, 1);
 	real *const topError = fused ? dx + rZOffsets[numLayers - 1] : errorTerm; /* the fused sweep works in the dx slots */
 	const HEAD_TERMS head = forward_pass(model, data, weights, z, topError, logLikelihood, modelError, nextDevPtr, isGradient, TRAIN_DATA);
 	if (fused) {

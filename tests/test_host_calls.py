@@ -25,6 +25,13 @@ int fitre_hip_conv_prepare_weights(int count, const void *s, const void *const *
 	NOTE("\n");
 	return 0;
 }
+int fitre_hip_dense_product_fits(int ta, int tb, int m, int n, int k) { (void)ta, (void)tb, (void)m, (void)n, (void)k; return 1; }
+int fitre_hip_output_terms(int term, const void *target, const void *out, long n, float scale, void *to)
+{
+	(void)target, (void)out, (void)scale;
+	NOTE("terms %d %ld %zu\n", term, n, (size_t)to);
+	return 0;
+}
 int fitre_hip_accuracy_add(const void *p, const void *t, int rows, int classes, void *hits)
 {
 	(void)p, (void)t, (void)classes;
@@ -91,3 +98,23 @@ print("room", 4 * L.cnn.cnnForwardMemRequired(C.byref(m)))
     hits = [(int(c[1]), int(c[2])) for c in calls if c[0] == "hits"]
     assert [rows for _, rows in hits] == [100, 100, 50]
     assert all(at + 4 * rows <= min(copies) and at >= 1 << 34 for at, rows in hits) and max(copies) + 256 <= (1 << 34) + room
+
+
+@pytest.mark.parametrize("targets", [9, 10, 11])
+def test_error_term_of_other_than_one_target_a_point(noting, targets):
+    """It is as long as the targets are; the dx slot of the last layer, where the fused sweep has it, as the points are."""
+    calls = noting("""
+import sys
+m, data, scratch, p = S.NN_MODEL(), S.DEVICE_DATASET(), S.SCRATCH_AREA(), lambda i: C.c_void_p(i << 34)
+L.cnn.fitre_build_nn(C.byref(m), (C.c_int * 3)(6, 5, 4), (C.c_int * 2)(S.ACT_TANH, S.ACT_SOFTMAX), 2, S.MODEL_TYPE_CLASSIFICATION, 10)
+L.cnn.initRZOffsets(C.byref(m), 10)
+data.features, data.trainSizeX, data.trainSizeY = 6, 10, %d
+scratch.nextDevPtr = 1 << 34
+loss, error = C.c_float(), C.c_float()
+L.cnn.computeGradient(C.byref(m), C.byref(data), C.byref(scratch), p(2), p(3), p(4), p(5), C.byref(loss), C.byref(error), S.FULL_DATASET)
+print("slot", (4 << 34) + 4 * m.rZOffsets[1], 4 * (m.rFullSize - m.rZOffsets[1]))
+""" % targets)
+    slot, size = map(int, calls[-1][1:])
+    error = [c for c in calls if c[0] == "terms"][-1]  # behind the terms of the loss
+    assert int(error[2]) == 4 * targets and size == 160
+    assert int(error[3]) == (slot if targets == 10 else 1 << 34)
